@@ -271,3 +271,112 @@ def tolerance(case):
     if case["kind"] == "experts":
         return {"rel": 1e-4, "max": 6e-3} if case["math"] == "bf16" else {"rel": 1e-3, "max": 1e-1}
     return {"rel": 2e-4, "max": 8e-3} if case["y"] == "bf16" else {"rel": 5e-7, "max": 4e-6}
+
+
+# ---- the same outputs in 64 bits, without the library ---------------------------------------------------------------
+
+
+def _e2m1(v):
+    """The nearest e2m1 value (ties to the even code), saturating at 6."""
+    grid = torch.tensor([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0], device=v.device)
+    low, high = torch.tensor([0.25, 1.25, 2.5, 5.0], device=v.device), torch.tensor([0.75, 1.75, 3.5], device=v.device)
+    a = v.abs()
+    code = sum((a > t).int() for t in low) + sum((a >= t).int() for t in high)
+    return torch.copysign(grid[code.long()], v)
+
+
+def _e4m3(v):
+    return v.clamp(-448.0, 448.0).to(torch.float8_e4m3fn).float()
+
+
+def _divided(a, b):
+    """a / b in f32 as IEEE rounds it (a double holds the quotient closely enough for one rounding)."""
+    return (a.double() / b.double()).float()
+
+
+def _weight_values(master, fmt, top=None):
+    """What the stored rows stand for, before the row factor (f32, exact), and the row factor [rows, 1] (f64). `top` is
+    the largest magnitude of the whole matrix or stack that the rows are part of (NVFP4 has one global factor)."""
+    w = master.float()
+    if fmt == "bf16":
+        return w, torch.ones(w.shape[0], 1, device=w.device, dtype=torch.float64)
+    if fmt == "nvfp4":
+        scale = _divided(w.abs().max() if top is None else top, torch.tensor(2688.0, device=w.device))
+        blocks = w.view(w.shape[0], -1, 16)
+        s = _e4m3(_divided(blocks.abs().amax(2), 6.0 * scale))
+        step = (s * scale).unsqueeze(2)
+        codes = torch.where(step > 0, _e2m1(_divided(blocks, step)), torch.zeros_like(blocks))
+        return (codes * s.unsqueeze(2)).view_as(w), scale.double().expand(w.shape[0], 1)
+    s = _divided(w.abs().amax(1, keepdim=True), torch.tensor(127.0 if fmt == "int8" else 448.0, device=w.device))
+    v = _divided(w, s)
+    return (v.round().clamp(-127.0, 127.0) if fmt == "int8" else _e4m3(v)), s.double()
+
+
+def _activation_values(x, math_name):
+    """The same of bf16 activation rows under a math: quantised per row, by a reciprocal (f32)."""
+    x = x.float()
+    if math_name == "bf16":
+        return x, torch.ones(x.shape[0], 1, device=x.device, dtype=torch.float64)
+    a = x.abs().amax(1, keepdim=True)
+    if math_name == "fp4":
+        g = _divided(a, torch.full_like(a, 2688.0))
+        blocks = x.view(x.shape[0], -1, 16)
+        s = _e4m3(_divided(blocks.abs().amax(2), 6.0 * g))
+        step = (s * g).unsqueeze(2)
+        codes = torch.where(step > 0, _e2m1(blocks * _divided(torch.ones_like(step), step)), torch.zeros_like(blocks))
+        return (codes * s.unsqueeze(2)).view_as(x), g.double()
+    top = torch.full_like(a, 127.0 if math_name == "int8" else 448.0)
+    v = x * _divided(top, a)
+    return (v.round().clamp(-127.0, 127.0) if math_name == "int8" else _e4m3(v)), _divided(a, top).double()
+
+
+def _product(x, master, fmt, math_name, top=None):
+    values, factor = _weight_values(master, fmt, top)
+    rows, scale = _activation_values(x, math_name)
+    return (rows.double() @ values.double().t().contiguous()) * scale * factor.t()
+
+
+def _routing(logits, top_k):
+    """Ids (in the order of the scores), weights, entropy and confidence of every token."""
+    logits = logits.double()
+    picked, ids = logits.topk(top_k, dim=1)
+    p = torch.softmax(logits, 1)
+    return ids, torch.softmax(picked, 1), -(p * p.clamp_min(1e-9).log()).sum(1), p.amax(1)
+
+
+def exact(case, seed):
+    """What run() returns, computed in 64 bits from the same inputs (ids, which are whole numbers, have None). The
+    quantised values themselves are the formats' own and taken as given, and so are the experts' bf16 intermediate rows."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+
+    def normal(*shape, dtype=torch.float32):
+        return torch.randn(*shape, generator=g, device="cuda", dtype=dtype)
+
+    outputs, fmt, math_name = [], case["format"], case["math"]
+    for _ in range(case["layers"]):
+        if case["kind"] == "linear":
+            master = normal(case["n"], case["k"], dtype=torch.bfloat16).mul_(0.02)
+            outputs.append(_product(normal(case["rows"], case["k"], dtype=torch.bfloat16), master, fmt, math_name))
+            continue
+        t, e, top_k, latent, inter = (case[key] for key in ("tokens", "experts", "top_k", "latent", "inter"))
+        gate_up = normal(e * 2 * inter, latent, dtype=torch.bfloat16).mul_(0.02)
+        down = normal(e * latent, inter, dtype=torch.bfloat16).mul_(0.02)
+        x = normal(t, latent, dtype=torch.bfloat16)
+        if t <= 8 and latent <= 2048:
+            logits = x.double() @ normal(e, latent).mul_(latent**-0.5).double().t().contiguous()
+        else:
+            logits = normal(t, e)
+        ids, weights, entropy, confidence = _routing(logits, top_k)
+        out = torch.zeros(t, latent, dtype=torch.float64, device="cuda")
+        tops = [m.float().abs().max() if fmt == "nvfp4" else None for m in (gate_up, down)]
+        for expert in range(e):
+            token, slot = (ids == expert).nonzero(as_tuple=True)
+            if not len(token):
+                continue
+            first = _product(x[token], gate_up[expert * 2 * inter:(expert + 1) * 2 * inter], fmt, math_name, tops[0])
+            gate, up = first[:, :inter], first[:, inter:]
+            middle = (gate / (1.0 + torch.exp(-gate)) * up).to(torch.bfloat16)
+            last = _product(middle, down[expert * latent:(expert + 1) * latent], fmt, math_name, tops[1])
+            out.index_add_(0, token, last * weights[token, slot].unsqueeze(1))
+        outputs += [None, weights, entropy, confidence, out]
+    return outputs
