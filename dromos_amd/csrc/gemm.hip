@@ -1410,6 +1410,35 @@ int launch_skinny(GemmArgs a, hipStream_t stream) {
                               : launch_skinny_x<F, MT, false, false>(a, lds, n_tiles, S * kWave, stream);
 }
 
+// More rows than a decode step has: the block kernel (gemm_block.h), which takes all of them in one launch, each weight read
+// and decoded once per 64 or 128 rows: with the passes of 64 rows below, 14336 x 4096 fp8 at 128 / 256 / 1024 / 4096 rows took
+// 42 / 84 / 334 / 1450 us. Where the product has too few blocks for the device, one slice of K a workgroup, the slices
+// added by the slab kernel's second half (the stream's partial-tile buffer permitting).
+template <int F, int MATH>
+bool launch_block(GemmArgs a, int* status, hipStream_t stream) {
+  auto launch = [&] {
+    if constexpr (MATH == LX_MATH_INT8) return launch_block_int8_math(a, status, stream);
+    else if constexpr (MATH == LX_MATH_FP8) return launch_block_fp8_math(a, status, stream);
+    else if constexpr (F == LX_W_BF16) return launch_block_bf16(a, status, stream);
+    else if constexpr (F == LX_W_INT8) return launch_block_int8(a, status, stream);
+    else if constexpr (F == LX_W_FP8) return launch_block_fp8(a, status, stream);
+    else return launch_block_nvfp4(a, status, stream);
+  };
+  const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave, mts = (a.M + 15) / 16;
+  const int64_t vectors = static_cast<int64_t>((a.N + kTileRows - 1) / kTileRows) * mts * kWave;  // of one slice
+  if (slices > 1 && (a.partial = slab_scratch(stream, static_cast<size_t>(slices * vectors * 16)))) {
+    if (launch()) {
+      if (*status) return true;
+      a.S = slices;
+      hipLaunchKernelGGL((slab_reduce_kernel<F, MATH>), dim3(static_cast<unsigned>((vectors + 255) / 256)), dim3(256), 0, stream, a, mts);
+      *status = status_of(hipGetLastError());
+      return true;
+    }
+    a.partial = nullptr;
+  }
+  return launch();
+}
+
 template <int F>
 int launch_format(GemmArgs a, const char* x0, char* y0, int M, int x_esize, int y_esize, hipStream_t stream) {
   const int64_t rb = row_bytes<F>(a.K);
@@ -1430,6 +1459,13 @@ int launch_format(GemmArgs a, const char* x0, char* y0, int M, int x_esize, int 
   // Slices are whole weight batches (the row's last one may be cut short by the row's end).
   a.steps_per_wave = ((a.steps + S - 1) / S + kLoadsInFlight - 1) / kLoadsInFlight * kLoadsInFlight;
   a.S = S;
+  if (M > 64 && a.xs.dtype == LX_BF16) {
+    a.M = M;
+    a.xs.x = x0;
+    a.y = y0;
+    int st = kOk;
+    if (launch_block<F, LX_MATH_BF16>(a, &st, stream)) return st;
+  }
   const float* const act_scale0 = a.act_scale;
   // Up to 64 activation rows a pass; every pass is the same arithmetic per row.
   for (int m0 = 0; m0 < M; m0 += 64) {
@@ -1562,7 +1598,15 @@ int gemm_bytes_math(const void* x, int x_dtype, int64_t ld_x, const lx_weight& w
     a.S = S;
     a.steps_per_wave = ((a.steps + S - 1) / S + kLoadsInFlight - 1) / kLoadsInFlight * kLoadsInFlight;
     const unsigned n_tiles = static_cast<unsigned>((N + kTileRows - 1) / kTileRows);
-    for (int m0 = 0; m0 < M && !st; m0 += 64) {
+    bool done = false;
+    if (M > 64) {
+      a.M = M;
+      a.xq = q;
+      a.xscale = scales;
+      a.y = y;
+      done = launch_block<F, MATH>(a, &st, s);
+    }
+    for (int m0 = done ? M : 0; m0 < M && !st; m0 += 64) {
       a.M = M - m0 < 64 ? M - m0 : 64;
       a.xq = q + static_cast<int64_t>(m0) * K;
       a.xscale = scales + m0;

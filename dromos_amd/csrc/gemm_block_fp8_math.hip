@@ -1,0 +1,6 @@
+// The block kernel under the FP8 math.
+#include "gemm_block.h"
+
+namespace dro {
+bool launch_block_fp8_math(const GemmArgs& a, int* status, hipStream_t stream) { return block::launch_format<LX_W_FP8, LX_MATH_FP8>(a, status, stream); }
+}  // namespace dro

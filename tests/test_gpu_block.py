@@ -1,0 +1,63 @@
+"""GPU: the block kernels (more rows than a decode step has) against the kernels for up to 64 rows, bit for bit: the same
+rows in calls of 64 at most. Row counts, output counts and row lengths around the edges of blocks, K tiles, slices and
+load steps; every format and math; the epilogue's operands; a stream with and without the partial-tile buffer."""
+
+import ctypes
+
+import pytest
+import torch
+
+import checks
+import ops
+from dromos_amd.abi import BF16, DTYPE, F32, FORMATS, MATH_BF16, MATH_FP4, MATH_FP8, MATH_INT8
+from dromos_amd.formats import random_weight
+
+pytestmark = pytest.mark.gpu
+MATHS = [("bf16", MATH_BF16), ("int8", MATH_BF16), ("fp8", MATH_BF16), ("nvfp4", MATH_BF16), ("int8", MATH_INT8), ("fp8", MATH_FP8),
+         ("nvfp4", MATH_FP8), ("nvfp4", MATH_FP4)]
+
+
+def chunks_of_64(hip, x, w, math, y, **kw):
+    return torch.cat([ops.gemm_w(hip, x[m : m + 64].contiguous(), w, math, y=y[m : m + 64].clone(), **kw) for m in range(0, x.shape[0], 64)])
+
+
+# Few blocks (a slice a workgroup), one block past a multiple of 64 / 128 rows and columns, an odd N, many blocks of each shape;
+# K of one slice, of slices whose last is short, of a last step and a last K tile cut short.
+@pytest.mark.parametrize("fmt,math", MATHS)
+@pytest.mark.parametrize("M,N,K", [(65, 300, 4096), (129, 257, 1056), (128, 1000, 544), (191, 2064, 8224), (515, 4096, 1056), (1030, 3001, 2080),
+                                   (2050, 4112, 1024), (66, 30000, 544)])
+def test_rows_are_those_of_calls_of_64(hip, fmt, math, M, N, K):
+    g = torch.Generator().manual_seed(M + N + K)
+    w = random_weight(FORMATS[fmt], N, K, N + K).to("cuda")
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    y = torch.full((M, N), float("nan"), device="cuda")
+    assert torch.equal(ops.gemm_w(hip, x, w, math, y=y.clone()), chunks_of_64(hip, x, w, math, y))
+
+
+@pytest.mark.parametrize("fmt,math", [("fp8", MATH_BF16), ("nvfp4", MATH_FP4), ("int8", MATH_INT8)])
+@pytest.mark.parametrize("y_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("bias,alpha,beta", [(None, 0.5, 0.0), (torch.float32, 1.0, 0.0), (torch.bfloat16, 1.5, 0.25)])
+@pytest.mark.parametrize("M,N,K", [(70, 132, 4096), (300, 1001, 1056)])
+def test_epilogue_operands(hip, fmt, math, y_dtype, bias, alpha, beta, M, N, K):
+    g = torch.Generator().manual_seed(N)
+    w = random_weight(FORMATS[fmt], N, K, N).to("cuda")
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    y = torch.randn(M, N, generator=g).to(y_dtype).cuda()
+    kw = dict(bias=None if bias is None else torch.randn(N, generator=g).to(bias).cuda(), alpha=alpha, beta=beta)
+    assert torch.equal(ops.gemm_w(hip, x, w, math, y=y.clone(), **kw), chunks_of_64(hip, x, w, math, y, **kw))
+
+
+@pytest.mark.parametrize("fmt", checks.FMT_NAMES)
+def test_strides_and_a_stream_without_the_partial_buffer(hip, fmt):
+    M, N, K, pad = 130, 264, 4096, 8
+    w = random_weight(FORMATS[fmt], N, K, 5).to("cuda")
+    x = torch.randn(M, K + pad, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16).cuda()
+    want = ops.gemm_w(hip, x[:, :K].contiguous(), w, MATH_BF16)
+    struct, stream = w.lx(), torch.cuda.Stream()
+    for y_dtype, ld_y in ((torch.float32, N + 1), (torch.bfloat16, N + 4)):
+        y = torch.full((M, ld_y), -3.0, dtype=y_dtype, device="cuda")
+        torch.cuda.synchronize()
+        assert hip.status("gemm_w", x, BF16, K + pad, ctypes.pointer(struct), MATH_BF16, None, F32, y, DTYPE[y_dtype], ld_y, M, N, K, 1.0, 0.0,
+                          None, stream.cuda_stream) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(y[:, :N], want.to(y_dtype)) and bool((y[:, N:] == -3.0).all())
