@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "moe_block.h"
 #include "moe_common.h"
 #include "tile_mfma.h"
 
@@ -49,7 +50,7 @@ struct Tables {
   int* n_tiles;      // [1]
 };
 
-int max_tiles(int P, int E) { return (P < E ? P : E) + P / kTileTokens + 1; }
+int max_tiles(int P, int E, int height = kTileTokens) { return (P < E ? P : E) + P / height + 1; }
 
 struct Layout {
   int64_t tables, inter, contrib, total;
@@ -111,7 +112,7 @@ __device__ __forceinline__ int block_scan(int v, int* buf) {
   return x + base;
 }
 
-__global__ void __launch_bounds__(kMaxExperts) group_kernel(const int32_t* __restrict__ ids, int P, int E, Tables t) {
+__global__ void __launch_bounds__(kMaxExperts) group_kernel(const int32_t* __restrict__ ids, int P, int E, int height, Tables t) {
   __shared__ int count[kMaxExperts], cursor[kMaxExperts], buf[kMaxExperts];
   const int e = threadIdx.x;
   count[e] = 0;
@@ -127,12 +128,12 @@ __global__ void __launch_bounds__(kMaxExperts) group_kernel(const int32_t* __res
   if (e == E - 1) t.offsets[E] = begin + mine;
   cursor[e] = begin;
   __syncthreads();
-  const int my_tiles = e < E ? (mine + kTileTokens - 1) / kTileTokens : 0;
+  const int my_tiles = e < E ? (mine + height - 1) / height : 0;
   const int tile0 = block_scan(my_tiles, buf) - my_tiles;
   for (int j = 0; j < my_tiles; ++j) {
     t.tile_expert[tile0 + j] = e;
-    t.tile_begin[tile0 + j] = begin + j * kTileTokens;
-    t.tile_rows[tile0 + j] = min(kTileTokens, mine - j * kTileTokens);
+    t.tile_begin[tile0 + j] = begin + j * height;
+    t.tile_rows[tile0 + j] = min(height, mine - j * height);
   }
   if (e == kMaxExperts - 1) *t.n_tiles = tile0 + my_tiles;
   for (int p = e; p < P; p += kMaxExperts) {
@@ -309,6 +310,49 @@ int launch_stage(Kernel kernel, GroupedArgs a, int64_t K, int NT, int out_rows, 
   return status_of(hipGetLastError());
 }
 
+// How a stage of rows of K values is cut for the block kernels: the same slices launch_stage walks.
+struct BlockCut {
+  bool fits;
+  int tiles, slice;
+};
+
+template <int F>
+BlockCut block_cut(int64_t K, int NT, int64_t out_rows) {
+  constexpr int kSteps = F == LX_W_BF16 ? 2 : 1, kTilesPerStep = F == LX_W_NVFP4 ? 2 : 1;
+  const int steps = load_steps_for<F>(K);
+  int S = split_for<F>(K, NT);
+  if (S > kGroupedSplit) S = kGroupedSplit;
+  const int per = (steps + S - 1) / S;
+  // 32-bit offsets inside a block (gate/up: from a gate row to the up rows).
+  return {(out_rows + 256) * row_bytes<F>(K) < (1ll << 31) && K * 2 * kBlockTokens < (1ll << 31),
+          ((steps * kTilesPerStep + kSteps - 1) / kSteps + 1) / 2 * 2, per * kTilesPerStep};
+}
+
+BlockCut block_cut_any(int type, int64_t K, int NT, int64_t out_rows) {
+  switch (type) {
+    case LX_W_BF16: return block_cut<LX_W_BF16>(K, NT, out_rows);
+    case LX_W_INT8: return block_cut<LX_W_INT8>(K, NT, out_rows);
+    case LX_W_FP8: return block_cut<LX_W_FP8>(K, NT, out_rows);
+    default: return block_cut<LX_W_NVFP4>(K, NT, out_rows);
+  }
+}
+
+int launch_expert_block(int type, ExpertBlock a, const Stack& w, int64_t K, int cols, const BlockCut& cut, int tiles, hipStream_t s) {
+  a.w = w;
+  a.K = static_cast<int>(K);
+  a.cols = cols;
+  a.row_bytes = row_bytes_of(type, K);
+  a.scale_row_bytes = type == LX_W_NVFP4 ? K / 16 : 0;
+  a.tiles = cut.tiles;
+  a.slice = cut.slice;
+  switch (type) {
+    case LX_W_BF16: return launch_expert_block_bf16(a, tiles, s);
+    case LX_W_INT8: return launch_expert_block_int8(a, tiles, s);
+    case LX_W_FP8: return launch_expert_block_fp8(a, tiles, s);
+    default: return launch_expert_block_nvfp4(a, tiles, s);
+  }
+}
+
 }  // namespace
 
 int64_t grouped_workspace_bytes(int T, int L, int I, int E, int top_k, int math) {
@@ -359,7 +403,14 @@ int experts_grouped(const void* latent, const int32_t* ids, const float* weights
     d.top_k = top_k;
     return experts_plain(d, gate_up.type, down.type, s);
   }
-  hipLaunchKernelGGL(group_kernel, dim3(1), dim3(kMaxExperts), 0, s, ids, P, E, a.t);
+  const BlockCut cut1 = block_cut_any(gate_up.type, L, 2, I), cut2 = block_cut_any(down.type, I, 1, L);
+  // Many rows an expert: the block kernels, which read and decode a weight once per 128 of them. Measured (64 and 128 experts,
+  // top-8): at 16 rows an expert on average NVFP4 4096 x 1536 724 -> 542 us, fp8 2048 x 1024 129 -> 110; at 8 the kernels
+  // here are ahead (93 / 107). bf16 weights, which have no decode to save, from 24 (at 16: 173 / 196, at 32: 254 / 204).
+  const int rows_wanted = gate_up.type == LX_W_BF16 ? 24 : 16;
+  const bool blocks = cut1.fits && cut2.fits && static_cast<int64_t>(T) * L * 2 < (1ll << 31) && P >= static_cast<int64_t>(rows_wanted) * E;
+  const int tiles = max_tiles(P, E, blocks ? kBlockTokens : kTileTokens);
+  hipLaunchKernelGGL(group_kernel, dim3(1), dim3(kMaxExperts), 0, s, ids, P, E, blocks ? kBlockTokens : kTileTokens, a.t);
   if (int st = status_of(hipGetLastError())) return st;
   if (quantised) {
     uint16_t* const image1 = reinterpret_cast<uint16_t*>(ws + lay.image1);
@@ -368,9 +419,20 @@ int experts_grouped(const void* latent, const int32_t* ids, const float* weights
     a.latent = image1;
     a.xs1 = scale1;
   }
-  const int tiles = max_tiles(P, E);
+  ExpertBlock b{};
+  b.top_k = top_k;
+  b.tile_expert = a.t.tile_expert;
+  b.tile_begin = a.t.tile_begin;
+  b.tile_rows = a.t.tile_rows;
+  b.n_tiles = a.t.n_tiles;
   int st;
-  switch (gate_up.type) {
+  if (blocks) {
+    b.x = a.latent;
+    b.xs = a.xs1;
+    b.order = a.t.order;
+    b.out = a.inter;
+    st = launch_expert_block(gate_up.type, b, a.gu, L, I, cut1, tiles, s);
+  } else switch (gate_up.type) {
     case LX_W_BF16: st = launch_stage<LX_W_BF16>(grouped_gate_up_kernel<LX_W_BF16, false>, a, L, 2, I, tiles, s); break;
     case LX_W_INT8: st = launch_stage<LX_W_INT8>(grouped_gate_up_kernel<LX_W_INT8, false>, a, L, 2, I, tiles, s); break;
     case LX_W_FP8: st = launch_stage<LX_W_FP8>(grouped_gate_up_kernel<LX_W_FP8, false>, a, L, 2, I, tiles, s); break;
@@ -390,7 +452,13 @@ int experts_grouped(const void* latent, const int32_t* ids, const float* weights
     a.down_in = image2;
     a.xs2 = scale2;
   }
-  switch (down.type) {
+  if (blocks) {
+    b.x = a.down_in;
+    b.xs = a.xs2;
+    b.order = nullptr;
+    b.out = a.contrib;
+    st = launch_expert_block(down.type, b, a.dn, I, L, cut2, tiles, s);
+  } else switch (down.type) {
     case LX_W_BF16: st = launch_stage<LX_W_BF16>(grouped_down_kernel<LX_W_BF16, false>, a, I, 1, L, tiles, s); break;
     case LX_W_INT8: st = launch_stage<LX_W_INT8>(grouped_down_kernel<LX_W_INT8, false>, a, I, 1, L, tiles, s); break;
     case LX_W_FP8: st = launch_stage<LX_W_FP8>(grouped_down_kernel<LX_W_FP8, false>, a, I, 1, L, tiles, s); break;

@@ -10,7 +10,7 @@ import torch
 import checks
 import ops
 from dromos_amd.abi import BF16, DTYPE, F32, FORMATS, MATH_BF16, MATH_FP4, MATH_FP8, MATH_INT8
-from dromos_amd.formats import random_weight
+from dromos_amd.formats import random_stack, random_weight
 
 pytestmark = pytest.mark.gpu
 MATHS = [("bf16", MATH_BF16), ("int8", MATH_BF16), ("fp8", MATH_BF16), ("nvfp4", MATH_BF16), ("int8", MATH_INT8), ("fp8", MATH_FP8),
@@ -61,3 +61,18 @@ def test_strides_and_a_stream_without_the_partial_buffer(hip, fmt):
                           None, stream.cuda_stream) == 0
         torch.cuda.synchronize()
         assert torch.equal(y[:, :N], want.to(y_dtype)) and bool((y[:, N:] == -3.0).all())
+
+
+# Experts: tiles of every height up to two of 128, slices that end on odd load steps (and, in bf16, inside a K tile), a
+# last block of columns cut short, ids outside the range.
+@pytest.mark.parametrize("fmt,math", MATHS)
+@pytest.mark.parametrize("T,L,I,E,top_k", [(96, 1056, 544, 2, 1), (160, 1088, 288, 4, 2), (300, 2112, 544, 8, 4), (700, 512, 160, 6, 3)])
+def test_experts_are_those_of_few_tokens(hip, fmt, math, T, L, I, E, top_k):
+    gu, dn = random_stack(FORMATS[fmt], E, 2 * I, L, 3).to("cuda"), random_stack(FORMATS[fmt], E, L, I, 4).to("cuda")
+    latent, ids, weights = (t.cuda() for t in checks.make_routing(T, E, L, top_k, T))
+    ids = torch.where(torch.rand(ids.shape, generator=torch.Generator().manual_seed(T)).cuda() < 0.03, torch.full_like(ids, E), ids)
+    got = ops.experts_grouped(hip, latent, ids, weights, gu, dn, I, E, top_k, math=math)
+    step = max(1, 12 * E // top_k)  # fewer rows an expert than the block kernels are taken for
+    few = [ops.experts_grouped(hip, latent[t : t + step].contiguous(), ids[t : t + step].contiguous(), weights[t : t + step].contiguous(), gu, dn,
+                               I, E, top_k, math=math) for t in range(0, T, step)]
+    assert torch.equal(got, torch.cat(few))
