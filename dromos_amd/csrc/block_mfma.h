@@ -30,8 +30,12 @@ __device__ __forceinline__ int die_order(int b, int total) {
   return die * share + min(die, extra) + (b >> 3);
 }
 
-// WM x WN wavefronts, each MT x NT tiles of 16 x 16. SPLIT: the row is more than one slice.
-template <int F, int MATH, int WM, int WN, int MT, int NT, bool SPLIT>
+// WM x WN wavefronts, each MT x NT tiles of 16 x 16. SPLIT: the row is more than one slice. ONE_X: one set of registers for
+// the activations' fragments, each read anew as soon as its products are issued, and the barrier behind a step's first products.
+// Reads and products then alternate more evenly and 16 registers are free: the experts' NVFP4 blocks of 128 x 256 at 2048 tokens
+// (128 of 4096 x 1536, both products and their sum) 1495 -> 1407 us; lx_gemm_w's blocks of 128 x 128 are 3 % faster without
+// (fp8 14336 x 4096 at 4096 rows 577 / 598).
+template <int F, int MATH, int WM, int WN, int MT, int NT, bool SPLIT, bool ONE_X = false>
 struct Block {
   static constexpr bool kBytes = MATH != LX_MATH_BF16;  // one-byte operands on both sides
   static constexpr int D = 2;  // sets of staging registers (four made no difference: 64 x 64 .. 128 x 128, any row count)
@@ -169,17 +173,21 @@ struct Block {
     for (int nt = 0; nt < NT; ++nt) f.w[nt] = *reinterpret_cast<const i32x4*>(p + nt * 256);
   }
 
-  __device__ __forceinline__ void fetch_x(Frags& f, const uint8_t* buf, int j) const {
+  __device__ __forceinline__ i32x4 fetch_x(const uint8_t* buf, int j, int mt) const {
     const uint8_t* const p = buf + ((4 * j + (lane >> 4)) * BM + wave % WM * 16 + ((lane & 15) ^ x_turn(4 * j + (lane >> 4)))) * 16;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) f.x[mt] = *reinterpret_cast<const i32x4*>(p + mt * WM * 256);
+    return *reinterpret_cast<const i32x4*>(p + mt * WM * 256);
   }
 
-  static __device__ __forceinline__ void multiply(const Frags& f, int mt, Acc (&acc)[NT][MT]) {
+  __device__ __forceinline__ void fetch_x(Frags& f, const uint8_t* buf, int j) const {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) f.x[mt] = fetch_x(buf, j, mt);
+  }
+
+  static __device__ __forceinline__ void multiply(const i32x4 (&w)[NT], const i32x4& x, int mt, Acc (&acc)[NT][MT]) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      if constexpr (kBytes) acc[nt][mt] = byte_mfma<MATH>(f.w[nt], f.x[mt], acc[nt][mt]);
-      else acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f.w[nt]), __builtin_bit_cast(bf16x8, f.x[mt]), acc[nt][mt], 0, 0, 0);
+      if constexpr (kBytes) acc[nt][mt] = byte_mfma<MATH>(w[nt], x, acc[nt][mt]);
+      else acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[nt]), __builtin_bit_cast(bf16x8, x), acc[nt][mt], 0, 0, 0);
     }
   }
 
@@ -235,7 +243,7 @@ struct Block {
       for (int mt = 0; mt < MT; ++mt) {
         if (mt == 0) fetch_w(f1, here, 1);
         if (mt == (MT > 3 ? 1 : 0)) fetch_x(f1, here, 1);
-        multiply(f0, mt, acc);
+        multiply(f0.w, f0.x[mt], mt, acc);
         __builtin_amdgcn_sched_barrier(0);
       }
       __syncthreads();
@@ -250,13 +258,43 @@ struct Block {
         for (int u = 0; u < XU + WU; ++u)
           if (mt == kFirst + u * kGroups / (XU + WU)) store(set, u, first + kt + 2, here);
         if (mt == MT - 1) load(set, first + kt + 2 + D);
-        multiply(f1, mt, acc);
+        multiply(f1.w, f1.x[mt], mt, acc);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // The same with f0.x for both instructions (ONE_X). Tile kt's last fragment is asked for behind the first instruction's last
+    // products and used by the second's last; the barrier, which waits for it, stands behind the second's first.
+    auto step_one_x = [&](int kt, Set& set, uint8_t* here, const uint8_t* there) {
+      flush(kStepHalves ? 2 * kt : kt);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        if (mt == 0) fetch_w(f1, here, 1);
+        multiply(f0.w, f0.x[mt], mt, acc);
+        f0.x[mt] = fetch_x(here, 1, mt);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (kStepHalves) flush(2 * kt + 1);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        multiply(f1.w, f0.x[mt], mt, acc);
+        if (mt == 0) {
+          __builtin_amdgcn_sched_barrier(0);
+          __syncthreads();
+          fetch_w(f0, there, 0);
+        }
+        f0.x[mt] = fetch_x(there, 0, mt);
+#pragma unroll
+        for (int u = 0; u < XU + WU; ++u)
+          if (mt == u * MT / (XU + WU)) store(set, u, first + kt + 2, here);
+        if (mt == MT - 1) load(set, first + kt + 2 + D);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
     for (int kt = 0; kt < tiles; kt += D) {
 #pragma unroll
-      for (int d = 0; d < D; ++d) step(kt + d, s[(d + 2) % D], d % 2 ? b1 : b0, d % 2 ? b0 : b1);
+      for (int d = 0; d < D; ++d)
+        if constexpr (ONE_X) step_one_x(kt + d, s[(d + 2) % D], d % 2 ? b1 : b0, d % 2 ? b0 : b1);
+        else step(kt + d, s[(d + 2) % D], d % 2 ? b1 : b0, d % 2 ? b0 : b1);
     }
     const int wm = wave % WM, wn = wave / WM;
 #pragma unroll

@@ -10,7 +10,7 @@ namespace block {
 // so that a wavefront's four tiles are two pairs and SwiGLU is its epilogue.
 template <int F, int MT, bool GATE_UP, bool SPLIT>
 __device__ __forceinline__ void expert_tile(const ExpertBlock& a, int e, int g0, int rows, int c0, void* lds) {
-  using B = Block<F, LX_MATH_BF16, 2, 4, MT, 4, SPLIT>;
+  using B = Block<F, LX_MATH_BF16, 2, 4, MT, 4, SPLIT, true>;
   const int64_t first = static_cast<int64_t>(e) * (GATE_UP ? 2 : 1) * a.cols;  // the expert's first row in the stack
   // The stack row of the block's weight row, relative to c0's; a row past the last stands for the last.
   auto weight_row = [&](int row) {
