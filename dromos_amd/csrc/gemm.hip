@@ -1435,8 +1435,26 @@ bool launch_block(GemmArgs a, int* status, hipStream_t stream) {
       return true;
     }
     a.partial = nullptr;
+  } else if (a.M <= 64) {
+    return false;  // few blocks and no way to share them out: the kernels for up to 64 rows are ahead
   }
   return launch();
+}
+
+// Whether 33 .. 64 rows go to the block kernel too: on short matrices the windowed and slab kernels stage all of the rows
+// once per few weight tiles, and the block kernel's slices fill the device. Measured at 64 rows (before -> after, us): fp8
+// 2048 x 2048 16.9 -> 9.7, 4096 x 4096 22.4 -> 14.9, 6144 x 5120 34.8 -> 20.8, 6400 x 2048 14.6 -> 13.8; NVFP4 4096 x 4096 20.1 ->
+// 15.6, 4096 x 6144 21.5 -> 19.8; bf16 5120 x 5120 32.5 -> 24.8, 6144 x 5120 33.2 -> 27.1. The lines: 4096 x 2048 ties or is behind
+// in bf16 (33 rows 11.5 / 12.1) and NVFP4 (64 rows 18.7 / 19.7), bf16 6400 x 2048 too (13.8 / 15.6); up to 48 rows one-byte
+// weights are behind on 256 tiles at 33 rows (4096 x 6144 14.9 / 16.0) and tie from 320, and NVFP4 gains nothing; 4096 x 14336
+// ties and 14336 x 4096 is behind (fp8 at 64 rows 22.5 / 28.6).
+template <int F>
+bool block_wanted(int M, int n_tiles, int64_t K, int tuned) {
+  if (M > 64) return true;
+  if (M <= 32 || tuned >= 0 || n_tiles < 128 || K < 2048 || K > 6144) return false;
+  if (F == LX_W_BF16) return n_tiles <= 400 && K >= 3072;
+  if (F == LX_W_NVFP4) return M > 48 && n_tiles <= 256 && K >= 3072;
+  return n_tiles <= (M > 48 ? 400 : 192);
 }
 
 template <int F>
@@ -1459,7 +1477,8 @@ int launch_format(GemmArgs a, const char* x0, char* y0, int M, int x_esize, int 
   // Slices are whole weight batches (the row's last one may be cut short by the row's end).
   a.steps_per_wave = ((a.steps + S - 1) / S + kLoadsInFlight - 1) / kLoadsInFlight * kLoadsInFlight;
   a.S = S;
-  if (M > 64 && a.xs.dtype == LX_BF16) {
+  if (a.xs.dtype == LX_BF16 &&
+      block_wanted<F>(M, (a.N + kTileRows - 1) / kTileRows, a.K, M > 64 ? -1 : tuned_variant(gemm_key<F>(), M, a.N, a.K))) {
     a.M = M;
     a.xs.x = x0;
     a.y = y0;

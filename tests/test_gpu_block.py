@@ -1,5 +1,5 @@
 """GPU: the block kernels (more rows than a decode step has) against the kernels for up to 64 rows, bit for bit: the same
-rows in calls of 64 at most. Row counts, output counts and row lengths around the edges of blocks, K tiles, slices and
+rows in calls of 32 at most. Row counts, output counts and row lengths around the edges of blocks, K tiles, slices and
 load steps; every format and math; the epilogue's operands; a stream with and without the partial-tile buffer."""
 
 import ctypes
@@ -17,8 +17,8 @@ MATHS = [("bf16", MATH_BF16), ("int8", MATH_BF16), ("fp8", MATH_BF16), ("nvfp4",
          ("nvfp4", MATH_FP8), ("nvfp4", MATH_FP4)]
 
 
-def chunks_of_64(hip, x, w, math, y, **kw):
-    return torch.cat([ops.gemm_w(hip, x[m : m + 64].contiguous(), w, math, y=y[m : m + 64].clone(), **kw) for m in range(0, x.shape[0], 64)])
+def chunks_of_32(hip, x, w, math, y, **kw):
+    return torch.cat([ops.gemm_w(hip, x[m : m + 32].contiguous(), w, math, y=y[m : m + 32].clone(), **kw) for m in range(0, x.shape[0], 32)])
 
 
 # Few blocks (a slice a workgroup), one block past a multiple of 64 / 128 rows and columns, an odd N, many blocks of each shape;
@@ -26,12 +26,12 @@ def chunks_of_64(hip, x, w, math, y, **kw):
 @pytest.mark.parametrize("fmt,math", MATHS)
 @pytest.mark.parametrize("M,N,K", [(65, 300, 4096), (129, 257, 1056), (128, 1000, 544), (191, 2064, 8224), (515, 4096, 1056), (1030, 3001, 2080),
                                    (2050, 4112, 1024), (66, 30000, 544)])
-def test_rows_are_those_of_calls_of_64(hip, fmt, math, M, N, K):
+def test_rows_are_those_of_calls_of_32(hip, fmt, math, M, N, K):
     g = torch.Generator().manual_seed(M + N + K)
     w = random_weight(FORMATS[fmt], N, K, N + K).to("cuda")
     x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
     y = torch.full((M, N), float("nan"), device="cuda")
-    assert torch.equal(ops.gemm_w(hip, x, w, math, y=y.clone()), chunks_of_64(hip, x, w, math, y))
+    assert torch.equal(ops.gemm_w(hip, x, w, math, y=y.clone()), chunks_of_32(hip, x, w, math, y))
 
 
 @pytest.mark.parametrize("fmt,math", [("fp8", MATH_BF16), ("nvfp4", MATH_FP4), ("int8", MATH_INT8)])
@@ -44,7 +44,7 @@ def test_epilogue_operands(hip, fmt, math, y_dtype, bias, alpha, beta, M, N, K):
     x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
     y = torch.randn(M, N, generator=g).to(y_dtype).cuda()
     kw = dict(bias=None if bias is None else torch.randn(N, generator=g).to(bias).cuda(), alpha=alpha, beta=beta)
-    assert torch.equal(ops.gemm_w(hip, x, w, math, y=y.clone(), **kw), chunks_of_64(hip, x, w, math, y, **kw))
+    assert torch.equal(ops.gemm_w(hip, x, w, math, y=y.clone(), **kw), chunks_of_32(hip, x, w, math, y, **kw))
 
 
 @pytest.mark.parametrize("fmt", checks.FMT_NAMES)
@@ -76,3 +76,32 @@ def test_experts_are_those_of_few_tokens(hip, fmt, math, T, L, I, E, top_k):
     few = [ops.experts_grouped(hip, latent[t : t + step].contiguous(), ids[t : t + step].contiguous(), weights[t : t + step].contiguous(), gu, dn,
                                I, E, top_k, math=math) for t in range(0, T, step)]
     assert torch.equal(got, torch.cat(few))
+
+
+# 33 .. 64 rows on short matrices: both ends of the rule's rows, tiles and row lengths, and a last tile and K tile cut short,
+# on a stream with a partial-tile buffer; eagerly and from a graph.
+@pytest.mark.parametrize("fmt", checks.FMT_NAMES)
+@pytest.mark.parametrize("M,N,K", [(33, 2048, 2048), (48, 3072, 4096), (49, 2040, 2080), (64, 4096, 6144), (57, 6400, 5120)])
+def test_few_rows_on_short_matrices(hip, fmt, M, N, K):
+    g = torch.Generator().manual_seed(M)
+    w = random_weight(FORMATS[fmt], N, K, N + K).to("cuda")
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    want = chunks_of_32(hip, x, w, MATH_BF16, torch.full((M, N), float("nan"), device="cuda"))
+    struct, stream, graph = w.lx(), ctypes.c_void_p(), ctypes.c_void_p()
+    y = torch.full((M, N), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    assert hip.lib.lx_rt_stream_create(ctypes.byref(stream)) == 0
+    call = ("gemm_w", x, BF16, K, ctypes.pointer(struct), MATH_BF16, None, F32, y, F32, N, M, N, K, 1.0, 0.0, None, stream.value)
+    try:
+        assert hip.status(*call) == 0 and hip.lib.lx_rt_stream_sync(stream) == 0
+        assert torch.equal(y, want)
+        assert hip.lib.lx_rt_capture_begin(stream) == 0 and hip.status(*call) == 0
+        assert hip.lib.lx_rt_capture_end(stream, ctypes.byref(graph)) == 0
+        for _ in range(3):
+            y.fill_(float("nan"))
+            torch.cuda.synchronize()
+            assert hip.lib.lx_rt_graph_launch(graph, stream) == 0 and hip.lib.lx_rt_stream_sync(stream) == 0
+            assert torch.equal(y, want)
+        assert hip.lib.lx_rt_graph_destroy(graph) == 0
+    finally:
+        assert hip.lib.lx_rt_stream_destroy(stream) == 0
