@@ -328,6 +328,25 @@ BlockCut block_cut(int64_t K, int NT, int64_t out_rows) {
           ((steps * kTilesPerStep + kSteps - 1) / kSteps + 1) / 2 * 2, per * kTilesPerStep};
 }
 
+// Whether P pairs over E experts go to the block kernels, which read and decode a weight once per 128 rows but are one
+// workgroup per 128 intermediate (256 output) rows and tile, a unit holding one at a time. Two things count (sweep of 1 .. 128
+// experts, 512 x 2048 .. 4096 x 14336, 16 .. 400 rows an expert, every format, against the kernels for up to 64 rows):
+// - Rows an expert: 128 experts of 4096 x 1536 at 16 on average NVFP4 724 -> 542 us; at 8 the kernels here are ahead (fp8
+//   2048 x 1024 93 / 107). bf16 weights, which have no decode to save, from 24 (at 16 rows 173 / 196 us, at 32 254 / 204).
+// - How much of the device the blocks fill: the share of the units that have one, over both stages by their rows' lengths.
+//   Two NVFP4 experts of 4096 x 1536 at 16 rows are 24 and 32 blocks: 26.6 us by the kernels here, 77.5 by blocks.
+// Rows (48 at most) times that share from 12 on is where the blocks are ahead: of 1661 sweep points 10 lose 4 % or more (11 %
+// at most: bf16 12 experts of 2048 x 4096 at 25 rows; NVFP4 up to 8 % at 17 .. 25), and 2 % of the gain is left.
+bool blocks_wanted(int type, int64_t P, int64_t E, int64_t L, int64_t I, int units) {
+  if (P < (type == LX_W_BF16 ? 24 : 16) * E) return false;
+  const int64_t by_rows = (P + kBlockTokens - 1) / kBlockTokens, tiles = by_rows > E ? by_rows : E;
+  const int64_t w1 = tiles * ((I + 127) / 128), w2 = tiles * ((L + 255) / 256);
+  const double busy = static_cast<double>(L) * w1 + static_cast<double>(I) * w2;
+  const double held = units * (static_cast<double>(L) * ((w1 + units - 1) / units) + static_cast<double>(I) * ((w2 + units - 1) / units));
+  const double rows = static_cast<double>(P) / E;
+  return (rows < 48 ? rows : 48) * busy >= 12 * held;
+}
+
 BlockCut block_cut_any(int type, int64_t K, int NT, int64_t out_rows) {
   switch (type) {
     case LX_W_BF16: return block_cut<LX_W_BF16>(K, NT, out_rows);
@@ -404,11 +423,7 @@ int experts_grouped(const void* latent, const int32_t* ids, const float* weights
     return experts_plain(d, gate_up.type, down.type, s);
   }
   const BlockCut cut1 = block_cut_any(gate_up.type, L, 2, I), cut2 = block_cut_any(down.type, I, 1, L);
-  // Many rows an expert: the block kernels, which read and decode a weight once per 128 of them. Measured (64 and 128 experts,
-  // top-8): at 16 rows an expert on average NVFP4 4096 x 1536 724 -> 542 us, fp8 2048 x 1024 129 -> 110; at 8 the kernels
-  // here are ahead (93 / 107). bf16 weights, which have no decode to save, from 24 (at 16: 173 / 196, at 32: 254 / 204).
-  const int rows_wanted = gate_up.type == LX_W_BF16 ? 24 : 16;
-  const bool blocks = cut1.fits && cut2.fits && static_cast<int64_t>(T) * L * 2 < (1ll << 31) && P >= static_cast<int64_t>(rows_wanted) * E;
+  const bool blocks = cut1.fits && cut2.fits && static_cast<int64_t>(T) * L * 2 < (1ll << 31) && blocks_wanted(gate_up.type, P, E, L, I, compute_units());
   const int tiles = max_tiles(P, E, blocks ? kBlockTokens : kTileTokens);
   hipLaunchKernelGGL(group_kernel, dim3(1), dim3(kMaxExperts), 0, s, ids, P, E, blocks ? kBlockTokens : kTileTokens, a.t);
   if (int st = status_of(hipGetLastError())) return st;
@@ -479,6 +494,12 @@ int experts_grouped(const void* latent, const int32_t* ids, const float* weights
 using namespace dro;
 
 extern "C" {
+
+// Which kernels lx_moe_experts_grouped takes on a device of `units` compute units (0: the current device): 1 the block kernels, 0
+// the others. For tests of the rule: nothing is launched, and with `units` given no device is needed.
+LX_API int dromos_plan_experts(int gate_up_type, int T, int L, int I, int E, int top_k, int units) {
+  return blocks_wanted(gate_up_type, static_cast<int64_t>(T) * top_k, E, L, I, units > 0 ? units : compute_units());
+}
 
 int lx_moe_experts_grouped(const void* latent, const int32_t* ids, const float* weights, const lx_weight* gate_up,
                            const lx_weight* down, lx_math math, float* out, void* workspace, int T, int L, int I, int E, int top_k,

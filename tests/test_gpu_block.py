@@ -63,16 +63,20 @@ def test_strides_and_a_stream_without_the_partial_buffer(hip, fmt):
         assert torch.equal(y[:, :N], want.to(y_dtype)) and bool((y[:, N:] == -3.0).all())
 
 
-# Experts: tiles of every height up to two of 128, slices that end on odd load steps (and, in bf16, inside a K tile), a
-# last block of columns cut short, ids outside the range.
+# Experts: tiles of every height up to two of 128 (the experts' shares differ by about e^2), slices that end on odd load
+# steps (and, in bf16, inside a K tile), a last block of columns cut short, ids outside the range.
 @pytest.mark.parametrize("fmt,math", MATHS)
-@pytest.mark.parametrize("T,L,I,E,top_k", [(96, 1056, 544, 2, 1), (160, 1088, 288, 4, 2), (300, 2112, 544, 8, 4), (700, 512, 160, 6, 3)])
+@pytest.mark.parametrize("T,L,I,E,top_k", [(1000, 1056, 544, 16, 1), (800, 1088, 288, 32, 2), (300, 2112, 544, 16, 4), (700, 512, 160, 40, 3)])
 def test_experts_are_those_of_few_tokens(hip, fmt, math, T, L, I, E, top_k):
     gu, dn = random_stack(FORMATS[fmt], E, 2 * I, L, 3).to("cuda"), random_stack(FORMATS[fmt], E, L, I, 4).to("cuda")
-    latent, ids, weights = (t.cuda() for t in checks.make_routing(T, E, L, top_k, T))
-    ids = torch.where(torch.rand(ids.shape, generator=torch.Generator().manual_seed(T)).cuda() < 0.03, torch.full_like(ids, E), ids)
+    latent, _, weights = (t.cuda() for t in checks.make_routing(T, E, L, top_k, T))
+    g = torch.Generator().manual_seed(T)
+    ids = (torch.linspace(-1, 1, E) - torch.rand(T, E, generator=g).log().neg().log()).topk(top_k, 1).indices.int().cuda()
+    ids = torch.where(torch.rand(ids.shape, generator=g).cuda() < 0.03, torch.full_like(ids, E), ids)
+    assert hip.lib.dromos_plan_experts(FORMATS[fmt], T, L, I, E, top_k, 0) == 1
     got = ops.experts_grouped(hip, latent, ids, weights, gu, dn, I, E, top_k, math=math)
     step = max(1, 12 * E // top_k)  # fewer rows an expert than the block kernels are taken for
+    assert hip.lib.dromos_plan_experts(FORMATS[fmt], step, L, I, E, top_k, 0) == 0
     few = [ops.experts_grouped(hip, latent[t : t + step].contiguous(), ids[t : t + step].contiguous(), weights[t : t + step].contiguous(), gu, dn,
                                I, E, top_k, math=math) for t in range(0, T, step)]
     assert torch.equal(got, torch.cat(few))
