@@ -137,16 +137,24 @@ struct Block {
     }
   }
 
-  // Tile kt from the staging registers into a buffer; what lies past K is zero on the activations' side.
+  // Tile kt from the staging registers into a buffer. What lies past K is zero on the activations' side, and in bf16 on the
+  // weights' too: a load there repeats the row's last values, and zero times an infinity among them is no zero (the other
+  // formats have no infinities). EDGE: the tile may reach past K; bf16 has a loop of its own for the tiles that do not: with one
+  // loop the weights' zeros cost 2 % (14336 x 4096 at 4096 rows 593 / 606 us, with two 585). The experts' blocks (ONE_X) have
+  // one: 64 experts of 2048 x 1024 at 1024 tokens 398 us, 416 with two.
+  template <bool EDGE>
   __device__ __forceinline__ void store_x(const Set& s, int u, int kt, uint8_t* buf) const {
     u32x4 v = s.x[u];
-    if (xtile(kt) + xk[u] > xlast) v = u32x4{0u, 0u, 0u, 0u};
+    if (EDGE && xtile(kt) + xk[u] > xlast) v = u32x4{0u, 0u, 0u, 0u};
     *reinterpret_cast<u32x4*>(buf + xput[u]) = v;
   }
 
-  __device__ __forceinline__ void store_w(const Set& s, int u, uint8_t* buf) const {
+  template <bool EDGE>
+  __device__ __forceinline__ void store_w(const Set& s, int u, int kt, uint8_t* buf) const {
     if constexpr (kRaw) {
-      *reinterpret_cast<u32x4*>(buf + wput[u]) = s.w[u];
+      u32x4 v = s.w[u];
+      if (EDGE && F == LX_W_BF16 && wtile(kt) + wk[u] > wlast) v = u32x4{0u, 0u, 0u, 0u};
+      *reinterpret_cast<u32x4*>(buf + wput[u]) = v;
     } else {
       u32x4 w;
       if constexpr (F == LX_W_NVFP4) w = u32x4{s.w[u].x, s.w[u].y, 0u, 0u};
@@ -157,9 +165,10 @@ struct Block {
   }
 
   // Unit u of the staging registers: activations first.
+  template <bool EDGE>
   __device__ __forceinline__ void store(const Set& s, int u, int kt, uint8_t* buf) const {
-    if (u < XU) store_x(s, u, kt, buf);
-    else store_w(s, u - XU, buf);
+    if (u < XU) store_x<EDGE>(s, u, kt, buf);
+    else store_w<EDGE>(s, u - XU, kt, buf);
   }
 
   // The fragments of a tile's instruction j.
@@ -210,10 +219,10 @@ struct Block {
     uint8_t* const b0 = lds;
     uint8_t* const b1 = lds + kBufBytes;
 #pragma unroll
-    for (int u = 0; u < XU + WU; ++u) store(s[0], u, first, b0);
+    for (int u = 0; u < XU + WU; ++u) store<true>(s[0], u, first, b0);
     load(s[0], first + D);
 #pragma unroll
-    for (int u = 0; u < XU + WU; ++u) store(s[1], u, first + 1, b1);
+    for (int u = 0; u < XU + WU; ++u) store<true>(s[1], u, first + 1, b1);
     load(s[1], first + D + 1);
     __syncthreads();
     Frags f0, f1;
@@ -237,7 +246,7 @@ struct Block {
     // Tile kt, whose first instruction's fragments are in f0, from `here`. Under their products the second's are read; after
     // the barrier nobody reads `here` any more, and under the second's products tile kt + 1's first fragments are read and
     // tile kt + 2 is written where tile kt was: the writes have half a step until the next barrier waits for them.
-    auto step = [&](int kt, Set& set, uint8_t* here, const uint8_t* there) {
+    auto step = [&](auto edge, int kt, Set& set, uint8_t* here, const uint8_t* there) {
       flush(kStepHalves ? 2 * kt : kt);
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
@@ -256,7 +265,7 @@ struct Block {
         constexpr int kFirst = MT > 1 ? 1 : 0, kGroups = MT - kFirst;
 #pragma unroll
         for (int u = 0; u < XU + WU; ++u)
-          if (mt == kFirst + u * kGroups / (XU + WU)) store(set, u, first + kt + 2, here);
+          if (mt == kFirst + u * kGroups / (XU + WU)) store<decltype(edge)::value>(set, u, first + kt + 2, here);
         if (mt == MT - 1) load(set, first + kt + 2 + D);
         multiply(f1.w, f1.x[mt], mt, acc);
         __builtin_amdgcn_sched_barrier(0);
@@ -264,7 +273,7 @@ struct Block {
     };
     // The same with f0.x for both instructions (ONE_X). Tile kt's last fragment is asked for behind the first instruction's last
     // products and used by the second's last; the barrier, which waits for it, stands behind the second's first.
-    auto step_one_x = [&](int kt, Set& set, uint8_t* here, const uint8_t* there) {
+    auto step_one_x = [&](auto edge, int kt, Set& set, uint8_t* here, const uint8_t* there) {
       flush(kStepHalves ? 2 * kt : kt);
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
@@ -285,17 +294,22 @@ struct Block {
         f0.x[mt] = fetch_x(there, 0, mt);
 #pragma unroll
         for (int u = 0; u < XU + WU; ++u)
-          if (mt == u * MT / (XU + WU)) store(set, u, first + kt + 2, here);
+          if (mt == u * MT / (XU + WU)) store<decltype(edge)::value>(set, u, first + kt + 2, here);
         if (mt == MT - 1) load(set, first + kt + 2 + D);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    for (int kt = 0; kt < tiles; kt += D) {
+    auto steps = [&](auto edge, int kt) {
 #pragma unroll
       for (int d = 0; d < D; ++d)
-        if constexpr (ONE_X) step_one_x(kt + d, s[(d + 2) % D], d % 2 ? b1 : b0, d % 2 ? b0 : b1);
-        else step(kt + d, s[(d + 2) % D], d % 2 ? b1 : b0, d % 2 ? b0 : b1);
-    }
+        if constexpr (ONE_X) step_one_x(edge, kt + d, s[(d + 2) % D], d % 2 ? b1 : b0, d % 2 ? b0 : b1);
+        else step(edge, kt + d, s[(d + 2) % D], d % 2 ? b1 : b0, d % 2 ? b0 : b1);
+    };
+    int kt = 0;
+    // Steps kt and kt + 1 write tiles kt + 2 and kt + 3.
+    if constexpr (F == LX_W_BF16 && !ONE_X)
+      for (const int inside = min(tiles, ((wlast + 16) / 128 - first - 2) & ~1); kt < inside; kt += D) steps(std::false_type{}, kt);
+    for (; kt < tiles; kt += D) steps(std::true_type{}, kt);
     const int wm = wave % WM, wn = wave / WM;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {

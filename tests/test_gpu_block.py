@@ -109,3 +109,49 @@ def test_few_rows_on_short_matrices(hip, fmt, M, N, K):
         assert hip.lib.lx_rt_graph_destroy(graph) == 0
     finally:
         assert hip.lib.lx_rt_stream_destroy(stream) == 0
+
+
+def on_library_stream(hip, x, w, math, y):
+    """lx_gemm_w on a stream with a partial-tile buffer."""
+    stream, struct = ctypes.c_void_p(), w.lx()
+    (M, K), N = x.shape, y.shape[1]
+    ws = torch.empty(max(256, int(hip.size("gemm_workspace_bytes", M, K, math))), dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    assert hip.lib.lx_rt_stream_create(ctypes.byref(stream)) == 0
+    try:
+        assert hip.status("gemm_w", x, DTYPE[x.dtype], x.shape[1], ctypes.pointer(struct), math, None, F32, y, DTYPE[y.dtype], y.shape[1], M, N, K, 1.0,
+                          0.0, ws, stream.value) == 0
+        assert hip.lib.lx_rt_stream_sync(stream) == 0
+    finally:
+        assert hip.lib.lx_rt_stream_destroy(stream) == 0
+    return y
+
+
+# An infinity among a row's last values: the tiles past the row's end (K is no multiple of 128 here) must not meet it again.
+# All slices in a workgroup, one, and one slice a workgroup; everything but the two rows keeps its bits.
+@pytest.mark.parametrize("M,N,K", [(65, 300, 1056), (130, 257, 1088), (515, 2064, 8256), (80, 1000, 4104)])
+@pytest.mark.parametrize("run", [ops.gemm_w, on_library_stream])
+def test_infinite_weights_at_the_rows_end(hip, run, M, N, K):
+    w = random_weight(FORMATS["bf16"], N, K, N + K).to("cuda")
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(K)).to(torch.bfloat16).cuda()
+    clean = run(hip, x, w, MATH_BF16, y=torch.empty(M, N, device="cuda"))
+    w.data[3, K - 1], w.data[N - 1, K - 8] = float("inf"), float("-inf")
+    got = run(hip, x, w, MATH_BF16, y=torch.empty(M, N, device="cuda"))
+    assert torch.equal(got[:, 3], x[:, K - 1].float() * float("inf")) and torch.equal(got[:, N - 1], x[:, K - 8].float() * -float("inf"))
+    got[:, [3, N - 1]] = clean[:, [3, N - 1]]
+    assert torch.equal(got, clean)
+
+
+def test_infinite_expert_weights_at_the_rows_end(hip):
+    T, L, I, E, top_k = 1000, 1056, 544, 16, 1
+    gu, dn = random_stack(FORMATS["bf16"], E, 2 * I, L, 3).to("cuda"), random_stack(FORMATS["bf16"], E, L, I, 4).to("cuda")
+    latent, ids, weights = (t.cuda() for t in checks.make_routing(T, E, L, top_k, T))
+    assert hip.lib.dromos_plan_experts(FORMATS["bf16"], T, L, I, E, top_k, 0) == 1
+    clean = ops.experts_grouped(hip, latent, ids, weights, gu, dn, I, E, top_k)
+    assert bool(clean.isfinite().all())
+    to5, to7 = (ids == 5).any(1), (ids == 7).any(1)
+    dn.data[5, 9, I - 1], gu.data[7, I + 11, L - 8] = float("inf"), float("-inf")  # one output row; one up row, so one intermediate value
+    got = ops.experts_grouped(hip, latent, ids, weights, gu, dn, I, E, top_k)
+    assert bool(got[to5, 9].isinf().all()) and bool(got[to7].isinf().all())
+    got[to5, 9], got[to7] = clean[to5, 9], clean[to7]
+    assert torch.equal(got, clean)
