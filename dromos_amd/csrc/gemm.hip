@@ -15,7 +15,7 @@
 #include <utility>
 
 #include "common.h"
-#include "gemm_args.h"
+#include "gemm_block_plan.h"
 #include "tile_mfma.h"
 
 namespace dro {
@@ -1410,37 +1410,6 @@ int launch_skinny(GemmArgs a, hipStream_t stream) {
                               : launch_skinny_x<F, MT, false, false>(a, lds, n_tiles, S * kWave, stream);
 }
 
-// More rows than a decode step has: the block kernel (gemm_block.h), which takes all of them in one launch, each weight read
-// and decoded once per 64 or 128 rows: with the passes of 64 rows below, 14336 x 4096 fp8 at 128 / 256 / 1024 / 4096 rows took
-// 42 / 84 / 334 / 1450 us. Where the product has too few blocks for the device, one slice of K a workgroup, the slices
-// added by the slab kernel's second half (the stream's partial-tile buffer permitting).
-template <int F, int MATH>
-bool launch_block(GemmArgs a, int* status, hipStream_t stream) {
-  auto launch = [&] {
-    if constexpr (MATH == LX_MATH_INT8) return launch_block_int8_math(a, status, stream);
-    else if constexpr (MATH == LX_MATH_FP8) return launch_block_fp8_math(a, status, stream);
-    else if constexpr (F == LX_W_BF16) return launch_block_bf16(a, status, stream);
-    else if constexpr (F == LX_W_INT8) return launch_block_int8(a, status, stream);
-    else if constexpr (F == LX_W_FP8) return launch_block_fp8(a, status, stream);
-    else return launch_block_nvfp4(a, status, stream);
-  };
-  const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave, mts = (a.M + 15) / 16;
-  const int64_t vectors = static_cast<int64_t>((a.N + kTileRows - 1) / kTileRows) * mts * kWave;  // of one slice
-  if (slices > 1 && (a.partial = slab_scratch(stream, static_cast<size_t>(slices * vectors * 16)))) {
-    if (launch()) {
-      if (*status) return true;
-      a.S = slices;
-      hipLaunchKernelGGL((slab_reduce_kernel<F, MATH>), dim3(static_cast<unsigned>((vectors + 255) / 256)), dim3(256), 0, stream, a, mts);
-      *status = status_of(hipGetLastError());
-      return true;
-    }
-    a.partial = nullptr;
-  } else if (a.M <= 64) {
-    return false;  // few blocks and no way to share them out: the kernels for up to 64 rows are ahead
-  }
-  return launch();
-}
-
 // Whether 33 .. 64 rows go to the block kernel too: on short matrices the windowed and slab kernels stage all of the rows
 // once per few weight tiles, and the block kernel's slices fill the device. Measured at 64 rows (before -> after, us): fp8
 // 2048 x 2048 16.9 -> 9.7, 4096 x 4096 22.4 -> 14.9, 6144 x 5120 34.8 -> 20.8, 6400 x 2048 14.6 -> 13.8; NVFP4 4096 x 4096 20.1 ->
@@ -1449,12 +1418,57 @@ bool launch_block(GemmArgs a, int* status, hipStream_t stream) {
 // weights are behind on 256 tiles at 33 rows (4096 x 6144 14.9 / 16.0) and tie from 320, and NVFP4 gains nothing; 4096 x 14336
 // ties and 14336 x 4096 is behind (fp8 at 64 rows 22.5 / 28.6).
 template <int F>
-bool block_wanted(int M, int n_tiles, int64_t K, int tuned) {
-  if (M > 64) return true;
-  if (M <= 32 || tuned >= 0 || n_tiles < 128 || K < 2048 || K > 6144) return false;
+bool block_wanted(int M, int n_tiles, int64_t K) {
+  if (M <= 32 || n_tiles < 128 || K < 2048 || K > 6144) return false;
   if (F == LX_W_BF16) return n_tiles <= 400 && K >= 3072;
   if (F == LX_W_NVFP4) return M > 48 && n_tiles <= 256 && K >= 3072;
   return n_tiles <= (M > 48 ? 400 : 192);
+}
+
+// How the block kernel takes a call of a.M bf16 rows (mode -1: it does not). More rows than a decode step has: all of them in
+// one launch, each weight read and decoded once per 64 or 128 rows: with the passes of 64 rows below, 14336 x 4096 fp8 at 128 /
+// 256 / 1024 / 4096 rows took 42 / 84 / 334 / 1450 us. Where the product has too few blocks for the device, one slice of K a
+// workgroup, `buffer` (the stream's partial-tile buffer) permitting.
+template <int F, int MATH>
+block::Plan block_plan(const GemmArgs& a, int units, bool buffer) {
+  constexpr block::Plan kNone = {-1, 0, 0, 0};
+  const int n_tiles = (a.N + kTileRows - 1) / kTileRows;
+  if (a.M <= 64 && (MATH != LX_MATH_BF16 || !block_wanted<F>(a.M, n_tiles, a.K))) return kNone;
+  const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave, mts = (a.M + 15) / 16;
+  const bool partial = buffer && slices > 1 && static_cast<size_t>(slices) * n_tiles * mts * kWave * 16 <= kSlabScratchBytes;
+  if (a.M <= 64 && !partial) return kNone;  // few blocks and no way to share them out: the kernels for up to 64 rows are ahead
+  return block::plan<F, MATH>(a, units, partial);
+}
+
+// The block kernel (gemm_block.h) as the plan says. Slices that went to a workgroup each are added by the slab kernel's second half.
+template <int F, int MATH>
+int launch_block(GemmArgs a, const block::Plan& p, void* partial, hipStream_t stream) {
+  a.partial = p.mode == block::kPart ? partial : nullptr;
+  int st;
+  if constexpr (MATH == LX_MATH_INT8) st = launch_block_int8_math(a, p, stream);
+  else if constexpr (MATH == LX_MATH_FP8) st = launch_block_fp8_math(a, p, stream);
+  else if constexpr (F == LX_W_BF16) st = launch_block_bf16(a, p, stream);
+  else if constexpr (F == LX_W_INT8) st = launch_block_int8(a, p, stream);
+  else if constexpr (F == LX_W_FP8) st = launch_block_fp8(a, p, stream);
+  else st = launch_block_nvfp4(a, p, stream);
+  if (st || p.mode != block::kPart) return st;
+  a.S = (p.tiles + p.slice_tiles - 1) / p.slice_tiles;
+  const int mts = (a.M + 15) / 16;
+  const int64_t vectors = static_cast<int64_t>((a.N + kTileRows - 1) / kTileRows) * mts * kWave;
+  hipLaunchKernelGGL((slab_reduce_kernel<F, MATH>), dim3(static_cast<unsigned>((vectors + 255) / 256)), dim3(256), 0, stream, a, mts);
+  return status_of(hipGetLastError());
+}
+
+// The weight rows' bytes, load steps and K split.
+template <int F>
+void cut_rows(GemmArgs& a) {
+  a.row_bytes = row_bytes<F>(a.K);
+  a.scale_row_bytes = F == LX_W_NVFP4 ? a.K / 16 : 0;
+  a.chunks = static_cast<int>(a.row_bytes / 16);
+  a.steps = load_steps_for<F>(a.K);
+  a.S = split_for_shape<F>(a.K, a.N);
+  // Slices are whole weight batches (the row's last one may be cut short by the row's end).
+  a.steps_per_wave = ((a.steps + a.S - 1) / a.S + kLoadsInFlight - 1) / kLoadsInFlight * kLoadsInFlight;
 }
 
 template <int F>
@@ -1469,21 +1483,14 @@ int launch_format(GemmArgs a, const char* x0, char* y0, int M, int x_esize, int 
                        a.xs.dtype == LX_F32 ? 1 : 0);
     return status_of(hipGetLastError());
   }
-  a.row_bytes = rb;
-  a.scale_row_bytes = F == LX_W_NVFP4 ? a.K / 16 : 0;
-  a.chunks = static_cast<int>(rb / 16);
-  a.steps = load_steps_for<F>(a.K);
-  int S = split_for_shape<F>(a.K, a.N);
-  // Slices are whole weight batches (the row's last one may be cut short by the row's end).
-  a.steps_per_wave = ((a.steps + S - 1) / S + kLoadsInFlight - 1) / kLoadsInFlight * kLoadsInFlight;
-  a.S = S;
-  if (a.xs.dtype == LX_BF16 &&
-      block_wanted<F>(M, (a.N + kTileRows - 1) / kTileRows, a.K, M > 64 ? -1 : tuned_variant(gemm_key<F>(), M, a.N, a.K))) {
+  cut_rows<F>(a);
+  if (a.xs.dtype == LX_BF16 && (M > 64 || tuned_variant(gemm_key<F>(), M, a.N, a.K) < 0)) {
     a.M = M;
     a.xs.x = x0;
     a.y = y0;
-    int st = kOk;
-    if (launch_block<F, LX_MATH_BF16>(a, &st, stream)) return st;
+    void* const partial = slab_scratch(stream, 0);
+    const block::Plan p = block_plan<F, LX_MATH_BF16>(a, compute_units(), partial != nullptr);
+    if (p.mode >= 0) return launch_block<F, LX_MATH_BF16>(a, p, partial, stream);
   }
   const float* const act_scale0 = a.act_scale;
   // Up to 64 activation rows a pass; every pass is the same arithmetic per row.
@@ -1611,11 +1618,8 @@ int gemm_bytes_math(const void* x, int x_dtype, int64_t ld_x, const lx_weight& w
     hipLaunchKernelGGL(gemm_bytes_plain_kernel<MATH>, dim3(static_cast<unsigned>((N + 3) / 4)), dim3(256), 0, s, a);
     st = status_of(hipGetLastError());
   } else if (!st) {
-    a.chunks = K / 16;
-    a.steps = load_steps_for<F>(K);
-    const int S = split_for_shape<F>(K, N);
-    a.S = S;
-    a.steps_per_wave = ((a.steps + S - 1) / S + kLoadsInFlight - 1) / kLoadsInFlight * kLoadsInFlight;
+    cut_rows<F>(a);
+    const int S = a.S;
     const unsigned n_tiles = static_cast<unsigned>((N + kTileRows - 1) / kTileRows);
     bool done = false;
     if (M > 64) {
@@ -1623,7 +1627,9 @@ int gemm_bytes_math(const void* x, int x_dtype, int64_t ld_x, const lx_weight& w
       a.xq = q;
       a.xscale = scales;
       a.y = y;
-      done = launch_block<F, MATH>(a, &st, s);
+      void* const partial = slab_scratch(s, 0);
+      const block::Plan p = block_plan<F, MATH>(a, compute_units(), partial != nullptr);
+      if ((done = p.mode >= 0)) st = launch_block<F, MATH>(a, p, partial, s);
     }
     for (int m0 = done ? M : 0; m0 < M && !st; m0 += 64) {
       a.M = M - m0 < 64 ? M - m0 : 64;
@@ -1745,6 +1751,35 @@ int slab_release(hipStream_t stream) {
 using namespace dro;
 
 extern "C" {
+
+// How lx_gemm_w's block kernel takes a call on bf16 rows that lie as its vector paths want them, on a device of `units` compute
+// units (0: the current device) and a stream with or without a partial-tile buffer, the variant table aside: 4 * mode + shape
+// (gemm_block_plan.h), or -1 where the kernels for up to 64 rows take it. For tests of the rule: nothing is launched, and with
+// `units` given no device is needed.
+LX_API int dromos_plan_gemm(int format, int math, int M, int N, int K, int units, int buffer) {
+  if (units <= 0) units = compute_units();
+  auto ask = [&](auto f, auto m) {
+    GemmArgs a{};
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.xs.ld = K;
+    cut_rows<f()>(a);
+    const block::Plan p = block_plan<f(), m()>(a, units, buffer != 0);
+    return p.mode < 0 ? -1 : 4 * p.mode + p.shape;
+  };
+  constexpr std::integral_constant<int, LX_MATH_BF16> bf16{};
+  switch (format) {
+    case LX_W_BF16: return ask(std::integral_constant<int, LX_W_BF16>{}, bf16);
+    case LX_W_INT8:
+      if (math == LX_MATH_INT8) return ask(std::integral_constant<int, LX_W_INT8>{}, std::integral_constant<int, LX_MATH_INT8>{});
+      return ask(std::integral_constant<int, LX_W_INT8>{}, bf16);
+    case LX_W_FP8:
+      if (math == LX_MATH_FP8) return ask(std::integral_constant<int, LX_W_FP8>{}, std::integral_constant<int, LX_MATH_FP8>{});
+      return ask(std::integral_constant<int, LX_W_FP8>{}, bf16);
+    default: return ask(std::integral_constant<int, LX_W_NVFP4>{}, bf16);
+  }
+}
 
 int lx_gemv_w(const void* x, lx_dtype x_dtype, int ld_x, const lx_weight* w, const void* bias, lx_dtype bias_dtype, void* y,
               lx_dtype y_dtype, int ld_y, int M, int N, int K, float alpha, float beta, void* stream) {

@@ -64,13 +64,16 @@ bool launch_walk_int8(const GemmArgs& a, int W, int* status, hipStream_t stream)
 bool launch_walk_fp8(const GemmArgs& a, int W, int* status, hipStream_t stream);
 bool launch_walk_nvfp4(const GemmArgs& a, int W, int* status, hipStream_t stream);
 
-// gemm_block_<format>.hip: the block kernel (gemm_block.h) for any number of bf16 activation rows, gemm_block_<format>_math.hip the same under the
-// INT8 and FP8 maths; false when it does not apply to the call, otherwise *status holds the launch's status.
-bool launch_block_bf16(const GemmArgs& a, int* status, hipStream_t stream);
-bool launch_block_int8(const GemmArgs& a, int* status, hipStream_t stream);
-bool launch_block_fp8(const GemmArgs& a, int* status, hipStream_t stream);
-bool launch_block_nvfp4(const GemmArgs& a, int* status, hipStream_t stream);
-bool launch_block_int8_math(const GemmArgs& a, int* status, hipStream_t stream);
-bool launch_block_fp8_math(const GemmArgs& a, int* status, hipStream_t stream);
+// gemm_block_<format>.hip: the block kernel (gemm_block.h) for any number of bf16 activation rows, gemm_block_<format>_math.hip the
+// same under the INT8 and FP8 maths, as the plan says (gemm_block_plan.h). Returns the launch's status.
+namespace block {
+struct Plan;
+}
+int launch_block_bf16(const GemmArgs& a, const block::Plan& p, hipStream_t stream);
+int launch_block_int8(const GemmArgs& a, const block::Plan& p, hipStream_t stream);
+int launch_block_fp8(const GemmArgs& a, const block::Plan& p, hipStream_t stream);
+int launch_block_nvfp4(const GemmArgs& a, const block::Plan& p, hipStream_t stream);
+int launch_block_int8_math(const GemmArgs& a, const block::Plan& p, hipStream_t stream);
+int launch_block_fp8_math(const GemmArgs& a, const block::Plan& p, hipStream_t stream);
 
 }  // namespace dro

@@ -2,14 +2,10 @@
 #pragma once
 
 #include "block_mfma.h"
-#include "gemm_args.h"
+#include "gemm_block_plan.h"
 
 namespace dro {
 namespace block {
-
-// What a workgroup does with the slices of its rows: there is one; their sums are added in registers; or it takes one of
-// them (blockIdx.y) and leaves its sums in a.partial, as the slab kernel does, for slab_reduce_kernel.
-enum Slices { kOne, kAdded, kPart };
 
 template <int F, int MATH, int WM, int WN, int MT, int NT, int MODE>
 __global__ void __launch_bounds__(WM* WN* kWave) __attribute__((amdgpu_waves_per_eu(2))) gemm_block_kernel(const GemmArgs a, int tiles, int slice_tiles) {
@@ -97,70 +93,24 @@ int launch_mode(const GemmArgs& a, int tiles, int slice_tiles, hipStream_t strea
   return status_of(hipGetLastError());
 }
 
-// The block shapes and what they were measured to take (us for 64 K tiles when every compute unit has n of them:
-// per_block * n + once; MI355X, K = 4096 / 11008, 65 .. 4096 rows): small blocks leave no unit idle, large ones read less.
-struct Shape {
-  int bm, bn;
-  float per_block, once;
-};
-template <int F, int MATH>
-constexpr Shape shape(int i) {
-  constexpr Shape bf16_math[4] = {{64, 64, 11, 10}, {64, 128, 20, 8}, {128, 128, 37, 2}, {128, 256, 74, 8}};
-  constexpr Shape nvfp4[4] = {{64, 64, 17, 2}, {64, 128, 27, 6}, {128, 128, 50, 1}, {128, 256, 82, 2}};
-  constexpr Shape int8_math[4] = {{64, 64, 14, 24}, {64, 128, 24, 22}, {128, 128, 45, 8}, {128, 256, 80, 10}};
-  constexpr Shape fp8_math[4] = {{64, 64, 15, 28}, {64, 128, 28, 30}, {128, 128, 62, 2}, {128, 256, 106, 40}};
-  return MATH == LX_MATH_INT8 ? int8_math[i] : MATH == LX_MATH_FP8 ? fp8_math[i] : F == LX_W_NVFP4 ? nvfp4[i] : bf16_math[i];
-}
-
-// The shape that is estimated to take least for `slices` launches of `tiles` K tiles a block, and that time.
-template <int F, int MATH>
-int best_shape(const GemmArgs& a, int tiles, int slices, float* us) {
-  int best = 0;
-  for (int i = 0; i < 4; ++i) {
-    const Shape s = shape<F, MATH>(i);
-    const int64_t blocks = static_cast<int64_t>((a.M + s.bm - 1) / s.bm) * ((a.N + s.bn - 1) / s.bn) * slices;
-    const int64_t a_unit = (blocks + compute_units() - 1) / compute_units();
-    const float t = (s.per_block * a_unit + s.once) * tiles * (1.0f / 64);
-    if (i == 0 || t < *us) {
-      best = i;
-      *us = t;
-    }
-  }
-  return best;
-}
-
 template <int F, int MATH, int MODE>
-int launch_shape(int i, const GemmArgs& a, int tiles, int slice_tiles, hipStream_t stream) {
-  switch (i) {
-    case 0: return launch_mode<F, MATH, 2, 2, 2, 2, MODE>(a, tiles, slice_tiles, stream);
-    case 1: return launch_mode<F, MATH, 2, 2, 2, 4, MODE>(a, tiles, slice_tiles, stream);
-    case 2: return launch_mode<F, MATH, 2, 4, 4, 2, MODE>(a, tiles, slice_tiles, stream);
-    default: return launch_mode<F, MATH, 2, 4, 4, 4, MODE>(a, tiles, slice_tiles, stream);
+int launch_shape(const GemmArgs& a, const Plan& p, hipStream_t stream) {
+  switch (p.shape) {
+    case 0: return launch_mode<F, MATH, 2, 2, 2, 2, MODE>(a, p.tiles, p.slice_tiles, stream);
+    case 1: return launch_mode<F, MATH, 2, 2, 2, 4, MODE>(a, p.tiles, p.slice_tiles, stream);
+    case 2: return launch_mode<F, MATH, 2, 4, 4, 2, MODE>(a, p.tiles, p.slice_tiles, stream);
+    default:
+      if constexpr (kShapes<F, MATH> > 3) return launch_mode<F, MATH, 2, 4, 4, 4, MODE>(a, p.tiles, p.slice_tiles, stream);
+      else return kNotSupported;
   }
 }
 
 template <int F, int MATH>
-bool launch_format(const GemmArgs& a, int* status, hipStream_t stream) {
-  constexpr bool kBytes = MATH != LX_MATH_BF16;
-  // Load steps a K tile holds (NVFP4: two tiles a step).
-  constexpr int kSteps = kBytes || F == LX_W_BF16 ? 2 : 1, kTilesPerStep = F == LX_W_NVFP4 ? 2 : 1;
-  // Offsets inside a block are 32 bits; a slice is whole pairs of tiles.
-  if (a.row_bytes * 256 >= (1ll << 31) || (!kBytes && a.xs.ld * 2 * 256 >= (1ll << 31)) || a.steps_per_wave % (2 * kSteps)) return false;
-  const int tiles = ((a.steps * kTilesPerStep + kSteps - 1) / kSteps + 1) / 2 * 2;
-  const int slice_tiles = a.steps_per_wave * kTilesPerStep / kSteps, slices = (tiles + slice_tiles - 1) / slice_tiles;
-  float us = 0.0f, us_part = 0.0f;
-  const int whole = best_shape<F, MATH>(a, tiles, 1, &us);
-  if (a.partial) {
-    // One slice a workgroup: a second launch, and every slice's sums written and read once more (4.5 us and about 4 TB/s).
-    const int part = best_shape<F, MATH>(a, slice_tiles, slices, &us_part);
-    us_part += 4.5f + 8e-6f * a.M * a.N * slices / 4.0f;
-    if (us_part >= us) return false;
-    *status = launch_shape<F, MATH, kPart>(part, a, tiles, slice_tiles, stream);
-    return true;
-  }
-  *status = MATH != LX_MATH_INT8 && slices > 1 ? launch_shape<F, MATH, MATH != LX_MATH_INT8 ? kAdded : kOne>(whole, a, tiles, slice_tiles, stream)
-                                               : launch_shape<F, MATH, kOne>(whole, a, tiles, slice_tiles, stream);
-  return true;
+int launch_format(const GemmArgs& a, const Plan& p, hipStream_t stream) {
+  if (p.mode == kPart) return launch_shape<F, MATH, kPart>(a, p, stream);
+  if constexpr (MATH != LX_MATH_INT8)  // (int32 sums need no slices)
+    if (p.mode == kAdded) return launch_shape<F, MATH, kAdded>(a, p, stream);
+  return launch_shape<F, MATH, kOne>(a, p, stream);
 }
 
 }  // namespace block

@@ -1,0 +1,77 @@
+// How the block kernel (gemm_block.h) takes a call: its block shape and what a workgroup does with a row's slices. Host code
+// only, a function of the sizes and the device's compute units, so that it can be asked without launching anything.
+#pragma once
+
+#include "gemm_args.h"
+
+namespace dro {
+namespace block {
+
+// What a workgroup does with the slices of its rows: there is one; their sums are added in registers; or it takes one of
+// them (blockIdx.y) and leaves its sums in a.partial, as the slab kernel does, for slab_reduce_kernel.
+enum Slices { kOne, kAdded, kPart };
+
+// The block shapes and what they were measured to take (us for 64 K tiles when every compute unit has n of them:
+// per_block * n + once; MI355X, K = 4096 / 11008, 65 .. 4096 rows): small blocks leave no unit idle, large ones read less.
+// bf16 and one-byte weights under the BF16 math have no 128 x 256: it takes twice a 128 x 128 block's time (74 n + 8), and a
+// product never has more than twice as many of the smaller.
+struct Shape {
+  int bm, bn;
+  float per_block, once;
+};
+template <int F, int MATH>
+constexpr int kShapes = MATH == LX_MATH_BF16 && F != LX_W_NVFP4 ? 3 : 4;
+template <int F, int MATH>
+constexpr Shape shape(int i) {
+  constexpr Shape bf16_math[4] = {{64, 64, 11, 10}, {64, 128, 20, 8}, {128, 128, 37, 2}, {}};
+  constexpr Shape nvfp4[4] = {{64, 64, 17, 2}, {64, 128, 27, 6}, {128, 128, 50, 1}, {128, 256, 82, 2}};
+  constexpr Shape int8_math[4] = {{64, 64, 14, 24}, {64, 128, 24, 22}, {128, 128, 45, 8}, {128, 256, 80, 10}};
+  constexpr Shape fp8_math[4] = {{64, 64, 15, 28}, {64, 128, 28, 30}, {128, 128, 62, 2}, {128, 256, 106, 40}};
+  return MATH == LX_MATH_INT8 ? int8_math[i] : MATH == LX_MATH_FP8 ? fp8_math[i] : F == LX_W_NVFP4 ? nvfp4[i] : bf16_math[i];
+}
+
+// mode: Slices, or -1 where the kernel does not apply. K tiles of a row and of a slice.
+struct Plan {
+  int mode, shape, tiles, slice_tiles;
+};
+
+// The shape that is estimated to take least for `slices` launches of `tiles` K tiles a block, and that time.
+template <int F, int MATH>
+int best_shape(const GemmArgs& a, int tiles, int slices, int units, float* us) {
+  int best = 0;
+  for (int i = 0; i < kShapes<F, MATH>; ++i) {
+    const Shape s = shape<F, MATH>(i);
+    const int64_t blocks = static_cast<int64_t>((a.M + s.bm - 1) / s.bm) * ((a.N + s.bn - 1) / s.bn) * slices;
+    const int64_t a_unit = (blocks + units - 1) / units;
+    const float t = (s.per_block * a_unit + s.once) * tiles * (1.0f / 64);
+    if (i == 0 || t < *us) {
+      best = i;
+      *us = t;
+    }
+  }
+  return best;
+}
+
+// partial: there is a buffer for the slices' sums.
+template <int F, int MATH>
+Plan plan(const GemmArgs& a, int units, bool partial) {
+  constexpr bool kBytes = MATH != LX_MATH_BF16;
+  // Load steps a K tile holds (NVFP4: two tiles a step).
+  constexpr int kSteps = kBytes || F == LX_W_BF16 ? 2 : 1, kTilesPerStep = F == LX_W_NVFP4 ? 2 : 1;
+  // Offsets inside a block are 32 bits; a slice is whole pairs of tiles.
+  if (a.row_bytes * 256 >= (1ll << 31) || (!kBytes && a.xs.ld * 2 * 256 >= (1ll << 31)) || a.steps_per_wave % (2 * kSteps)) return {-1, 0, 0, 0};
+  const int tiles = ((a.steps * kTilesPerStep + kSteps - 1) / kSteps + 1) / 2 * 2;
+  const int slice_tiles = a.steps_per_wave * kTilesPerStep / kSteps, slices = (tiles + slice_tiles - 1) / slice_tiles;
+  float us = 0.0f, us_part = 0.0f;
+  const int whole = best_shape<F, MATH>(a, tiles, 1, units, &us);
+  if (partial && slices > 1) {
+    // One slice a workgroup: a second launch, and every slice's sums written and read once more (4.5 us and about 4 TB/s).
+    const int part = best_shape<F, MATH>(a, slice_tiles, slices, units, &us_part);
+    us_part += 4.5f + 8e-6f * a.M * a.N * slices / 4.0f;
+    if (us_part < us) return {kPart, part, tiles, slice_tiles};
+  }
+  return {MATH != LX_MATH_INT8 && slices > 1 ? kAdded : kOne, whole, tiles, slice_tiles};
+}
+
+}  // namespace block
+}  // namespace dro

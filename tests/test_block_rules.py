@@ -25,3 +25,20 @@ def lib():
     ("nvfp4", 4096, 14336, 12, 2, 1536, 1), ("fp8", 4096, 1536, 1, 1, 2048, 1)])
 def test_experts(lib, fmt, L, I, E, top_k, T, taken):
     assert lib.dromos_plan_experts(FORMATS[fmt], T, L, I, E, top_k, UNITS) == taken
+
+
+# lx_gemm_w: 4 * mode + shape, or -1 for the kernels for up to 64 rows.
+@pytest.mark.parametrize("fmt,math,M,N,K,buffer,taken", [
+    ("fp8", 0, 32, 4096, 4096, 1, False), ("fp8", 0, 64, 4096, 4096, 1, True), ("fp8", 0, 64, 4096, 4096, 0, False), ("fp8", 0, 48, 4096, 4096, 1, False),
+    ("fp8", 0, 48, 3072, 3072, 1, True), ("fp8", 0, 64, 14336, 4096, 1, False), ("fp8", 0, 64, 4096, 14336, 1, False), ("fp8", 0, 64, 1024, 4096, 1, False),
+    ("bf16", 0, 33, 5120, 5120, 1, True), ("bf16", 0, 64, 4096, 2048, 1, False), ("nvfp4", 0, 48, 4096, 4096, 1, False), ("nvfp4", 0, 49, 4096, 4096, 1, True),
+    ("nvfp4", 0, 64, 5120, 5120, 1, False), ("int8", 1, 64, 4096, 4096, 1, False), ("int8", 1, 65, 4096, 4096, 0, True), ("fp8", 2, 65, 300, 512, 1, True),
+    ("bf16", 0, 65, 300, 40, 0, True), ("nvfp4", 3, 4096, 14336, 4096, 1, True)])
+def test_gemm(lib, fmt, math, M, N, K, buffer, taken):
+    assert (lib.dromos_plan_gemm(FORMATS[fmt], math, M, N, K, UNITS, buffer) >= 0) == taken
+
+
+def test_sums_of_slices_that_do_not_fit_the_buffer_stay_in_the_workgroup(lib):
+    part = lambda M: lib.dromos_plan_gemm(FORMATS["fp8"], 0, M, 1024, 14336, UNITS, 1) // 4 == 2
+    assert part(128) and not lib.dromos_plan_gemm(FORMATS["fp8"], 0, 128, 1024, 14336, UNITS, 0) // 4 == 2
+    assert not part(8192)

@@ -21,6 +21,61 @@ def chunks_of_32(hip, x, w, math, y, **kw):
     return torch.cat([ops.gemm_w(hip, x[m : m + 32].contiguous(), w, math, y=y[m : m + 32].clone(), **kw) for m in range(0, x.shape[0], 32)])
 
 
+def on_a_stream(hip, buffer, x, w, math, y):
+    """lx_gemm_w on a stream of the library's with or without its partial-tile buffer."""
+    stream, struct = ctypes.c_void_p(), w.lx()
+    (M, K), N = x.shape, y.shape[1]
+    ws = torch.empty(max(256, int(hip.size("gemm_workspace_bytes", M, K, math))), dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    assert hip.lib.lx_rt_stream_create(ctypes.byref(stream)) == 0
+    assert buffer or hip.lib.lx_rt_stream_release(stream) == 0
+    try:
+        assert hip.status("gemm_w", x, DTYPE[x.dtype], x.shape[1], ctypes.pointer(struct), math, None, F32, y, DTYPE[y.dtype], y.shape[1], M, N, K, 1.0,
+                          0.0, ws, stream.value) == 0
+        assert hip.lib.lx_rt_stream_sync(stream) == 0
+    finally:
+        assert hip.lib.lx_rt_stream_destroy(stream) == 0
+    return y
+
+
+# Every block shape in every mode that the rule takes it in ("one slice a row", "added" in registers, "part": a slice a workgroup),
+# each near the smallest product that it is taken for.
+PLANS = ["one", "added", "part"]
+SHAPES = ["64x64", "64x128", "128x128", "128x256"]
+COVER = [("bf16", MATH_BF16, "one", "64x64", 66, 131, 224), ("bf16", MATH_BF16, "one", "64x128", 1605, 598, 224), ("bf16", MATH_BF16, "one", "128x128", 2312, 849, 256),
+         ("bf16", MATH_BF16, "added", "64x64", 66, 129, 520), ("bf16", MATH_BF16, "added", "64x128", 1605, 598, 512), ("bf16", MATH_BF16, "added", "128x128", 2312, 849, 1064),
+         ("bf16", MATH_BF16, "part", "64x64", 67, 139, 1184), ("bf16", MATH_BF16, "part", "64x128", 520, 132, 2336), ("bf16", MATH_BF16, "part", "128x128", 1097, 134, 2368),
+         ("int8", MATH_BF16, "one", "64x64", 76, 139, 512), ("int8", MATH_BF16, "one", "64x128", 2086, 454, 512), ("int8", MATH_BF16, "one", "128x128", 2559, 806, 512),
+         ("int8", MATH_BF16, "added", "64x64", 68, 131, 544), ("int8", MATH_BF16, "added", "64x128", 2368, 422, 544), ("int8", MATH_BF16, "added", "128x128", 2547, 789, 544),
+         ("int8", MATH_BF16, "part", "64x64", 75, 130, 1344), ("int8", MATH_BF16, "part", "64x128", 782, 201, 2144), ("int8", MATH_BF16, "part", "128x128", 611, 513, 2592),
+         ("fp8", MATH_BF16, "one", "64x64", 77, 131, 512), ("fp8", MATH_BF16, "one", "64x128", 2120, 470, 512), ("fp8", MATH_BF16, "one", "128x128", 2055, 1009, 512),
+         ("fp8", MATH_BF16, "added", "64x64", 68, 136, 544), ("fp8", MATH_BF16, "added", "64x128", 2719, 330, 544), ("fp8", MATH_BF16, "added", "128x128", 1703, 1156, 544),
+         ("fp8", MATH_BF16, "part", "64x64", 76, 133, 1312), ("fp8", MATH_BF16, "part", "64x128", 1124, 131, 2080), ("fp8", MATH_BF16, "part", "128x128", 901, 350, 2592),
+         ("nvfp4", MATH_BF16, "one", "64x64", 68, 134, 512), ("nvfp4", MATH_BF16, "one", "64x128", 1843, 520, 512), ("nvfp4", MATH_BF16, "one", "128x128", 3014, 643, 512),
+         ("nvfp4", MATH_FP4, "one", "128x256", 1719, 2384, 512), ("nvfp4", MATH_BF16, "added", "64x64", 129, 257, 1056),
+         ("nvfp4", MATH_FP8, "added", "64x128", 1129, 897, 1056), ("nvfp4", MATH_BF16, "added", "128x128", 2181, 905, 1056),
+         ("nvfp4", MATH_BF16, "added", "128x256", 1667, 2413, 1088), ("nvfp4", MATH_BF16, "part", "64x64", 95, 130, 2048), ("nvfp4", MATH_BF16, "part", "64x128", 802, 264, 3264),
+         ("nvfp4", MATH_FP4, "part", "128x128", 1603, 195, 4640), ("nvfp4", MATH_BF16, "part", "128x256", 643, 743, 7264),
+         ("int8", MATH_INT8, "one", "64x64", 68, 133, 512), ("int8", MATH_INT8, "one", "64x128", 1497, 641, 512), ("int8", MATH_INT8, "one", "128x128", 2411, 847, 512),
+         ("int8", MATH_INT8, "one", "128x256", 2404, 1702, 528), ("int8", MATH_INT8, "part", "64x64", 71, 136, 1408), ("int8", MATH_INT8, "part", "64x128", 782, 194, 2112),
+         ("int8", MATH_INT8, "part", "128x128", 1606, 195, 2368), ("int8", MATH_INT8, "part", "128x256", 2883, 130, 3648),
+         ("fp8", MATH_FP8, "one", "64x64", 85, 137, 512), ("fp8", MATH_FP8, "one", "64x128", 783, 4663, 512), ("fp8", MATH_FP8, "one", "128x128", 1311, 1548, 512),
+         ("fp8", MATH_FP8, "one", "128x256", 2255, 10704, 512), ("fp8", MATH_FP8, "added", "64x64", 73, 132, 608), ("fp8", MATH_FP8, "added", "64x128", 1073, 3631, 544),
+         ("fp8", MATH_FP8, "added", "128x128", 2065, 1001, 560), ("fp8", MATH_FP8, "added", "128x256", 2749, 8363, 576), ("fp8", MATH_FP8, "part", "64x64", 82, 130, 1376),
+         ("fp8", MATH_FP8, "part", "64x128", 777, 258, 6240), ("fp8", MATH_FP8, "part", "128x128", 773, 464, 2240)]
+
+
+@pytest.mark.parametrize("fmt,math,mode,shape,M,N,K", COVER)
+def test_every_shape_and_mode(hip, fmt, math, mode, shape, M, N, K):
+    buffer = mode == "part"
+    assert hip.lib.dromos_plan_gemm(FORMATS[fmt], math, M, N, K, 0, buffer) == 4 * PLANS.index(mode) + SHAPES.index(shape)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    w = random_weight(FORMATS[fmt], N, K, N + K).to("cuda")
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    y = torch.full((M, N), float("nan"), device="cuda")
+    assert torch.equal(on_a_stream(hip, buffer, x, w, math, y.clone()), chunks_of_32(hip, x, w, math, y))
+
+
 # Few blocks (a slice a workgroup), one block past a multiple of 64 / 128 rows and columns, an odd N, many blocks of each shape;
 # K of one slice, of slices whose last is short, of a last step and a last K tile cut short.
 @pytest.mark.parametrize("fmt,math", MATHS)
@@ -82,11 +137,15 @@ def test_experts_are_those_of_few_tokens(hip, fmt, math, T, L, I, E, top_k):
     assert torch.equal(got, torch.cat(few))
 
 
-# 33 .. 64 rows on short matrices: both ends of the rule's rows, tiles and row lengths, and a last tile and K tile cut short,
-# on a stream with a partial-tile buffer; eagerly and from a graph.
-@pytest.mark.parametrize("fmt", checks.FMT_NAMES)
-@pytest.mark.parametrize("M,N,K", [(33, 2048, 2048), (48, 3072, 4096), (49, 2040, 2080), (64, 4096, 6144), (57, 6400, 5120)])
+# 33 .. 64 rows on short matrices: both ends of the rule's rows, tiles and row lengths in every format, and a last tile and K
+# tile cut short, on a stream with a partial-tile buffer; eagerly and from a graph.
+FEW = {"bf16": [(33, 2048, 3072), (48, 3072, 4096), (57, 6400, 5120), (64, 4096, 6144)], "int8": [(33, 2048, 2048), (48, 3072, 4096), (49, 2040, 2080), (57, 6400, 5120)],
+       "fp8": [(33, 2048, 2048), (48, 3072, 6144), (49, 2040, 2080), (57, 6400, 5120)], "nvfp4": [(49, 2040, 3104), (57, 3072, 4096), (64, 4096, 6144)]}
+
+
+@pytest.mark.parametrize("fmt,M,N,K", [(f, *c) for f in checks.FMT_NAMES for c in FEW[f]])
 def test_few_rows_on_short_matrices(hip, fmt, M, N, K):
+    assert hip.lib.dromos_plan_gemm(FORMATS[fmt], MATH_BF16, M, N, K, 0, 1) >= 0
     g = torch.Generator().manual_seed(M)
     w = random_weight(FORMATS[fmt], N, K, N + K).to("cuda")
     x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
@@ -111,32 +170,16 @@ def test_few_rows_on_short_matrices(hip, fmt, M, N, K):
         assert hip.lib.lx_rt_stream_destroy(stream) == 0
 
 
-def on_library_stream(hip, x, w, math, y):
-    """lx_gemm_w on a stream with a partial-tile buffer."""
-    stream, struct = ctypes.c_void_p(), w.lx()
-    (M, K), N = x.shape, y.shape[1]
-    ws = torch.empty(max(256, int(hip.size("gemm_workspace_bytes", M, K, math))), dtype=torch.uint8, device="cuda")
-    torch.cuda.synchronize()
-    assert hip.lib.lx_rt_stream_create(ctypes.byref(stream)) == 0
-    try:
-        assert hip.status("gemm_w", x, DTYPE[x.dtype], x.shape[1], ctypes.pointer(struct), math, None, F32, y, DTYPE[y.dtype], y.shape[1], M, N, K, 1.0,
-                          0.0, ws, stream.value) == 0
-        assert hip.lib.lx_rt_stream_sync(stream) == 0
-    finally:
-        assert hip.lib.lx_rt_stream_destroy(stream) == 0
-    return y
-
-
 # An infinity among a row's last values: the tiles past the row's end (K is no multiple of 128 here) must not meet it again.
 # All slices in a workgroup, one, and one slice a workgroup; everything but the two rows keeps its bits.
 @pytest.mark.parametrize("M,N,K", [(65, 300, 1056), (130, 257, 1088), (515, 2064, 8256), (80, 1000, 4104)])
-@pytest.mark.parametrize("run", [ops.gemm_w, on_library_stream])
-def test_infinite_weights_at_the_rows_end(hip, run, M, N, K):
+@pytest.mark.parametrize("buffer", [False, True])
+def test_infinite_weights_at_the_rows_end(hip, buffer, M, N, K):
     w = random_weight(FORMATS["bf16"], N, K, N + K).to("cuda")
     x = torch.randn(M, K, generator=torch.Generator().manual_seed(K)).to(torch.bfloat16).cuda()
-    clean = run(hip, x, w, MATH_BF16, y=torch.empty(M, N, device="cuda"))
+    clean = on_a_stream(hip, buffer, x, w, MATH_BF16, torch.empty(M, N, device="cuda"))
     w.data[3, K - 1], w.data[N - 1, K - 8] = float("inf"), float("-inf")
-    got = run(hip, x, w, MATH_BF16, y=torch.empty(M, N, device="cuda"))
+    got = on_a_stream(hip, buffer, x, w, MATH_BF16, torch.empty(M, N, device="cuda"))
     assert torch.equal(got[:, 3], x[:, K - 1].float() * float("inf")) and torch.equal(got[:, N - 1], x[:, K - 8].float() * -float("inf"))
     got[:, [3, N - 1]] = clean[:, [3, N - 1]]
     assert torch.equal(got, clean)
