@@ -844,9 +844,10 @@ void* slab_scratch(hipStream_t stream, size_t bytes) {
   return it == b.of.end() ? nullptr : it->second;
 }
 
-// Which of the tile kernels' own choices the variant table fixes ("gemm_w_<format>": 4 = never the slab kernel,
-// 5 = the slab kernel wherever it fits); anything else leaves the measured rule.
-constexpr int kVariantWindow = 4, kVariantSlab = 5, kVariantWalkParts = 6, kVariantWalkSplit = 7;
+// The variants of "gemm_w_<format>" in the variant table: 0 = the tile kernels by their own rule, 1 .. 3 = walk with 1, 2, 4 tiles a
+// workgroup, 4 / 5 = the tile kernels without the slab kernel / with it wherever it fits, 6 / 7 = the walk kernel by single
+// slices / split over a workgroup, 8 = the block kernel wherever it fits. None changes a sum.
+constexpr int kVariantWindow = 4, kVariantSlab = 5, kVariantWalkParts = 6, kVariantWalkSplit = 7, kVariantBlock = 8;
 
 template <int F>
 const char* gemm_key() {
@@ -1195,14 +1196,12 @@ int launch_skinny_x(const GemmArgs& a, size_t lds, unsigned grid, unsigned threa
 // wins where a wavefront's walk is at most 16 groups of four load steps (K = 4096 of one-byte weights) and the matrix
 // has the tiles to give most compute units a workgroup: 14336 x 4096 int8 at 16 / 32 / 64 rows 16.0 / 20.7 / 29.9 ->
 // 15.2 / 18.1 / 25.4 us, 16384 x 4096 fp8 at 32 rows 21.5 -> 17.5 us, 6144 x 4096 14.2 -> 12.7 us, 4096 x 4096
-// 13.6 -> 12.7 us; on 4096 x 8192 (32 groups) and at 8 rows and fewer the tile kernels are faster. The variant table
-// ("gemm_w_<format>": 0 = the tile kernels by their own rule, 1 .. 3 = walk with 1, 2, 4 tiles a workgroup, 4 / 5 = the
-// tile kernels without / with the slab kernel) overrides; no variant changes a sum.
+// 13.6 -> 12.7 us; on 4096 x 8192 (32 groups) and at 8 rows and fewer the tile kernels are faster. The variant table overrides.
 template <int F>
 bool try_walk(const GemmArgs& a, int* status, hipStream_t stream) {
   if (a.xs.dtype != LX_BF16) return false;
   const int n_tiles = (a.N + kTileRows - 1) / kTileRows;
-  const int tuned = tuned_variant(gemm_key<F>(), a.M, a.N, a.K);
+  const int tuned = a.tuned;
   int W;
   if (tuned == 0 || tuned >= kVariantWindow) return false;
   if (tuned >= 1 && tuned <= 3) {
@@ -1354,13 +1353,13 @@ int launch_skinny(GemmArgs a, hipStream_t stream) {
   const unsigned n_tiles = static_cast<unsigned>((a.N + kTileRows - 1) / kTileRows);
   {
     int st = kOk;
-    if (walk_parts_wanted<F>(a.M, static_cast<int>(n_tiles), a.K, tuned_variant(gemm_key<F>(), a.M, a.N, a.K)) && launch_walk_parts<F>(a, &st, stream)) return st;
-    if (walk_split_wanted(a.M, static_cast<int>(n_tiles), a.K, tuned_variant(gemm_key<F>(), a.M, a.N, a.K)) && launch_walk_split<F>(a, &st, stream)) return st;
+    if (walk_parts_wanted<F>(a.M, static_cast<int>(n_tiles), a.K, a.tuned) && launch_walk_parts<F>(a, &st, stream)) return st;
+    if (walk_split_wanted(a.M, static_cast<int>(n_tiles), a.K, a.tuned) && launch_walk_split<F>(a, &st, stream)) return st;
     if (try_walk<F>(a, &st, stream)) return st;
   }
   // More than eight rows: the windowed kernel (for 9 .. 16 rows where the matrix has the tiles to fill its
   // sixteen-wavefront workgroups; the lean kernel's image of all of K leaves too few of them resident there).
-  const int tuned = tuned_variant(gemm_key<F>(), a.M, a.N, a.K);
+  const int tuned = a.tuned;
   if (MT > 1 || (a.M > 8 && n_tiles >= 320) || tuned == kVariantWindow || tuned == kVariantSlab) {
     int st = kOk;
     if (slab_wanted(a.M, static_cast<int>(n_tiles), a.K, tuned) && launch_slab<F, LX_MATH_BF16>(a, &st, stream)) return st;
@@ -1428,15 +1427,19 @@ bool block_wanted(int M, int n_tiles, int64_t K) {
 // How the block kernel takes a call of a.M bf16 rows (mode -1: it does not). More rows than a decode step has: all of them in
 // one launch, each weight read and decoded once per 64 or 128 rows: with the passes of 64 rows below, 14336 x 4096 fp8 at 128 /
 // 256 / 1024 / 4096 rows took 42 / 84 / 334 / 1450 us. Where the product has too few blocks for the device, one slice of K a
-// workgroup, `buffer` (the stream's partial-tile buffer) permitting.
+// workgroup, `buffer` (the stream's partial-tile buffer) permitting. tuned: the variant table's entry for the call's own
+// row count: another family's keeps the call from the block kernel (more than 64 rows go to it in passes), "block" asks for it at
+// any row count.
 template <int F, int MATH>
-block::Plan block_plan(const GemmArgs& a, int units, bool buffer) {
+block::Plan block_plan(const GemmArgs& a, int tuned, int units, bool buffer) {
   constexpr block::Plan kNone = {-1, 0, 0, 0};
+  const bool forced = tuned == kVariantBlock;
+  if (tuned >= 0 && !forced) return kNone;
   const int n_tiles = (a.N + kTileRows - 1) / kTileRows;
-  if (a.M <= 64 && (MATH != LX_MATH_BF16 || !block_wanted<F>(a.M, n_tiles, a.K))) return kNone;
+  if (!forced && a.M <= 64 && (MATH != LX_MATH_BF16 || !block_wanted<F>(a.M, n_tiles, a.K))) return kNone;
   const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave, mts = (a.M + 15) / 16;
   const bool partial = buffer && slices > 1 && static_cast<size_t>(slices) * n_tiles * mts * kWave * 16 <= kSlabScratchBytes;
-  if (a.M <= 64 && !partial) return kNone;  // few blocks and no way to share them out: the kernels for up to 64 rows are ahead
+  if (!forced && a.M <= 64 && !partial) return kNone;  // few blocks and no way to share them out: the kernels for up to 64 rows are ahead
   return block::plan<F, MATH>(a, units, partial);
 }
 
@@ -1457,6 +1460,14 @@ int launch_block(GemmArgs a, const block::Plan& p, void* partial, hipStream_t st
   const int64_t vectors = static_cast<int64_t>((a.N + kTileRows - 1) / kTileRows) * mts * kWave;
   hipLaunchKernelGGL((slab_reduce_kernel<F, MATH>), dim3(static_cast<unsigned>((vectors + 255) / 256)), dim3(256), 0, stream, a, mts);
   return status_of(hipGetLastError());
+}
+
+// The variant for a pass of a.M of a call's M rows: the call's own entry, else (M > 64) the one for the pass's row count. (The block
+// kernel takes a whole call or none of it.)
+template <int F>
+int pass_variant(int tuned, int M, const GemmArgs& a) {
+  if (tuned < 0 && M > 64) tuned = tuned_variant(gemm_key<F>(), a.M, a.N, a.K);
+  return tuned == kVariantBlock ? -1 : tuned;
 }
 
 // The weight rows' bytes, load steps and K split.
@@ -1484,18 +1495,20 @@ int launch_format(GemmArgs a, const char* x0, char* y0, int M, int x_esize, int 
     return status_of(hipGetLastError());
   }
   cut_rows<F>(a);
-  if (a.xs.dtype == LX_BF16 && (M > 64 || tuned_variant(gemm_key<F>(), M, a.N, a.K) < 0)) {
+  const int tuned = tuned_variant(gemm_key<F>(), M, a.N, a.K);
+  if (a.xs.dtype == LX_BF16) {
     a.M = M;
     a.xs.x = x0;
     a.y = y0;
     void* const partial = slab_scratch(stream, 0);
-    const block::Plan p = block_plan<F, LX_MATH_BF16>(a, compute_units(), partial != nullptr);
+    const block::Plan p = block_plan<F, LX_MATH_BF16>(a, tuned, compute_units(), partial != nullptr);
     if (p.mode >= 0) return launch_block<F, LX_MATH_BF16>(a, p, partial, stream);
   }
   const float* const act_scale0 = a.act_scale;
   // Up to 64 activation rows a pass; every pass is the same arithmetic per row.
   for (int m0 = 0; m0 < M; m0 += 64) {
     a.M = M - m0 < 64 ? M - m0 : 64;
+    a.tuned = pass_variant<F>(tuned, M, a);
     a.xs.x = x0 + static_cast<int64_t>(m0) * a.xs.ld * x_esize;
     a.y = y0 + static_cast<int64_t>(m0) * a.ld_y * y_esize;
     if (act_scale0) a.act_scale = act_scale0 + m0;
@@ -1621,16 +1634,15 @@ int gemm_bytes_math(const void* x, int x_dtype, int64_t ld_x, const lx_weight& w
     cut_rows<F>(a);
     const int S = a.S;
     const unsigned n_tiles = static_cast<unsigned>((N + kTileRows - 1) / kTileRows);
-    bool done = false;
-    if (M > 64) {
-      a.M = M;
-      a.xq = q;
-      a.xscale = scales;
-      a.y = y;
-      void* const partial = slab_scratch(s, 0);
-      const block::Plan p = block_plan<F, MATH>(a, compute_units(), partial != nullptr);
-      if ((done = p.mode >= 0)) st = launch_block<F, MATH>(a, p, partial, s);
-    }
+    const int tuned = tuned_variant(gemm_key<F>(), M, N, K);
+    a.M = M;
+    a.xq = q;
+    a.xscale = scales;
+    a.y = y;
+    void* const partial = slab_scratch(s, 0);
+    const block::Plan p = block_plan<F, MATH>(a, tuned, compute_units(), partial != nullptr);
+    const bool done = p.mode >= 0;
+    if (done) st = launch_block<F, MATH>(a, p, partial, s);
     for (int m0 = done ? M : 0; m0 < M && !st; m0 += 64) {
       a.M = M - m0 < 64 ? M - m0 : 64;
       a.xq = q + static_cast<int64_t>(m0) * K;
@@ -1649,7 +1661,7 @@ int gemm_bytes_math(const void* x, int x_dtype, int64_t ld_x, const lx_weight& w
         return status_of(hipGetLastError());
       };
       const int mt = (a.M + 15) / 16;
-      if ((mt > 1 || (a.M > 8 && n_tiles >= 320)) && slab_wanted(a.M, static_cast<int>(n_tiles), K, tuned_variant(gemm_key<F>(), a.M, N, K)) && launch_slab<F, MATH>(a, &st, s)) continue;
+      if ((mt > 1 || (a.M > 8 && n_tiles >= 320)) && slab_wanted(a.M, static_cast<int>(n_tiles), K, pass_variant<F>(tuned, M, a)) && launch_slab<F, MATH>(a, &st, s)) continue;
       if ((mt > 1 || (a.M > 8 && n_tiles >= 320)) && launch_window<F, MATH>(a, &st, s)) continue;
       if (mt == 1 && launch_tile16<F, MATH>(a, &st, s)) continue;
       if (mt == 1) {
@@ -1753,8 +1765,8 @@ using namespace dro;
 extern "C" {
 
 // How lx_gemm_w's block kernel takes a call on bf16 rows that lie as its vector paths want them, on a device of `units` compute
-// units (0: the current device) and a stream with or without a partial-tile buffer, the variant table aside: 4 * mode + shape
-// (gemm_block_plan.h), or -1 where the kernels for up to 64 rows take it. For tests of the rule: nothing is launched, and with
+// units (0: the current device) and a stream with or without a partial-tile buffer: 4 * mode + shape (gemm_block_plan.h), or -1
+// where the kernels for up to 64 rows take it. For tests of the rule: nothing is launched, and with
 // `units` given no device is needed.
 LX_API int dromos_plan_gemm(int format, int math, int M, int N, int K, int units, int buffer) {
   if (units <= 0) units = compute_units();
@@ -1765,7 +1777,7 @@ LX_API int dromos_plan_gemm(int format, int math, int M, int N, int K, int units
     a.K = K;
     a.xs.ld = K;
     cut_rows<f()>(a);
-    const block::Plan p = block_plan<f(), m()>(a, units, buffer != 0);
+    const block::Plan p = block_plan<f(), m()>(a, tuned_variant(gemm_key<f()>(), M, N, K), units, buffer != 0);
     return p.mode < 0 ? -1 : 4 * p.mode + p.shape;
   };
   constexpr std::integral_constant<int, LX_MATH_BF16> bf16{};

@@ -38,6 +38,7 @@ struct GemmArgs {
   int pass_begin, pass_steps, pass_continues;  // slab kernel: the part of every slice this launch takes, and whether it goes on from `partial`
   void* partial;  // slab kernel with S > 1: the slices' partial tiles, [S][tile][16 rows][lane] x 4 words (f32, or i32 for the INT8 math)
   int walk_slices;  // walk kernel with partial tiles: the slices a workgroup walks; split over a workgroup's wavefronts: the slices a wavefront walks
+  int tuned;        // the variant table's entry for the call, or -1
   int walk_split;   // walk kernel: the wavefronts of a workgroup take one tile between them (two or four of them)
 };
 

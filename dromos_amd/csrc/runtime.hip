@@ -78,19 +78,18 @@ struct Registered {
 };
 
 // The kernels with variants. The GEMV of each format has three: its K split of 1, 2 or 4 wavefronts (admitted where the
-// split is the shape's order class). The matrix-core product of each format (9 .. 64 activation rows) has four: the tile
-// kernels by their own rule, the walk kernel with 1, 2 or 4 tiles a workgroup, the tile kernels without or with the slab
-// kernel; none changes a sum, so all are admitted.
+// split is the shape's order class). The matrix-core product of each format has its kernel families (gemm.hip: kVariant...);
+// none changes a sum, so all are admitted.
 const std::map<std::string, Registered>& registry() {
   static const auto* r = new std::map<std::string, Registered>{
       {"gemv_w_bf16", {{"s1", "s2", "s4"}, LX_W_BF16}},
       {"gemv_w_int8", {{"s1", "s2", "s4"}, LX_W_INT8}},
       {"gemv_w_fp8", {{"s1", "s2", "s4"}, LX_W_FP8}},
       {"gemv_w_nvfp4", {{"s1", "s2", "s4"}, LX_W_NVFP4}},
-      {"gemm_w_bf16", {{"tiles", "walk1", "walk2", "walk4", "window", "slab", "walkparts", "walksplit"}, -1}},
-      {"gemm_w_int8", {{"tiles", "walk1", "walk2", "walk4", "window", "slab", "walkparts", "walksplit"}, -1}},
-      {"gemm_w_fp8", {{"tiles", "walk1", "walk2", "walk4", "window", "slab", "walkparts", "walksplit"}, -1}},
-      {"gemm_w_nvfp4", {{"tiles", "walk1", "walk2", "walk4", "window", "slab", "walkparts", "walksplit"}, -1}},
+      {"gemm_w_bf16", {{"tiles", "walk1", "walk2", "walk4", "window", "slab", "walkparts", "walksplit", "block"}, -1}},
+      {"gemm_w_int8", {{"tiles", "walk1", "walk2", "walk4", "window", "slab", "walkparts", "walksplit", "block"}, -1}},
+      {"gemm_w_fp8", {{"tiles", "walk1", "walk2", "walk4", "window", "slab", "walkparts", "walksplit", "block"}, -1}},
+      {"gemm_w_nvfp4", {{"tiles", "walk1", "walk2", "walk4", "window", "slab", "walkparts", "walksplit", "block"}, -1}},
   };
   return *r;
 }

@@ -42,3 +42,25 @@ def test_sums_of_slices_that_do_not_fit_the_buffer_stay_in_the_workgroup(lib):
     part = lambda M: lib.dromos_plan_gemm(FORMATS["fp8"], 0, M, 1024, 14336, UNITS, 1) // 4 == 2
     assert part(128) and not lib.dromos_plan_gemm(FORMATS["fp8"], 0, 128, 1024, 14336, UNITS, 0) // 4 == 2
     assert not part(8192)
+
+
+@pytest.mark.parametrize("fmt,math", [("bf16", 0), ("int8", 1), ("fp8", 0), ("fp8", 2), ("nvfp4", 0)])
+def test_the_variant_table_has_the_last_word(lib, fmt, math):
+    # An entry is for a row count (the next power of two) of a matrix: "block" asks for the block kernel at any count, every other
+    # family keeps the call from it, and an entry for up to 64 rows leaves calls of more rows alone.
+    key, N, K = f"gemm_w_{fmt}".encode(), 4096, 4096
+    plan = lambda M: lib.dromos_plan_gemm(FORMATS[fmt], math, M, N, K, UNITS, 1) >= 0
+    variants = lib.lx_tune_variants(key)
+    lib.lx_tune_variant_name.restype = ctypes.c_char_p
+    names = [lib.lx_tune_variant_name(key, v).decode() for v in range(variants)]
+    try:
+        assert plan(130) and not plan(20)
+        for M in (20, 64, 130):
+            for v, name in enumerate(names):
+                lib.lx_tune_clear()
+                assert lib.lx_tune_set(key, M, N, K, v) == 0
+                assert plan(M) == (name == "block"), (M, name)
+                assert M > 64 or plan(130), "an entry for fewer rows holds here"
+    finally:
+        lib.lx_tune_clear()
+    assert names[-1] == "block" and plan(130)

@@ -2,7 +2,7 @@
 tile) against float64 on the decoded values, and bit for bit against the tile kernels it replaces on the shapes it
 takes: the variant table forces each family ("gemm_w_<format>": 0 = the tile kernels, 1 .. 3 = walk with 1, 2, 4 tiles
 a workgroup, 4 / 5 = the tile kernels without / with the slab kernel, 6 = walks of single slices whose sums meet in the
-stream's partial-tile buffer, 7 = a tile's slices split over the wavefronts of a workgroup), and no variant may change an output bit, a row's bits may not depend on the batch."""
+stream's partial-tile buffer, 7 = a tile's slices split over the wavefronts of a workgroup, 8 = the block kernel), and no variant may change an output bit, a row's bits may not depend on the batch."""
 
 import pytest
 import torch
@@ -36,10 +36,10 @@ def test_variants_are_registered(hip):
     hip.lib.lx_tune_variant_name.restype = ctypes.c_char_p
     for fmt in FMT:
         key = f"gemm_w_{fmt}".encode()
-        assert hip.lib.lx_tune_variants(key) == 8
-        assert [hip.lib.lx_tune_variant_name(key, v).decode() for v in range(8)] == ["tiles", "walk1", "walk2", "walk4", "window", "slab", "walkparts", "walksplit"]
-        assert all(hip.lib.lx_tune_set(key, 32, 4096, 4096, v) == 0 for v in range(8))  # none changes a sum: all admitted
-        assert hip.lib.lx_tune_set(key, 32, 4096, 4096, 8) == 803
+        assert hip.lib.lx_tune_variants(key) == 9
+        assert [hip.lib.lx_tune_variant_name(key, v).decode() for v in range(9)] == ["tiles", "walk1", "walk2", "walk4", "window", "slab", "walkparts", "walksplit", "block"]
+        assert all(hip.lib.lx_tune_set(key, 32, 4096, 4096, v) == 0 for v in range(9))  # none changes a sum: all admitted
+        assert hip.lib.lx_tune_set(key, 32, 4096, 4096, 9) == 803
 
 
 @pytest.mark.parametrize("M", [9, 16, 17, 33, 48, 64])
@@ -53,7 +53,7 @@ def test_every_variant_gives_the_same_bits(hip, fmt, M):
         want = ops.gemv_reference(x, w.dense(), bias, 1.0, 0.0, None)
         wd, xd, bd = w.to("cuda"), x.cuda(), bias.cuda()
         outs = {}
-        for variant in (0, 1, 2, 3, 4, 5, 6, 7, None):
+        for variant in (0, 1, 2, 3, 4, 5, 6, 7, 8, None):
             force(hip, fmt, M, N, K, variant)
             y = torch.full((M, N), float("nan"), device="cuda")
             outs[variant] = ops.gemm_w(hip, xd, wd, MATH_BF16, bias=bd, y=y).clone()
@@ -80,7 +80,7 @@ def test_rows_that_are_not_whole_walks(hip, fmt, M):
         want = ops.gemv_reference(x, w.dense(), bias, 1.0, 0.0, None)
         wd, xd, bd = w.to("cuda"), x.cuda(), bias.cuda()
         outs = {}
-        for variant in (0, 1, 2, 3, 6, 7, None):
+        for variant in (0, 1, 2, 3, 6, 7, 8, None):
             force(hip, fmt, M, N, K, variant)
             y = torch.full((M, N), float("nan"), device="cuda")
             outs[variant] = ops.gemm_w(hip, xd, wd, MATH_BF16, bias=bd, y=y).clone()
