@@ -1410,18 +1410,19 @@ int launch_skinny(GemmArgs a, hipStream_t stream) {
 }
 
 // Whether 33 .. 64 rows go to the block kernel too: on short matrices the windowed and slab kernels stage all of the rows
-// once per few weight tiles, and the block kernel's slices fill the device. Measured at 64 rows (before -> after, us): fp8
-// 2048 x 2048 16.9 -> 9.7, 4096 x 4096 22.4 -> 14.9, 6144 x 5120 34.8 -> 20.8, 6400 x 2048 14.6 -> 13.8; NVFP4 4096 x 4096 20.1 ->
-// 15.6, 4096 x 6144 21.5 -> 19.8; bf16 5120 x 5120 32.5 -> 24.8, 6144 x 5120 33.2 -> 27.1. The lines: 4096 x 2048 ties or is behind
-// in bf16 (33 rows 11.5 / 12.1) and NVFP4 (64 rows 18.7 / 19.7), bf16 6400 x 2048 too (13.8 / 15.6); up to 48 rows one-byte
-// weights are behind on 256 tiles at 33 rows (4096 x 6144 14.9 / 16.0) and tie from 320, and NVFP4 gains nothing; 4096 x 14336
-// ties and 14336 x 4096 is behind (fp8 at 64 rows 22.5 / 28.6).
+// once per few weight tiles, and the block kernel's slices fill the device. Measured at 64 rows on cold weights (before ->
+// after, us): fp8 2048 x 2048 16.8 -> 10.2, 4096 x 4096 21.2 -> 15.3, 6144 x 5120 34.7 -> 20.6, 4608 x 2560 16.4 -> 14.4; NVFP4
+// 4096 x 4096 19.4 -> 14.7, 4096 x 6144 20.9 -> 20.5; bf16 4096 x 4096 20.1 -> 15.1, 6400 x 3072 24.3 -> 16.7. The lines: one-byte
+// weights of more than 288 tiles are behind below K = 3072 (fp8 6400 x 2048 13.2 / 15.3, 6400 x 2560 16.5 / 18.0; 5120 x 2048 13.0 /
+// 15.3) and tie there; up to 48 rows they are behind from 192 tiles of K = 2048, where the walk kernel starts (fp8 3072 x 2048 9.6 /
+// 10.6, 2560 x 2048 14.7 / 10.1), and beyond 192 of any K. Blocks are also ahead on some shapes outside these lines (64 to 127
+// tiles, bf16 from K = 2560 and to 448 tiles, NVFP4 from 33 rows and on 9216 x 11008: 70 / 49 us), which stay as they were.
 template <int F>
 bool block_wanted(int M, int n_tiles, int64_t K) {
   if (M <= 32 || n_tiles < 128 || K < 2048 || K > 6144) return false;
   if (F == LX_W_BF16) return n_tiles <= 400 && K >= 3072;
   if (F == LX_W_NVFP4) return M > 48 && n_tiles <= 256 && K >= 3072;
-  return n_tiles <= (M > 48 ? 400 : 192);
+  return M > 48 ? n_tiles <= (K >= 3072 ? 400 : 288) : n_tiles <= (K >= 3072 ? 192 : 191);
 }
 
 // How the block kernel takes a call of a.M bf16 rows (mode -1: it does not). More rows than a decode step has: all of them in

@@ -32,6 +32,8 @@ def test_experts(lib, fmt, L, I, E, top_k, T, taken):
 @pytest.mark.parametrize("fmt,math,M,N,K,buffer,taken", [
     ("fp8", 0, 32, 4096, 4096, 1, False), ("fp8", 0, 64, 4096, 4096, 1, True), ("fp8", 0, 64, 4096, 4096, 0, False), ("fp8", 0, 48, 4096, 4096, 1, False),
     ("fp8", 0, 48, 3072, 3072, 1, True), ("fp8", 0, 64, 14336, 4096, 1, False), ("fp8", 0, 64, 4096, 14336, 1, False), ("fp8", 0, 64, 1024, 4096, 1, False),
+    ("fp8", 0, 64, 6400, 2048, 1, False), ("int8", 0, 49, 5120, 2048, 1, False), ("fp8", 0, 64, 6400, 2560, 1, False), ("fp8", 0, 40, 3072, 2048, 1, False),
+    ("fp8", 0, 64, 4608, 2560, 1, True), ("int8", 0, 64, 4096, 2048, 1, True), ("fp8", 0, 33, 2048, 2048, 1, True), ("fp8", 0, 48, 2560, 2048, 1, True), ("fp8", 0, 64, 6400, 3072, 1, True),
     ("bf16", 0, 33, 5120, 5120, 1, True), ("bf16", 0, 64, 4096, 2048, 1, False), ("nvfp4", 0, 48, 4096, 4096, 1, False), ("nvfp4", 0, 49, 4096, 4096, 1, True),
     ("nvfp4", 0, 64, 5120, 5120, 1, False), ("int8", 1, 64, 4096, 4096, 1, False), ("int8", 1, 65, 4096, 4096, 0, True), ("fp8", 2, 65, 300, 512, 1, True),
     ("bf16", 0, 65, 300, 40, 0, True), ("nvfp4", 3, 4096, 14336, 4096, 1, True)])
