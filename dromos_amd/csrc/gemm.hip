@@ -1441,7 +1441,18 @@ block::Plan block_plan(const GemmArgs& a, int tuned, int units, bool buffer) {
   const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave, mts = (a.M + 15) / 16;
   const bool partial = buffer && slices > 1 && static_cast<size_t>(slices) * n_tiles * mts * kWave * 16 <= kSlabScratchBytes;
   if (!forced && a.M <= 64 && !partial) return kNone;  // few blocks and no way to share them out: the kernels for up to 64 rows are ahead
-  return block::plan<F, MATH>(a, units, partial);
+  const block::Plan p = block::plan<F, MATH>(a, units, partial);
+  if constexpr (F == LX_W_NVFP4) {
+    // NVFP4 blocks that walk all of a long row, a few rows past 64: a chain of K tiles a block, at 8.2 us per 1000 values, on fewer
+    // blocks than units, behind a pass of 64 rows and one of the rest. Blocks of 64 x 64, passes / blocks in us: without the partial-tile buffer
+    // 1500 x 8192 at 65 / 80 / 96 / 128 rows 44 / 67, 46 / 68, 54 / 68, 69 / 68; 4096 x 14336 85 / 118, 88 / 123, 106 / 124, 134 / 126;
+    // 1024 x 7168 at 88 rows 46 / 57; 4096 x 4096 33 / 36, 35 / 36, 42 / 36; with it 6144 x 4096 30 / 36, 33 / 36, 37 / 36. Rows of up to 3328
+    // values tie.
+    const int blocks = (a.N + 63) / 64 * 2;
+    if (!forced && p.mode == block::kAdded && a.M <= 96 && a.K >= 3584 && (a.M <= 80 ? blocks <= 192 : blocks <= (a.K > 4096 ? 128 : 100)))
+      return kNone;
+  }
+  return p;
 }
 
 // The block kernel (gemm_block.h) as the plan says. Slices that went to a workgroup each are added by the slab kernel's second half.

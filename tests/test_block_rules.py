@@ -34,7 +34,9 @@ def test_experts(lib, fmt, L, I, E, top_k, T, taken):
     ("fp8", 0, 48, 3072, 3072, 1, True), ("fp8", 0, 64, 14336, 4096, 1, False), ("fp8", 0, 64, 4096, 14336, 1, False), ("fp8", 0, 64, 1024, 4096, 1, False),
     ("fp8", 0, 64, 6400, 2048, 1, False), ("int8", 0, 49, 5120, 2048, 1, False), ("fp8", 0, 64, 6400, 2560, 1, False), ("fp8", 0, 40, 3072, 2048, 1, False),
     ("fp8", 0, 64, 4608, 2560, 1, True), ("int8", 0, 64, 4096, 2048, 1, True), ("fp8", 0, 33, 2048, 2048, 1, True), ("fp8", 0, 48, 2560, 2048, 1, True), ("fp8", 0, 64, 6400, 3072, 1, True),
-    ("bf16", 0, 33, 5120, 5120, 1, True), ("bf16", 0, 64, 4096, 2048, 1, False), ("nvfp4", 0, 48, 4096, 4096, 1, False), ("nvfp4", 0, 49, 4096, 4096, 1, True),
+    ("nvfp4", 0, 65, 1500, 8192, 0, False), ("nvfp4", 0, 96, 4096, 14336, 0, False), ("nvfp4", 3, 80, 6144, 4096, 1, False), ("nvfp4", 2, 96, 256, 4096, 0, False),
+    ("nvfp4", 0, 65, 1500, 8192, 1, True), ("nvfp4", 0, 97, 1500, 8192, 0, True), ("nvfp4", 0, 96, 4096, 4096, 0, True), ("nvfp4", 0, 65, 9216, 11008, 0, True),
+    ("nvfp4", 0, 72, 2048, 2048, 0, True), ("fp8", 0, 65, 1500, 8192, 0, True), ("bf16", 0, 33, 5120, 5120, 1, True), ("bf16", 0, 64, 4096, 2048, 1, False), ("nvfp4", 0, 48, 4096, 4096, 1, False), ("nvfp4", 0, 49, 4096, 4096, 1, True),
     ("nvfp4", 0, 64, 5120, 5120, 1, False), ("int8", 1, 64, 4096, 4096, 1, False), ("int8", 1, 65, 4096, 4096, 0, True), ("fp8", 2, 65, 300, 512, 1, True),
     ("bf16", 0, 65, 300, 40, 0, True), ("nvfp4", 3, 4096, 14336, 4096, 1, True)])
 def test_gemm(lib, fmt, math, M, N, K, buffer, taken):
