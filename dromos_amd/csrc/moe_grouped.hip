@@ -335,16 +335,16 @@ BlockCut block_cut(int64_t K, int NT, int64_t out_rows) {
 //   2048 x 1024 93 / 107). bf16 weights, which have no decode to save, from 24 (at 16 rows 173 / 196 us, at 32 254 / 204).
 // - How much of the device the blocks fill: the share of the units that have one, over both stages by their rows' lengths.
 //   Two NVFP4 experts of 4096 x 1536 at 16 rows are 24 and 32 blocks: 27.5 us by the kernels here, 95.5 by blocks.
-// Rows (48 at most) times that share from 12 on is where the blocks are ahead; bf16 56 and 14; NVFP4, whose blocks decode more a
-// row, 80 and 16. Of 1661 sweep points 10 lose 4 % or more that way (16 % at most: NVFP4 8 experts of 1024 x 2048 at 64 rows, bf16
-// 12 of 2048 x 4096 at 25 rows 13 %), and 1 % of the gain is left.
+// Rows (48 at most) times that share from 12 on is where FP8 blocks are ahead; INT8 60 and 12, bf16 56 and 14; NVFP4, whose blocks
+// decode more a row, 80 and 16. Of 1661 sweep points 11 lose 4 % or more that way (16 % at most: NVFP4 8 experts of 1024 x 2048 at
+// 64 rows, bf16 12 of 2048 x 4096 at 25 rows 13 %), and 1 % of the gain is left.
 bool blocks_wanted(int type, int64_t P, int64_t E, int64_t L, int64_t I, int units) {
   if (P < (type == LX_W_BF16 ? 24 : 16) * E) return false;
   const int64_t by_rows = (P + kBlockTokens - 1) / kBlockTokens, tiles = by_rows > E ? by_rows : E;
   const int64_t w1 = tiles * ((I + 127) / 128), w2 = tiles * ((L + 255) / 256);
   const double busy = static_cast<double>(L) * w1 + static_cast<double>(I) * w2;
   const double held = units * (static_cast<double>(L) * ((w1 + units - 1) / units) + static_cast<double>(I) * ((w2 + units - 1) / units));
-  const double rows = static_cast<double>(P) / E, most = type == LX_W_NVFP4 ? 80 : type == LX_W_BF16 ? 56 : 48;
+  const double rows = static_cast<double>(P) / E, most = type == LX_W_NVFP4 ? 80 : type == LX_W_INT8 ? 60 : type == LX_W_BF16 ? 56 : 48;
   return (rows < most ? rows : most) * busy >= (type == LX_W_NVFP4 ? 16 : type == LX_W_BF16 ? 14 : 12) * held;
 }
 

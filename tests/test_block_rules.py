@@ -20,7 +20,7 @@ def lib():
     ("nvfp4", 4096, 1536, 2, 1, 32, 0), ("bf16", 1024, 512, 2, 1, 256, 0), ("fp8", 2048, 1024, 2, 1, 256, 0),
     ("int8", 2048, 1024, 8, 2, 64, 0), ("nvfp4", 1024, 2048, 4, 2, 64, 0), ("bf16", 512, 2048, 12, 2, 540, 0),
     ("fp8", 4096, 1536, 4, 2, 128, 0), ("nvfp4", 2048, 1024, 16, 4, 96, 0), ("nvfp4", 2048, 4096, 12, 2, 150, 0),
-    ("bf16", 1024, 2048, 16, 2, 192, 0), ("nvfp4", 4096, 1536, 128, 8, 255, 0), ("bf16", 4096, 1536, 128, 8, 256, 0),
+    ("bf16", 1024, 2048, 16, 2, 192, 0), ("int8", 4096, 1536, 4, 2, 128, 1), ("nvfp4", 4096, 1536, 128, 8, 255, 0), ("bf16", 4096, 1536, 128, 8, 256, 0),
     ("nvfp4", 4096, 1536, 128, 8, 256, 1), ("nvfp4", 4096, 1536, 128, 8, 2048, 1), ("bf16", 4096, 1536, 128, 8, 384, 1),
     ("fp8", 2048, 1024, 64, 8, 128, 1), ("int8", 4096, 1536, 8, 2, 128, 1), ("bf16", 2048, 1024, 16, 4, 256, 1),
     ("nvfp4", 4096, 14336, 12, 2, 1536, 1), ("fp8", 4096, 1536, 1, 1, 2048, 1)])
