@@ -13,8 +13,9 @@
 // multiple of 256 bytes apart (the LDS's fast pattern), and so are the staging writes, whose 16-lane groups hold sixteen
 // rows of one piece. Weights are expanded to bf16 on their way from the staging registers into LDS.
 //
-// Two LDS buffers, one barrier a tile, two sets of staging registers: while tile t is multiplied tile t + 1 goes from
-// registers into the other buffer and tile t + 3 is asked for.
+// Two LDS buffers, one barrier a tile, two sets of staging registers. Tile t is multiplied from one buffer while tile t + 1 lies
+// complete in the other. Its fragments are read ahead, so behind tile t's barrier nobody reads its buffer any more: tile t + 2
+// goes there from the registers while tile t + 1's first fragments are read, and tile t + 4 is asked for into those registers.
 #pragma once
 
 #include "common.h"
@@ -33,8 +34,11 @@ __device__ __forceinline__ int die_order(int b, int total) {
 // WM x WN wavefronts, each MT x NT tiles of 16 x 16. SPLIT: the row is more than one slice. ONE_X: one set of registers for
 // the activations' fragments, each read anew as soon as its products are issued, and the barrier behind a step's first products.
 // Reads and products then alternate more evenly and 16 registers are free: the experts' NVFP4 blocks of 128 x 256 at 2048 tokens
-// (128 of 4096 x 1536, both products and their sum) 1495 -> 1407 us; lx_gemm_w's blocks of 128 x 128 are 3 % faster without
-// (fp8 14336 x 4096 at 4096 rows 577 / 598).
+// (128 of 4096 x 1536, a pass of the layer) 1476 -> 1388 us; lx_gemm_w's blocks of 128 x 128 are 4 % faster without (fp8 14336 x
+// 4096 at 4096 rows 552 / 573, int8 math 4096 x 11008 at 515 rows 162 / 165).
+// With SPLIT a 128 x 256 block holds two sets of 64 sums a lane and does not fit 256 registers: the compiler spills 84 .. 200 of
+// them (116 .. 180 bytes a lane: the experts in every format, lx_gemm_w's on NVFP4 and under the FP8 math), moved where a slice ends. No
+// other block spills.
 template <int F, int MATH, int WM, int WN, int MT, int NT, bool SPLIT, bool ONE_X = false>
 struct Block {
   static constexpr bool kBytes = MATH != LX_MATH_BF16;  // one-byte operands on both sides

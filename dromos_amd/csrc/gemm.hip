@@ -1508,7 +1508,7 @@ int launch_format(GemmArgs a, const char* x0, char* y0, int M, int x_esize, int 
   }
   cut_rows<F>(a);
   const int tuned = tuned_variant(gemm_key<F>(), M, a.N, a.K);
-  if (a.xs.dtype == LX_BF16) {
+  if (a.xs.dtype == LX_BF16 && (M > 32 || tuned == kVariantBlock)) {  // (fewer are never the block kernel's: no buffer to look up)
     a.M = M;
     a.xs.x = x0;
     a.y = y0;
@@ -1517,7 +1517,7 @@ int launch_format(GemmArgs a, const char* x0, char* y0, int M, int x_esize, int 
     if (p.mode >= 0) return launch_block<F, LX_MATH_BF16>(a, p, partial, stream);
   }
   const float* const act_scale0 = a.act_scale;
-  // Up to 64 activation rows a pass; every pass is the same arithmetic per row.
+  // Up to 64 activation rows a pass (f32 activations at any row count); every pass is the same arithmetic per row.
   for (int m0 = 0; m0 < M; m0 += 64) {
     a.M = M - m0 < 64 ? M - m0 : 64;
     a.tuned = pass_variant<F>(tuned, M, a);

@@ -275,11 +275,24 @@ def test_c3_shape_under_the_fp4_math(hip, oracle):
 # ---- the slab kernel (a workgroup per K slice of many tiles, partial tiles added by a second kernel) ----------------
 
 
+@pytest.fixture
+def partial_sum_buffer(hip):
+    """The current stream with the buffer that the slab kernel's slices need."""
+    stream = torch.cuda.current_stream().cuda_stream
+    assert hip.lib.lx_rt_stream_reserve(stream) == 0
+    yield
+    torch.cuda.synchronize()
+    assert hip.lib.lx_rt_stream_release(stream) == 0
+    hip.lib.lx_tune_clear()
+
+
 @pytest.mark.parametrize("fmt", FMT)
 @pytest.mark.parametrize("M,N,K", [(64, 6144, 4096), (32, 4096, 8192), (40, 2048, 8192), (57, 6000, 2048)])
-def test_slab_shapes_give_the_bits_of_every_other_kernel(hip, fmt, M, N, K):
-    # Shapes the slab kernel takes by itself: their rows equal the same rows computed sixteen at a time (the lean tile
-    # kernel) bit for bit, with bias, alpha and a bf16 output in the epilogue of the second pass.
+def test_slab_shapes_give_the_bits_of_every_other_kernel(hip, partial_sum_buffer, fmt, M, N, K):
+    # Shapes the slab kernel takes by its rule (the table asks for it where the block kernel or the walks go first): their rows
+    # equal the same rows computed sixteen at a time (the lean tile kernel) bit for bit, with bias, alpha and a bf16 output in
+    # the epilogue of the second pass.
+    assert hip.lib.lx_tune_force(f"gemm_w_{fmt}".encode(), M, N, K, 5) == 0
     g = torch.Generator().manual_seed(M + N)
     w = random_weight(FORMATS[fmt], N, K, N + K).to("cuda")
     x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
@@ -373,7 +386,7 @@ def test_streams_with_and_without_the_partial_sum_buffer(hip):
 
 
 @pytest.mark.parametrize("math,fmt", [(MATH_INT8, "int8"), (MATH_FP8, "fp8")])
-def test_slab_under_the_byte_maths(hip, oracle, math, fmt):
+def test_slab_under_the_byte_maths(hip, oracle, partial_sum_buffer, math, fmt):
     M, N, K = 64, 6144, 4096
     g = torch.Generator().manual_seed(9)
     w = random_weight(FORMATS[fmt], N, K, 5)
