@@ -198,3 +198,23 @@ def test_infinite_expert_weights_at_the_rows_end(hip):
     assert bool(got[to5, 9].isinf().all()) and bool(got[to7].isinf().all())
     got[to5, 9], got[to7] = clean[to5, 9], clean[to7]
     assert torch.equal(got, clean)
+
+
+# Asked for through the variant table: row counts that the rule never sends there, in every format and math, with the
+# partial-tile buffer and without.
+@pytest.mark.parametrize("fmt,math", MATHS)
+@pytest.mark.parametrize("M,N,K", [(1, 300, 1056), (17, 1000, 4096), (64, 257, 2080)])
+@pytest.mark.parametrize("buffer", [False, True])
+def test_asked_for_by_the_table(hip, buffer, fmt, math, M, N, K):
+    g = torch.Generator().manual_seed(M)
+    w = random_weight(FORMATS[fmt], N, K, N + K).to("cuda")
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    y = torch.full((M, N), float("nan"), device="cuda")
+    assert hip.lib.dromos_plan_gemm(FORMATS[fmt], math, M, N, K, 0, buffer) == -1
+    want = on_a_stream(hip, buffer, x, w, math, y.clone())
+    try:
+        assert hip.lib.lx_tune_force(f"gemm_w_{fmt}".encode(), M, N, K, 8) == 0
+        assert hip.lib.dromos_plan_gemm(FORMATS[fmt], math, M, N, K, 0, buffer) >= 0
+        assert torch.equal(on_a_stream(hip, buffer, x, w, math, y.clone()), want)
+    finally:
+        hip.lib.lx_tune_clear()
