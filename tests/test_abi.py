@@ -1,4 +1,4 @@
-"""The C-ABI library loads and exports exactly what include/dromos_hip.h declares (no compute calls: this runs
+"""The C-ABI library loads and exports what include/dromos_hip.h declares (no compute calls: this runs
 without a GPU)."""
 
 import ctypes
