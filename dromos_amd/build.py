@@ -20,6 +20,9 @@ SOURCES = ["runtime.hip", "quant.hip", "gemv.hip", "gemv_bf16.hip", "gemv_int8.h
 
 # -ffp-contract=off: the epilogues and the ordered sums are written as separate multiplies and adds, as the
 # CPU reference computes them; fused operations are spelled __builtin_fmaf where they are meant.
+# amdgpu-mfma-vgpr-form: a wavefront that may have 512 registers keeps the running sums of its matrix products in vector registers
+# and moves what is seldom touched to accumulation registers; left alone the compiler does it the other way round and copies sums
+# between accumulation registers in the walk (124 moves for 64 matrix instructions).
 # packed-fp32-ops off: scalar float code must not be turned into v_pk_*_f32 by the optimiser.
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -28,6 +31,7 @@ HIPCC_FLAGS = [
     "-fPIC",
     "-fvisibility=hidden",
     "-ffp-contract=off",
+    "-mllvm", "-amdgpu-mfma-vgpr-form=1",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     f"-I{ROOT / 'include'}",
     f"-I{CSRC}",

@@ -2,22 +2,68 @@
 #pragma once
 
 #include "block_mfma.h"
+#include "block_wide.h"
 #include "gemm_block_plan.h"
 
 namespace dro {
 namespace block {
 
+// Where blocks lie: by bands of kBand blocks of activation rows, across a band first, so that the blocks a die holds at once
+// are about as many rows high as wide, which is the least they read between them.
+__device__ __forceinline__ void block_of(int b, int blocks_m, int blocks_n, int* bm, int* bn) {
+  constexpr int kBand = 8;
+  const int at = die_order(b, blocks_m * blocks_n);
+  const int band = at / (kBand * blocks_n), high = min(kBand, blocks_m - band * kBand), in_band = at - band * kBand * blocks_n;
+  *bn = in_band / high;
+  *bm = band * kBand + in_band - *bn * high;
+}
+
+// Four columns can be written at a time.
+__device__ __forceinline__ bool wide_stores(const GemmArgs& a) {
+  return !a.bias && a.beta == 0.0f && a.ld_y % 4 == 0 && reinterpret_cast<uintptr_t>(a.y) % 16 == 0;
+}
+
+// Four outputs at y[at] without bias and beta: write_out four columns at a time (rf: the row factors).
+template <class Acc>
+__device__ __forceinline__ void write_four(const GemmArgs& a, int64_t at, const Acc& sums, const float (&rf)[4]) {
+  f32x4 v;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = a.alpha * (rf[r] * static_cast<float>(sums[r]));
+  if (a.y_dtype == LX_F32) {
+    *reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + at) = v;
+  } else {
+    const bf16x2 p[2] = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+    *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.y) + at) = __builtin_bit_cast(u32x2, p);
+  }
+}
+
+// Columns n .. n + 3 of row m (of the matrix), as far as they exist, one at a time.
+template <class Acc>
+__device__ __forceinline__ void write_each(const GemmArgs& a, int m, int n, const Acc& sums, const float (&rf)[4]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (n + r < a.N) {
+      float t = rf[r] * static_cast<float>(sums[r]);
+      if (a.bias) t += a.bias_dtype == LX_F32 ? static_cast<const float*>(a.bias)[n + r] : load_as_f32(a.bias, a.bias_dtype, n + r);
+      float v = a.alpha * t;
+      const int64_t at = m * a.ld_y + n + r;
+      if (a.beta != 0.0f) v = a.beta * load_as_f32(a.y, a.y_dtype, at) + v;
+      store_from_f32(a.y, a.y_dtype, at, v);
+    }
+}
+
+// The activation row's factor: its scale under a quantised math.
+template <bool BYTES>
+__device__ __forceinline__ float row_scale(const GemmArgs& a, int m) {
+  return BYTES ? a.xscale[m] : a.act_scale ? a.act_scale[m] : 1.0f;
+}
+
 template <int F, int MATH, int WM, int WN, int MT, int NT, int MODE>
 __global__ void __launch_bounds__(WM* WN* kWave) __attribute__((amdgpu_waves_per_eu(2))) gemm_block_kernel(const GemmArgs a, int tiles, int slice_tiles) {
   using B = Block<F, MATH, WM, WN, MT, NT, MODE == kAdded>;
   extern __shared__ __align__(16) f32x4 lds4[];
-  const int blocks_m = (a.M + B::BM - 1) / B::BM, blocks_n = (a.N + B::BN - 1) / B::BN;
-  // Blocks go by bands of kBand blocks of activation rows, across a band first: the blocks a die holds at once are about
-  // as many rows high as wide, which is the least they read between them.
-  constexpr int kBand = 8;
-  const int at = die_order(blockIdx.x, blocks_m * blocks_n);
-  const int band = at / (kBand * blocks_n), high = min(kBand, blocks_m - band * kBand), in_band = at - band * kBand * blocks_n;
-  const int bn = in_band / high, bm = band * kBand + in_band - bn * high;
+  int bm, bn;
+  block_of(blockIdx.x, (a.M + B::BM - 1) / B::BM, (a.N + B::BN - 1) / B::BN, &bm, &bn);
   const int m0 = bm * B::BM, n0 = bn * B::BN;
   const int rows = min(B::BM, a.M - m0), cols = min(B::BN, a.N - n0);
   constexpr int xe = B::kBytes ? 1 : 2;
@@ -43,41 +89,19 @@ __global__ void __launch_bounds__(WM* WN* kWave) __attribute__((amdgpu_waves_per
     });
     return;
   }
-  const bool wide = !a.bias && a.beta == 0.0f && a.ld_y % 4 == 0 && reinterpret_cast<uintptr_t>(a.y) % 16 == 0;
-  const bool bias_f32 = a.bias && a.bias_dtype == LX_F32;
+  const bool wide = wide_stores(a);
   b.run(0, tiles, B::kStepHalves ? 2 * slice_tiles : slice_tiles, [&](int m, int tile, const typename B::Acc(&sums)[NT]) {
     if (m >= rows) return;
+    const float xs = row_scale<B::kBytes>(a, m0 + m);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const int n = 16 * (tile + t) + g4;
       if (n >= cols) continue;
       float rf[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        rf[r] = row_factor(F, a.scale, a.global, n0 + min(n + r, cols - 1));
-        if (B::kBytes) rf[r] *= a.xscale[m0 + m];
-      }
-      if (wide && n + 3 < cols) {
-        // write_out without bias and beta, four columns at a time.
-        f32x4 v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = a.alpha * ((!B::kBytes && a.act_scale ? rf[r] * a.act_scale[m0 + m] : rf[r]) * static_cast<float>(sums[t][r]));
-        const int64_t at_y = static_cast<int64_t>(m0 + m) * a.ld_y + n0 + n;
-        if (a.y_dtype == LX_F32) {
-          *reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + at_y) = v;
-        } else {
-          const u32x2 p = {f32_to_bf16_bits(v[0]) | static_cast<uint32_t>(f32_to_bf16_bits(v[1])) << 16,
-                           f32_to_bf16_bits(v[2]) | static_cast<uint32_t>(f32_to_bf16_bits(v[3])) << 16};
-          *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.y) + at_y) = p;
-        }
-        continue;
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (n + r < cols) {
-          const float bias = !a.bias ? 0.0f : bias_f32 ? static_cast<const float*>(a.bias)[n0 + n + r] : load_as_f32(a.bias, a.bias_dtype, n0 + n + r);
-          write_out(a, m0 + m, n0 + n + r, static_cast<float>(sums[t][r]), rf[r], bias);
-        }
+      for (int r = 0; r < 4; ++r) rf[r] = row_factor(F, a.scale, a.global, n0 + min(n + r, cols - 1)) * xs;
+      if (wide && n + 3 < cols) write_four(a, (m0 + m) * a.ld_y + n0 + n, sums[t], rf);
+      else write_each(a, m0 + m, n0 + n, sums[t], rf);
     }
   });
 }
@@ -93,8 +117,73 @@ int launch_mode(const GemmArgs& a, int tiles, int slice_tiles, hipStream_t strea
   return status_of(hipGetLastError());
 }
 
+// The wide block (block_wide.h): 128 x 256, all of K in a workgroup.
+template <int F, int MATH, int MODE>
+__global__ void __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) gemm_wide_kernel(const GemmArgs a, int stages, int slice) {
+  using B = Wide<F, MATH, 8, MODE == kAdded>;
+  extern __shared__ __align__(16) f32x4 lds4[];
+  int bm, bn;
+  block_of(blockIdx.x, (a.M + B::BM - 1) / B::BM, (a.N + B::BN - 1) / B::BN, &bm, &bn);
+  const int m0 = bm * B::BM, n0 = bn * B::BN;
+  const int rows = min(B::BM, a.M - m0), cols = min(B::BN, a.N - n0);
+  constexpr int xe = B::kBytes ? 1 : 2;
+  const int64_t ld = (B::kBytes ? a.K : a.xs.ld) * xe;
+  const char* const x = B::kBytes ? reinterpret_cast<const char*>(a.xq) : static_cast<const char*>(a.xs.x);
+  B b;
+  b.init(x + m0 * ld, (rows - 1) * ld + a.K * xe, a.w + n0 * a.row_bytes, cols * a.row_bytes, F == LX_W_NVFP4 ? a.scale + n0 * a.scale_row_bytes : a.scale,
+         cols * a.scale_row_bytes, a.row_bytes, a.K, lds4, [&](int row) { return static_cast<uint32_t>(min(row, rows - 1)) * static_cast<uint32_t>(ld); },
+         [&](int row) { return static_cast<uint32_t>(min(row, cols - 1)) * static_cast<uint32_t>(a.row_bytes); },
+         [&](int row) { return static_cast<uint32_t>(min(row, cols - 1)) * static_cast<uint32_t>(a.scale_row_bytes); });
+  const bool wide = wide_stores(a);
+  b.run(stages, slice);
+  // A wavefront writes every fourth row, a lane its four columns. What comes from memory is asked for in front of the loop (a load in
+  // it would wait behind the stores: 700 cycles a row).
+  const int n = 4 * b.lane;
+  float rf[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) rf[r] = row_factor(F, a.scale, a.global, n0 + min(n + r, cols - 1));
+  float xs[2];  // rows lane and 64 + lane
+#pragma unroll
+  for (int h = 0; h < 2; ++h) xs[h] = row_scale<B::kBytes>(a, m0 + min(64 * h + b.lane, rows - 1));
+  // (Everything is here: no wait in the loops, where it would be one for the stores too.)
+  asm volatile("" ::"v"(rf[0]), "v"(rf[1]), "v"(rf[2]), "v"(rf[3]), "v"(xs[0]), "v"(xs[1]));
+  auto factors = [&](int m, float(&f)[4]) {
+    // (One lane's value each time: lanes without columns take no part in a choice between two.)
+    const uint32_t s0 = __builtin_amdgcn_readlane(__float_as_uint(xs[0]), m & 63), s1 = __builtin_amdgcn_readlane(__float_as_uint(xs[1]), m & 63);
+    const float s = __uint_as_float(m < 64 ? s0 : s1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) f[r] = rf[r] * s;
+  };
+  float f[4];
+  if (wide && n + 3 < cols) {
+#pragma unroll 4
+    for (int m = b.wave; m < rows; m += B::kWaves) {
+      factors(m, f);
+      write_four(a, (m0 + m) * a.ld_y + n0 + n, b.sum(m, b.lane), f);
+    }
+  } else if (n < cols) {
+    for (int m = b.wave; m < rows; m += B::kWaves) {
+      factors(m, f);
+      write_each(a, m0 + m, n0 + n, b.sum(m, b.lane), f);
+    }
+  }
+}
+
+template <int F, int MATH, int MODE>
+int launch_wide(const GemmArgs& a, const Plan& p, hipStream_t stream) {
+  using B = Wide<F, MATH, 8, MODE == kAdded>;
+  const auto kernel = gemm_wide_kernel<F, MATH, MODE>;
+  allow_lds(reinterpret_cast<const void*>(kernel), kLdsMax);
+  const int64_t blocks = static_cast<int64_t>((a.M + B::BM - 1) / B::BM) * ((a.N + B::BN - 1) / B::BN);
+  constexpr int kSteps = B::kBytes ? 2 : 1;  // load steps a stage
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(B::kThreads), B::kLdsBytes, stream, a, (a.steps + kSteps - 1) / kSteps, a.steps_per_wave / kSteps);
+  return status_of(hipGetLastError());
+}
+
 template <int F, int MATH, int MODE>
 int launch_shape(const GemmArgs& a, const Plan& p, hipStream_t stream) {
+  if constexpr (F != LX_W_BF16 && MODE != kPart)
+    if (p.shape == kWide) return launch_wide<F, MATH, MODE>(a, p, stream);
   switch (p.shape) {
     case 0: return launch_mode<F, MATH, 2, 2, 2, 2, MODE>(a, p.tiles, p.slice_tiles, stream);
     case 1: return launch_mode<F, MATH, 2, 2, 2, 4, MODE>(a, p.tiles, p.slice_tiles, stream);

@@ -2,6 +2,8 @@
 // only, a function of the sizes and the device's compute units, so that it can be asked without launching anything.
 #pragma once
 
+#include <math.h>
+
 #include "gemm_args.h"
 
 namespace dro {
@@ -28,6 +30,30 @@ constexpr Shape shape(int i) {
   constexpr Shape int8_math[4] = {{64, 64, 14, 24}, {64, 128, 24, 22}, {128, 128, 45, 8}, {128, 256, 80, 10}};
   constexpr Shape fp8_math[4] = {{64, 64, 15, 28}, {64, 128, 28, 30}, {128, 128, 62, 2}, {128, 256, 106, 40}};
   return MATH == LX_MATH_INT8 ? int8_math[i] : MATH == LX_MATH_FP8 ? fp8_math[i] : F == LX_W_NVFP4 ? nvfp4[i] : bf16_math[i];
+}
+
+// The wide block (block_wide.h) as a plan's shape: 128 x 256, one wavefront a SIMD, quantised weights. It takes per_stage us a
+// stage of K and per_block us a block besides (its first loads, the sums' way out), and once. Measured on 65 .. 4096 rows, N 1024 ..
+// 16384, K 1024 .. 14336: fp8 14336 x 4096 at 4096 rows 547 us by blocks of 128 x 128, 420 wide; NVFP4 632 / 445, INT8 math 280 / 230,
+// FP8 math 497 / 351. A unit holds one block at a time and a block is a long chain: products of few blocks or short rows stay with
+// the smaller shapes (fp8 2656 x 9600 at 347 rows 48 / 106).
+constexpr int kWide = 16;
+struct WideCost {
+  float per_stage, per_block, once;
+};
+template <int F, int MATH>
+constexpr WideCost wide_cost() {
+  return MATH == LX_MATH_INT8 ? WideCost{0.82f, 8.5f, 3} : MATH == LX_MATH_FP8 ? WideCost{1.55f, 10, 4} : F == LX_W_NVFP4 ? WideCost{1.65f, 10, 4} : WideCost{0.75f, 8, 4};
+}
+
+// What the wide block is estimated to take, in us; infinite where it does not apply (block scales are loaded four bytes at a time).
+template <int F, int MATH>
+float wide_us(const GemmArgs& a, int units) {
+  if (F == LX_W_BF16 || (F == LX_W_NVFP4 && (a.scale_row_bytes % 4 != 0 || reinterpret_cast<uintptr_t>(a.scale) % 4 != 0))) return INFINITY;
+  constexpr WideCost c = wide_cost<F, MATH>();
+  const int stages = MATH == LX_MATH_BF16 ? a.steps : (a.steps + 1) / 2;
+  const int64_t blocks = static_cast<int64_t>((a.M + 127) / 128) * ((a.N + 255) / 256);
+  return ((blocks + units - 1) / units) * (c.per_stage * stages + c.per_block) + c.once;
 }
 
 // mode: Slices, or -1 where the kernel does not apply. K tiles of a row and of a slice.
@@ -63,7 +89,11 @@ Plan plan(const GemmArgs& a, int units, bool partial) {
   const int tiles = ((a.steps * kTilesPerStep + kSteps - 1) / kSteps + 1) / 2 * 2;
   const int slice_tiles = a.steps_per_wave * kTilesPerStep / kSteps, slices = (tiles + slice_tiles - 1) / slice_tiles;
   float us = 0.0f, us_part = 0.0f;
-  const int whole = best_shape<F, MATH>(a, tiles, 1, units, &us);
+  int whole = best_shape<F, MATH>(a, tiles, 1, units, &us);
+  if (const float wide = wide_us<F, MATH>(a, units); wide < us) {
+    whole = kWide;
+    us = wide;
+  }
   if (partial && slices > 1) {
     // One slice a workgroup: a second launch, and every slice's sums written and read once more (4.5 us and about 4 TB/s).
     const int part = best_shape<F, MATH>(a, slice_tiles, slices, units, &us_part);

@@ -76,6 +76,25 @@ def test_every_shape_and_mode(hip, fmt, math, mode, shape, M, N, K):
     assert torch.equal(on_a_stream(hip, buffer, x, w, math, y.clone()), chunks_of_32(hip, x, w, math, y))
 
 
+# The wide block (128 x 256, plan shape 16): blocks cut short in rows and columns, odd and even numbers of columns, rows that end
+# inside a stage of K and inside its pieces, two stages past a slice, the epilogue's operands.
+WIDE = [("int8", MATH_BF16, 20, 834, 7039, 1568, 0), ("int8", MATH_BF16, 20, 1921, 3332, 1600, 1), ("fp8", MATH_BF16, 20, 2731, 2203, 1568, 2), ("fp8", MATH_BF16, 20, 769, 7668, 1600, 0),
+        ("nvfp4", MATH_BF16, 20, 518, 7603, 1856, 0), ("nvfp4", MATH_BF16, 20, 897, 4612, 1984, 1), ("nvfp4", MATH_FP4, 20, 3896, 1033, 1856, 2), ("nvfp4", MATH_FP8, 20, 1512, 2703, 1856, 0),
+        ("int8", MATH_INT8, 16, 2691, 1491, 2336, 0), ("int8", MATH_INT8, 16, 477, 8257, 2416, 2), ("fp8", MATH_FP8, 20, 2049, 7169, 4112, 0)]
+
+
+@pytest.mark.parametrize("fmt,math,plan,M,N,K,epilogue", WIDE)
+def test_wide_block(hip, fmt, math, plan, M, N, K, epilogue):
+    assert hip.lib.dromos_plan_gemm(FORMATS[fmt], math, M, N, K, 0, 0) == plan
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    w = random_weight(FORMATS[fmt], N, K, N + K).to("cuda")
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    y = torch.randn(M, N, generator=g, device="cuda").to([torch.float32, torch.bfloat16, torch.bfloat16][epilogue])
+    bias = torch.randn(N, generator=g, device="cuda")
+    kw = [{}, {"alpha": 0.5}, {"bias": bias, "alpha": 1.5, "beta": 0.25}][epilogue]
+    assert torch.equal(ops.gemm_w(hip, x, w, math, y=y.clone(), **kw), chunks_of_32(hip, x, w, math, y, **kw))
+
+
 # Few blocks (a slice a workgroup), one block past a multiple of 64 / 128 rows and columns, an odd N, many blocks of each shape;
 # K of one slice, of slices whose last is short, of a last step and a last K tile cut short.
 @pytest.mark.parametrize("fmt,math", MATHS)
