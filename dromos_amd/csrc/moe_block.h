@@ -22,6 +22,8 @@ struct ExpertBlock {
   int K, cols;
   int64_t row_bytes, scale_row_bytes;
   int tiles, slice;  // K tiles, and what a slice is of them (block_mfma.h: Block::run)
+  int x_rows;        // rows of x
+  bool wide;         // by block_wide.h (whose stages are a tile each, two of NVFP4's)
 };
 
 // moe_block_<format>.hip. max_tiles bounds *n_tiles (which only the device knows).

@@ -112,7 +112,7 @@ __device__ __forceinline__ int block_scan(int v, int* buf) {
   return x + base;
 }
 
-__global__ void __launch_bounds__(kMaxExperts) group_kernel(const int32_t* __restrict__ ids, int P, int E, int height, Tables t) {
+__global__ void __launch_bounds__(kMaxExperts) group_kernel(const int32_t* __restrict__ ids, int P, int E, int height, bool even, Tables t) {
   __shared__ int count[kMaxExperts], cursor[kMaxExperts], buf[kMaxExperts];
   const int e = threadIdx.x;
   count[e] = 0;
@@ -130,10 +130,12 @@ __global__ void __launch_bounds__(kMaxExperts) group_kernel(const int32_t* __res
   __syncthreads();
   const int my_tiles = e < E ? (mine + height - 1) / height : 0;
   const int tile0 = block_scan(my_tiles, buf) - my_tiles;
+  // even: an expert's tiles are of one height, in whole sixteens (140 rows: 80 and 60, not 128 and 12); no more of them.
+  const int rows = even && my_tiles > 0 ? ((mine + my_tiles - 1) / my_tiles + 15) / 16 * 16 : height;
   for (int j = 0; j < my_tiles; ++j) {
     t.tile_expert[tile0 + j] = e;
-    t.tile_begin[tile0 + j] = begin + j * height;
-    t.tile_rows[tile0 + j] = min(height, mine - j * height);
+    t.tile_begin[tile0 + j] = begin + j * rows;
+    t.tile_rows[tile0 + j] = min(rows, mine - j * rows);
   }
   if (e == kMaxExperts - 1) *t.n_tiles = tile0 + my_tiles;
   for (int p = e; p < P; p += kMaxExperts) {
@@ -348,6 +350,14 @@ bool blocks_wanted(int type, int64_t P, int64_t E, int64_t L, int64_t I, int uni
   return (rows < most ? rows : most) * busy >= (type == LX_W_NVFP4 ? 16 : type == LX_W_BF16 ? 14 : 12) * held;
 }
 
+// Whether a stack of rows of K values is taken by the wide block (block_wide.h): quantised rows, NVFP4's with block scales that can be
+// loaded four bytes at a time. It is ahead wherever blocks are taken at all (72 products of 8 .. 128 experts, 1088 .. 4096 x 512 ..
+// 1984, 17 .. 1388 rows an expert: 0.70 .. 1.02 of the other blocks' time; 128 NVFP4 experts of 4096 x 1536 at 2048 tokens 1372 ->
+// 990 us, at 512 646 -> 477, FP8 at 2048 1260 -> 980).
+bool wide_fits(int type, const Stack& w, int64_t K) {
+  return type == LX_W_INT8 || type == LX_W_FP8 || (type == LX_W_NVFP4 && K % 64 == 0 && reinterpret_cast<uintptr_t>(w.scale) % 4 == 0);
+}
+
 BlockCut block_cut_any(int type, int64_t K, int NT, int64_t out_rows) {
   switch (type) {
     case LX_W_BF16: return block_cut<LX_W_BF16>(K, NT, out_rows);
@@ -425,8 +435,9 @@ int experts_grouped(const void* latent, const int32_t* ids, const float* weights
   }
   const BlockCut cut1 = block_cut_any(gate_up.type, L, 2, I), cut2 = block_cut_any(down.type, I, 1, L);
   const bool blocks = cut1.fits && cut2.fits && static_cast<int64_t>(T) * L * 2 < (1ll << 31) && blocks_wanted(gate_up.type, P, E, L, I, compute_units());
+  const bool wide1 = blocks && wide_fits(gate_up.type, a.gu, L), wide2 = blocks && wide_fits(down.type, a.dn, I);
   const int tiles = max_tiles(P, E, blocks ? kBlockTokens : kTileTokens);
-  hipLaunchKernelGGL(group_kernel, dim3(1), dim3(kMaxExperts), 0, s, ids, P, E, blocks ? kBlockTokens : kTileTokens, a.t);
+  hipLaunchKernelGGL(group_kernel, dim3(1), dim3(kMaxExperts), 0, s, ids, P, E, blocks ? kBlockTokens : kTileTokens, wide1, a.t);
   if (int st = status_of(hipGetLastError())) return st;
   if (quantised) {
     uint16_t* const image1 = reinterpret_cast<uint16_t*>(ws + lay.image1);
@@ -446,6 +457,8 @@ int experts_grouped(const void* latent, const int32_t* ids, const float* weights
     b.x = a.latent;
     b.xs = a.xs1;
     b.order = a.t.order;
+    b.x_rows = T;
+    b.wide = wide1;
     b.out = a.inter;
     st = launch_expert_block(gate_up.type, b, a.gu, L, I, cut1, tiles, s);
   } else switch (gate_up.type) {
@@ -472,6 +485,7 @@ int experts_grouped(const void* latent, const int32_t* ids, const float* weights
     b.x = a.down_in;
     b.xs = a.xs2;
     b.order = nullptr;
+    b.wide = wide2;
     b.out = a.contrib;
     st = launch_expert_block(down.type, b, a.dn, I, L, cut2, tiles, s);
   } else switch (down.type) {
