@@ -53,6 +53,31 @@ __device__ __forceinline__ uint32_t e2m1_encode(float x) {
   return idx | ((x < 0.0f && idx > 0u) ? 8u : 0u);
 }
 
+// Four e4m3_encode()s as a dword by the conversion instruction, which does not saturate by itself and gives every NaN one sign.
+// Equal to e4m3_encode() on all 2^32 arguments, as e2m1_encode_eight() is to e2m1_encode().
+__device__ __forceinline__ uint32_t e4m3_encode_four(const float* v) {
+  const float sum = (v[0] + v[1]) + (v[2] + v[3]);
+  if (__builtin_expect(sum != sum, 0)) return e4m3_encode(v[0]) | e4m3_encode(v[1]) << 8 | e4m3_encode(v[2]) << 16 | e4m3_encode(v[3]) << 24;
+  float c[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) c[j] = fminf(fmaxf(v[j], -448.0f), 448.0f);
+  return __builtin_amdgcn_cvt_pk_fp8_f32(c[2], c[3], __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[1], 0, false), true);
+}
+
+// Eight e2m1_encode()s as a dword by the conversion instruction, without the signs it leaves on zeros (a NaN is a six).
+__device__ __forceinline__ uint32_t e2m1_encode_eight(const float* v) {
+  float c[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) c[j] = fmaxf(fminf(v[j], 6.0f), -6.0f);
+  uint32_t d = 0;
+  d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, c[0], c[1], 1.0f, 0);
+  d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, c[2], c[3], 1.0f, 1);
+  d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, c[4], c[5], 1.0f, 2);
+  d = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(d, c[6], c[7], 1.0f, 3);
+  const uint32_t mag = d & 0x77777777u;
+  return mag | (d & (mag + 0x77777777u) & 0x88888888u);
+}
+
 __device__ __forceinline__ float block_max(float v, float* shared) {
   v = wave_max(v);
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
@@ -112,12 +137,30 @@ __global__ void __launch_bounds__(kThreads) quantize_act_kernel(const void* __re
   }
 }
 
-// The INT8 / FP8 rules of quantize_act_kernel for rows that can be read 16 bytes at a time and fit a workgroup's
-// registers (K <= 8 * kActVecs * kThreads): every value is read once, eight bf16 or two times four f32 per thread
-// and pass, and eight codes are stored at a time. The same operations on the same values: the same bytes.
-constexpr int kActVecs = 4;
-
+// Eight values from 16-byte aligned p as f32 (XF32: they are f32, else bf16).
 template <bool XF32>
+__device__ __forceinline__ void load_eight(const char* p, float (&v)[8]) {
+  if constexpr (XF32) {
+    const f32x4 lo = *reinterpret_cast<const f32x4*>(p), hi = *reinterpret_cast<const f32x4*>(p + 16);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[j] = lo[j];
+      v[4 + j] = hi[j];
+    }
+  } else {
+    const u32x4 w = *reinterpret_cast<const u32x4*>(p);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[2 * j] = __uint_as_float(w[j] << 16);
+      v[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
+    }
+  }
+}
+
+// The INT8 / FP8 rules of quantize_act_kernel for rows that can be read 16 bytes at a time and fit a workgroup's
+// registers (K <= 8 * VECS * kThreads): every value is read once, eight a thread and piece, and eight codes are stored at a time.
+// The same operations on the same values: the same bytes. Bound by memory: see the launch.
+template <bool XF32, int VECS>
 __global__ void __launch_bounds__(kThreads) quantize_act_rows_kernel(const void* __restrict__ x, int64_t ld_x, int math,
                                                                      uint8_t* __restrict__ q, int64_t ld_q, float* __restrict__ scale,
                                                                      int K) {
@@ -125,52 +168,88 @@ __global__ void __launch_bounds__(kThreads) quantize_act_rows_kernel(const void*
   const int64_t m = blockIdx.x;
   const char* const row = static_cast<const char*>(x) + m * ld_x * (XF32 ? 4 : 2);
   const int vecs = K >> 3;
-  float v[kActVecs][8];
+  float v[VECS][8];
   float a = 0.0f;
 #pragma unroll
-  for (int u = 0; u < kActVecs; ++u) {
+  for (int u = 0; u < VECS; ++u) {
     const int vi = threadIdx.x + u * kThreads;
-    const int vc = min(vi, vecs - 1);  // clamped: no predicated loads; a piece past the row is not stored
-    if constexpr (XF32) {
-      const f32x4 lo = *reinterpret_cast<const f32x4*>(row + vc * 32), hi = *reinterpret_cast<const f32x4*>(row + vc * 32 + 16);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[u][j] = lo[j];
-        v[u][4 + j] = hi[j];
-      }
-    } else {
-      const u32x4 w = *reinterpret_cast<const u32x4*>(row + vc * 16);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[u][2 * j] = __uint_as_float(w[j] << 16);
-        v[u][2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
-      }
-    }
-    if (vi < vecs) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) a = fmaxf(a, fabsf(v[u][j]));
-    }
+    load_eight<XF32>(row + min(vi, vecs - 1) * (XF32 ? 32 : 16), v[u]);  // clamped: no predicated loads; a piece past the row is not stored
   }
+#pragma unroll
+  for (int u = 0; u < VECS; ++u)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) a = fmaxf(a, fabsf(v[u][j]));  // (the row's last piece again, past its end)
   a = block_max(a, shared);
   const float qmax = math == LX_MATH_INT8 ? 127.0f : 448.0f;
   const float inv = a > 0.0f ? qmax / a : 0.0f;
   uint8_t* const out = q + m * ld_q;
 #pragma unroll
-  for (int u = 0; u < kActVecs; ++u) {
+  for (int u = 0; u < VECS; ++u) {
     const int vi = threadIdx.x + u * kThreads;
     if (vi < vecs) {
       uint32_t packed[2] = {0u, 0u};
+      float t[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float t = v[u][j] * inv;
-        const uint32_t code = math == LX_MATH_INT8 ? static_cast<uint32_t>(static_cast<int>(fminf(fmaxf(rintf(t), -127.0f), 127.0f))) & 0xffu
-                                                   : e4m3_encode(t);
-        packed[j >> 2] |= code << (8 * (j & 3));
+      for (int j = 0; j < 8; ++j) t[j] = v[u][j] * inv;
+      if (math == LX_MATH_INT8) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          packed[j >> 2] |= (static_cast<uint32_t>(static_cast<int>(fminf(fmaxf(rintf(t[j]), -127.0f), 127.0f))) & 0xffu) << (8 * (j & 3));
+      } else {
+        packed[0] = e4m3_encode_four(t);
+        packed[1] = e4m3_encode_four(t + 4);
       }
       *reinterpret_cast<uint2*>(out + vi * 8) = uint2{packed[0], packed[1]};
     }
   }
   if (threadIdx.x == 0) scale[m] = a > 0.0f ? a / qmax : 1.0f;
+}
+
+// The FP4 rule the same way: a thread holds VECS blocks of sixteen (K <= 16 * VECS * kThreads) and stores a block's eight bytes.
+template <bool XF32, int VECS>
+__global__ void __launch_bounds__(kThreads) quantize_act_blocks_kernel(const void* __restrict__ x, int64_t ld_x, uint8_t* __restrict__ q, int64_t ld_q, float* __restrict__ scale,
+                                                                       uint8_t* __restrict__ block_scale, int64_t ld_bs, int K) {
+  __shared__ float shared[kWaves];
+  const int64_t m = blockIdx.x;
+  const char* const row = static_cast<const char*>(x) + m * ld_x * (XF32 ? 4 : 2);
+  const int blocks = K >> 4;
+  float v[VECS][2][8], amax[VECS], a = 0.0f;
+#pragma unroll
+  for (int u = 0; u < VECS; ++u) {
+    const char* const p = row + min(static_cast<int>(threadIdx.x) + u * kThreads, blocks - 1) * (XF32 ? 64 : 32);
+    load_eight<XF32>(p, v[u][0]);
+    load_eight<XF32>(p + (XF32 ? 32 : 16), v[u][1]);
+  }
+#pragma unroll
+  for (int u = 0; u < VECS; ++u) {
+    amax[u] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) amax[u] = fmaxf(amax[u], fabsf(v[u][j >> 3][j & 7]));
+    a = fmaxf(a, amax[u]);
+  }
+  a = block_max(a, shared);
+  const float g = a > 0.0f ? a / 2688.0f : 1.0f;
+  if (threadIdx.x == 0) scale[m] = g;
+#pragma unroll
+  for (int u = 0; u < VECS; ++u) {
+    const int b = threadIdx.x + u * kThreads;
+    if (b >= blocks) break;
+    const uint32_t s8 = e4m3_encode(amax[u] / (6.0f * g));
+    block_scale[m * ld_bs + b] = static_cast<uint8_t>(s8);
+    const float d = e4m3_decode(s8) * g;
+    const float r = d > 0.0f ? 1.0f / d : 0.0f;
+    uint32_t packed[2] = {0u, 0u};
+    if (d > 0.0f) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float t[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) t[j] = v[u][h][j] * r;
+        packed[h] = e2m1_encode_eight(t);
+      }
+    }
+    *reinterpret_cast<uint2*>(q + m * ld_q + b * 8) = uint2{packed[0], packed[1]};
+  }
 }
 
 // One workgroup per row: absmax, then the row's codes. FP8 = false is INT8.
@@ -311,15 +390,31 @@ namespace dro {
 // The launch behind lx_quantize_act (arguments already validated), shared with the INT8 math of lx_gemm_w.
 int quantize_act_rows(const void* x, int x_dtype, int64_t ld_x, int math, void* q, int64_t ld_q, float* scale, void* block_scale,
                       int64_t ld_bs, int M, int K, hipStream_t stream) {
+  // Rows that are read 16 bytes at a time and held in registers; longer and unaligned ones are read twice. Calls
+  // back to back (an empty one is 7 us): INT8 on 515 bf16 rows of 11008 values 18.9 us read twice, 7.3 held, FP8 24.1 / 7.5; INT8 on 4096
+  // of 14336 91 / 27, FP4 151 / 26 (4.5 TB/s).
   const int esize = x_dtype == LX_F32 ? 4 : 2;
-  const bool fast = math != LX_MATH_FP4 && K % 8 == 0 && K <= 8 * kActVecs * kThreads && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+  const int unit = math == LX_MATH_FP4 ? 16 : 8, pieces = (K / unit + kThreads - 1) / kThreads;
+  const bool fast = K % unit == 0 && pieces <= (math == LX_MATH_FP4 ? 4 : 8) && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
                     (ld_x * esize) % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 8 == 0 && ld_q % 8 == 0;
-  if (fast && x_dtype == LX_F32)
-    hipLaunchKernelGGL(quantize_act_rows_kernel<true>, dim3(static_cast<unsigned>(M)), dim3(kThreads), 0, stream, x, ld_x, math,
-                       static_cast<uint8_t*>(q), ld_q, scale, K);
-  else if (fast)
-    hipLaunchKernelGGL(quantize_act_rows_kernel<false>, dim3(static_cast<unsigned>(M)), dim3(kThreads), 0, stream, x, ld_x, math,
-                       static_cast<uint8_t*>(q), ld_q, scale, K);
+  const dim3 grid(static_cast<unsigned>(M)), block(kThreads);
+  uint8_t *const codes = static_cast<uint8_t*>(q), *const scales = static_cast<uint8_t*>(block_scale);
+  auto rows = [&](auto f32, auto vecs) {
+    if (math == LX_MATH_FP4) {
+      if constexpr (decltype(vecs)::value <= 4)
+        hipLaunchKernelGGL((quantize_act_blocks_kernel<decltype(f32)::value, decltype(vecs)::value>), grid, block, 0, stream, x, ld_x, codes, ld_q, scale, scales, ld_bs, K);
+    } else {
+      hipLaunchKernelGGL((quantize_act_rows_kernel<decltype(f32)::value, decltype(vecs)::value>), grid, block, 0, stream, x, ld_x, math, codes, ld_q, scale, K);
+    }
+  };
+  auto held = [&](auto f32) {
+    if (pieces <= 1) rows(f32, std::integral_constant<int, 1>{});
+    else if (pieces <= 2) rows(f32, std::integral_constant<int, 2>{});
+    else if (pieces <= 4) rows(f32, std::integral_constant<int, 4>{});
+    else rows(f32, std::integral_constant<int, 8>{});
+  };
+  if (fast && x_dtype == LX_F32) held(std::true_type{});
+  else if (fast) held(std::false_type{});
   else
     hipLaunchKernelGGL(quantize_act_kernel, dim3(static_cast<unsigned>(M)), dim3(kThreads), 0, stream, x, x_dtype, ld_x, math,
                        static_cast<uint8_t*>(q), ld_q, scale, static_cast<uint8_t*>(block_scale), ld_bs, K);
@@ -355,6 +450,31 @@ __global__ void __launch_bounds__(kThreads) act_values_kernel(const uint8_t* __r
   }
 }
 
+// The same for rows of whole eights whose codes and values can be moved at once: a thread's eight codes in one load, its values in one
+// store of 16 bytes. A row is blockIdx.x's.
+template <int MATH>
+__global__ void __launch_bounds__(kThreads) act_values_rows_kernel(const uint8_t* __restrict__ q, int64_t ld_q, const uint8_t* __restrict__ bs, int64_t ld_bs,
+                                                                   uint16_t* __restrict__ xhat, int64_t ld_o, int K) {
+  const int64_t m = blockIdx.x;
+  const int k0 = (blockIdx.y * kThreads + threadIdx.x) * 8;
+  if (k0 >= K) return;
+  float v[8];
+  if constexpr (MATH == LX_MATH_FP4) {
+    decode_dword<LX_W_NVFP4>(*reinterpret_cast<const uint32_t*>(q + m * ld_q + (k0 >> 1)), v);
+    const float s = e4m3_decode(bs[m * ld_bs + (k0 >> 4)]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] *= s;
+  } else {
+    const u32x2 w = *reinterpret_cast<const u32x2*>(q + m * ld_q + k0);
+    decode_dword<MATH == LX_MATH_INT8 ? LX_W_INT8 : LX_W_FP8>(w.x, v);
+    decode_dword<MATH == LX_MATH_INT8 ? LX_W_INT8 : LX_W_FP8>(w.y, v + 4);
+  }
+  uint32_t h[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) h[j] = f32_to_bf16_bits(v[2 * j]) | static_cast<uint32_t>(f32_to_bf16_bits(v[2 * j + 1])) << 16;
+  *reinterpret_cast<u32x4*>(xhat + m * ld_o + k0) = u32x4{h[0], h[1], h[2], h[3]};
+}
+
 }  // namespace
 
 // The rows of x [M, K] as a quantised math sees them: quantised per row by lx_quantize_act's rule for `math` (bytes into
@@ -366,6 +486,14 @@ int act_images(const void* x, int x_dtype, int64_t ld_x, int math, uint8_t* q, u
   const int64_t ld_q = math == LX_MATH_FP4 ? K / 2 : K, ld_bs = K / 16;
   uint8_t* const bs = q + static_cast<int64_t>(M) * ld_q;
   if (int st = quantize_act_rows(x, x_dtype, ld_x, math, q, ld_q, scale, bs, ld_bs, M, K, stream)) return st;
+  if (K % 8 == 0 && reinterpret_cast<uintptr_t>(q) % 8 == 0 && reinterpret_cast<uintptr_t>(xhat) % 16 == 0) {
+    const dim3 grid(static_cast<unsigned>(M), static_cast<unsigned>((K / 8 + kThreads - 1) / kThreads));
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, q, ld_q, bs, ld_bs, xhat, static_cast<int64_t>(K), K); };
+    if (math == LX_MATH_INT8) go(act_values_rows_kernel<LX_MATH_INT8>);
+    else if (math == LX_MATH_FP8) go(act_values_rows_kernel<LX_MATH_FP8>);
+    else go(act_values_rows_kernel<LX_MATH_FP4>);
+    return status_of(hipGetLastError());
+  }
   const int64_t items = static_cast<int64_t>(M) * ((K + 7) / 8);
   hipLaunchKernelGGL(act_values_kernel, dim3(static_cast<unsigned>((items + kThreads - 1) / kThreads)), dim3(kThreads), 0, stream, q, ld_q,
                      bs, ld_bs, math, xhat, static_cast<int64_t>(K), M, K);

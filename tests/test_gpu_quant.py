@@ -90,6 +90,15 @@ def test_quantize_act_matches_the_rules(hip, M, K, math, x_dtype, pad):
     checks.quantize_act_case(hip, math, M, K, seed=M * 31 + K + math, x_dtype=x_dtype, pad=pad * 2, x_pad=pad)
 
 
+# Rows held in registers: the ends of each number of pieces a thread (256 threads, eight values a piece; sixteen under FP4), and past the
+# longest; rows with a NaN-free maximum at either end.
+@pytest.mark.parametrize("x_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("math", [1, 2, 3])
+@pytest.mark.parametrize("M,K", [(3, 2064), (2, 4112), (5, 8192), (3, 8208), (4, 11008), (2, 16384), (3, 16400)])
+def test_quantize_act_long_rows(hip, M, K, math, x_dtype):
+    checks.quantize_act_case(hip, math, M, K, seed=M * 31 + K + math, x_dtype=x_dtype)
+
+
 @pytest.mark.parametrize("math", [1, 2])
 def test_quantize_act_odd_k(hip, math):
     checks.quantize_act_case(hip, math, 9, 1001, seed=5, x_pad=3, pad=7)
