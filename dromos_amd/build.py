@@ -15,6 +15,7 @@ CSRC = ROOT / "dromos_amd" / "csrc"
 LIB_DIR = ROOT / "dromos_amd" / "lib"
 HIP_LIB = LIB_DIR / "libdromos_hip.so"
 SOURCES = ["runtime.hip", "quant.hip", "gemv.hip", "gemv_bf16.hip", "gemv_int8.hip", "gemv_fp8.hip", "gemv_nvfp4.hip", "gemv_bf16x.hip", "bf16x.hip", "gemm.hip", "gemm_walk_bf16.hip", "gemm_walk_int8.hip", "gemm_walk_fp8.hip", "gemm_walk_nvfp4.hip",
+           "gemm_ring_bf16.hip", "gemm_ring_int8.hip", "gemm_ring_fp8.hip", "gemm_ring_nvfp4.hip",
            "gemm_block_bf16.hip", "gemm_block_int8.hip", "gemm_block_fp8.hip", "gemm_block_nvfp4.hip", "gemm_block_int8_math.hip", "gemm_block_fp8_math.hip",
            "moe.hip", "moe_grouped.hip", "moe_block_bf16.hip", "moe_block_int8.hip", "moe_block_fp8.hip", "moe_block_nvfp4.hip", "router.hip", "checkpoint.hip"]
 
@@ -33,7 +34,7 @@ HIPCC_FLAGS = [
     f"-I{CSRC}",
 ]
 
-# The kernels whose wavefronts may have 512 registers for themselves (block_wide.h) keep the running sums of their matrix
+# The kernels whose wavefronts may have 512 registers for themselves (block_wide.h, gemm_ring.h) keep the running sums of their matrix
 # products in vector registers and what is seldom touched in accumulation registers; left alone the compiler does it the other way
 # round and copies sums between accumulation registers in the walk (124 moves for 64 matrix instructions). The walk kernels are
 # better off left alone (NVFP4 14336 x 4096 at 64 rows 28.3 us, with it 33.7).
@@ -41,7 +42,7 @@ MFMA_VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 
 
 def _flags(source):
-    return HIPCC_FLAGS + (MFMA_VGPR_FORM if source.startswith(("gemm_block_", "moe_block_")) else [])
+    return HIPCC_FLAGS + (MFMA_VGPR_FORM if source.startswith(("gemm_block_", "gemm_ring_", "moe_block_")) else [])
 
 
 def _hipcc():

@@ -1347,12 +1347,52 @@ bool walk_parts_wanted(int M, int n_tiles, int64_t K, int tuned) {
   return K >= mid_k && K < 8192 && n_tiles > 256 && n_tiles <= 384;
 }
 
+// Weight rows a workgroup of the ring kernel (gemm_ring.h) takes, 32 up to 512 tiles and 64 beyond, or 0 where another kernel is
+// ahead. From a sweep on cold weights (176 products of 9 .. 64 rows, 289 .. 1021 tiles, K 2048 .. 14336; ratios are ring to the kernels
+// it replaces). It was not measured outside 289 .. 1024 tiles.
+// - NVFP4 from 17 rows, whose other kernels are short of wavefronts: 0.52 .. 0.93 to K = 4096 (6208 x 2048 at 56 rows 19.8 -> 10.3 us,
+//   7264 x 4096 at 32 rows 17.4 -> 10.4, 9088 x 4096 at 64 rows 36 -> 26), beyond it where the slices fill the wavefronts (8192 values:
+//   0.78 .. 0.81, 11008: 0.75 .. 0.97; three slices of 5120 .. 7168 values for four wavefronts 1.08 .. 1.20). Up to 16 rows 0.98 .. 1.06.
+//   Four slices of 64 rows leave the ring two stages: on 896 tiles, where the walk kernel takes four tiles a workgroup, 28.3 / 29.0.
+// - bf16 on more than 383 tiles: 0.61 .. 0.97 at every row count (7984 x 4096 at 56 rows 33.4 -> 20.3 us, 12048 x 4096 at 32 rows 33.4 ->
+//   24.7, 12512 x 4096 at 9 rows 24.6 -> 20.9); short rows on more than 900 tiles at 64 rows 1.07.
+// - One-byte weights of 4096 .. 8192 values: from 17 rows up to 512 tiles (0.80 .. 0.94, once 1.01: int8 5360 x 4096 at 32 rows 15.5 -> 12.1
+//   us, fp8 7280 x 4096 at 24 rows 13.8 -> 12.1; up to 16 rows 0.80 .. 1.18), beyond 512 tiles from 33 rows, K = 4096 from 49 (0.65 .. 0.95: fp8
+//   8704 x 5120 at 56 rows 46.8 -> 31.2, int8 16192 x 7168 at 40 rows 48.8 -> 42.7; at 24 .. 32 rows 0.91 .. 1.10).
+template <int F>
+int ring_cols(const GemmArgs& a, int n_tiles) {
+  if (a.M <= 8 || n_tiles < 289 || n_tiles > 1024 || a.K < 2048 || a.K > 11264) return 0;
+  const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave, waves = slices > 2 ? 4 : slices;
+  if (slices > 4) return 0;
+  const int cols = n_tiles <= 512 ? 32 : 64;
+  if (F == LX_W_NVFP4 && a.M > 48 && slices > 2 && n_tiles > 768) return 0;
+  if (F == LX_W_NVFP4) return a.M > 16 && (a.K <= 4096 || a.steps * 100 >= a.steps_per_wave * waves * 89) ? cols : 0;
+  if (F == LX_W_BF16) return n_tiles > 383 && (a.K >= 4096 || n_tiles <= 900) ? cols : 0;
+  if (a.K < 4096 || a.K > 8192) return 0;
+  return n_tiles <= 512 ? (a.M > 16 ? cols : 0) : a.M > (a.K == 4096 ? 48 : 32) ? cols : 0;
+}
+
+// The ring kernel where it is the faster one.
+template <int F>
+bool try_ring(const GemmArgs& a, int* status, hipStream_t stream) {
+  if (a.tuned >= 0 || a.xs.dtype != LX_BF16) return false;
+  const int cols = ring_cols<F>(a, (a.N + kTileRows - 1) / kTileRows);
+  if (cols == 0 || a.row_bytes * 64 >= (1ll << 31) || a.xs.ld * 2 * 64 >= (1ll << 31)) return false;  // 32-bit offsets
+  // (Block scales are loaded four bytes at a time.)
+  if (F == LX_W_NVFP4 && (a.scale_row_bytes % 4 != 0 || reinterpret_cast<uintptr_t>(a.scale) % 4 != 0)) return false;
+  if constexpr (F == LX_W_BF16) return launch_ring_bf16(a, cols, status, stream);
+  else if constexpr (F == LX_W_INT8) return launch_ring_int8(a, cols, status, stream);
+  else if constexpr (F == LX_W_FP8) return launch_ring_fp8(a, cols, status, stream);
+  else return launch_ring_nvfp4(a, cols, status, stream);
+}
+
 template <int F, int MT>
 int launch_skinny(GemmArgs a, hipStream_t stream) {
   const int S = a.S;
   const unsigned n_tiles = static_cast<unsigned>((a.N + kTileRows - 1) / kTileRows);
   {
     int st = kOk;
+    if (try_ring<F>(a, &st, stream)) return st;
     if (walk_parts_wanted<F>(a.M, static_cast<int>(n_tiles), a.K, a.tuned) && launch_walk_parts<F>(a, &st, stream)) return st;
     if (walk_split_wanted(a.M, static_cast<int>(n_tiles), a.K, a.tuned) && launch_walk_split<F>(a, &st, stream)) return st;
     if (try_walk<F>(a, &st, stream)) return st;

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "common.h"
+#include "tile_mfma.h"
 
 namespace dro {
 
@@ -56,6 +57,40 @@ __device__ __forceinline__ void write_out(const GemmArgs& a, int wtype, int m, i
   write_out(a, m, n, sum, row_factor(wtype, a.scale, a.global, n), a.bias ? load_as_f32(a.bias, a.bias_dtype, n) : 0.0f);
 }
 
+// Four columns can be written at a time.
+__device__ __forceinline__ bool wide_stores(const GemmArgs& a) {
+  return !a.bias && a.beta == 0.0f && a.ld_y % 4 == 0 && reinterpret_cast<uintptr_t>(a.y) % 16 == 0;
+}
+
+// Four outputs at y[at] without bias and beta: write_out four columns at a time (rf: the row factors).
+template <class Acc>
+__device__ __forceinline__ void write_four(const GemmArgs& a, int64_t at, const Acc& sums, const float (&rf)[4]) {
+  f32x4 v;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = a.alpha * (rf[r] * static_cast<float>(sums[r]));
+  if (a.y_dtype == LX_F32) {
+    *reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + at) = v;
+  } else {
+    const bf16x2 p[2] = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+    *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.y) + at) = __builtin_bit_cast(u32x2, p);
+  }
+}
+
+// Columns n .. n + 3 of row m (of the matrix), as far as they exist, one at a time.
+template <class Acc>
+__device__ __forceinline__ void write_each(const GemmArgs& a, int m, int n, const Acc& sums, const float (&rf)[4]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (n + r < a.N) {
+      float t = rf[r] * static_cast<float>(sums[r]);
+      if (a.bias) t += a.bias_dtype == LX_F32 ? static_cast<const float*>(a.bias)[n + r] : load_as_f32(a.bias, a.bias_dtype, n + r);
+      float v = a.alpha * t;
+      const int64_t at = m * a.ld_y + n + r;
+      if (a.beta != 0.0f) v = a.beta * load_as_f32(a.y, a.y_dtype, at) + v;
+      store_from_f32(a.y, a.y_dtype, at, v);
+    }
+}
+
 // gemm_walk_<format>.hip: the walk kernel (gemm_walk.h) for up to 64 bf16 activation rows with W tiles a workgroup
 // (1, 2 or 4; with a.partial set, 4 or 8, and a workgroup walks a.walk_slices slices and leaves their sums there; with a.walk_split
 // set, W = 2 or 4 wavefronts on one tile); false when it does not apply to the call (the caller then takes another kernel), otherwise *status holds
@@ -64,6 +99,13 @@ bool launch_walk_bf16(const GemmArgs& a, int W, int* status, hipStream_t stream)
 bool launch_walk_int8(const GemmArgs& a, int W, int* status, hipStream_t stream);
 bool launch_walk_fp8(const GemmArgs& a, int W, int* status, hipStream_t stream);
 bool launch_walk_nvfp4(const GemmArgs& a, int W, int* status, hipStream_t stream);
+
+// gemm_ring_<format>.hip: the ring kernel (gemm_ring.h) for up to 64 bf16 activation rows with `cols` (32 or 64) weight rows a workgroup;
+// false when it does not apply, otherwise *status holds the launch's status.
+bool launch_ring_bf16(const GemmArgs& a, int cols, int* status, hipStream_t stream);
+bool launch_ring_int8(const GemmArgs& a, int cols, int* status, hipStream_t stream);
+bool launch_ring_fp8(const GemmArgs& a, int cols, int* status, hipStream_t stream);
+bool launch_ring_nvfp4(const GemmArgs& a, int cols, int* status, hipStream_t stream);
 
 // gemm_block_<format>.hip: the block kernel (gemm_block.h) for any number of bf16 activation rows, gemm_block_<format>_math.hip the
 // same under the INT8 and FP8 maths, as the plan says (gemm_block_plan.h). Returns the launch's status.

@@ -18,40 +18,6 @@ __device__ __forceinline__ void block_of(int b, int blocks_m, int blocks_n, int*
   *bm = band * kBand + in_band - *bn * high;
 }
 
-// Four columns can be written at a time.
-__device__ __forceinline__ bool wide_stores(const GemmArgs& a) {
-  return !a.bias && a.beta == 0.0f && a.ld_y % 4 == 0 && reinterpret_cast<uintptr_t>(a.y) % 16 == 0;
-}
-
-// Four outputs at y[at] without bias and beta: write_out four columns at a time (rf: the row factors).
-template <class Acc>
-__device__ __forceinline__ void write_four(const GemmArgs& a, int64_t at, const Acc& sums, const float (&rf)[4]) {
-  f32x4 v;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) v[r] = a.alpha * (rf[r] * static_cast<float>(sums[r]));
-  if (a.y_dtype == LX_F32) {
-    *reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + at) = v;
-  } else {
-    const bf16x2 p[2] = {pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
-    *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.y) + at) = __builtin_bit_cast(u32x2, p);
-  }
-}
-
-// Columns n .. n + 3 of row m (of the matrix), as far as they exist, one at a time.
-template <class Acc>
-__device__ __forceinline__ void write_each(const GemmArgs& a, int m, int n, const Acc& sums, const float (&rf)[4]) {
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-    if (n + r < a.N) {
-      float t = rf[r] * static_cast<float>(sums[r]);
-      if (a.bias) t += a.bias_dtype == LX_F32 ? static_cast<const float*>(a.bias)[n + r] : load_as_f32(a.bias, a.bias_dtype, n + r);
-      float v = a.alpha * t;
-      const int64_t at = m * a.ld_y + n + r;
-      if (a.beta != 0.0f) v = a.beta * load_as_f32(a.y, a.y_dtype, at) + v;
-      store_from_f32(a.y, a.y_dtype, at, v);
-    }
-}
-
 // The activation row's factor: its scale under a quantised math.
 template <bool BYTES>
 __device__ __forceinline__ float row_scale(const GemmArgs& a, int m) {

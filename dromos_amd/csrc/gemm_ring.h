@@ -1,0 +1,301 @@
+// lx_gemm_w for a decode step's rows (up to 64) on wide matrices, on block_wide.h's loads: a workgroup takes all of the activation
+// rows by BN weight rows, its four wavefronts KS slices of K by 4 / KS parts of the columns. Weights and activations go from memory
+// into a ring in LDS that belongs to the wavefront (KS = 4: nothing is shared and nobody waits for anybody) or to the wavefronts of
+// a slice. The slices' sums meet in LDS and are added in ascending order; the bits are the other kernels' (tile_mfma.h).
+//
+// Bound by bytes on their way: a unit's ring holds 80 .. 160 KB of which the activations, which every workgroup reads anew from
+// its die's L2, are the larger part from 32 rows on (fp8 14336 x 4096 at 64 rows, 23 us: 17 with the weights alone loaded, 13 with the
+// activations alone; the order of a row's lanes, the row stride and the activations asked for ahead make no difference). The
+// kernels that stage windows of the activations through registers for all wavefronts (gemm_walk.h) stay ahead up to 16 rows. Where:
+// gemm.hip, ring_cols().
+#pragma once
+
+#include "block_wide.h"
+#include "gemm_args.h"
+
+namespace dro {
+namespace ring {
+
+using block::Rsrc;
+using block::load_to_lds16;
+using block::load_to_lds4;
+using block::wait_loads;
+
+template <int F, int MT, int KS, int BN>
+struct Ring {
+  static constexpr bool kNv = F == LX_W_NVFP4, kRaw = F == LX_W_BF16;
+  static constexpr int kWaves = 4, kThreads = kWaves * kWave, WN = kWaves / KS, NT = BN / 16 / WN;
+  static_assert(NT >= 1, "a tile of weight rows a wavefront at least");
+  static constexpr int BM = MT * 16;
+  static constexpr int kSteps = kRaw ? 2 : 1;  // load steps a stage
+  static constexpr int J = kNv ? 4 : 2;
+  static constexpr int kXRow = kNv ? 256 : 128, kWRow = kRaw ? 128 : 64;
+  // Wave-sized loads a stage and wavefront: its part of its slice's activations, its own weights and block scales.
+  static constexpr int kXLoads = (BM * kXRow / 1024 + WN - 1) / WN, kWLoads = NT * 16 * kWRow / 1024, kSLoads = kNv ? (NT + 1) / 2 : 0;
+  static constexpr int kLoads = kXLoads + kWLoads + kSLoads;
+  static constexpr int kXBytes = kXLoads * WN * 1024, kWBytes = kWLoads * 1024, kOwn = kWBytes + kSLoads * 256;
+  static constexpr int kStage = KS * kXBytes + kWaves * kOwn;
+  static constexpr int fit(int a, int b) { return a < b ? a : b; }
+  static constexpr int kStages = fit(fit(160 * 1024 / kStage, 8), 63 / kLoads + 2);
+  static constexpr bool kFits = kStages >= 2;
+  static constexpr int kSums = KS * BM * BN * 4;
+  static constexpr int kLdsBytes = kStages * kStage > kSums ? kStages * kStage : kSums;
+};
+
+template <int F, int MT, int KS, int BN>
+__global__ void __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(1, 2))) ring_kernel(const GemmArgs a, int slices) {
+  using R = Ring<F, MT, KS, BN>;
+  constexpr int WN = R::WN, NT = R::NT, J = R::J, kStages = R::kStages, kLoads = R::kLoads;
+  extern __shared__ __align__(16) f32x4 lds4[];
+  uint8_t* const lds = reinterpret_cast<uint8_t*>(lds4);
+  const uint32_t lds_at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds)));
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), g = lane >> 4, i = lane & 15;
+  const int ks = wave % KS, wn = wave / KS;
+  const int n0 = blockIdx.x * BN, cols = min(BN, a.N - n0);
+  const int xbytes = a.K * 2, wbytes = static_cast<int>(a.row_bytes), sbytes = a.K / 16;
+  const int64_t ld = a.xs.ld * 2;
+  const Rsrc xbuf = block::buffer_of(a.xs.x, (a.M - 1) * ld + xbytes), wbuf = block::buffer_of(a.w + n0 * a.row_bytes, cols * a.row_bytes),
+             sbuf = block::buffer_of(R::kNv ? a.scale + n0 * a.scale_row_bytes : a.scale, cols * a.scale_row_bytes);
+  // This slice's stages (all slices walk as many; what lies past the row's end is zero), and the last one with anything in it.
+  const int per = a.steps_per_wave / R::kSteps, first = ks * per, end = (a.steps + R::kSteps - 1) / R::kSteps - 1;
+  uint32_t xrow[R::kXLoads], wrow[R::kWLoads], srow[R::kSLoads > 0 ? R::kSLoads : 1];
+  int xpiece = 0, wpiece = 0;
+  const int spiece = (lane & 1) * 4;
+  // Places in a row as in block_wide.h: slot s of activation row r holds place s ^ r (instruction p / 4's, lane group p % 4's); of a
+  // weight row piece s ^ (r / 2), of a bf16 weight row s ^ r.
+#pragma unroll
+  for (int u = 0; u < R::kXLoads; ++u) {
+    constexpr int kSlots = R::kXRow / 16;
+    const int at = (u * WN + wn) * kWave + lane, row = at / kSlots, place = (at ^ row) % kSlots;
+    xpiece = (R::kRaw ? place : J * (place & 3) + (place >> 2)) * 16;
+    xrow[u] = static_cast<uint32_t>(min(row, a.M - 1)) * static_cast<uint32_t>(ld) + xpiece;
+  }
+#pragma unroll
+  for (int u = 0; u < R::kWLoads; ++u) {
+    constexpr int kSlots = R::kWRow / 16;
+    const int at = u * kWave + lane, row = at / kSlots;
+    wpiece = ((at % kSlots) ^ (R::kRaw ? row & 7 : (row >> 1) & 3)) * 16;
+    wrow[u] = static_cast<uint32_t>(min(wn * NT * 16 + row, cols - 1)) * static_cast<uint32_t>(wbytes) + wpiece;
+  }
+#pragma unroll
+  for (int u = 0; u < R::kSLoads; ++u)
+    srow[u] = static_cast<uint32_t>(min(wn * NT * 16 + min(u * 32 + (lane >> 1), NT * 16 - 1), cols - 1)) * static_cast<uint32_t>(a.scale_row_bytes) + spiece;
+  const uint32_t x_at = ks * R::kXBytes, own_at = KS * R::kXBytes + wave * R::kOwn;  // in a stage
+  // Load u of the slice's stage st: what lies past the row's end is asked for at its start (its last stage's) and zeroed by finish().
+  auto load = [&](int st, int slot, int u) {
+    const int t = min(first + st, end);
+    const uint32_t to = lds_at + slot * R::kStage;
+    if (u < R::kWLoads) {
+      load_to_lds16(to + own_at + u * 1024, wrow[u] - (wpiece + t * R::kWRow >= wbytes ? wpiece : 0), wbuf, t * R::kWRow);
+    } else if (u < R::kWLoads + R::kSLoads) {
+      load_to_lds4(to + own_at + R::kWBytes + (u - R::kWLoads) * 256, srow[u - R::kWLoads] - (spiece + t * 8 >= sbytes ? spiece : 0), sbuf, t * 8);
+    } else {
+      const int v = u - R::kWLoads - R::kSLoads;
+      load_to_lds16(to + x_at + (v * WN + wn) * 1024, xrow[v] - (xpiece + t * R::kXRow >= xbytes ? xpiece : 0), xbuf, t * R::kXRow);
+    }
+  };
+  auto finish = [&](int st, int slot) {
+    uint8_t* const to = lds + slot * R::kStage;
+    const int t = first + st;
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    if (xpiece + static_cast<int64_t>(t) * R::kXRow >= xbytes) {
+#pragma unroll
+      for (int u = 0; u < R::kXLoads; ++u) *reinterpret_cast<u32x4*>(to + x_at + (u * WN + wn) * 1024 + lane * 16) = zero;
+    }
+    if (wpiece + static_cast<int64_t>(t) * R::kWRow >= wbytes) {
+#pragma unroll
+      for (int u = 0; u < R::kWLoads; ++u) *reinterpret_cast<u32x4*>(to + own_at + u * 1024 + lane * 16) = zero;
+    }
+#pragma unroll
+    for (int u = 0; u < R::kSLoads; ++u) {
+      uint8_t* const s = to + own_at + R::kWBytes + u * 256 + lane * 4;
+      if (spiece + t * 8 >= sbytes) *reinterpret_cast<uint32_t*>(s) = 0;
+      else if (spiece + t * 8 + 2 >= sbytes) *reinterpret_cast<uint16_t*>(s + 2) = 0;
+    }
+  };
+  uint32_t xat[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) xat[j] = x_at + i * R::kXRow + ((4 * j + g) ^ (i % (R::kXRow / 16))) * 16;
+  const uint32_t wat = own_at + i * R::kWRow + (R::kRaw ? g ^ (i & 7) : g ^ ((i >> 1) & 3)) * 16, sat = own_at + R::kWBytes + i * 8 + g * 2;
+  f32x4 acc[NT][MT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 raw[NT], wf[2][NT], xf[2][MT];
+  uint32_t sc[NT];
+  auto fetch_raw = [&](const uint8_t* st, int nt) {
+    sc[nt] = 0;
+    if constexpr (!R::kRaw) raw[nt] = *reinterpret_cast<const u32x4*>(st + wat + nt * 16 * R::kWRow);
+    if constexpr (R::kNv) sc[nt] = *reinterpret_cast<const uint16_t*>(st + sat + nt * 128);
+  };
+  auto fetch_w = [&](u32x4(&w)[NT], const uint8_t* st, int j, int nt) {
+    if constexpr (R::kRaw) w[nt] = *reinterpret_cast<const u32x4*>(st + (wat ^ (j ? 64 : 0)) + nt * 16 * R::kWRow);
+    else
+#pragma unroll
+      for (int p = 0; p < 4; ++p) w[nt][p] = block::weight_pair<F>(raw[nt], sc[nt], j, p);
+  };
+  auto fetch_x = [&](u32x4(&x)[MT], const uint8_t* st, int j, int mt) { x[mt] = *reinterpret_cast<const u32x4*>(st + xat[j] + mt * 16 * R::kXRow); };
+  // Stage st is here: this wavefront's loads, and the others' of the slice.
+  auto arrive = [&](auto steady, int st, int slot) {
+    if constexpr (decltype(steady)::value) {
+      wait_loads<(kStages - 2) * kLoads>();
+    } else {
+      const int behind = min(per - 1 - st, kStages - 2);
+      if (behind == kStages - 2) wait_loads<(kStages - 2) * kLoads>();
+      else if (behind == 1) wait_loads<kLoads>();
+      else if (kStages > 4 && behind == 2) wait_loads<(kStages > 4 ? 2 : 0) * kLoads>();
+      else if (kStages > 5 && behind == 3) wait_loads<(kStages > 5 ? 3 : 0) * kLoads>();
+      else if (kStages > 6 && behind == 4) wait_loads<(kStages > 6 ? 4 : 0) * kLoads>();
+      else if (kStages > 7 && behind == 5) wait_loads<(kStages > 7 ? 5 : 0) * kLoads>();
+      else wait_loads<0>();
+    }
+    if (first + st >= end) {  // (the row may end inside it, or before it)
+      finish(st, slot);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    if constexpr (WN > 1) asm volatile("s_barrier" ::: "memory");
+  };
+  // All workgroups walk K together, so an activation row's next piece would come from memory for every one of them. The workgroups
+  // of a die (every eighth) share out the activations' 128-byte lines and ask for them once, at the start: the walk then finds
+  // them in the die's L2. (Into the ring's last slot, which is not in use before these have arrived.) NVFP4 8192 x 8192 at
+  // 33 rows 23.7 -> 22.8 us; one-byte weights lose 4 .. 6 %.
+  if constexpr (R::kNv) {
+    const int line_row = (xbytes + 127) / 128, lines = line_row * a.M, share = (lines + (gridDim.x >> 3)) / ((gridDim.x >> 3) + 1);
+    for (int at = static_cast<int>(threadIdx.x); at - lane < share; at += R::kThreads) {
+      const int line = min(static_cast<int>(blockIdx.x >> 3) * share + min(at, share - 1), lines - 1), row = line / line_row;
+      load_to_lds4(lds_at + (kStages - 1) * R::kStage + wave * 256, static_cast<uint32_t>(row) * static_cast<uint32_t>(ld) + (line - row * line_row) * 128, xbuf, 0);
+    }
+  }
+#pragma unroll
+  for (int st = 0; st < kStages - 1; ++st)
+    if (st < per) {
+#pragma unroll
+      for (int u = 0; u < kLoads; ++u) load(st, st, u);
+    }
+  arrive(std::false_type{}, 0, 0);
+  if (kStages - 1 < per) {
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) load(kStages - 1, kStages - 1, u);
+  }
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    fetch_raw(lds, nt);
+    fetch_w(wf[0], lds, 0, nt);
+  }
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) fetch_x(xf[0], lds, 0, mt);
+  int slot = 0;
+  // As block_wide.h's step: under an instruction's products the next one's fragments are read and expanded.
+  auto step = [&](auto steady, int st) {
+    const int next = slot + 1 == kStages ? 0 : slot + 1;
+    const uint8_t *const here = lds + slot * R::kStage, *const there = lds + next * R::kStage;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const bool last = j == J - 1;
+      const uint8_t* const from = last ? there : here;
+      __builtin_amdgcn_sched_barrier(0);
+      if (last) {
+        if (decltype(steady)::value || st + 1 < per) arrive(steady, st + 1, next);
+        if constexpr (decltype(steady)::value) {
+#pragma unroll
+          for (int u = 0; u < kLoads; ++u) load(st + kStages, slot, u);
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) fetch_raw(from, nt);
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) fetch_x(xf[(j + 1) & 1], from, (j + 1) % J, mt);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[j & 1][nt]), __builtin_bit_cast(bf16x8, xf[j & 1][mt]), acc[nt][mt], 0, 0, 0);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) fetch_w(wf[(j + 1) & 1], from, (j + 1) % J, nt);
+#pragma unroll
+      for (int n = 0; n < MT * NT; ++n) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, R::kNv ? 4 : 3, 0);
+      }
+    }
+    slot = next;
+  };
+  int st = 0;
+  for (; st + kStages < per; ++st) step(std::true_type{}, st);
+  for (; st < per; ++st) step(std::false_type{}, st);
+  __builtin_amdgcn_sched_barrier(0);
+  // The slices' sums side by side in LDS, a row's pieces of four turned by the row; then everyone adds up what it writes.
+  constexpr int kPieces = BN / 4, kSlice = R::BM * BN * 4;
+  __syncthreads();
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      *reinterpret_cast<f32x4*>(lds + ks * kSlice + (mt * 16 + i) * BN * 4 + ((((wn * NT + nt) * 4 + g) ^ i) & (kPieces - 1)) * 16) = acc[nt][mt];
+  __syncthreads();
+  const int piece = threadIdx.x % kPieces, n = 4 * piece;
+  if (n >= cols) return;
+  const bool wide = wide_stores(a) && n + 3 < cols;
+  constexpr int kRows = R::kThreads / kPieces, kTimes = (R::BM + kRows - 1) / kRows;
+  float rf[4], xs[kTimes];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) rf[r] = row_factor(F, a.scale, a.global, n0 + min(n + r, cols - 1));
+#pragma unroll
+  for (int q = 0; q < kTimes; ++q) xs[q] = a.act_scale ? a.act_scale[min(static_cast<int>(threadIdx.x) / kPieces + q * kRows, a.M - 1)] : 1.0f;
+#pragma unroll
+  for (int q = 0; q < kTimes; ++q) {
+    const int m = threadIdx.x / kPieces + q * kRows;
+    if (m >= a.M || m >= R::BM) break;
+    const uint8_t* const at = lds + m * BN * 4 + ((piece ^ (m & 15)) & (kPieces - 1)) * 16;
+    f32x4 s = *reinterpret_cast<const f32x4*>(at);
+#pragma unroll
+    for (int k = 1; k < KS; ++k)
+      if (k < slices) s += *reinterpret_cast<const f32x4*>(at + k * kSlice);
+    float f[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) f[r] = rf[r] * xs[q];
+    if (wide) write_four(a, m * a.ld_y + n0 + n, s, f);
+    else write_each(a, m, n0 + n, s, f);
+  }
+}
+
+template <int F, int MT, int KS, int BN>
+int launch(const GemmArgs& a, int slices, hipStream_t stream) {
+  using R = Ring<F, MT, KS, BN>;
+  const auto kernel = ring_kernel<F, MT, KS, BN>;
+  allow_lds(reinterpret_cast<const void*>(kernel), R::kLdsBytes);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((a.N + BN - 1) / BN)), dim3(R::kThreads), R::kLdsBytes, stream, a, slices);
+  return status_of(hipGetLastError());
+}
+
+// The launch for `cols` (32 or 64) weight rows a workgroup; false where the slices are too many.
+template <int F>
+bool launch_ring(const GemmArgs& a, int cols, int* status, hipStream_t stream) {
+  const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave;
+  auto rows = [&](auto mt) {
+    constexpr int MT = decltype(mt)::value;
+    if (slices < 2 || slices > 4) return false;
+    if (slices > 2) {
+      if constexpr (Ring<F, MT, 4, 64>::kFits)
+        if (cols == 64) {
+          *status = launch<F, MT, 4, 64>(a, slices, stream);
+          return true;
+        }
+      *status = launch<F, MT, 4, 32>(a, slices, stream);
+    } else {
+      *status = cols == 32 ? launch<F, MT, 2, 32>(a, slices, stream) : launch<F, MT, 2, 64>(a, slices, stream);
+    }
+    return true;
+  };
+  switch ((a.M + 15) / 16) {
+    case 1: return rows(std::integral_constant<int, 1>{});
+    case 2: return rows(std::integral_constant<int, 2>{});
+    case 3: return rows(std::integral_constant<int, 3>{});
+    default: return rows(std::integral_constant<int, 4>{});
+  }
+}
+
+}  // namespace ring
+}  // namespace dro
