@@ -37,7 +37,7 @@ __device__ __forceinline__ int die_order(int b, int total) {
 // (128 of 4096 x 1536, a pass of the layer) 1476 -> 1388 us; lx_gemm_w's blocks of 128 x 128 are 4 % faster without (fp8 14336 x
 // 4096 at 4096 rows 552 / 573, int8 math 4096 x 11008 at 515 rows 162 / 165).
 // With SPLIT a 128 x 256 block holds two sets of 64 sums a lane and does not fit 256 registers: the compiler spills 84 .. 200 of
-// them (116 .. 180 bytes a lane: the experts in every format, lx_gemm_w's on NVFP4 and under the FP8 math), moved where a slice ends. No
+// them (116 .. 180 bytes a lane: the experts in bf16 and NVFP4, lx_gemm_w's on NVFP4 and under the FP8 math), moved where a slice ends. No
 // other block spills.
 template <int F, int MATH, int WM, int WN, int MT, int NT, bool SPLIT, bool ONE_X = false>
 struct Block {
