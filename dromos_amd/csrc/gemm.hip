@@ -16,6 +16,7 @@
 
 #include "common.h"
 #include "gemm_block_plan.h"
+#include "gemm_ring.h"
 #include "tile_mfma.h"
 
 namespace dro {
@@ -1842,6 +1843,42 @@ LX_API int dromos_plan_gemm(int format, int math, int M, int N, int K, int units
       if (math == LX_MATH_FP8) return ask(std::integral_constant<int, LX_W_FP8>{}, std::integral_constant<int, LX_MATH_FP8>{});
       return ask(std::integral_constant<int, LX_W_FP8>{}, bf16);
     default: return ask(std::integral_constant<int, LX_W_NVFP4>{}, bf16);
+  }
+}
+
+// The same of the ring kernel, for a pass of up to 64 bf16 rows under the BF16 math: 8 * its weight rows a workgroup + the slices of K, or
+// 0 where another kernel takes it. lds, if given: thirteen numbers, the bytes of a stage of its ring and for each of its four
+// wavefronts where its look-ahead goes, where its own part begins and how many bytes that has.
+LX_API int dromos_plan_ring(int format, int M, int N, int K, int units, int buffer, int* lds) {
+  if (M < 1 || M > 64 || dromos_plan_gemm(format, LX_MATH_BF16, M, N, K, units, buffer) >= 0) return 0;
+  auto ask = [&](auto f) {
+    GemmArgs a{};
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    cut_rows<f()>(a);
+    const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave;
+    int plan = 0;
+    const int cols = tuned_variant(gemm_key<f()>(), M, N, K) >= 0 ? 0 : ring_cols<f()>(a, (N + kTileRows - 1) / kTileRows);
+    if (cols > 0)
+      ring::with_ring<f()>(M, slices, cols, [&](auto ring) {
+        using R = decltype(ring);
+        plan = 8 * R::BN + slices;
+        if (!lds) return;
+        *lds = R::kStage;
+        for (int w = 0; w < R::kWaves; ++w) {
+          lds[1 + 3 * w] = R::ahead_at(w);
+          lds[2 + 3 * w] = R::own_at(w);
+          lds[3 + 3 * w] = R::kOwn;
+        }
+      });
+    return plan;
+  };
+  switch (format) {
+    case LX_W_BF16: return ask(std::integral_constant<int, LX_W_BF16>{});
+    case LX_W_INT8: return ask(std::integral_constant<int, LX_W_INT8>{});
+    case LX_W_FP8: return ask(std::integral_constant<int, LX_W_FP8>{});
+    default: return ask(std::integral_constant<int, LX_W_NVFP4>{});
   }
 }
 

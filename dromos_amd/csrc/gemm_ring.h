@@ -21,8 +21,9 @@ using block::load_to_lds16;
 using block::load_to_lds4;
 using block::wait_loads;
 
-template <int F, int MT, int KS, int BN>
+template <int F, int MT_, int KS_, int BN_>
 struct Ring {
+  static constexpr int MT = MT_, KS = KS_, BN = BN_;
   static constexpr bool kNv = F == LX_W_NVFP4, kRaw = F == LX_W_BF16;
   static constexpr int kWaves = 4, kThreads = kWaves * kWave, WN = kWaves / KS, NT = BN / 16 / WN;
   static_assert(NT >= 1, "a tile of weight rows a wavefront at least");
@@ -35,6 +36,12 @@ struct Ring {
   static constexpr int kLoads = kXLoads + kWLoads + kSLoads;
   static constexpr int kXBytes = kXLoads * WN * 1024, kWBytes = kWLoads * 1024, kOwn = kWBytes + kSLoads * 256;
   static constexpr int kStage = KS * kXBytes + kWaves * kOwn;
+  // Where in a stage: a slice's activations, which its WN wavefronts load and read; what one wavefront alone loads and reads; and
+  // (NVFP4, in the ring's last stage) where a wavefront's look-ahead goes, 256 bytes.
+  static constexpr int x_at(int ks) { return ks * kXBytes; }
+  static constexpr int own_at(int wave) { return KS * kXBytes + wave * kOwn; }
+  static constexpr int ahead_at(int wave) { return own_at(wave); }
+  static_assert(kOwn >= 256, "room for a look-ahead");
   static constexpr int fit(int a, int b) { return a < b ? a : b; }
   static constexpr int kStages = fit(fit(160 * 1024 / kStage, 8), 63 / kLoads + 2);
   static constexpr bool kFits = kStages >= 2;
@@ -80,7 +87,7 @@ __global__ void __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
   for (int u = 0; u < R::kSLoads; ++u)
     srow[u] = static_cast<uint32_t>(min(wn * NT * 16 + min(u * 32 + (lane >> 1), NT * 16 - 1), cols - 1)) * static_cast<uint32_t>(a.scale_row_bytes) + spiece;
-  const uint32_t x_at = ks * R::kXBytes, own_at = KS * R::kXBytes + wave * R::kOwn;  // in a stage
+  const uint32_t x_at = R::x_at(ks), own_at = R::own_at(wave);  // in a stage
   // Load u of the slice's stage st: what lies past the row's end is asked for at its start (its last stage's) and zeroed by finish().
   auto load = [&](int st, int slot, int u) {
     const int t = min(first + st, end);
@@ -158,13 +165,14 @@ __global__ void __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(
   };
   // All workgroups walk K together, so an activation row's next piece would come from memory for every one of them. The workgroups
   // of a die (every eighth) share out the activations' 128-byte lines and ask for them once, at the start: the walk then finds
-  // them in the die's L2. (Into the ring's last slot, which is not in use before these have arrived.) NVFP4 8192 x 8192 at
+  // them in the die's L2. They land in the wavefront's own part of the ring's last slot: with a slice a wavefront nobody waits for
+  // anybody else's loads, and its own stage kStages - 1 is asked for behind a wait for these. NVFP4 8192 x 8192 at
   // 33 rows 23.7 -> 22.8 us; one-byte weights lose 4 .. 6 %.
   if constexpr (R::kNv) {
     const int line_row = (xbytes + 127) / 128, lines = line_row * a.M, share = (lines + (gridDim.x >> 3)) / ((gridDim.x >> 3) + 1);
     for (int at = static_cast<int>(threadIdx.x); at - lane < share; at += R::kThreads) {
       const int line = min(static_cast<int>(blockIdx.x >> 3) * share + min(at, share - 1), lines - 1), row = line / line_row;
-      load_to_lds4(lds_at + (kStages - 1) * R::kStage + wave * 256, static_cast<uint32_t>(row) * static_cast<uint32_t>(ld) + (line - row * line_row) * 128, xbuf, 0);
+      load_to_lds4(lds_at + (kStages - 1) * R::kStage + R::ahead_at(wave), static_cast<uint32_t>(row) * static_cast<uint32_t>(ld) + (line - row * line_row) * 128, xbuf, 0);
     }
   }
 #pragma unroll
@@ -261,40 +269,46 @@ __global__ void __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(
   }
 }
 
-template <int F, int MT, int KS, int BN>
+template <class R, int F>
 int launch(const GemmArgs& a, int slices, hipStream_t stream) {
-  using R = Ring<F, MT, KS, BN>;
-  const auto kernel = ring_kernel<F, MT, KS, BN>;
+  const auto kernel = ring_kernel<F, R::MT, R::KS, R::BN>;
   allow_lds(reinterpret_cast<const void*>(kernel), R::kLdsBytes);
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((a.N + BN - 1) / BN)), dim3(R::kThreads), R::kLdsBytes, stream, a, slices);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((a.N + R::BN - 1) / R::BN)), dim3(R::kThreads), R::kLdsBytes, stream, a, slices);
   return status_of(hipGetLastError());
 }
 
-// The launch for `cols` (32 or 64) weight rows a workgroup; false where the slices are too many.
-template <int F>
-bool launch_ring(const GemmArgs& a, int cols, int* status, hipStream_t stream) {
-  const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave;
+// fn(the Ring for M rows in `slices` slices with `cols` (32 or 64) weight rows a workgroup); false where the slices are too many.
+template <int F, class Fn>
+bool with_ring(int M, int slices, int cols, Fn&& fn) {
   auto rows = [&](auto mt) {
     constexpr int MT = decltype(mt)::value;
     if (slices < 2 || slices > 4) return false;
     if (slices > 2) {
       if constexpr (Ring<F, MT, 4, 64>::kFits)
         if (cols == 64) {
-          *status = launch<F, MT, 4, 64>(a, slices, stream);
+          fn(Ring<F, MT, 4, 64>{});
           return true;
         }
-      *status = launch<F, MT, 4, 32>(a, slices, stream);
+      fn(Ring<F, MT, 4, 32>{});
+    } else if (cols == 32) {
+      fn(Ring<F, MT, 2, 32>{});
     } else {
-      *status = cols == 32 ? launch<F, MT, 2, 32>(a, slices, stream) : launch<F, MT, 2, 64>(a, slices, stream);
+      fn(Ring<F, MT, 2, 64>{});
     }
     return true;
   };
-  switch ((a.M + 15) / 16) {
+  switch ((M + 15) / 16) {
     case 1: return rows(std::integral_constant<int, 1>{});
     case 2: return rows(std::integral_constant<int, 2>{});
     case 3: return rows(std::integral_constant<int, 3>{});
     default: return rows(std::integral_constant<int, 4>{});
   }
+}
+
+template <int F>
+bool launch_ring(const GemmArgs& a, int cols, int* status, hipStream_t stream) {
+  const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave;
+  return with_ring<F>(a.M, slices, cols, [&](auto ring) { *status = launch<decltype(ring), F>(a, slices, stream); });
 }
 
 }  // namespace ring
