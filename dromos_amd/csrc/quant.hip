@@ -20,6 +20,9 @@ __device__ __forceinline__ float e4m3_decode(uint32_t b) {
   return (b & 0x80u) ? -v : v;
 }
 
+// Whether one of four e4m3 codes is 0x7f or 0xff. (No carry leaves a byte.)
+__device__ __forceinline__ bool has_nan_code(uint32_t d) { return (((d & 0x7f7f7f7fu) + 0x01010101u) & 0x80808080u) != 0; }
+
 // f32 -> e4m3fn, nearest even, saturating at 448, NaN -> 0x7f with the sign (engine/cpu/quant.cpp:20-39).
 __device__ __forceinline__ uint32_t e4m3_encode(float f) {
   uint32_t u = __float_as_uint(f);
@@ -468,6 +471,11 @@ __global__ void __launch_bounds__(kThreads) act_values_rows_kernel(const uint8_t
     const u32x2 w = *reinterpret_cast<const u32x2*>(q + m * ld_q + k0);
     decode_dword<MATH == LX_MATH_INT8 ? LX_W_INT8 : LX_W_FP8>(w.x, v);
     decode_dword<MATH == LX_MATH_INT8 ? LX_W_INT8 : LX_W_FP8>(w.y, v + 4);
+    // A NaN's codes 0x7f / 0xff read as +-480 (e4m3_decode), which the conversion instruction does not know.
+    if (MATH == LX_MATH_FP8 && __builtin_expect(has_nan_code(w.x) | has_nan_code(w.y), 0)) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = e4m3_decode(w[j >> 2] >> (8 * (j & 3)) & 0xffu);
+    }
   }
   uint32_t h[4];
 #pragma unroll

@@ -12,7 +12,7 @@ import checks
 import ops
 from conftest import rel_l2
 from dromos_amd.abi import FORMATS, MATH_BF16, MATH_FP4, MATH_FP8, MATH_INT8
-from dromos_amd.formats import master_weight, quantize_with, random_weight
+from dromos_amd.formats import Weight, master_weight, quantize_with, random_weight
 
 pytestmark = pytest.mark.gpu
 FMT = checks.FMT_NAMES
@@ -257,6 +257,23 @@ def test_nvfp4_maths_rows_do_not_depend_on_the_batch(hip, math):
     for M in (1, 7, 16, 33):
         part = ops.gemm_w(hip, x[:M].contiguous(), w, math)
         assert torch.equal(part, full[:M]), M
+
+
+# Every e4m3 code an activation can be quantised to, against identity weights: a NaN's codes 0x7f / 0xff count as +-480, as the
+# oracle has it (engine/cpu/quant.cpp:12-18), whichever kernel expands them.
+@pytest.mark.parametrize("M", [1, 20, 130])
+@pytest.mark.parametrize("x_dtype", [torch.float32, torch.bfloat16])
+def test_fp8_math_on_every_activation_code(hip, oracle, M, x_dtype):
+    codes = torch.arange(256, dtype=torch.int32).to(torch.uint8)
+    values = codes.view(torch.float8_e4m3fn).float()
+    values[0x7F], values[0xFF] = float("nan"), -float("nan")
+    x = values.to(x_dtype).repeat(M, 1)  # the largest is 448: the row's scale is 1
+    data = torch.zeros(256, 128, dtype=torch.uint8)
+    data[torch.arange(256), torch.arange(256) // 2] = torch.tensor([0x02, 0x20], dtype=torch.uint8).repeat(128)  # e2m1 1.0
+    w = Weight(FORMATS["nvfp4"], data, torch.full((256, 16), 0x38, dtype=torch.uint8), glob=1.0)
+    want = ops.gemm_w(oracle, x, w, MATH_FP8)
+    assert want[0, 0x7F].abs() == 480 and torch.equal(want[0, :0x7F], values[:0x7F])
+    assert torch.equal(ops.gemm_w(hip, x.cuda(), w.to("cuda"), MATH_FP8).cpu(), want)
 
 
 def test_c3_shape_under_the_fp4_math(hip, oracle):

@@ -155,6 +155,21 @@ def test_grouped_under_a_math_against_the_oracle(hip, oracle, fmt, math, T, L, I
     assert err <= 1e-2 and err <= (1e-2 if math == MATH_FP4 else 3e-3), err
 
 
+# A NaN among the latents: its token's output is the oracle's (whose codes 0x7f / 0xff count as +-480), the others' what they were.
+# (Not the FP4 math: a NaN's e2m1 code is 6 on the device and 0 in the oracle.)
+@pytest.mark.parametrize("fmt,math", [("int8", MATH_INT8), ("fp8", MATH_FP8), ("nvfp4", MATH_FP8)])
+def test_grouped_under_a_math_with_a_nan(hip, oracle, fmt, math):
+    L, I, E, top_k = 256, 128, 4, 2
+    latent, ids, weights, gu, dn = make(fmt, 24, L, I, E, top_k, 5 + math)
+    clean = ops.experts_grouped(hip, latent, ids, weights, gu, dn, I, E, top_k, math=math)
+    latent[3, 17] = float("nan")
+    got = ops.experts_grouped(hip, latent, ids, weights, gu, dn, I, E, top_k, math=math)
+    want = ops.experts_grouped(oracle, latent.cpu(), ids.cpu(), weights.cpu(), gu.to("cpu"), dn.to("cpu"), I, E, top_k, math=math)
+    others = torch.arange(24) != 3
+    assert torch.equal(got.cpu()[others], clean.cpu()[others])
+    assert rel_l2(got[3], want[3]) <= 3e-3  # (as for finite latents)
+
+
 @pytest.mark.parametrize("fmt,math", GROUPED_MATHS)
 def test_grouped_under_a_math_rows_do_not_depend_on_the_batch(hip, fmt, math):
     L, I, E, top_k = 1024, 512, 32, 4
