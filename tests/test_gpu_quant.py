@@ -119,6 +119,32 @@ def test_quantize_act_equals_the_oracle(hip, oracle, math):
         assert torch.equal(a[2].cpu(), b[2])
 
 
+# NaNs of both signs, infinities, zeros of both signs, values that underflow: rows that are held in registers against rows that are read
+# twice (an odd leading dimension) byte for byte, INT8 and FP8 also against the oracle. (An infinity makes its row's other codes zeros and
+# its own a NaN's, whose sign is the multiplication's, not the format's. A NaN's e2m1 code is 6 here and 0 in the oracle.)
+@pytest.mark.parametrize("x_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("math", [1, 2, 3])
+@pytest.mark.parametrize("K", [2080, 5008, 10000])
+def test_quantize_act_values_that_are_not_finite(hip, oracle, math, x_dtype, K):
+    x = (torch.randn(8, K + 1, generator=torch.Generator().manual_seed(math)) * 3).to(x_dtype)
+    nan, inf = float("nan"), float("inf")
+    x[0, 5], x[0, K - 1], x[1, 17], x[2] = nan, -nan, -nan, nan
+    x[3, 100], x[4, K - 1], x[5, :2] = inf, -inf, torch.tensor([inf, nan])
+    x[6, ::2], x[6, 1::2] = 0.0, -0.0
+    x[7] *= 1e-3
+    x[7, ::16] = -0.0
+    x[7, 1] = 400.0
+    held, twice = (ops.quantize_act(hip, v.cuda(), math, K=K) for v in (x[:, :K].contiguous(), x))
+    for a, b in zip(held, twice):
+        assert a is b or torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    if math != 3:
+        q, scale, _ = ops.quantize_act(oracle, x, math, K=K)
+        ours = held[0].cpu()
+        if math == 2:
+            ours[3:6], q[3:6] = ours[3:6] & 0x7F, q[3:6] & 0x7F
+        assert torch.equal(ours, q) and torch.equal(held[1].cpu().view(torch.int32), scale.view(torch.int32))
+
+
 def test_quantize_act_invalid(hip):
     x = torch.zeros(4, 24, device="cuda")
     assert ops.quantize_act(hip, x, 3, status=True) == 1
