@@ -113,24 +113,28 @@ __global__ void __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(
   for (int h = 0; h < 2; ++h) xs[h] = row_scale<B::kBytes>(a, m0 + min(64 * h + b.lane, rows - 1));
   // (Everything is here: no wait in the loops, where it would be one for the stores too.)
   asm volatile("" ::"v"(rf[0]), "v"(rf[1]), "v"(rf[2]), "v"(rf[3]), "v"(xs[0]), "v"(xs[1]));
+  // (One lane's value each time, and the loops are walked by every lane: a value taken from a lane that is switched off would be
+  // whatever the register allocation left there. Lanes without columns only do not store.)
   auto factors = [&](int m, float(&f)[4]) {
-    // (One lane's value each time: lanes without columns take no part in a choice between two.)
     const uint32_t s0 = __builtin_amdgcn_readlane(__float_as_uint(xs[0]), m & 63), s1 = __builtin_amdgcn_readlane(__float_as_uint(xs[1]), m & 63);
     const float s = __uint_as_float(m < 64 ? s0 : s1);
 #pragma unroll
     for (int r = 0; r < 4; ++r) f[r] = rf[r] * s;
   };
   float f[4];
-  if (wide && n + 3 < cols) {
+  if (wide && cols % 4 == 0) {
 #pragma unroll 4
     for (int m = b.wave; m < rows; m += B::kWaves) {
       factors(m, f);
-      write_four(a, (m0 + m) * a.ld_y + n0 + n, b.sum(m, b.lane), f);
+      const typename B::Acc sums = b.sum(m, b.lane);
+      if (n < cols) write_four(a, (m0 + m) * a.ld_y + n0 + n, sums, f);
     }
-  } else if (n < cols) {
+  } else {
     for (int m = b.wave; m < rows; m += B::kWaves) {
       factors(m, f);
-      write_each(a, m0 + m, n0 + n, b.sum(m, b.lane), f);
+      const typename B::Acc sums = b.sum(m, b.lane);
+      if (wide && n + 3 < cols) write_four(a, (m0 + m) * a.ld_y + n0 + n, sums, f);
+      else if (n < cols) write_each(a, m0 + m, n0 + n, sums, f);
     }
   }
 }
