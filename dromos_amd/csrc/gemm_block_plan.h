@@ -33,17 +33,21 @@ constexpr Shape shape(int i) {
 }
 
 // The wide block (block_wide.h) as a plan's shape: 128 x 256, one wavefront a SIMD, quantised weights. It takes per_stage us a
-// stage of K and per_block us a block besides (its first loads, the sums' way out), and once. Measured on 65 .. 4096 rows, N 1024 ..
-// 16384, K 1024 .. 14336: fp8 14336 x 4096 at 4096 rows 547 us by blocks of 128 x 128, 420 wide; NVFP4 632 / 445, INT8 math 280 / 230,
-// FP8 math 497 / 351. A unit holds one block at a time and a block is a long chain: products of few blocks or short rows stay with
-// the smaller shapes (fp8 2656 x 9600 at 347 rows 48 / 106).
+// stage of K and per_block us a block besides (its first loads, the sums' way out), and once; under the FP8 math the blocks that
+// start together take `first` more a stage. Measured on 65 .. 4096 rows, N 1024 .. 16384, K 1024 .. 14336, whole calls by the blocks of
+// 64 .. 128 x 64 .. 256 and wide: 14336 x 4096 at 4096 rows fp8 582 / 433 us, NVFP4 700 / 497, INT8 math 318 / 285, FP8 math 551 / 387. A
+// unit holds one block at a time and a block is a long chain: products of few blocks or short rows stay with the smaller shapes (fp8
+// 3206 x 11968 at 338 rows 78 / 180, NVFP4 7536 x 3712 at 340 rows 66 / 79). The FP8 math's line was where its estimate of 1.55 a
+// stage put it and kept 14336 x 4096 at 4096 rows from the wide block; of 24 other calls that `first` moved all are ahead (3 .. 35 %:
+// 5194 x 6464 at 3747 rows 286 / 279, 12608 x 3840 at 2471 339 / 221), calls of one block a unit stay (behind: 3352 x 4672 at 1635 83 / 89; ahead:
+// 12070 x 5248 at 456 103 / 92).
 constexpr int kWide = 16;
 struct WideCost {
-  float per_stage, per_block, once;
+  float per_stage, per_block, once, first = 0;
 };
 template <int F, int MATH>
 constexpr WideCost wide_cost() {
-  return MATH == LX_MATH_INT8 ? WideCost{0.82f, 8.5f, 3} : MATH == LX_MATH_FP8 ? WideCost{1.55f, 10, 4} : F == LX_W_NVFP4 ? WideCost{1.65f, 10, 4} : WideCost{0.75f, 8, 4};
+  return MATH == LX_MATH_INT8 ? WideCost{0.82f, 8.5f, 3} : MATH == LX_MATH_FP8 ? WideCost{1.35f, 10, 4, 0.2f} : F == LX_W_NVFP4 ? WideCost{1.65f, 10, 4} : WideCost{0.75f, 8, 4};
 }
 
 // What the wide block is estimated to take, in us; infinite where it does not apply (block scales are loaded four bytes at a time).
@@ -53,7 +57,7 @@ float wide_us(const GemmArgs& a, int units) {
   constexpr WideCost c = wide_cost<F, MATH>();
   const int stages = MATH == LX_MATH_BF16 ? a.steps : (a.steps + 1) / 2;
   const int64_t blocks = static_cast<int64_t>((a.M + 127) / 128) * ((a.N + 255) / 256);
-  return ((blocks + units - 1) / units) * (c.per_stage * stages + c.per_block) + c.once;
+  return ((blocks + units - 1) / units) * (c.per_stage * stages + c.per_block) + c.first * stages + c.once;
 }
 
 // mode: Slices, or -1 where the kernel does not apply. K tiles of a row and of a slice.

@@ -43,6 +43,15 @@ def test_gemm(lib, fmt, math, M, N, K, buffer, taken):
     assert (lib.dromos_plan_gemm(FORMATS[fmt], math, M, N, K, UNITS, buffer) >= 0) == taken
 
 
+# The wide block (shape 16, whole rows or added slices) where it was measured ahead, and not where its blocks are few or a unit's only ones.
+@pytest.mark.parametrize("fmt,math,M,N,K,wide", [
+    ("fp8", 0, 4096, 14336, 4096, True), ("nvfp4", 0, 4096, 14336, 4096, True), ("int8", 1, 4096, 14336, 4096, True), ("fp8", 2, 4096, 14336, 4096, True),
+    ("fp8", 2, 2471, 12608, 3840, True), ("fp8", 2, 1563, 13731, 4176, True), ("fp8", 2, 3708, 3601, 3712, False), ("fp8", 2, 1635, 3352, 4672, False),
+    ("fp8", 2, 1024, 4096, 14336, False), ("int8", 1, 515, 4096, 11008, False), ("fp8", 0, 338, 3206, 11968, False)])
+def test_wide_block(lib, fmt, math, M, N, K, wide):
+    assert (lib.dromos_plan_gemm(FORMATS[fmt], math, M, N, K, UNITS, 1) in (16, 20)) == wide
+
+
 def test_sums_of_slices_that_do_not_fit_the_buffer_stay_in_the_workgroup(lib):
     part = lambda M: lib.dromos_plan_gemm(FORMATS["fp8"], 0, M, 1024, 14336, UNITS, 1) // 4 == 2
     assert part(128) and not lib.dromos_plan_gemm(FORMATS["fp8"], 0, 128, 1024, 14336, UNITS, 0) // 4 == 2
