@@ -1348,29 +1348,58 @@ bool walk_parts_wanted(int M, int n_tiles, int64_t K, int tuned) {
   return K >= mid_k && K < 8192 && n_tiles > 256 && n_tiles <= 384;
 }
 
-// Weight rows a workgroup of the ring kernel (gemm_ring.h) takes, 32 up to 512 tiles and 64 beyond, or 0 where another kernel is
-// ahead. From a sweep on cold weights (176 products of 9 .. 64 rows, 289 .. 1021 tiles, K 2048 .. 14336; ratios are ring to the kernels
-// it replaces). It was not measured outside 289 .. 1024 tiles.
-// - NVFP4 from 17 rows, whose other kernels are short of wavefronts: 0.52 .. 0.93 to K = 4096 (6208 x 2048 at 56 rows 19.8 -> 10.3 us,
-//   7264 x 4096 at 32 rows 17.4 -> 10.4, 9088 x 4096 at 64 rows 36 -> 26), beyond it where the slices fill the wavefronts (8192 values:
-//   0.78 .. 0.81, 11008: 0.75 .. 0.97; three slices of 5120 .. 7168 values for four wavefronts 1.08 .. 1.20). Up to 16 rows 0.98 .. 1.06.
-//   Four slices of 64 rows leave the ring two stages: on 896 tiles, where the walk kernel takes four tiles a workgroup, 28.3 / 29.0.
-// - bf16 on more than 383 tiles: 0.61 .. 0.97 at every row count (7984 x 4096 at 56 rows 33.4 -> 20.3 us, 12048 x 4096 at 32 rows 33.4 ->
-//   24.7, 12512 x 4096 at 9 rows 24.6 -> 20.9); short rows on more than 900 tiles at 64 rows 1.07.
-// - One-byte weights of 4096 .. 8192 values: from 17 rows up to 512 tiles (0.80 .. 0.94, once 1.01: int8 5360 x 4096 at 32 rows 15.5 -> 12.1
-//   us, fp8 7280 x 4096 at 24 rows 13.8 -> 12.1; up to 16 rows 0.80 .. 1.18), beyond 512 tiles from 33 rows, K = 4096 from 49 (0.65 .. 0.95: fp8
-//   8704 x 5120 at 56 rows 46.8 -> 31.2, int8 16192 x 7168 at 40 rows 48.8 -> 42.7; at 24 .. 32 rows 0.91 .. 1.10).
+// Weight rows a workgroup of the ring kernel (gemm_ring.h) takes, or 0 where another kernel is ahead: 32 up to 512 tiles and 64 beyond
+// (NVFP4 at 49 .. 64 rows in three or four slices always 32: two stages of 64 do not fit). From 8000 calls on cold weights that a wider
+// rule took: 9 .. 64 rows, 289 .. 1024 tiles with and without a cut last one, K 2048 .. 11264 in steps of a row's alignment, f32
+// outputs. Ratios are ring to the kernels it replaces, means of groups; outside those sizes it was not measured. What decides besides
+// rows and tiles: whether the activations' rows start on 128-byte lines (a stage takes one line of every row, off the lines two);
+// how much of the slices K fills (every slice walks as many stages); and whole tiles a unit (512, 768 tiles), where the other
+// kernels come out even.
+// - One-byte weights from 17 rows, K 4096 .. 8192. To 384 tiles on lines 0.83 to K = 6144, beyond 1.2 (off the lines to 1.54: fp8 5136 x 7504 at 35
+//   rows 21.3 / 29.9 us). 385 .. 512 tiles: from 33 rows 0.72, fewer on lines 0.87 where the slices are filled, else 0.97 .. 1.03; fp8 on 512 tiles
+//   0.75 .. 0.86 to K = 4096 and 0.77 .. 0.98 from 49 rows from 5120, else to 1.16. More tiles with K a multiple of 512 that fills the slices: 513 .. 767 from 49 rows
+//   0.79 (8784 x 5120 at 54 rows 45.9 / 30.0), from 769 at 33 .. 40 rows 0.88; everything else there 1.06 .. 1.34 (14400 x 6576 at 42 rows 29.5 / 46.4).
+// - bf16 from 384 tiles. To 512, K <= 8192: from 33 rows 0.70, fewer on lines 0.87; on 512 tiles beyond 24 rows only K = 2048, 3072 and 4096
+//   (0.68 .. 1.0, else to 1.12). More tiles on lines: up to 24 rows 0.92 (rows of 16 KB 0.98 .. 1.28), with full slices to 32 rows 0.91 and beyond 0.90 below 768
+//   tiles between 3 K and 8 K; everything else 1.0 .. 1.17 (15010 x 7064 at 56 rows 51.7 / 64.1).
+// - NVFP4 from 17 rows. Rows of a cut load step (K % 128), where the walk kernel does not apply, 0.39 .. 0.73. Whole ones 0.78 where a workgroup takes 32
+//   (K above 4096 on more than 512 tiles, and 768, 1.07) and 0.74 at 33 .. 64 rows to 768 tiles; else 0.95 .. 1.03. Three slices of 5120 .. 7168
+//   values for four wavefronts 1.08 .. 1.20. Four slices of 64 rows leave the ring two stages: on 896 tiles, where the walk kernel
+//   takes four tiles a workgroup, 28.3 / 29.0 (bf16 outputs 30.8 / 28.8).
 template <int F>
 int ring_cols(const GemmArgs& a, int n_tiles) {
   if (a.M <= 8 || n_tiles < 289 || n_tiles > 1024 || a.K < 2048 || a.K > 11264) return 0;
-  const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave, waves = slices > 2 ? 4 : slices;
-  if (slices > 4) return 0;
-  const int cols = n_tiles <= 512 ? 32 : 64;
-  if (F == LX_W_NVFP4 && a.M > 48 && slices > 2 && n_tiles > 768) return 0;
-  if (F == LX_W_NVFP4) return a.M > 16 && (a.K <= 4096 || a.steps * 100 >= a.steps_per_wave * waves * 89) ? cols : 0;
-  if (F == LX_W_BF16) return n_tiles > 383 && (a.K >= 4096 || n_tiles <= 900) ? cols : 0;
-  if (a.K < 4096 || a.K > 8192) return 0;
-  return n_tiles <= 512 ? (a.M > 16 ? cols : 0) : a.M > (a.K == 4096 ? 48 : 32) ? cols : 0;
+  const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave, waves = slices > 2 ? 4 : 2;
+  if (slices < (F == LX_W_NVFP4 ? 2 : 3) || slices > 4) return 0;
+  const int filled = a.steps * 100 / (a.steps_per_wave * waves);  // percent of the slices
+  const bool lines = a.K % 64 == 0 && a.xs.ld % 64 == 0, whole = n_tiles % 256 == 0;
+  if (F == LX_W_NVFP4) {
+    if (a.scale_row_bytes % 4 != 0 || reinterpret_cast<uintptr_t>(a.scale) % 4 != 0) return 0;  // (loaded four bytes at a time)
+    const bool deep = a.M > 48 && slices > 2;
+    if (a.M <= 16 || (a.K > 4096 && filled < 89) || (deep && n_tiles > 768)) return 0;
+    const int cols = n_tiles <= 512 || deep ? 32 : 64;
+    if (a.K % 128 != 0) return cols;
+    return (cols == 32 ? n_tiles <= 512 || (a.K <= 4096 && !whole) : a.M > 32 && n_tiles <= 768) ? cols : 0;
+  }
+  if (F == LX_W_BF16) {
+    if (n_tiles <= 383) return 0;
+    if (n_tiles <= 512) {
+      if (a.K > 8192 || (!lines && (a.M <= 32 || whole))) return 0;
+      return !whole || (a.M <= 24 && a.K < 8192) || (a.K <= 4096 && a.K % 1024 == 0) ? 32 : 0;
+    }
+    if (!lines || a.K % 8192 == 0 || (a.K < 4096 && n_tiles > 900)) return 0;
+    if (a.M <= 32) return a.M <= 24 || filled == 100 ? 64 : 0;
+    return filled == 100 && a.K > 3008 && a.K < 8192 && (n_tiles < 768 || (n_tiles == 768 && a.M <= 40)) ? 64 : 0;
+  }
+  if (a.M <= 16 || a.K < 4096 || a.K > 8192) return 0;
+  if (n_tiles <= 384) return lines && a.K <= 6144 && (a.M > 32 || filled >= 84) ? 32 : 0;
+  if (n_tiles <= 512) {
+    if (whole && F == LX_W_FP8) return lines && (a.K < 4608 || (a.M > 48 && a.K >= 5120 && a.K < 8192)) ? 32 : 0;
+    if (a.M > 32) return (lines || (n_tiles > 400 && !whole)) && (a.K < 8192 || a.M <= 48) ? 32 : 0;
+    return lines && filled > (whole ? 90 : 86) ? 32 : 0;
+  }
+  if (!lines || a.K % 512 != 0 || filled < 83) return 0;
+  return n_tiles < 768 ? (a.M > 48 ? 64 : 0) : n_tiles > 768 && a.M > 32 && a.M <= 40 && a.K > 4096 ? 64 : 0;
 }
 
 // The ring kernel where it is the faster one.
@@ -1379,8 +1408,6 @@ bool try_ring(const GemmArgs& a, int* status, hipStream_t stream) {
   if (a.tuned >= 0 || a.xs.dtype != LX_BF16) return false;
   const int cols = ring_cols<F>(a, (a.N + kTileRows - 1) / kTileRows);
   if (cols == 0 || a.row_bytes * 64 >= (1ll << 31) || a.xs.ld * 2 * 64 >= (1ll << 31)) return false;  // 32-bit offsets
-  // (Block scales are loaded four bytes at a time.)
-  if (F == LX_W_NVFP4 && (a.scale_row_bytes % 4 != 0 || reinterpret_cast<uintptr_t>(a.scale) % 4 != 0)) return false;
   if constexpr (F == LX_W_BF16) return launch_ring_bf16(a, cols, status, stream);
   else if constexpr (F == LX_W_INT8) return launch_ring_int8(a, cols, status, stream);
   else if constexpr (F == LX_W_FP8) return launch_ring_fp8(a, cols, status, stream);
@@ -1856,6 +1883,7 @@ LX_API int dromos_plan_ring(int format, int M, int N, int K, int units, int buff
     a.M = M;
     a.N = N;
     a.K = K;
+    a.xs.ld = K;
     cut_rows<f()>(a);
     const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave;
     int plan = 0;

@@ -277,28 +277,35 @@ int launch(const GemmArgs& a, int slices, hipStream_t stream) {
   return status_of(hipGetLastError());
 }
 
-// fn(the Ring for M rows in `slices` slices with `cols` (32 or 64) weight rows a workgroup); false where the slices are too many.
+// fn(the Ring for M rows in `slices` slices with `cols` (32 or 64) weight rows a workgroup); false where ring_cols() has no such call: only
+// NVFP4 rows are ever cut in two, only bf16 weights taken at 16 rows and fewer, one-byte weights with 64 columns from 33 rows.
 template <int F, class Fn>
 bool with_ring(int M, int slices, int cols, Fn&& fn) {
   auto rows = [&](auto mt) {
     constexpr int MT = decltype(mt)::value;
     if (slices < 2 || slices > 4) return false;
-    if (slices > 2) {
-      if constexpr (Ring<F, MT, 4, 64>::kFits)
-        if (cols == 64) {
-          fn(Ring<F, MT, 4, 64>{});
-          return true;
-        }
-      fn(Ring<F, MT, 4, 32>{});
-    } else if (cols == 32) {
-      fn(Ring<F, MT, 2, 32>{});
-    } else {
-      fn(Ring<F, MT, 2, 64>{});
+    if (slices == 2) {
+      if constexpr (F == LX_W_NVFP4) {
+        if (cols == 32) fn(Ring<F, MT, 2, 32>{});
+        else fn(Ring<F, MT, 2, 64>{});
+        return true;
+      }
+      return false;
     }
-    return true;
+    if (cols == 32) {
+      fn(Ring<F, MT, 4, 32>{});
+      return true;
+    }
+    if constexpr (Ring<F, MT, 4, 64>::kFits && (MT > 2 || F == LX_W_BF16 || F == LX_W_NVFP4)) {
+      fn(Ring<F, MT, 4, 64>{});
+      return true;
+    }
+    return false;
   };
   switch ((M + 15) / 16) {
-    case 1: return rows(std::integral_constant<int, 1>{});
+    case 1:
+      if constexpr (F == LX_W_BF16) return rows(std::integral_constant<int, 1>{});
+      return false;
     case 2: return rows(std::integral_constant<int, 2>{});
     case 3: return rows(std::integral_constant<int, 3>{});
     default: return rows(std::integral_constant<int, 4>{});

@@ -1,6 +1,6 @@
-"""GPU: the ring kernel of lx_gemm_w (up to 64 bf16 rows on wide matrices) against the tile kernels, bit for bit: two, three and four
-slices, 32 and 64 weight rows a workgroup, ragged rows and columns, rows that end inside a stage and inside a slice; the epilogue's
-operands and strides; from a graph as well."""
+"""GPU: the ring kernel of lx_gemm_w (up to 64 bf16 rows on wide matrices) against the tile kernels, bit for bit: every kernel that is
+built (row tiles, two to four slices, 32 and 64 weight rows a workgroup), ragged rows and columns, rows that end inside a stage and inside a slice;
+the epilogue's operands, strides and activation scales; from a graph as well. Every case asks the library first whether the ring takes it."""
 
 import ctypes
 
@@ -8,14 +8,21 @@ import pytest
 import torch
 
 import ops
-from dromos_amd.abi import BF16, DTYPE, F32, FORMATS, MATH_BF16
+from dromos_amd.abi import BF16, DTYPE, F32, FORMATS, MATH_BF16, MATH_FP4, MATH_FP8
 from dromos_amd.formats import random_weight
 
 pytestmark = pytest.mark.gpu
-# N: 290 .. 1000 tiles; K: whole stages, and rows cut short in every format's way.
-CASES = [("nvfp4", m, n, k) for m, n, k in [(17, 4625, 2048), (33, 8190, 2112), (48, 6400, 3136), (64, 14336, 4032), (49, 15999, 4096), (40, 8208, 11008)]]
-CASES += [("bf16", m, n, k) for m, n, k in [(9, 6145, 4096), (16, 8190, 2056), (33, 12001, 4104), (48, 6400, 8200), (64, 14336, 3072)]]
-CASES += [(f, m, n, k) for f in ("int8", "fp8") for m, n, k in [(17, 6145, 4096), (32, 8190, 4112), (48, 7008, 8192), (49, 8705, 4096), (33, 16127, 5136), (64, 14336, 8176)]]
+# Row tiles 1 .. 4; 8 * columns a workgroup + slices.
+CASES = [("nvfp4", *c) for c in [(17, 4625, 2048, 258), (33, 7190, 2048, 258), (63, 7001, 2048, 258), (25, 16007, 2112, 514), (35, 10274, 2048, 514), (51, 11853, 2048, 514),
+                                 (50, 12000, 2112, 259), (40, 8208, 2112, 515), (17, 5201, 3136, 260), (33, 5762, 3136, 260), (64, 8209, 4032, 260), (48, 6400, 4096, 260),
+                                 (24, 11047, 3392, 516), (40, 11047, 3392, 516), (40, 10288, 11008, 516)]]
+CASES += [("bf16", *c) for c in [(9, 7345, 4608, 260), (30, 7414, 6144, 260), (33, 8001, 4104, 260), (64, 7001, 2056, 259), (16, 12293, 2560, 516), (17, 13930, 3072, 516),
+                                 (34, 10109, 3072, 516), (64, 11697, 5120, 516)]]
+CASES += [(f, *c) for f in ("int8", "fp8") for c in [(17, 5182, 4096, 260), (32, 5937, 6144, 260), (33, 7990, 4112, 259), (51, 7442, 4976, 260), (36, 12922, 5120, 516), (52, 11697, 5120, 516)]]
+
+
+def plan(hip, fmt, M, N, K):
+    return hip.lib.dromos_plan_ring(FORMATS[fmt], M, N, K, 0, 1, None)
 
 
 @pytest.fixture(autouse=True)
@@ -24,17 +31,18 @@ def clear_table(hip):
     hip.lib.lx_tune_clear()
 
 
-def tiles(hip, fmt, x, w, y, **kw):
+def tiles(hip, fmt, x, w, y, math=MATH_BF16, **kw):
     (M, K), N = x.shape, y.shape[1]
     assert hip.lib.lx_tune_force(f"gemm_w_{fmt}".encode(), M, N, K, 0) == 0
     try:
-        return ops.gemm_w(hip, x, w, MATH_BF16, y=y.clone(), **kw)
+        return ops.gemm_w(hip, x, w, math, y=y.clone(), **kw)
     finally:
         hip.lib.lx_tune_clear()
 
 
-@pytest.mark.parametrize("fmt,M,N,K", CASES)
-def test_ring_gives_the_tile_kernels_bits(hip, fmt, M, N, K):
+@pytest.mark.parametrize("fmt,M,N,K,taken", CASES)
+def test_ring_gives_the_tile_kernels_bits(hip, fmt, M, N, K, taken):
+    assert plan(hip, fmt, M, N, K) == taken
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     w = random_weight(FORMATS[fmt], N, K, N + K).to("cuda")
     x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
@@ -47,7 +55,8 @@ def test_ring_gives_the_tile_kernels_bits(hip, fmt, M, N, K):
 
 @pytest.mark.parametrize("fmt", ["bf16", "int8", "fp8", "nvfp4"])
 def test_ring_strides_and_graph(hip, fmt):
-    M, N, K, pad = 50, 8704, 4096, 8
+    M, N, K, pad = 50, 8704, 4096, 64
+    assert plan(hip, fmt, M, N, K) > 0
     w = random_weight(FORMATS[fmt], N, K, 5).to("cuda")
     x = torch.randn(M, K + pad, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16).cuda()
     want = tiles(hip, fmt, x[:, :K].contiguous(), w, torch.empty(M, N, device="cuda"))
@@ -71,7 +80,8 @@ def test_ring_strides_and_graph(hip, fmt):
 
 # An infinity among a bf16 row's last values: what lies past the row's end must not meet it.
 def test_ring_infinite_weights_at_the_rows_end(hip):
-    M, N, K = 20, 12008, 4104
+    M, N, K = 33, 8008, 4104
+    assert plan(hip, "bf16", M, N, K) == 260
     w = random_weight(FORMATS["bf16"], N, K, N + K).to("cuda")
     x = torch.randn(M, K, generator=torch.Generator().manual_seed(K)).to(torch.bfloat16).cuda()
     clean = ops.gemm_w(hip, x, w, MATH_BF16, y=torch.empty(M, N, device="cuda"))
@@ -80,3 +90,15 @@ def test_ring_infinite_weights_at_the_rows_end(hip):
     assert torch.equal(got[:, 3], x[:, K - 1].float() * float("inf")) and torch.equal(got[:, N - 1], x[:, K - 8].float() * -float("inf"))
     got[:, [3, N - 1]] = clean[:, [3, N - 1]]
     assert torch.equal(got, clean)
+
+
+# The activations' scales in the epilogue.
+@pytest.mark.parametrize("math", [MATH_FP8, MATH_FP4])
+@pytest.mark.parametrize("M,N,K", [(17, 4625, 2048), (40, 11047, 3392), (64, 8209, 4032)])
+def test_ring_under_the_maths_of_activation_images(hip, math, M, N, K):
+    assert plan(hip, "nvfp4", M, N, K) > 0
+    g = torch.Generator(device="cuda").manual_seed(M)
+    w = random_weight(FORMATS["nvfp4"], N, K, N + K).to("cuda")
+    x = (torch.randn(M, K, generator=g, device="cuda") * torch.rand(M, 1, generator=g, device="cuda")).to(torch.bfloat16)
+    y = torch.full((M, N), float("nan"), device="cuda")
+    assert torch.equal(ops.gemm_w(hip, x, w, math, y=y.clone()), tiles(hip, "nvfp4", x, w, y, math=math))
