@@ -16,7 +16,7 @@ import sys
 
 import torch
 
-from .abi import load_hip
+from .abi import BF16, F32, FORMATS, LxWeight, load_hip
 
 FLUSH_BYTES = 512 << 20
 
@@ -33,61 +33,93 @@ def variants(lx, kernel):
     return [lib.lx_tune_variant_name(kernel.encode(), v).decode() for v in range(lib.lx_tune_variants(kernel.encode()))]
 
 
+class Stopwatch:
+    """median(call): the median microseconds of `repeats` calls on the current stream, cold weights each time."""
+
+    def __init__(self, lx, repeats):
+        self.lib, self.repeats = lx.lib, repeats
+        self.stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        self.flush = torch.empty(FLUSH_BYTES, dtype=torch.uint8, device="cuda")
+        self.events = []
+        for _ in range(2):
+            e = ctypes.c_void_p()
+            assert self.lib.lx_rt_event_create_timed(ctypes.byref(e)) == 0
+            self.events.append(e)
+        # The variants that keep partial sums in the stream's buffer run only on a stream that has one; the stream keeps it
+        # afterwards (reserving twice is harmless, and releasing here would take away a buffer the caller had reserved).
+        assert self.lib.lx_rt_stream_reserve(self.stream) == 0
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *_):
+        for e in self.events:
+            self.lib.lx_rt_event_destroy(e)
+
+    def median(self, call):
+        times = []
+        for _ in range(self.repeats):
+            self.flush.fill_(1)
+            assert self.lib.lx_rt_event_record(self.events[0], self.stream) == 0
+            assert call() == 0
+            assert self.lib.lx_rt_event_record(self.events[1], self.stream) == 0
+            torch.cuda.synchronize()
+            ms = ctypes.c_float()
+            assert self.lib.lx_rt_event_elapsed(self.events[0], self.events[1], ctypes.byref(ms)) == 0
+            times.append(ms.value * 1e3)
+        return round(sorted(times)[len(times) // 2], 2)
+
+
 def time_variants(lx, kernel, M, N, K, repeats=7):
     """{variant name: (median microseconds of one launch, bits equal variant 0's)} for the variants that run here."""
-    lib = lx.lib
     name = kernel.encode()
-    if not lib.lx_tune_runnable(name):
+    if not lx.lib.lx_tune_runnable(name):
         raise ValueError(f"{kernel} has no runner")
     problem = Problem(M, N, K, 1, 0, 0)
-    events = []
-    for _ in range(2):
-        e = ctypes.c_void_p()
-        assert lib.lx_rt_event_create_timed(ctypes.byref(e)) == 0
-        events.append(e)
-    flush = torch.empty(FLUSH_BYTES, dtype=torch.uint8, device="cuda")
-    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    # The variants that keep partial sums in the stream's buffer run only on a stream that has one; the stream keeps it
-    # afterwards (reserving twice is harmless, and releasing here would take away a buffer the caller had reserved).
-    assert lib.lx_rt_stream_reserve(stream) == 0
     first, result = None, {}
-    try:
+    with Stopwatch(lx, repeats) as watch:
         for v, vname in enumerate(variants(lx, kernel)):
             out = torch.empty(M, N, dtype=torch.float32, device="cuda")
-            if lx.status("tune_run", name, v, ctypes.byref(problem), out) != 0:
+            run = lambda: lx.status("tune_run", name, v, ctypes.byref(problem), out)
+            if run() != 0:
                 continue  # LX_ERR_NOT_SUPPORTED: this variant or problem does not run here
             torch.cuda.synchronize()
             first = out if first is None else first
             same = bool(torch.equal(out.view(torch.int32), first.view(torch.int32)))
-            times = []
-            for _ in range(repeats):
-                flush.fill_(1)
-                assert lib.lx_rt_event_record(events[0], stream) == 0
-                assert lx.status("tune_run", name, v, ctypes.byref(problem), out) == 0
-                assert lib.lx_rt_event_record(events[1], stream) == 0
-                torch.cuda.synchronize()
-                ms = ctypes.c_float()
-                assert lib.lx_rt_event_elapsed(events[0], events[1], ctypes.byref(ms)) == 0
-                times.append(ms.value * 1e3)
-            times.sort()
-            result[vname] = (round(times[len(times) // 2], 2), same)
-    finally:
-        for e in events:
-            lib.lx_rt_event_destroy(e)
+            result[vname] = (watch.median(run), same)
     return result
+
+
+def time_own_rule(lx, kernel, M, N, K, repeats=7):
+    """Median microseconds of the call without a table entry, or None where one of the variants is what it takes. (The ring kernel of
+    lx_gemm_w has no variant: an entry, whatever it names, keeps a call from it.)"""
+    fmt = FORMATS.get(kernel.removeprefix("gemm_w_"))
+    if not kernel.startswith("gemm_w_") or lx.lib.dromos_plan_ring(fmt, M, N, K, 0, 1, None) <= 0:
+        return None
+    device = {"device": "cuda"}
+    data = torch.randint(0, 64, (N, 2 * K), dtype=torch.uint8, **device)  # any bytes that hold no NaN: times only
+    scale = torch.ones(N, **device) if fmt != FORMATS["nvfp4"] else torch.full((N, K // 16), 0x38, dtype=torch.uint8, **device)
+    w = LxWeight(type=fmt, data=data.data_ptr(), scale=scale.data_ptr(), global_=1.0, expert_global=None)
+    x, out = torch.randn(M, K, **device).to(torch.bfloat16), torch.empty(M, N, **device)
+    run = lambda: lx.status("gemm_w", x, BF16, K, ctypes.pointer(w), 0, None, F32, out, F32, N, M, N, K, 1.0, 0.0, None)
+    with Stopwatch(lx, repeats) as watch:
+        return watch.median(run)
 
 
 def tune(lx, kernel, M, N, K, repeats=7, tolerance=1e-5):
     """Times the variants, stores the fastest one the kernel admits for the shape (lx_tune_set), and returns
     {"key", "us": {variant: microseconds}, "pick": variant name or None}. A variant whose result is neither variant 0's
-    bits nor within `tolerance` (relative L2) of it is never picked."""
+    bits nor within `tolerance` (relative L2) of it is never picked, and none where the library's own rule takes a kernel that has
+    no variant and is faster: the table then stays without an entry."""
     lib = lx.lib
     names = variants(lx, kernel)
     timed = time_variants(lx, kernel, M, N, K, repeats)
     key = ctypes.create_string_buffer(128)
     lib.lx_tune_key(kernel.encode(), ctypes.byref(Problem(M, N, K, 1, 0, 0)), key, 128)
-    pick = None
+    pick, own = None, time_own_rule(lx, kernel, M, N, K, repeats)
     for vname, (us, same) in sorted(timed.items(), key=lambda kv: kv[1][0]):
+        if own is not None and own <= us:
+            break
         if not same and not _close(lx, kernel, names.index(vname), M, N, K, tolerance):
             continue
         if lib.lx_tune_set(kernel.encode(), M, N, K, names.index(vname)) == 0:  # 802: the order-class rule refuses it

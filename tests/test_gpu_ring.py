@@ -102,3 +102,15 @@ def test_ring_under_the_maths_of_activation_images(hip, math, M, N, K):
     x = (torch.randn(M, K, generator=g, device="cuda") * torch.rand(M, 1, generator=g, device="cuda")).to(torch.bfloat16)
     y = torch.full((M, N), float("nan"), device="cuda")
     assert torch.equal(ops.gemm_w(hip, x, w, math, y=y.clone()), tiles(hip, "nvfp4", x, w, y, math=math))
+
+
+# A table entry keeps a call from the ring kernel, so the tuner stores none where the ring is faster than every variant (here about
+# half of the best one's time), and still stores the fastest where another kernel takes the call.
+def test_the_tuner_leaves_the_rings_calls_to_it(hip):
+    from dromos_amd import tune
+
+    M, N, K = 40, 8192, 2048
+    assert plan(hip, "nvfp4", M, N, K) > 0
+    got = tune.tune(hip, "gemm_w_nvfp4", M, N, K, repeats=5)
+    assert got["pick"] is None and hip.lib.lx_tune_get(b"gemm_w_nvfp4", M, N, K) == -1 and plan(hip, "nvfp4", M, N, K) > 0
+    assert tune.time_own_rule(hip, "gemm_w_nvfp4", M, 2048, K) is None and tune.time_own_rule(hip, "gemv_w_fp8", 4, N, K) is None
