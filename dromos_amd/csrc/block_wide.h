@@ -29,12 +29,12 @@ __device__ __forceinline__ Rsrc buffer_of(const void* base, int64_t bytes) {
 }
 
 // 16 (4) bytes a lane from buffer + voffset + soffset to LDS address `lds` + 16 (4) * lane. Counted by vmcnt; the compiler does not
-// know of them (it would wait for all of them before any LDS read), so wait_loads() does.
+// know of them (it would wait for all of them before any LDS read), so wait_loads() does. (M0 is reserved: the compiler keeps nothing in it.)
 __device__ __forceinline__ void load_to_lds16(uint32_t lds, uint32_t voffset, const Rsrc& rsrc, uint32_t soffset) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voffset), "s"(rsrc), "s"(soffset));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voffset), "s"(rsrc), "s"(soffset) : "memory");
 }
 __device__ __forceinline__ void load_to_lds4(uint32_t lds, uint32_t voffset, const Rsrc& rsrc, uint32_t soffset) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voffset), "s"(rsrc), "s"(soffset));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voffset), "s"(rsrc), "s"(soffset) : "memory");
 }
 
 // Waits until at most LEFT of this wavefront's loads are on their way and all of its LDS reads and writes are done.
