@@ -847,7 +847,8 @@ void* slab_scratch(hipStream_t stream, size_t bytes) {
 
 // The variants of "gemm_w_<format>" in the variant table: 0 = the tile kernels by their own rule, 1 .. 3 = walk with 1, 2, 4 tiles a
 // workgroup, 4 / 5 = the tile kernels without the slab kernel / with it wherever it fits, 6 / 7 = the walk kernel by single
-// slices / split over a workgroup, 8 = the block kernel wherever it fits. None changes a sum.
+// slices / split over a workgroup, 8 = the block kernel wherever it fits. None changes a sum. The ring kernel has none: a call with an
+// entry of 0 .. 7 does not go there.
 constexpr int kVariantWindow = 4, kVariantSlab = 5, kVariantWalkParts = 6, kVariantWalkSplit = 7, kVariantBlock = 8;
 
 template <int F>
@@ -1355,17 +1356,18 @@ bool walk_parts_wanted(int M, int n_tiles, int64_t K, int tuned) {
 // rows and tiles: whether the activations' rows start on 128-byte lines (a stage takes one line of every row, off the lines two);
 // how much of the slices K fills (every slice walks as many stages); and whole tiles a unit (512, 768 tiles), where the other
 // kernels come out even.
-// - One-byte weights from 17 rows, K 4096 .. 8192. To 384 tiles on lines 0.83 to K = 6144, beyond 1.2 (off the lines to 1.54: fp8 5136 x 7504 at 35
-//   rows 21.3 / 29.9 us). 385 .. 512 tiles: from 33 rows 0.72, fewer on lines 0.87 where the slices are filled, else 0.97 .. 1.03; fp8 on 512 tiles
-//   0.75 .. 0.86 to K = 4096 and 0.77 .. 0.98 from 49 rows from 5120, else to 1.16. More tiles with K a multiple of 512 that fills the slices: 513 .. 767 from 49 rows
-//   0.79 (8784 x 5120 at 54 rows 45.9 / 30.0), from 769 at 33 .. 40 rows 0.88; everything else there 1.06 .. 1.34 (14400 x 6576 at 42 rows 29.5 / 46.4).
+// - One-byte weights from 17 rows, K 4096 .. 8192. To 384 tiles on lines 0.82 to K = 6144, beyond 1.2 (off the lines to 1.54: fp8 5136 x 7504 at 35
+//   rows 21.3 / 29.9 us). 385 .. 512 tiles: from 33 rows 0.73, fewer on lines 0.87 where the slices are filled, else 0.97 .. 1.05; fp8 on 512 tiles
+//   0.75 .. 0.86 to K = 4096 and 0.77 .. 0.98 from 49 rows from 5120, else to 1.16. Beyond, on lines: above 768 tiles at 33 .. 40 rows from K = 4160 0.90, from 49 rows
+//   on 4096 and 8192 values 0.94 (8192 from 41), below 768 from 49 rows where K is a multiple of 512 that fills the slices 0.79 (8784 x 5120 at 54 rows
+//   45.9 / 30.0); everything else 1.06 .. 1.45 (14400 x 6576 at 42 rows 29.5 / 46.4).
 // - bf16 from 384 tiles. To 512, K <= 8192: from 33 rows 0.70, fewer on lines 0.87; on 512 tiles beyond 24 rows only K = 2048, 3072 and 4096
-//   (0.68 .. 1.0, else to 1.12). More tiles on lines: up to 24 rows 0.92 (rows of 16 KB 0.98 .. 1.28), with full slices to 32 rows 0.91 and beyond 0.90 below 768
-//   tiles between 3 K and 8 K; everything else 1.0 .. 1.17 (15010 x 7064 at 56 rows 51.7 / 64.1).
-// - NVFP4 from 17 rows. Rows of a cut load step (K % 128), where the walk kernel does not apply, 0.39 .. 0.73. Whole ones 0.78 where a workgroup takes 32
-//   (K above 4096 on more than 512 tiles, and 768, 1.07) and 0.74 at 33 .. 64 rows to 768 tiles; else 0.95 .. 1.03. Three slices of 5120 .. 7168
-//   values for four wavefronts 1.08 .. 1.20. Four slices of 64 rows leave the ring two stages: on 896 tiles, where the walk kernel
-//   takes four tiles a workgroup, 28.3 / 29.0 (bf16 outputs 30.8 / 28.8).
+//   (0.68 .. 1.0, else to 1.12). Beyond, on lines: up to 24 rows 0.92 (rows of 16 KB 0.98 .. 1.28), with full slices to 32 rows 0.91; from 33 rows between
+//   3 K and 8 K with full slices below 768 tiles, and above at 33 .. 40 rows, 0.90; everything else 1.0 .. 1.17 (15010 x 7064 at 56 rows 51.7 / 64.1).
+// - NVFP4 from 17 rows. Rows of a cut load step (K % 128), where the walk kernel does not apply, 0.39 .. 0.75. Whole ones 0.78 where a workgroup takes 32
+//   (K above 4096 on more than 512 tiles, and 768, 1.07); at 33 .. 64 rows to 768 tiles 0.74, above where a slice is eight steps 0.92; else 0.98 .. 1.06.
+//   Three slices of 5120 .. 7168 values for four wavefronts 1.08 .. 1.20. Four slices of 64 rows leave the ring two stages: on 896 tiles, where
+//   the walk kernel takes four tiles a workgroup, 28.3 / 29.0 (bf16 outputs 30.8 / 28.8).
 template <int F>
 int ring_cols(const GemmArgs& a, int n_tiles) {
   if (a.M <= 8 || n_tiles < 289 || n_tiles > 1024 || a.K < 2048 || a.K > 11264) return 0;
@@ -1379,7 +1381,7 @@ int ring_cols(const GemmArgs& a, int n_tiles) {
     if (a.M <= 16 || (a.K > 4096 && filled < 89) || (deep && n_tiles > 768)) return 0;
     const int cols = n_tiles <= 512 || deep ? 32 : 64;
     if (a.K % 128 != 0) return cols;
-    return (cols == 32 ? n_tiles <= 512 || (a.K <= 4096 && !whole) : a.M > 32 && n_tiles <= 768) ? cols : 0;
+    return (cols == 32 ? n_tiles <= 512 || (a.K <= 4096 && !whole) : a.M > 32 && (n_tiles <= 768 || a.steps_per_wave == 8)) ? cols : 0;
   }
   if (F == LX_W_BF16) {
     if (n_tiles <= 383) return 0;
@@ -1389,17 +1391,20 @@ int ring_cols(const GemmArgs& a, int n_tiles) {
     }
     if (!lines || a.K % 8192 == 0 || (a.K < 4096 && n_tiles > 900)) return 0;
     if (a.M <= 32) return a.M <= 24 || filled == 100 ? 64 : 0;
+    if (a.M <= 40 && n_tiles > 768 && a.K > 2304 && a.K < 8192) return 64;
     return filled == 100 && a.K > 3008 && a.K < 8192 && (n_tiles < 768 || (n_tiles == 768 && a.M <= 40)) ? 64 : 0;
   }
   if (a.M <= 16 || a.K < 4096 || a.K > 8192) return 0;
   if (n_tiles <= 384) return lines && a.K <= 6144 && (a.M > 32 || filled >= 84) ? 32 : 0;
   if (n_tiles <= 512) {
     if (whole && F == LX_W_FP8) return lines && (a.K < 4608 || (a.M > 48 && a.K >= 5120 && a.K < 8192)) ? 32 : 0;
-    if (a.M > 32) return (lines || (n_tiles > 400 && !whole)) && (a.K < 8192 || a.M <= 48) ? 32 : 0;
+    if (a.M > 32) return (lines || a.M > 48 || (n_tiles > 400 && !whole)) && (a.K < 8192 || a.M <= 40) ? 32 : 0;
     return lines && filled > (whole ? 90 : 86) ? 32 : 0;
   }
-  if (!lines || a.K % 512 != 0 || filled < 83) return 0;
-  return n_tiles < 768 ? (a.M > 48 ? 64 : 0) : n_tiles > 768 && a.M > 32 && a.M <= 40 && a.K > 4096 ? 64 : 0;
+  if (!lines) return 0;
+  if (n_tiles > 768 && a.M > 32 && a.M <= 40 && a.K > 4096) return 64;
+  if (n_tiles >= 768) return a.K % 4096 == 0 && (a.M > 48 || (a.M > 40 && a.K > 4096)) ? 64 : 0;
+  return a.M > 48 && a.K % 512 == 0 && filled >= 83 ? 64 : 0;
 }
 
 // The ring kernel where it is the faster one.
@@ -1484,7 +1489,8 @@ int launch_skinny(GemmArgs a, hipStream_t stream) {
 // weights of more than 288 tiles are behind below K = 3072 (fp8 6400 x 2048 13.2 / 15.3, 6400 x 2560 16.5 / 18.0; 5120 x 2048 13.0 /
 // 15.3) and tie there; up to 48 rows they are behind from 192 tiles of K = 2048, where the walk kernel starts (fp8 3072 x 2048 9.6 /
 // 10.6, 2560 x 2048 14.7 / 10.1), and beyond 192 of any K. Blocks are also ahead on some shapes outside these lines (64 to 127
-// tiles, bf16 from K = 2560 and to 448 tiles, NVFP4 from 33 rows and on 9216 x 11008: 70 / 49 us), which stay as they were.
+// tiles, bf16 from K = 2560 and to 448 tiles, NVFP4 from 33 rows and on 9216 x 11008: 70 / 49 us), which stay as they were. (All against
+// the windowed and slab kernels: this rule goes before the ring kernel's and has not been compared with it on 289 .. 400 tiles.)
 template <int F>
 bool block_wanted(int M, int n_tiles, int64_t K) {
   if (M <= 32 || n_tiles < 128 || K < 2048 || K > 6144) return false;

@@ -36,10 +36,10 @@ def test_look_ahead_stays_in_the_wavefronts_own_part(lib, M, N, K, plan):
     ("fp8", 32, 6144, 4096, True), ("fp8", 35, 5136, 7504, False), ("fp8", 49, 5328, 6448, False), ("fp8", 46, 5584, 7168, False), ("fp8", 27, 5952, 6400, False),
     ("fp8", 40, 8192, 4096, True), ("fp8", 48, 8192, 5120, False), ("int8", 48, 8192, 5120, True), ("fp8", 35, 8192, 5008, False), ("fp8", 64, 8192, 6144, True),
     ("fp8", 29, 7744, 7056, False), ("fp8", 43, 6480, 7136, True), ("fp8", 54, 8784, 5120, True), ("fp8", 42, 14400, 6576, False), ("fp8", 63, 11280, 6976, False),
-    ("int8", 46, 14752, 7120, False), ("int8", 40, 9600, 4112, False), ("fp8", 64, 12288, 6144, False), ("int8", 40, 16192, 7168, True), ("int8", 24, 16192, 7168, False),
+    ("int8", 46, 14752, 7120, False), ("int8", 40, 9600, 4112, False), ("fp8", 64, 12288, 6144, False), ("int8", 40, 16192, 7168, True), ("int8", 64, 14336, 4096, True), ("fp8", 48, 14336, 4096, False), ("fp8", 37, 15104, 6592, True), ("nvfp4", 40, 14336, 2048, True), ("bf16", 38, 14336, 5120, True), ("int8", 24, 16192, 7168, False),
     ("bf16", 56, 15010, 7064, False), ("bf16", 56, 7984, 4096, True), ("bf16", 48, 8192, 4096, True), ("bf16", 48, 8192, 7680, False), ("bf16", 9, 16384, 8192, False),
     ("bf16", 9, 12512, 4096, True), ("bf16", 48, 12288, 6144, False), ("bf16", 40, 12288, 6144, True), ("bf16", 30, 9472, 2464, False), ("bf16", 29, 10544, 2432, False), ("bf16", 36, 11040, 8064, False), ("int8", 32, 8192, 7168, False),
     ("nvfp4", 32, 7264, 4096, True), ("nvfp4", 64, 12288, 3072, False), ("nvfp4", 32, 14336, 4096, False), ("nvfp4", 30, 14336, 2112, True), ("nvfp4", 64, 14336, 4096, False),
-    ("nvfp4", 40, 12368, 4096, False), ("nvfp4", 24, 8970, 3616, False), ("nvfp4", 16, 7264, 4096, False)])
+    ("nvfp4", 40, 12368, 4096, True), ("fp8", 47, 7867, 8192, False), ("nvfp4", 24, 8970, 3616, False), ("nvfp4", 16, 7264, 4096, False)])
 def test_what_the_ring_takes(lib, fmt, M, N, K, taken):
     assert (lib.dromos_plan_ring(FORMATS[fmt], M, N, K, UNITS, 1, None) > 0) == taken
