@@ -36,8 +36,10 @@ HIPCC_FLAGS = [
 
 # The kernels whose wavefronts may have 512 registers for themselves (block_wide.h, gemm_ring.h) keep the running sums of their matrix
 # products in vector registers and what is seldom touched in accumulation registers; left alone the compiler does it the other way
-# round and copies sums between accumulation registers in the walk (124 moves for 64 matrix instructions). The walk kernels are
-# better off left alone (NVFP4 14336 x 4096 at 64 rows 28.3 us, with it 33.7).
+# round and copies sums between accumulation registers in the walk (124 moves for 64 matrix instructions). The flag is a source's, so the
+# blocks of eight wavefronts (256 registers) beside the wide one, and bf16's, have it too: 64 x 64 and 64 x 128 take 0.93 .. 0.99 of the
+# time without, 128 x 128 and more, a slice a workgroup and the bf16 experts 0.99 .. 1.01 (averages over 1100 calls). The walk
+# kernels are better off left alone (NVFP4 14336 x 4096 at 64 rows 28.3 us, with it 33.7).
 MFMA_VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 
 

@@ -123,7 +123,6 @@ __global__ void __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(
   };
   float f[4];
   if (wide && cols % 4 == 0) {
-#pragma unroll 4
     for (int m = b.wave; m < rows; m += B::kWaves) {
       factors(m, f);
       const typename B::Acc sums = b.sum(m, b.lane);

@@ -6,8 +6,8 @@
 // Bound by bytes on their way: a unit's ring holds 80 .. 160 KB of which the activations, which every workgroup reads anew from
 // its die's L2, are the larger part from 32 rows on (fp8 14336 x 4096 at 64 rows, 23 us: 17 with the weights alone loaded, 13 with the
 // activations alone; the order of a row's lanes, the row stride and the activations asked for ahead make no difference). The
-// kernels that stage windows of the activations through registers for all wavefronts (gemm_walk.h) stay ahead up to 16 rows. Where:
-// gemm.hip, ring_cols().
+// kernels that stage windows of the activations through registers for all wavefronts (gemm_walk.h) tie or are ahead on many sizes
+// (on that one 22.9 / 22.2). Which it takes: gemm.hip, ring_cols().
 #pragma once
 
 #include "block_wide.h"

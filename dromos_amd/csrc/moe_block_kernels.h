@@ -114,7 +114,6 @@ __device__ __forceinline__ void expert_wide_tile(const ExpertBlock& a, int e, in
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) asm volatile("" ::"v"(fg[r]), "v"(fu[r]), "v"(xs[r & 1]));
-#pragma unroll 2
     for (int m0 = 2 * b.wave; m0 < rows; m0 += 2 * B::kWaves) {
       const int m = m0 + (b.lane >> 5);
       const float lo = __shfl(xs[0], m & 63), hi = __shfl(xs[1], m & 63), s = m < 64 ? lo : hi;
@@ -131,7 +130,6 @@ __device__ __forceinline__ void expert_wide_tile(const ExpertBlock& a, int e, in
 #pragma unroll
     for (int r = 0; r < 4; ++r) f[r] = stack_factor(F, a.w, e, first + min(c + r, a.cols - 1));
     asm volatile("" ::"v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(xs[0]), "v"(xs[1]));
-#pragma unroll 4
     for (int m = b.wave; m < rows; m += B::kWaves) {
       // (One lane's value each time: lanes without columns take no part in a choice between two.)
       const uint32_t s0 = __builtin_amdgcn_readlane(__float_as_uint(xs[0]), m & 63), s1 = __builtin_amdgcn_readlane(__float_as_uint(xs[1]), m & 63);

@@ -339,7 +339,8 @@ BlockCut block_cut(int64_t K, int NT, int64_t out_rows) {
 //   Two NVFP4 experts of 4096 x 1536 at 16 rows are 24 and 32 blocks: 27.5 us by the kernels here, 95.5 by blocks.
 // Rows (48 at most) times that share from 12 on is where FP8 blocks are ahead; INT8 60 and 12, bf16 56 and 14; NVFP4, whose blocks
 // decode more a row, 80 and 16. Of 1661 sweep points 11 lose 4 % or more that way (16 % at most: NVFP4 8 experts of 1024 x 2048 at
-// 64 rows, bf16 12 of 2048 x 4096 at 25 rows 13 %), and 1 % of the gain is left.
+// 64 rows, bf16 12 of 2048 x 4096 at 25 rows 13 %), and 1 % of the gain is left. (The quantised formats' lines are the blocks' of eight wavefronts:
+// since the wide block they may lie too high, never too low.)
 bool blocks_wanted(int type, int64_t P, int64_t E, int64_t L, int64_t I, int units) {
   if (P < (type == LX_W_BF16 ? 24 : 16) * E) return false;
   const int64_t by_rows = (P + kBlockTokens - 1) / kBlockTokens, tiles = by_rows > E ? by_rows : E;
@@ -351,8 +352,8 @@ bool blocks_wanted(int type, int64_t P, int64_t E, int64_t L, int64_t I, int uni
 }
 
 // Whether a stack of rows of K values is taken by the wide block (block_wide.h): quantised rows, NVFP4's with block scales that can be
-// loaded four bytes at a time. It is ahead wherever blocks are taken at all (72 products of 8 .. 128 experts, 1088 .. 4096 x 512 ..
-// 1984, 17 .. 1388 rows an expert: 0.70 .. 1.02 of the other blocks' time; 128 NVFP4 experts of 4096 x 1536 at 2048 tokens 1372 ->
+// loaded four bytes at a time. It is ahead wherever blocks are taken at all (120 products of 4 .. 128 experts, 512 .. 4096 x 256 ..
+// 4096, 16 .. 1388 rows an expert: 0.69 .. 1.02 of the other blocks' time, 0.84 on average; 128 NVFP4 experts of 4096 x 1536 at 2048 tokens 1372 ->
 // 990 us, at 512 646 -> 477, FP8 at 2048 1260 -> 980).
 bool wide_fits(int type, const Stack& w, int64_t K) {
   return type == LX_W_INT8 || type == LX_W_FP8 || (type == LX_W_NVFP4 && K % 64 == 0 && reinterpret_cast<uintptr_t>(w.scale) % 4 == 0);

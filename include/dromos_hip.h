@@ -331,6 +331,7 @@ LX_API int lx_probe_empty(void* stream);
  * shape's own (so the rows' bits never depend on the table). The matrix-core products (lx_gemm_w, lx_gemm_skinny)
  * register theirs under gemm_w_<format>: which kernel family runs ("tiles", "walk1", "walk2", "walk4", "window",
  * "slab", "walkparts", "walksplit" for up to 64 rows, "block" for any); none changes a sum, so every one is admitted.
+ * The ring kernel (some calls of 9 .. 64 rows, by the library's own rule) has no variant: an entry other than "block" keeps a call from it.
  * An entry holds for the row counts of its power of two: calls of more than 64 rows, which the block kernel takes by the
  * library's own rule, go 64 rows a pass where an entry of theirs names another family. */
 LX_API int lx_arch(void);
