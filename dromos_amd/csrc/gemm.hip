@@ -1407,12 +1407,43 @@ int ring_cols(const GemmArgs& a, int n_tiles) {
   return a.M > 48 && a.K % 512 == 0 && filled >= 83 ? 64 : 0;
 }
 
-// The ring kernel where it is the faster one.
+// Whether NVFP4 rows go to the ring kernel with loader wavefronts (gemm_ring.h: fed_kernel), of the calls that ring_cols() leaves: more than
+// 512 tiles (fewer are up to 1.6 times the present time: 192 workgroups at 384 tiles) in up to four slices. From 6200 random calls on
+// cold weights (9 .. 64 rows, 128 .. 1536 tiles, K 1024 .. 14336 in steps of 64, f32 and bf16 outputs), times over the kernels it replaces: the 3014
+// calls of them that this takes 0.69 on average, none above 1.01.
+// - Rows of a cut load step (K % 128), where no walk kernel applies, from 17 rows 0.23 .. 0.95; at 9 .. 16 rows 0.75 .. 1.0 to 1024 tiles
+//   (beyond, a second round of workgroups, 0.96 .. 1.26).
+// - Whole steps from 33 rows 0.29 .. 1.0, but not slices of 32 steps (1.04 .. 1.14).
+// - At 17 .. 32 rows the walk kernels' bytes count for more: beyond 1024 tiles 0.65 .. 0.99; to 1024 where K leaves slices unfilled, which this kernel
+//   does not walk (filled ones 0.92 .. 1.13), not three slices of 16 steps that are four fifths full, nor four of 24 and more (to 1.46).
+bool fed_wanted(const GemmArgs& a, int n_tiles) {
+  if (a.M <= 8 || n_tiles <= 512 || a.K < 1024 || a.K > 14336) return false;
+  if (a.scale_row_bytes % 4 != 0 || reinterpret_cast<uintptr_t>(a.scale) % 4 != 0) return false;  // (loaded four bytes at a time)
+  const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave;
+  if (slices > 4) return false;
+  if (a.K % 128 != 0) return a.M > 16 || n_tiles <= 1024;
+  if (a.M <= 16) return false;
+  if (a.M > 32) return slices < 4 || a.steps_per_wave <= 24;
+  if (n_tiles > 1024) return true;
+  const int filled = a.steps * 100 / (a.steps_per_wave * slices);  // percent of the slices
+  if (filled > 94) return false;
+  return slices == 3 ? a.steps_per_wave != 16 || filled < 80 : slices < 4 || a.steps_per_wave <= 16;
+}
+
+// The ring kernels where one is the fastest.
 template <int F>
 bool try_ring(const GemmArgs& a, int* status, hipStream_t stream) {
   if (a.tuned >= 0 || a.xs.dtype != LX_BF16) return false;
-  const int cols = ring_cols<F>(a, (a.N + kTileRows - 1) / kTileRows);
-  if (cols == 0 || a.row_bytes * 64 >= (1ll << 31) || a.xs.ld * 2 * 64 >= (1ll << 31)) return false;  // 32-bit offsets
+  const int n_tiles = (a.N + kTileRows - 1) / kTileRows;
+  const int cols = ring_cols<F>(a, n_tiles);
+  if (a.row_bytes * 64 >= (1ll << 31) || a.xs.ld * 2 * 64 >= (1ll << 31)) return false;  // 32-bit offsets
+  if constexpr (F == LX_W_NVFP4) {
+    if (cols == 0 && fed_wanted(a, n_tiles)) {
+      *status = launch_fed_nvfp4(a, stream);
+      return true;
+    }
+  }
+  if (cols == 0) return false;
   if constexpr (F == LX_W_BF16) return launch_ring_bf16(a, cols, status, stream);
   else if constexpr (F == LX_W_INT8) return launch_ring_int8(a, cols, status, stream);
   else if constexpr (F == LX_W_FP8) return launch_ring_fp8(a, cols, status, stream);
@@ -1914,6 +1945,20 @@ LX_API int dromos_plan_ring(int format, int M, int N, int K, int units, int buff
     case LX_W_FP8: return ask(std::integral_constant<int, LX_W_FP8>{});
     default: return ask(std::integral_constant<int, LX_W_NVFP4>{});
   }
+}
+
+// The same of its form with loader wavefronts: the slices of K, or 0.
+LX_API int dromos_plan_fed(int format, int M, int N, int K, int units, int buffer) {
+  if (format != LX_W_NVFP4 || M < 1 || M > 64 || K % 32 != 0 || dromos_plan_gemm(format, LX_MATH_BF16, M, N, K, units, buffer) >= 0) return 0;
+  GemmArgs a{};
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.xs.ld = K;
+  cut_rows<LX_W_NVFP4>(a);
+  const int n_tiles = (N + kTileRows - 1) / kTileRows;
+  if (tuned_variant(gemm_key<LX_W_NVFP4>(), M, N, K) >= 0 || ring_cols<LX_W_NVFP4>(a, n_tiles) > 0 || !fed_wanted(a, n_tiles)) return 0;
+  return (a.steps + a.steps_per_wave - 1) / a.steps_per_wave;
 }
 
 int lx_gemv_w(const void* x, lx_dtype x_dtype, int ld_x, const lx_weight* w, const void* bias, lx_dtype bias_dtype, void* y,

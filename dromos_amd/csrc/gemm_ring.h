@@ -49,6 +49,37 @@ struct Ring {
   static constexpr int kLdsBytes = kStages * kStage > kSums ? kStages * kStage : kSums;
 };
 
+// What a kernel below leaves in LDS, SL slices' sums of BM rows by BN columns side by side, added up in ascending order and written out by
+// THREADS threads.
+template <int F, int BM, int BN, int SL, int THREADS>
+__device__ __forceinline__ void write_slices(const GemmArgs& a, const uint8_t* lds, int n0, int cols, int slices) {
+  constexpr int kPieces = BN / 4, kSlice = BM * BN * 4;
+  const int piece = threadIdx.x % kPieces, n = 4 * piece;
+  if (n >= cols) return;
+  const bool wide = wide_stores(a) && n + 3 < cols;
+  constexpr int kRows = THREADS / kPieces, kTimes = (BM + kRows - 1) / kRows;
+  float rf[4], xs[kTimes];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) rf[r] = row_factor(F, a.scale, a.global, n0 + min(n + r, cols - 1));
+#pragma unroll
+  for (int q = 0; q < kTimes; ++q) xs[q] = a.act_scale ? a.act_scale[min(static_cast<int>(threadIdx.x) / kPieces + q * kRows, a.M - 1)] : 1.0f;
+#pragma unroll
+  for (int q = 0; q < kTimes; ++q) {
+    const int m = threadIdx.x / kPieces + q * kRows;
+    if (m >= a.M || m >= BM) break;
+    const uint8_t* const at = lds + m * BN * 4 + ((piece ^ (m & 15)) & (kPieces - 1)) * 16;
+    f32x4 s = *reinterpret_cast<const f32x4*>(at);
+#pragma unroll
+    for (int k = 1; k < SL; ++k)
+      if (k < slices) s += *reinterpret_cast<const f32x4*>(at + k * kSlice);
+    float f[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) f[r] = rf[r] * xs[q];
+    if (wide) write_four(a, m * a.ld_y + n0 + n, s, f);
+    else write_each(a, m, n0 + n, s, f);
+  }
+}
+
 template <int F, int MT, int KS, int BN>
 __global__ void __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(1, 2))) ring_kernel(const GemmArgs a, int slices) {
   using R = Ring<F, MT, KS, BN>;
@@ -243,30 +274,255 @@ __global__ void __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(
     for (int mt = 0; mt < MT; ++mt)
       *reinterpret_cast<f32x4*>(lds + ks * kSlice + (mt * 16 + i) * BN * 4 + ((((wn * NT + nt) * 4 + g) ^ i) & (kPieces - 1)) * 16) = acc[nt][mt];
   __syncthreads();
-  const int piece = threadIdx.x % kPieces, n = 4 * piece;
-  if (n >= cols) return;
-  const bool wide = wide_stores(a) && n + 3 < cols;
-  constexpr int kRows = R::kThreads / kPieces, kTimes = (R::BM + kRows - 1) / kRows;
-  float rf[4], xs[kTimes];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) rf[r] = row_factor(F, a.scale, a.global, n0 + min(n + r, cols - 1));
-#pragma unroll
-  for (int q = 0; q < kTimes; ++q) xs[q] = a.act_scale ? a.act_scale[min(static_cast<int>(threadIdx.x) / kPieces + q * kRows, a.M - 1)] : 1.0f;
-#pragma unroll
-  for (int q = 0; q < kTimes; ++q) {
-    const int m = threadIdx.x / kPieces + q * kRows;
-    if (m >= a.M || m >= R::BM) break;
-    const uint8_t* const at = lds + m * BN * 4 + ((piece ^ (m & 15)) & (kPieces - 1)) * 16;
-    f32x4 s = *reinterpret_cast<const f32x4*>(at);
-#pragma unroll
-    for (int k = 1; k < KS; ++k)
-      if (k < slices) s += *reinterpret_cast<const f32x4*>(at + k * kSlice);
-    float f[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) f[r] = rf[r] * xs[q];
-    if (wide) write_four(a, m * a.ld_y + n0 + n, s, f);
-    else write_each(a, m, n0 + n, s, f);
+  write_slices<F, R::BM, BN, KS, R::kThreads>(a, lds, n0, cols, slices);
+}
+
+// The same product on NVFP4 weights with the loads on wavefronts of their own: of a workgroup's eight, four multiply (two slices by two
+// parts of 64 columns; PER slices one after the other), two load a slice's activations each and two its weights (the feeders). A wavefront's
+// loads return in the order they were asked for, so in ring_kernel the activations, which come from the die's L2, wait behind weights from
+// memory; here the two wait apart, and the weights' ring is as deep as LDS allows. What the row does not fill of the last slices is not
+// walked (ring_kernel multiplies zeros there).
+// 14336 x 4096 at 64 rows 28.3 -> 21.1 us (by gemm_walk.h before), 16384 x 4096 28.4 -> 21.0, 8256 x 4416 at 50 rows 67 -> 26 (by the windows before).
+// Bound by what a multiplying wavefront, alone on its SIMD but for a feeder, issues: an instruction every four cycles whatever its kind, about
+// 300 a stage of which 32 are matrix instructions and 128 conversions. (With every load from one row, out of L2, 16.7 us; the loads on
+// the multiplying wavefronts the same time at 64 rows and 1 us more at 32; a stage's codes read a quarter earlier 1 us more.)
+// A barrier a stage: behind stage st's it is in LDS, and nobody reads stage st - 1 any more.
+template <int MT_, int PER_>
+struct Fed {
+  static constexpr int MT = MT_, PER = PER_, KS = 2, BN = 64;
+  using R = Ring<LX_W_NVFP4, MT, KS, BN>;
+  static_assert(R::WN == 2 && R::NT == 2);
+  static constexpr int kThreads = 2 * R::kThreads;
+  // A stage: the slices' activations; of weights the multiplying wavefronts' parts, codes and block scales.
+  static constexpr int kXStage = KS * R::kXBytes, kWStage = R::kWaves * R::kOwn;
+  static constexpr int kXL = R::kXLoads * R::WN, kWL = (R::kWLoads + R::kSLoads) * R::WN;  // a feeder's loads a stage
+  static constexpr int fit(int a, int b) { return a < b ? a : b; }
+  static constexpr int kXStages = MT == 4 ? 3 : 4;
+  static constexpr int kWAt = kXStages * kXStage;
+  static constexpr int kWStages = fit(fit((160 * 1024 - kWAt) / kWStage, 10), 63 / kWL + 1);
+  static_assert(kXStages <= 63 / kXL + 2 && kWStages >= 3);
+  static constexpr int kSums = KS * PER * R::BM * BN * 4, kRing = kWAt + kWStages * kWStage, kLdsBytes = kRing > kSums ? kRing : kSums;
+};
+
+// Waits until at most `behind` (0 .. MOST) stages of L loads each are on their way.
+template <int L, int MOST>
+__device__ __forceinline__ void wait_stages(int behind) {
+  if constexpr (MOST == 0) wait_loads<0>();
+  else if (behind >= MOST) wait_loads<MOST * L>();
+  else wait_stages<L, MOST - 1>(behind);
+}
+
+// A feeder's walk over `stages` stages by a ring of STAGES: load(st, slot) asks for stage st's L loads, finish(st, slot) writes zeros where
+// stage `cut`, which has arrived, reaches past the row's end. `all` stages have a barrier.
+template <int L, int STAGES, class Load, class Finish>
+__device__ __forceinline__ void feed(int stages, int all, int cut, Load&& load, Finish&& finish) {
+  for (int st = 0; st < STAGES - 1; ++st)
+    if (st < stages) load(st, st);
+  int slot = 0, free = STAGES - 1;  // stage st's slot, and the one that stage st - 1 + STAGES takes
+  for (int st = 0; st < stages; ++st) {
+    wait_stages<L, STAGES - 2>(stages - 1 - st);
+    if (st == cut) {
+      finish(st, slot);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    asm volatile("s_barrier" ::: "memory");
+    if (st - 1 + STAGES < stages) load(st - 1 + STAGES, free);
+    slot = slot + 1 == STAGES ? 0 : slot + 1;
+    free = free + 1 == STAGES ? 0 : free + 1;
   }
+  for (int st = stages; st < all; ++st) asm volatile("s_barrier" ::: "memory");
+}
+
+template <int MT, int PER>
+__global__ void __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(2, 2))) fed_kernel(const GemmArgs a, int slices) {
+  using D = Fed<MT, PER>;
+  using R = typename D::R;
+  constexpr int F = LX_W_NVFP4, WN = R::WN, NT = R::NT, J = R::J, KS = D::KS, BN = D::BN;
+  extern __shared__ __align__(16) f32x4 lds4[];
+  uint8_t* const lds = reinterpret_cast<uint8_t*>(lds4);
+  const uint32_t lds_at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds)));
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), g = lane >> 4, i = lane & 15;
+  const int ks = wave % KS, wn = wave / KS % WN;
+  const int n0 = blockIdx.x * BN, cols = min(BN, a.N - n0);
+  const int xbytes = a.K * 2, wbytes = static_cast<int>(a.row_bytes), sbytes = a.K / 16;
+  const int64_t ld = a.xs.ld * 2;
+  // The stages of this wavefront's slices, and those of them that the row has (the others are barriers only). The row's last one, `end`,
+  // may be cut short by K: zeros there.
+  const int per = PER * a.steps_per_wave, first = ks * per, end = a.steps - 1, stages = max(0, min(per, a.steps - first));
+  constexpr int kSlice = R::BM * BN * 4;
+  if (wave >= R::kWaves + KS) {
+    // Slice ks's weights and block scales, for the WN wavefronts that multiply them; a stage is a load step, 64 bytes of a row (8 of scales).
+    const Rsrc wbuf = block::buffer_of(a.w + n0 * a.row_bytes, cols * a.row_bytes), sbuf = block::buffer_of(a.scale + n0 * a.scale_row_bytes, cols * a.scale_row_bytes);
+    const int wpiece = ((lane & 3) ^ ((lane >> 3) & 3)) * 16, spiece = (lane & 1) * 4;  // piece s ^ (r / 2) of row r at slot s, as in ring_kernel
+    uint32_t wrow[WN][R::kWLoads], srow[WN];
+    static_assert(R::kWRow == 64 && R::kSLoads == 1 && NT * 16 == 32);
+#pragma unroll
+    for (int h = 0; h < WN; ++h) {
+#pragma unroll
+      for (int u = 0; u < R::kWLoads; ++u)
+        wrow[h][u] = static_cast<uint32_t>(min(h * 32 + u * 16 + (lane >> 2), cols - 1)) * static_cast<uint32_t>(wbytes) + wpiece;
+      srow[h] = static_cast<uint32_t>(min(h * 32 + (lane >> 1), cols - 1)) * static_cast<uint32_t>(a.scale_row_bytes) + spiece;
+    }
+    feed<D::kWL, D::kWStages>(
+        stages, per, end - first,
+        [&](int st, int slot) {
+          const int t = first + st;
+          const uint32_t to = lds_at + D::kWAt + slot * D::kWStage + ks * R::kOwn;
+          const uint32_t wback = wpiece + t * 64 >= wbytes ? wpiece : 0, sback = spiece + t * 8 >= sbytes ? spiece : 0;
+#pragma unroll
+          for (int h = 0; h < WN; ++h) {
+#pragma unroll
+            for (int u = 0; u < R::kWLoads; ++u) load_to_lds16(to + h * KS * R::kOwn + u * 1024, wrow[h][u] - wback, wbuf, t * 64);
+            load_to_lds4(to + h * KS * R::kOwn + R::kWBytes, srow[h] - sback, sbuf, t * 8);
+          }
+        },
+        [&](int st, int slot) {
+          const int t = first + st;
+#pragma unroll
+          for (int h = 0; h < WN; ++h) {
+            uint8_t* const to = lds + D::kWAt + slot * D::kWStage + (h * KS + ks) * R::kOwn;
+            if (wpiece + t * 64 >= wbytes) {
+#pragma unroll
+              for (int u = 0; u < R::kWLoads; ++u) *reinterpret_cast<u32x4*>(to + u * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+            }
+            uint8_t* const s = to + R::kWBytes + lane * 4;
+            if (spiece + t * 8 >= sbytes) *reinterpret_cast<uint32_t*>(s) = 0;
+            else if (spiece + t * 8 + 2 >= sbytes) *reinterpret_cast<uint16_t*>(s + 2) = 0;
+          }
+        });
+  } else if (wave >= R::kWaves) {
+    // Slice ks's activations, 256 bytes of every row a stage. Places in a row as in ring_kernel.
+    const Rsrc xbuf = block::buffer_of(a.xs.x, (a.M - 1) * ld + xbytes);
+    uint32_t xrow[D::kXL];
+    int xpiece[D::kXL > 3 ? 4 : D::kXL];
+    static_assert(R::kXRow == 256 && J == 4);
+#pragma unroll
+    for (int u = 0; u < D::kXL; ++u) {
+      const int row = u * 4 + (lane >> 4), place = (lane ^ row) & 15;
+      const int piece = (J * (place & 3) + (place >> 2)) * 16;
+      if (u < 4) xpiece[u] = piece;  // (the same for every sixteen rows)
+      xrow[u] = static_cast<uint32_t>(min(row, a.M - 1)) * static_cast<uint32_t>(ld) + piece;
+    }
+    const uint32_t own = ks * R::kXBytes;
+    // All workgroups walk K together, so an activation row's next piece would come from memory for every one of them. The workgroups of
+    // a die (every eighth) share out the activations' 128-byte lines and ask for them once, at the start. They land where this
+    // feeder loads the last slot's stage, which it asks for behind a wait for these.
+    {
+      const int line_row = (xbytes + 127) / 128, lines = line_row * a.M, share = (lines + (gridDim.x >> 3)) / ((gridDim.x >> 3) + 1);
+      for (int at = ks * kWave + lane; at - lane < share; at += KS * kWave) {
+        const int line = min(static_cast<int>(blockIdx.x >> 3) * share + min(at, share - 1), lines - 1), row = line / line_row;
+        load_to_lds4(lds_at + (D::kXStages - 1) * D::kXStage + own, static_cast<uint32_t>(row) * static_cast<uint32_t>(ld) + (line - row * line_row) * 128, xbuf, 0);
+      }
+    }
+    feed<D::kXL, D::kXStages>(
+        stages, per, end - first,
+        [&](int st, int slot) {
+          const int t = first + st;
+          uint32_t back[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) back[q] = xpiece[q] + t * 256 >= xbytes ? xpiece[q] : 0;
+#pragma unroll
+          for (int u = 0; u < D::kXL; ++u) load_to_lds16(lds_at + slot * D::kXStage + own + u * 1024, xrow[u] - back[u & 3], xbuf, t * 256);
+        },
+        [&](int st, int slot) {
+#pragma unroll
+          for (int u = 0; u < D::kXL; ++u)
+            if (xpiece[u & 3] + (first + st) * 256 >= xbytes)
+              *reinterpret_cast<u32x4*>(lds + slot * D::kXStage + own + u * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+        });
+  }
+  if (wave >= R::kWaves) {
+    __syncthreads();
+  } else {
+    uint32_t xat[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) xat[j] = ks * R::kXBytes + i * R::kXRow + ((4 * j + g) ^ i) * 16;
+    const uint32_t own = D::kWAt + wave * R::kOwn, wat = own + i * 64 + (g ^ ((i >> 1) & 3)) * 16, sat = own + R::kWBytes + i * 8 + g * 2;
+    f32x4 acc[NT][MT], done[PER][NT][MT];  // the slice at hand, and the slices walked
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    u32x4 raw[NT], wf[2][NT], xf[2][MT];
+    uint32_t sc[NT];
+    auto fetch_raw = [&](const uint8_t* st, int nt) {
+      raw[nt] = *reinterpret_cast<const u32x4*>(st + wat + nt * 1024);
+      sc[nt] = *reinterpret_cast<const uint16_t*>(st + sat + nt * 128);
+    };
+    auto fetch_w = [&](u32x4(&w)[NT], int j, int nt) {
+#pragma unroll
+      for (int p = 0; p < 4; ++p) w[nt][p] = block::weight_pair<F>(raw[nt], sc[nt], j, p);
+    };
+    auto fetch_x = [&](u32x4(&x)[MT], const uint8_t* st, int j, int mt) { x[mt] = *reinterpret_cast<const u32x4*>(st + xat[j] + mt * 16 * R::kXRow); };
+    // (What was read of the stage before is in registers.)
+    auto arrive = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    arrive();
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      fetch_raw(lds, nt);
+      fetch_w(wf[0], 0, nt);
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) fetch_x(xf[0], lds, 0, mt);
+    const uint8_t *x_here = lds, *w_here = lds;  // the stage's slots
+    const uint8_t *const x_end = lds + D::kXStages * D::kXStage, *const w_end = lds + D::kWStages * D::kWStage;
+    int st = 0;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      for (const int all = min((q + 1) * a.steps_per_wave, stages); st < all; ++st) {
+        const uint8_t *x_next = x_here + D::kXStage, *w_next = w_here + D::kWStage;
+        x_next = x_next == x_end ? lds : x_next;
+        w_next = w_next == w_end ? lds : w_next;
+        // As block_wide.h's step: under an instruction's products the next one's fragments are read and expanded.
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          const bool last = j == J - 1;
+          __builtin_amdgcn_sched_barrier(0);
+          if (last) {
+            if (st + 1 < stages) arrive();
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) fetch_raw(w_next, nt);
+          }
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) fetch_x(xf[(j + 1) & 1], last ? x_next : x_here, (j + 1) % J, mt);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+              acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[j & 1][nt]), __builtin_bit_cast(bf16x8, xf[j & 1][mt]), acc[nt][mt], 0, 0, 0);
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) fetch_w(wf[(j + 1) & 1], (j + 1) % J, nt);
+#pragma unroll
+          for (int n = 0; n < MT * NT; ++n) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+          }
+        }
+        x_here = x_next;
+        w_here = w_next;
+      }
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          done[q][nt][mt] = acc[nt][mt];
+          acc[nt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    for (int b = max(stages, 1); b < per; ++b) asm volatile("s_barrier" ::: "memory");
+    __syncthreads();
+    // The slices' sums side by side in LDS, a row's pieces of four turned by the row; then everyone adds up what it writes.
+#pragma unroll
+    for (int q = 0; q < PER; ++q)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          *reinterpret_cast<f32x4*>(lds + (ks * PER + q) * kSlice + (mt * 16 + i) * BN * 4 + ((((wn * NT + nt) * 4 + g) ^ i) & (BN / 4 - 1)) * 16) = done[q][nt][mt];
+  }
+  __syncthreads();
+  write_slices<F, R::BM, BN, KS * PER, D::kThreads>(a, lds, n0, cols, slices);
 }
 
 template <class R, int F>
@@ -316,6 +572,29 @@ template <int F>
 bool launch_ring(const GemmArgs& a, int cols, int* status, hipStream_t stream) {
   const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave;
   return with_ring<F>(a.M, slices, cols, [&](auto ring) { *status = launch<decltype(ring), F>(a, slices, stream); });
+}
+
+template <int MT, int PER>
+int launch_fed_as(const GemmArgs& a, int slices, hipStream_t stream) {
+  using D = Fed<MT, PER>;
+  const auto kernel = fed_kernel<MT, PER>;
+  allow_lds(reinterpret_cast<const void*>(kernel), D::kLdsBytes);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((a.N + D::BN - 1) / D::BN)), dim3(D::kThreads), D::kLdsBytes, stream, a, slices);
+  return status_of(hipGetLastError());
+}
+
+inline int launch_fed(const GemmArgs& a, hipStream_t stream) {
+  const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave;
+  auto go = [&](auto mt) {
+    constexpr int MT = decltype(mt)::value;
+    return slices > 2 ? launch_fed_as<MT, 2>(a, slices, stream) : launch_fed_as<MT, 1>(a, slices, stream);
+  };
+  switch ((a.M + 15) / 16) {
+    case 1:
+    case 2: return go(std::integral_constant<int, 2>{});
+    case 3: return go(std::integral_constant<int, 3>{});
+    default: return go(std::integral_constant<int, 4>{});
+  }
 }
 
 }  // namespace ring

@@ -91,10 +91,10 @@ def time_variants(lx, kernel, M, N, K, repeats=7):
 
 
 def time_own_rule(lx, kernel, M, N, K, repeats=7):
-    """Median microseconds of the call without a table entry, or None where one of the variants is what it takes. (The ring kernel of
-    lx_gemm_w has no variant: an entry, whatever it names, keeps a call from it.)"""
+    """Median microseconds of the call without a table entry, or None where one of the variants is what it takes. (The ring kernels
+    of lx_gemm_w have no variant: an entry, whatever it names, keeps a call from them.)"""
     fmt = FORMATS.get(kernel.removeprefix("gemm_w_"))
-    if not kernel.startswith("gemm_w_") or lx.lib.dromos_plan_ring(fmt, M, N, K, 0, 1, None) <= 0:
+    if not kernel.startswith("gemm_w_") or (lx.lib.dromos_plan_ring(fmt, M, N, K, 0, 1, None) <= 0 and lx.lib.dromos_plan_fed(fmt, M, N, K, 0, 1) <= 0):
         return None
     device = {"device": "cuda"}
     data = torch.randint(0, 64, (N, 2 * K), dtype=torch.uint8, **device)  # any bytes that hold no NaN: times only

@@ -43,3 +43,13 @@ def test_look_ahead_stays_in_the_wavefronts_own_part(lib, M, N, K, plan):
     ("nvfp4", 40, 12368, 4096, True), ("fp8", 47, 7867, 8192, False), ("nvfp4", 24, 8970, 3616, False), ("nvfp4", 16, 7264, 4096, False)])
 def test_what_the_ring_takes(lib, fmt, M, N, K, taken):
     assert (lib.dromos_plan_ring(FORMATS[fmt], M, N, K, UNITS, 1, None) > 0) == taken
+
+
+# The form with loader wavefronts: of the calls above none, of those that ring_cols() leaves what was measured faster.
+@pytest.mark.parametrize("M,N,K,slices", [
+    (64, 14336, 4096, 4), (50, 8256, 4416, 3), (33, 14336, 8192, 4), (57, 9408, 8704, 3), (40, 24000, 3072, 2), (20, 16400, 4096, 2), (12, 9600, 2112, 3), (64, 20000, 1024, 1),
+    (64, 8192, 4096, 0), (64, 9088, 4096, 0), (12, 16500, 2112, 0), (16, 14336, 4096, 0), (32, 14336, 4096, 0), (44, 8656, 13184, 0), (20, 12384, 6144, 0), (8, 14336, 4160, 0),
+    (64, 14336, 4112, 0), (40, 8704, 4096, 0)])
+def test_what_the_form_with_loaders_takes(lib, M, N, K, slices):
+    assert lib.dromos_plan_fed(FORMATS["nvfp4"], M, N, K, UNITS, 1) == slices
+    assert slices == 0 or lib.dromos_plan_ring(FORMATS["nvfp4"], M, N, K, UNITS, 1, None) == 0
