@@ -1554,9 +1554,10 @@ block::Plan block_plan(const GemmArgs& a, int tuned, int units, bool buffer) {
   const int n_tiles = (a.N + kTileRows - 1) / kTileRows;
   if (!forced && a.M <= 64 && (MATH != LX_MATH_BF16 || !block_wanted<F>(a.M, n_tiles, a.K))) return kNone;
   const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave, mts = (a.M + 15) / 16;
-  const bool partial = buffer && slices > 1 && static_cast<size_t>(slices) * n_tiles * mts * kWave * 16 <= kSlabScratchBytes;
+  const size_t fits = buffer ? kSlabScratchBytes / (static_cast<size_t>(n_tiles) * mts * kWave * 16) : 0;  // slices the buffer holds
+  const bool partial = slices > 1 && fits >= static_cast<size_t>(slices);
   if (!forced && a.M <= 64 && !partial) return kNone;  // few blocks and no way to share them out: the kernels for up to 64 rows are ahead
-  const block::Plan p = block::plan<F, MATH>(a, units, partial);
+  const block::Plan p = block::plan<F, MATH>(a, units, fits < kMaxSplit ? static_cast<int>(fits) : kMaxSplit);
   if constexpr (F == LX_W_NVFP4) {
     // NVFP4 blocks that walk all of a long row, a few rows past 64: a chain of K tiles a block, at 8.2 us per 1000 values, on fewer
     // blocks than units, behind a pass of 64 rows and one of the rest. Blocks of 64 x 64, passes / blocks in us: without the partial-tile buffer

@@ -82,9 +82,9 @@ int best_shape(const GemmArgs& a, int tiles, int slices, int units, float* us) {
   return best;
 }
 
-// partial: there is a buffer for the slices' sums.
+// most: how many slices' sums there is a buffer for (0: none; kMaxSplit at most).
 template <int F, int MATH>
-Plan plan(const GemmArgs& a, int units, bool partial) {
+Plan plan(const GemmArgs& a, int units, int most) {
   constexpr bool kBytes = MATH != LX_MATH_BF16;
   // Load steps a K tile holds (NVFP4: two tiles a step).
   constexpr int kSteps = kBytes || F == LX_W_BF16 ? 2 : 1, kTilesPerStep = F == LX_W_NVFP4 ? 2 : 1;
@@ -92,19 +92,46 @@ Plan plan(const GemmArgs& a, int units, bool partial) {
   if (a.row_bytes * 256 >= (1ll << 31) || (!kBytes && a.xs.ld * 2 * 256 >= (1ll << 31)) || a.steps_per_wave % (2 * kSteps)) return {-1, 0, 0, 0};
   const int tiles = ((a.steps * kTilesPerStep + kSteps - 1) / kSteps + 1) / 2 * 2;
   const int slice_tiles = a.steps_per_wave * kTilesPerStep / kSteps, slices = (tiles + slice_tiles - 1) / slice_tiles;
-  float us = 0.0f, us_part = 0.0f;
+  float us = 0.0f;
   int whole = best_shape<F, MATH>(a, tiles, 1, units, &us);
   if (const float wide = wide_us<F, MATH>(a, units); wide < us) {
     whole = kWide;
     us = wide;
   }
-  if (partial && slices > 1) {
-    // One slice a workgroup: a second launch, and every slice's sums written and read once more (4.5 us and about 4 TB/s).
-    const int part = best_shape<F, MATH>(a, slice_tiles, slices, units, &us_part);
-    us_part += 4.5f + 8e-6f * a.M * a.N * slices / 4.0f;
-    if (us_part < us) return {kPart, part, tiles, slice_tiles};
+  // One slice a workgroup: a second launch, and every slice's sums written and read once more (4.5 us and about 4 TB/s).
+  auto parts = [&](int cut, int cuts, int* part) {
+    float t;
+    *part = best_shape<F, MATH>(a, cut, cuts, units, &t);
+    return t + 4.5f + 8e-6f * a.M * a.N * cuts / 4.0f;
+  };
+  Plan best = {MATH != LX_MATH_INT8 && slices > 1 ? kAdded : kOne, whole, tiles, slice_tiles};
+  if (int part; slices > 1 && most >= slices) {
+    if (const float t = parts(slice_tiles, slices, &part); t < us) {
+      best = {kPart, part, tiles, slice_tiles};
+      us = t;
+    }
   }
-  return {MATH != LX_MATH_INT8 && slices > 1 ? kAdded : kOne, whole, tiles, slice_tiles};
+  if constexpr (MATH == LX_MATH_INT8) {
+    // int32 sums are the same however K is cut. Where the row's own slices are taken, fewer that are estimated to take less (1418 x 576 x
+    // 13312 13 -> 4 slices, 57.1 -> 40.5 us; 437 x 2608 x 10016 10 -> 3, 54.6 -> 36.9; 515 x 592 x 2656 6 -> 4 18.7 -> 17.2: rows, N, K; more
+    // slices lost where they were estimated ahead, 79 x 1328 x 2240 5 -> 9 11.6 / 12.7). Where a workgroup walks all of K it stays so unless
+    // its block is a large one and slices are estimated at 0.85 of the time: 515 x 4096 x 11008 in three 59.7 -> 53.1, 418 x 5216 x 13344 82 -> 70; of 14
+    // others that the estimate alone moved eight lost (66 x 5360 x 2464 12.4 / 16.7). 250 random calls of 65 .. 2048 rows, N 512 .. 16384, K 1024 ..
+    // 14336: 0.95 on average, none above 1.03; fewer columns were not measured.
+    const bool own = best.mode == kPart;
+    if (a.N >= 512 && (own || best.shape == 2 || best.shape == 3)) {
+      if (!own) us *= 0.85f;
+      for (int s = 2; s <= (own ? slices - 1 : most) && s * 2 <= tiles; ++s) {
+        const int cut = ((tiles + s - 1) / s + 1) / 2 * 2;
+        int part;
+        if (const float t = parts(cut, (tiles + cut - 1) / cut, &part); t < us) {
+          best = {kPart, part, tiles, cut};
+          us = t;
+        }
+      }
+    }
+  }
+  return best;
 }
 
 }  // namespace block

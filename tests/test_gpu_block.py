@@ -76,6 +76,23 @@ def test_every_shape_and_mode(hip, fmt, math, mode, shape, M, N, K):
     assert torch.equal(on_a_stream(hip, buffer, x, w, math, y.clone()), chunks_of_32(hip, x, w, math, y))
 
 
+# The INT8 math's sums are whole numbers, so K is cut as is estimated fastest: slices that are not the row's own, the last of them shorter, rows
+# that end inside a K tile, on every block shape; and where no number of slices fits the partial-tile buffer, none.
+@pytest.mark.parametrize("M,N,K,plan", [(193, 2703, 6528, 10), (515, 4096, 11008, 11), (437, 2608, 10016, 10), (585, 608, 4992, 9), (545, 576, 2752, 8), (133, 1968, 5136, 10),
+                                        (430, 5216, 13344, 11), (4000, 4096, 4096, None)])
+def test_int8_math_in_slices_of_its_own(hip, M, N, K, plan):
+    got = hip.lib.dromos_plan_gemm(FORMATS["int8"], MATH_INT8, M, N, K, 0, 1)
+    assert got == plan if plan else got // 4 != 2
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    w = random_weight(FORMATS["int8"], N, K, N + K).to("cuda")
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    for y in (torch.full((M, N), float("nan"), device="cuda"), torch.full((M, N), float("nan"), device="cuda", dtype=torch.bfloat16)):
+        want = on_a_stream(hip, False, x, w, MATH_INT8, y.clone())
+        assert torch.equal(on_a_stream(hip, True, x, w, MATH_INT8, y.clone()), want)
+    assert torch.equal(chunks_of_32(hip, x[:64].contiguous(), w, MATH_INT8, y[:64].clone()), want[:64])
+
+
+
 # The wide block (128 x 256, plan shape 16): blocks cut short in rows and columns, odd and even numbers of columns, rows that end
 # inside a stage of K and inside its pieces, two stages past a slice, the epilogue's operands.
 WIDE = [("int8", MATH_BF16, 20, 834, 7039, 1568, 0), ("int8", MATH_BF16, 20, 1921, 3332, 1600, 1), ("fp8", MATH_BF16, 20, 2731, 2203, 1568, 2), ("fp8", MATH_BF16, 20, 769, 7668, 1600, 0),
