@@ -19,10 +19,64 @@ constexpr int kSpecRows = 8;  // engine/cpu/spec.cpp:12
 // (blockIdx.y; the last block may hold fewer), a lane taking four consecutive k of every 256 (a 16-byte load where the
 // rows allow it), f32 FMAs in ascending k, the lane sums combined by one fixed tree. Nothing in a row's sums depends on
 // the other rows.
-template <bool VEC>
+
+// Rows that allow 16-byte loads, R (1, 2, 4, 8) of them at a time (one past the last repeats it and is not stored). Bound by latency: a
+// router is a few workgroups (64 experts: 16), and a loop that waited for a piece of the row before it asked for the next took a memory
+// latency per 256 values. All of a row's pieces of 256, up to C (4, 8), are asked for together, and the activations against as many
+// pieces as R rows leave registers for: 64 x 1024 at one row 2.9 -> 1.9 us (a launch is 1.6), 128 x 2048 at eight 9.8 -> 4.4, 4096 x 2048
+// at eight 22.4 -> 14.9.
+template <int R, int C>
 __global__ void __launch_bounds__(kThreads) spec_gemv_f32_kernel(const float* __restrict__ x, int64_t ld_x, const float* __restrict__ w,
                                                                  const float* __restrict__ bias, float* __restrict__ y, int64_t ld_y,
                                                                  int rows, int N, int K) {
+  constexpr int kAtOnce = R == 1 ? C : R == 2 ? 4 : R == 4 ? 2 : 1;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t n = static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + threadIdx.x / kWave;
+  if (n >= N) return;
+  const int m0 = blockIdx.y * kSpecRows, M = min(kSpecRows, rows - m0);
+  x += m0 * ld_x;
+  y += m0 * ld_y;
+  const float* wrow = w + n * K;
+  float acc[R];
+#pragma unroll
+  for (int m = 0; m < R; ++m) acc[m] = 0.0f;
+  for (int k0 = 0; k0 < K; k0 += C * kWave * 4) {
+    // (Past K: the row's last values, not multiplied.)
+    auto at = [&](int c) { return k0 + c * kWave * 4 + lane * 4; };
+    f32x4 wv[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) wv[c] = *reinterpret_cast<const f32x4*>(wrow + min(at(c), K - 4));
+#pragma unroll
+    for (int c0 = 0; c0 < C; c0 += kAtOnce) {
+      f32x4 xv[kAtOnce][R];
+#pragma unroll
+      for (int c = 0; c < kAtOnce; ++c)
+#pragma unroll
+        for (int m = 0; m < R; ++m) xv[c][m] = *reinterpret_cast<const f32x4*>(x + min(m, M - 1) * ld_x + min(at(c0 + c), K - 4));
+#pragma unroll
+      for (int c = 0; c < kAtOnce; ++c) {
+        if (at(c0 + c) >= K) continue;
+#pragma unroll
+        for (int m = 0; m < R; ++m) {
+          acc[m] = __builtin_fmaf(xv[c][m].x, wv[c0 + c].x, acc[m]);
+          acc[m] = __builtin_fmaf(xv[c][m].y, wv[c0 + c].y, acc[m]);
+          acc[m] = __builtin_fmaf(xv[c][m].z, wv[c0 + c].z, acc[m]);
+          acc[m] = __builtin_fmaf(xv[c][m].w, wv[c0 + c].w, acc[m]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < R; ++m) {
+    const float s = wave_sum(acc[m]);
+    if (lane == 0 && m < M) y[m * ld_y + n] = bias ? s + bias[n] : s;
+  }
+}
+
+// The same assignment of k to lanes and the same order, element by element.
+__global__ void __launch_bounds__(kThreads) spec_gemv_f32_plain_kernel(const float* __restrict__ x, int64_t ld_x, const float* __restrict__ w,
+                                                                       const float* __restrict__ bias, float* __restrict__ y, int64_t ld_y,
+                                                                       int rows, int N, int K) {
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t n = static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + threadIdx.x / kWave;
   if (n >= N) return;
@@ -33,29 +87,12 @@ __global__ void __launch_bounds__(kThreads) spec_gemv_f32_kernel(const float* __
   float acc[kSpecRows];
 #pragma unroll
   for (int m = 0; m < kSpecRows; ++m) acc[m] = 0.0f;
-  if constexpr (VEC) {
-    for (int k = lane * 4; k < K; k += kWave * 4) {
-      const f32x4 wv = *reinterpret_cast<const f32x4*>(wrow + k);
+  for (int k0 = lane * 4; k0 < K; k0 += kWave * 4) {
+    for (int k = k0; k < min(k0 + 4, K); ++k) {
+      const float wv = wrow[k];
 #pragma unroll
-      for (int m = 0; m < kSpecRows; ++m) {
-        if (m < M) {
-          const f32x4 xv = *reinterpret_cast<const f32x4*>(x + m * ld_x + k);
-          acc[m] = __builtin_fmaf(xv.x, wv.x, acc[m]);
-          acc[m] = __builtin_fmaf(xv.y, wv.y, acc[m]);
-          acc[m] = __builtin_fmaf(xv.z, wv.z, acc[m]);
-          acc[m] = __builtin_fmaf(xv.w, wv.w, acc[m]);
-        }
-      }
-    }
-  } else {
-    // The same assignment of k to lanes and the same order, element by element.
-    for (int k0 = lane * 4; k0 < K; k0 += kWave * 4) {
-      for (int k = k0; k < min(k0 + 4, K); ++k) {
-        const float wv = wrow[k];
-#pragma unroll
-        for (int m = 0; m < kSpecRows; ++m)
-          if (m < M) acc[m] = __builtin_fmaf(x[m * ld_x + k], wv, acc[m]);
-      }
+      for (int m = 0; m < kSpecRows; ++m)
+        if (m < M) acc[m] = __builtin_fmaf(x[m * ld_x + k], wv, acc[m]);
     }
   }
 #pragma unroll
@@ -68,8 +105,13 @@ __global__ void __launch_bounds__(kThreads) spec_gemv_f32_kernel(const float* __
 int spec_gemv(const float* x, int ld_x, const float* w, const float* bias, float* y, int ld_y, int M, int N, int K, hipStream_t s) {
   const bool vec = K % 4 == 0 && ld_x % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
   const dim3 grid((N + kThreads / kWave - 1) / (kThreads / kWave), (M + kSpecRows - 1) / kSpecRows);
-  if (vec) hipLaunchKernelGGL(spec_gemv_f32_kernel<true>, grid, dim3(kThreads), 0, s, x, ld_x, w, bias, y, ld_y, M, N, K);
-  else hipLaunchKernelGGL(spec_gemv_f32_kernel<false>, grid, dim3(kThreads), 0, s, x, ld_x, w, bias, y, ld_y, M, N, K);
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, s, x, ld_x, w, bias, y, ld_y, M, N, K); };
+  const bool few = K <= 4 * kWave * 4;
+  if (!vec) go(spec_gemv_f32_plain_kernel);
+  else if (M == 1) few ? go(spec_gemv_f32_kernel<1, 4>) : go(spec_gemv_f32_kernel<1, 8>);
+  else if (M == 2) few ? go(spec_gemv_f32_kernel<2, 4>) : go(spec_gemv_f32_kernel<2, 8>);
+  else if (M <= 4) few ? go(spec_gemv_f32_kernel<4, 4>) : go(spec_gemv_f32_kernel<4, 8>);
+  else few ? go(spec_gemv_f32_kernel<8, 4>) : go(spec_gemv_f32_kernel<8, 8>);
   return status_of(hipGetLastError());
 }
 

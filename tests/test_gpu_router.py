@@ -56,6 +56,19 @@ def test_gemm_f32(hip, oracle, M, N, K, pad):
     assert rel_l2(no_bias, x.double() @ w.double().T) <= 1e-5
 
 
+# Rows that 16-byte loads can read give the bits of the same rows one float off, which are read element by element: around the pieces of 256
+# values, the pieces asked for together (four to 1024 values, eight beyond), and the rows taken at a time.
+@pytest.mark.parametrize("K", [4, 252, 256, 260, 1020, 1024, 1028, 2044, 2048, 2052, 5000])
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 9, 19])
+def test_gemm_f32_read_either_way_gives_the_same_bits(hip, M, K):
+    N = 21
+    x, w, bias, _ = router_inputs(M, N, K, M + K)
+    x, w, bias = x.cuda(), w.cuda(), bias.cuda()
+    off = torch.empty(M * K + 1, device="cuda")[1:].view(M, K).copy_(x)
+    assert off.data_ptr() % 16 == 4
+    assert torch.equal(ops.gemm_f32(hip, x, w, bias).view(torch.int32), ops.gemm_f32(hip, off, w, bias).view(torch.int32))
+
+
 def test_gemm_f32_arguments(hip):
     w = torch.zeros(16, 64, device="cuda")
     assert ops.gemm_f32(hip, torch.zeros(0, 64, device="cuda"), w, None, status=True) == 0
