@@ -29,10 +29,25 @@ __device__ __forceinline__ uint32_t order_key(float b) {
   return b != b ? 0u : b == 0.0f ? 0x80000000u : k;
 }
 
+__device__ __forceinline__ uint32_t wave_max_key(uint32_t v) {
+  auto moved = [&](auto c) { return __float_as_uint(dpp_move<decltype(c)::value>(__uint_as_float(v))); };
+  v = max(v, moved(std::integral_constant<int, 0xB1>{}));
+  v = max(v, moved(std::integral_constant<int, 0x4E>{}));
+  v = max(v, moved(std::integral_constant<int, 0x141>{}));
+  v = max(v, moved(std::integral_constant<int, 0x140>{}));
+  float a, b;
+  swap_halves<true>(__uint_as_float(v), a, b);
+  v = max(__float_as_uint(a), __float_as_uint(b));
+  swap_halves<false>(__uint_as_float(v), a, b);
+  return max(__float_as_uint(a), __float_as_uint(b));
+}
+
 // One wavefront per token; a lane keeps its NPL logits (elements lane, lane + 64, ...) in registers, so the row
-// is read once. E <= 64 * NPL. The picks: with few experts (NPL <= 4) every element is ranked against all the
-// others (its rank among the biased logits, ties to the lower index, is its pick number); with many, top_k
-// rounds of a wave-wide argmax.
+// is read once. E <= 64 * NPL. The picks: rounds of a wave-wide maximum of order_key, the lowest index that holds it struck out. With
+// many picks of up to 256 experts instead every element's rank among all (its pick number), which takes as long whatever top_k is.
+// A launch's latency is what counts (a token is one wavefront): a round is 0.25 us, the ranks 1.3, 3.5 and 12 us at 64, 128 and 256
+// experts, so they are for more than 6, 16 and 40 picks. Eight of 128 experts 5.8 -> 4.1 us, of 256 14.0 -> 5.2 (by ranks before), of 512
+// 16.2 -> 11.6 (rounds through LDS before); 2048 tokens' 7.3 -> 4.7; two of 64 3.0 -> 2.1.
 template <int NPL>
 __global__ void __launch_bounds__(kThreads) route_kernel(const float* __restrict__ logits, const float* __restrict__ bias,
                                                          int32_t* __restrict__ ids, float* __restrict__ weights,
@@ -75,7 +90,7 @@ __global__ void __launch_bounds__(kThreads) route_kernel(const float* __restrict
     entropy[t] = h;
     confidence[t] = 1.0f / z;  // the largest probability is exp(0) / z
   }
-  if constexpr (NPL <= 4) {
+  if (NPL <= 4 && top_k > (NPL == 1 ? 6 : NPL == 2 ? 16 : 40)) {
     // Element (u, ~index) as one 64-bit number: another element is picked before this one exactly when its number
     // is the greater (a greater biased logit, or the same and a lower index).
     uint32_t key[NPL];
@@ -115,41 +130,34 @@ __global__ void __launch_bounds__(kThreads) route_kernel(const float* __restrict
       picked_logit[wave][lane] = NAN;
     }
   } else {
-    // A picked element is struck from the candidates by its bit in `taken` (bit j: this lane's element j), not by
-    // its value: an element whose logit is -inf can still be picked, once, lowest index first, as the reference's
-    // search over the indices not yet picked does (engine/cpu/moe.cpp:367-381).
-    uint64_t taken = 0;
+    // An element whose logit is -inf can still be picked, once, lowest index first, as the reference's search over the indices not yet
+    // picked does (engine/cpu/moe.cpp:367-381); a NaN, a picked or a missing element (key 0) cannot.
+    uint32_t key[NPL];
+#pragma unroll
+    for (int j = 0; j < NPL; ++j) key[j] = lane + j * kWave < E ? order_key(biased[j]) : 0u;
     for (int r = 0; r < top_k; ++r) {
-      float best = -INFINITY;
-      int best_i = E;
+      uint32_t most = key[0];
+#pragma unroll
+      for (int j = 1; j < NPL; ++j) most = max(most, key[j]);
+      most = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(wave_max_key(most))));
+      if (most == 0) {
+        // Fewer rankable logits than picks: the rest get the id E, as a search that finds nothing returns.
+        if (lane >= r && lane < top_k) {
+          ids[t * top_k + lane] = E;
+          picked_logit[wave][lane] = NAN;
+        }
+        break;
+      }
+      bool found = false;
 #pragma unroll
       for (int j = 0; j < NPL; ++j) {
-        const int i = lane + j * kWave;
-        if (i < E && !((taken >> j) & 1) && (biased[j] > best || (biased[j] == best && i < best_i))) {
-          best = biased[j];
-          best_i = i;
-        }
-      }
-#pragma unroll
-      for (int off = 1; off < kWave; off <<= 1) {
-        const float ov = __shfl_xor(best, off);
-        const int oi = __shfl_xor(best_i, off);
-        if (ov > best || (ov == best && oi < best_i)) {
-          best = ov;
-          best_i = oi;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < NPL; ++j) {
-        if (lane + j * kWave == best_i) {
-          ids[t * top_k + r] = best_i;
+        const uint64_t holds = __ballot(key[j] == most);
+        if (!found && holds != 0 && lane == __ffsll(static_cast<unsigned long long>(holds)) - 1) {
+          ids[t * top_k + r] = lane + j * kWave;
           picked_logit[wave][r] = v[j];
-          taken |= 1ull << j;
+          key[j] = 0;
         }
-      }
-      if (best_i >= E && lane == 0) {
-        ids[t * top_k + r] = E;
-        picked_logit[wave][r] = NAN;
+        found = found || holds != 0;
       }
     }
   }

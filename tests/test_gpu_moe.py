@@ -42,6 +42,14 @@ def test_route_picks_on_awkward_values_match_the_oracle(hip, oracle, E, top_k):
         checks.same_routes(ops.route(hip, logits.cuda(), None if b is None else b.cuda(), top_k), ops.route(oracle, logits, b, top_k), E)
 
 
+# The picks are made in rounds up to 6, 16 and 40 of them (64, 128, 256 experts) and by ranks beyond; in rounds always with more experts.
+@pytest.mark.parametrize("E,top_k", [(64, 6), (64, 7), (40, 1), (65, 16), (65, 17), (128, 16), (128, 17), (129, 40), (129, 41), (256, 40), (256, 41), (257, 64), (1024, 32), (1030, 3)])
+def test_route_either_side_of_the_rounds(hip, oracle, E, top_k):
+    logits, bias = checks.awkward_logits(E, top_k)
+    for b in (None, bias):
+        checks.same_routes(ops.route(hip, logits.cuda(), None if b is None else b.cuda(), top_k), ops.route(oracle, logits, b, top_k), E)
+
+
 def test_route_empty_and_invalid(hip):
     logits = torch.zeros(2, 8, device="cuda")
     ids = torch.zeros(2, 2, dtype=torch.int32, device="cuda")
