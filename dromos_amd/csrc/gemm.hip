@@ -1377,7 +1377,7 @@ bool walk_parts_wanted(int M, int n_tiles, int64_t K, int tuned) {
 // - NVFP4 from 17 rows. Rows of a cut load step (K % 128), where the walk kernel does not apply, 0.39 .. 0.75. Whole ones 0.78 where a workgroup takes 32
 //   (K above 4096 on more than 512 tiles, and 768, 1.07); at 33 .. 64 rows to 768 tiles 0.74, above where a slice is eight steps 0.92; else 0.98 .. 1.06.
 //   Three slices of 5120 .. 7168 values for four wavefronts 1.08 .. 1.20. Four slices of 64 rows leave the ring two stages: on 896 tiles, where
-//   the walk kernel takes four tiles a workgroup, 28.3 / 29.0 (bf16 outputs 30.8 / 28.8).
+//   the walk kernel takes four tiles a workgroup, 28.3 / 29.0 (bf16 outputs 30.8 / 28.8); fed_wanted() takes those (21.1).
 template <int F>
 int ring_cols(const GemmArgs& a, int n_tiles) {
   if (a.M <= 8 || n_tiles < 289 || n_tiles > 1024 || a.K < 2048 || a.K > 11264) return 0;

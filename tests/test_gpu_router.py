@@ -64,9 +64,9 @@ def test_gemm_f32_read_either_way_gives_the_same_bits(hip, M, K):
     N = 21
     x, w, bias, _ = router_inputs(M, N, K, M + K)
     x, w, bias = x.cuda(), w.cuda(), bias.cuda()
-    off = torch.empty(M * K + 1, device="cuda")[1:].view(M, K).copy_(x)
+    off = torch.empty(N * K + 1, device="cuda")[1:].view(N, K).copy_(w)
     assert off.data_ptr() % 16 == 4
-    assert torch.equal(ops.gemm_f32(hip, x, w, bias).view(torch.int32), ops.gemm_f32(hip, off, w, bias).view(torch.int32))
+    assert torch.equal(ops.gemm_f32(hip, x, w, bias).view(torch.int32), ops.gemm_f32(hip, x, off, bias).view(torch.int32))
 
 
 def test_gemm_f32_arguments(hip):
