@@ -1886,6 +1886,23 @@ int slab_release(hipStream_t stream) {
   return status_of(hipFree(buffer));
 }
 
+// What a feeder (gemm_ring.h) asks for and waits for, counted on the host.
+struct FeedOnHost {
+  int loads, stages, ahead, asked;  // a stage's loads, the stages, what was asked for before the walk and so far
+  int here = 0, barriers = 0;
+  bool early = false;
+  void load(int, int) { asked += loads; }
+  void finish(int, int) const {}
+  void written() const {}
+  template <int LEFT>
+  void wait() {
+    if (asked - LEFT > here) here = asked - LEFT;
+  }
+  void barrier() {
+    if (++barriers <= stages && here < ahead + loads * barriers) early = true;
+  }
+};
+
 }  // namespace dro
 
 using namespace dro;
@@ -1970,6 +1987,20 @@ LX_API int dromos_plan_fed(int format, int M, int N, int K, int units, int buffe
   const int n_tiles = (N + kTileRows - 1) / kTileRows;
   if (tuned_variant(gemm_key<LX_W_NVFP4>(), M, N, K) >= 0 || ring_cols<LX_W_NVFP4>(a, n_tiles) > 0 || !fed_wanted(a, n_tiles)) return 0;
   return (a.steps + a.steps_per_wave - 1) / a.steps_per_wave;
+}
+
+// Follows a feeder of that form (rows' activations, or weights with `weights` set) through its walk: how many of its loads are on their
+// way when it ends, or -1 where a barrier is passed with that stage's loads on their way. ahead: loads asked for before the walk.
+LX_API int dromos_feed_in_flight(int rows, int weights, int stages, int all, int ahead) {
+  auto follow = [&](auto d) {
+    using D = decltype(d);
+    const int loads = weights ? D::kWL : D::kXL;
+    FeedOnHost walk{loads, stages, ahead, ahead};
+    if (weights) ring::feed<D::kWL, D::kWStages>(stages, all, stages - 1, walk);
+    else ring::feed<D::kXL, D::kXStages>(stages, all, stages - 1, walk);
+    return walk.early || walk.barriers != all ? -1 : walk.asked - walk.here;
+  };
+  return rows > 48 ? follow(ring::Fed<4, 2>{}) : rows > 32 ? follow(ring::Fed<3, 2>{}) : follow(ring::Fed<2, 2>{});
 }
 
 int lx_gemv_w(const void* x, lx_dtype x_dtype, int ld_x, const lx_weight* w, const void* bias, lx_dtype bias_dtype, void* y,

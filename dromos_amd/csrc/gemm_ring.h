@@ -304,33 +304,53 @@ struct Fed {
   static constexpr int kSums = KS * PER * R::BM * BN * 4, kRing = kWAt + kWStages * kWStage, kLdsBytes = kRing > kSums ? kRing : kSums;
 };
 
-// Waits until at most `behind` (0 .. MOST) stages of L loads each are on their way.
-template <int L, int MOST>
-__device__ __forceinline__ void wait_stages(int behind) {
-  if constexpr (MOST == 0) wait_loads<0>();
-  else if (behind >= MOST) wait_loads<MOST * L>();
-  else wait_stages<L, MOST - 1>(behind);
+// What a feeder's walk does on the device: load(st, slot) asks for stage st's loads, finish(st, slot) writes zeros where a stage reaches past
+// the row's end. (A walk of its own because tests follow it on the host: gemm.hip, dromos_feed_in_flight().)
+template <class Load, class Finish>
+struct Feeder {
+  Load load;
+  Finish finish;
+  template <int LEFT>
+  __device__ __forceinline__ void wait() const {
+    wait_loads<LEFT>();
+  }
+  __device__ __forceinline__ void written() const { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+  __device__ __forceinline__ void barrier() const { asm volatile("s_barrier" ::: "memory"); }
+};
+template <class Load, class Finish>
+__device__ __forceinline__ Feeder<Load, Finish> feeder(Load load, Finish finish) {
+  return {load, finish};
 }
 
-// A feeder's walk over `stages` stages by a ring of STAGES: load(st, slot) asks for stage st's L loads, finish(st, slot) writes zeros where
-// stage `cut`, which has arrived, reaches past the row's end. `all` stages have a barrier.
-template <int L, int STAGES, class Load, class Finish>
-__device__ __forceinline__ void feed(int stages, int all, int cut, Load&& load, Finish&& finish) {
+// Waits until at most `behind` (0 .. MOST) stages of L loads each are on their way.
+template <int L, int MOST, class Walk>
+__host__ __device__ __forceinline__ void wait_stages(int behind, Walk& walk) {
+  if constexpr (MOST == 0) walk.template wait<0>();
+  else if (behind >= MOST) walk.template wait<MOST * L>();
+  else wait_stages<L, MOST - 1>(behind, walk);
+}
+
+// A feeder's walk over `stages` stages of L loads each by a ring of STAGES; stage `cut` is finished once it has arrived. `all` stages have a
+// barrier. Whatever was asked for before the walk (a look-ahead) is here when it ends, as the walk's own loads are: a feeder that has no
+// stage waits for nothing else, and behind the walk the ring's bytes are the sums'.
+template <int L, int STAGES, class Walk>
+__host__ __device__ __forceinline__ void feed(int stages, int all, int cut, Walk&& walk) {
   for (int st = 0; st < STAGES - 1; ++st)
-    if (st < stages) load(st, st);
+    if (st < stages) walk.load(st, st);
   int slot = 0, free = STAGES - 1;  // stage st's slot, and the one that stage st - 1 + STAGES takes
   for (int st = 0; st < stages; ++st) {
-    wait_stages<L, STAGES - 2>(stages - 1 - st);
+    wait_stages<L, STAGES - 2>(stages - 1 - st, walk);
     if (st == cut) {
-      finish(st, slot);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      walk.finish(st, slot);
+      walk.written();
     }
-    asm volatile("s_barrier" ::: "memory");
-    if (st - 1 + STAGES < stages) load(st - 1 + STAGES, free);
+    walk.barrier();
+    if (st - 1 + STAGES < stages) walk.load(st - 1 + STAGES, free);
     slot = slot + 1 == STAGES ? 0 : slot + 1;
     free = free + 1 == STAGES ? 0 : free + 1;
   }
-  for (int st = stages; st < all; ++st) asm volatile("s_barrier" ::: "memory");
+  for (int st = stages; st < all; ++st) walk.barrier();
+  if (stages == 0) walk.template wait<0>();
 }
 
 template <int MT, int PER>
@@ -365,7 +385,7 @@ __global__ void __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(
     }
     feed<D::kWL, D::kWStages>(
         stages, per, end - first,
-        [&](int st, int slot) {
+        feeder([&](int st, int slot) {
           const int t = first + st;
           const uint32_t to = lds_at + D::kWAt + slot * D::kWStage + ks * R::kOwn;
           const uint32_t wback = wpiece + t * 64 >= wbytes ? wpiece : 0, sback = spiece + t * 8 >= sbytes ? spiece : 0;
@@ -389,7 +409,7 @@ __global__ void __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(
             if (spiece + t * 8 >= sbytes) *reinterpret_cast<uint32_t*>(s) = 0;
             else if (spiece + t * 8 + 2 >= sbytes) *reinterpret_cast<uint16_t*>(s + 2) = 0;
           }
-        });
+        }));
   } else if (wave >= R::kWaves) {
     // Slice ks's activations, 256 bytes of every row a stage. Places in a row as in ring_kernel.
     const Rsrc xbuf = block::buffer_of(a.xs.x, (a.M - 1) * ld + xbytes);
@@ -406,7 +426,7 @@ __global__ void __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(
     const uint32_t own = ks * R::kXBytes;
     // All workgroups walk K together, so an activation row's next piece would come from memory for every one of them. The workgroups of
     // a die (every eighth) share out the activations' 128-byte lines and ask for them once, at the start. They land where this
-    // feeder loads the last slot's stage, which it asks for behind a wait for these.
+    // feeder loads the last slot's stage, which it asks for behind a wait for these (a feeder without stages waits at its walk's end).
     {
       const int line_row = (xbytes + 127) / 128, lines = line_row * a.M, share = (lines + (gridDim.x >> 3)) / ((gridDim.x >> 3) + 1);
       for (int at = ks * kWave + lane; at - lane < share; at += KS * kWave) {
@@ -416,7 +436,7 @@ __global__ void __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(
     }
     feed<D::kXL, D::kXStages>(
         stages, per, end - first,
-        [&](int st, int slot) {
+        feeder([&](int st, int slot) {
           const int t = first + st;
           uint32_t back[4];
 #pragma unroll
@@ -429,7 +449,7 @@ __global__ void __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(
           for (int u = 0; u < D::kXL; ++u)
             if (xpiece[u & 3] + (first + st) * 256 >= xbytes)
               *reinterpret_cast<u32x4*>(lds + slot * D::kXStage + own + u * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
-        });
+        }));
   }
   if (wave >= R::kWaves) {
     __syncthreads();

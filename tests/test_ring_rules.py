@@ -53,3 +53,14 @@ def test_what_the_ring_takes(lib, fmt, M, N, K, taken):
 def test_what_the_form_with_loaders_takes(lib, M, N, K, slices):
     assert lib.dromos_plan_fed(FORMATS["nvfp4"], M, N, K, UNITS, 1) == slices
     assert slices == 0 or lib.dromos_plan_ring(FORMATS["nvfp4"], M, N, K, UNITS, 1, None) == 0
+
+
+# A feeder of that form passes a stage's barrier with the stage's loads here, and ends its walk with nothing on its way: behind it the ring
+# is overwritten, and what it asked for ahead of the walk counts too (one without any stage, where K is one slice, asks for that only).
+@pytest.mark.parametrize("weights", [0, 1])
+@pytest.mark.parametrize("rows", [32, 48, 64])
+def test_a_feeder_leaves_nothing_in_flight(lib, rows, weights):
+    for ahead in (0, 1, 2, 7):
+        for stages in (0, 1, 2, 3, 4, 5, 9, 10, 11, 40):
+            for idle in (0, 1, 8):
+                assert lib.dromos_feed_in_flight(rows, weights, stages, max(1, stages + idle), ahead) == 0, (stages, idle, ahead)
