@@ -1911,9 +1911,10 @@ extern "C" {
 
 // How lx_gemm_w's block kernel takes a call on bf16 rows that lie as its vector paths want them, on a device of `units` compute
 // units (0: the current device) and a stream with or without a partial-tile buffer: 4 * mode + shape (gemm_block_plan.h), or -1
-// where the kernels for up to 64 rows take it. For tests of the rule: nothing is launched, and with
+// where the kernels for up to 64 rows take it or there is nothing to compute. For tests of the rule: nothing is launched, and with
 // `units` given no device is needed.
 LX_API int dromos_plan_gemm(int format, int math, int M, int N, int K, int units, int buffer) {
+  if (M < 1 || N < 1 || K < 1) return -1;
   if (units <= 0) units = compute_units();
   auto ask = [&](auto f, auto m) {
     GemmArgs a{};
@@ -1942,7 +1943,7 @@ LX_API int dromos_plan_gemm(int format, int math, int M, int N, int K, int units
 // 0 where another kernel takes it. lds, if given: thirteen numbers, the bytes of a stage of its ring and for each of its four
 // wavefronts where its look-ahead goes, where its own part begins and how many bytes that has.
 LX_API int dromos_plan_ring(int format, int M, int N, int K, int units, int buffer, int* lds) {
-  if (M < 1 || M > 64 || dromos_plan_gemm(format, LX_MATH_BF16, M, N, K, units, buffer) >= 0) return 0;
+  if (M < 1 || M > 64 || N < 1 || K < 1 || dromos_plan_gemm(format, LX_MATH_BF16, M, N, K, units, buffer) >= 0) return 0;
   auto ask = [&](auto f) {
     GemmArgs a{};
     a.M = M;
@@ -1977,7 +1978,7 @@ LX_API int dromos_plan_ring(int format, int M, int N, int K, int units, int buff
 
 // The same of its form with loader wavefronts: the slices of K, or 0.
 LX_API int dromos_plan_fed(int format, int M, int N, int K, int units, int buffer) {
-  if (format != LX_W_NVFP4 || M < 1 || M > 64 || K % 32 != 0 || dromos_plan_gemm(format, LX_MATH_BF16, M, N, K, units, buffer) >= 0) return 0;
+  if (format != LX_W_NVFP4 || M < 1 || M > 64 || N < 1 || K < 1 || K % 32 != 0 || dromos_plan_gemm(format, LX_MATH_BF16, M, N, K, units, buffer) >= 0) return 0;
   GemmArgs a{};
   a.M = M;
   a.N = N;

@@ -58,6 +58,14 @@ def test_sums_of_slices_that_do_not_fit_the_buffer_stay_in_the_workgroup(lib):
     assert not part(8192)
 
 
+# Sizes that are no product have no plan (the slices that fit the buffer are a quotient by the rows and columns).
+@pytest.mark.parametrize("M,N,K", [(128, 0, 4096), (0, 4096, 4096), (128, 4096, 0), (-5, 4096, 4096), (128, -16, 4096), (128, 4096, -64), (32, 0, 4096), (32, 4096, 0)])
+def test_nothing_to_compute(lib, M, N, K):
+    for fmt, math in (("bf16", 0), ("int8", 0), ("int8", 1), ("fp8", 0), ("fp8", 2), ("nvfp4", 0)):
+        assert lib.dromos_plan_gemm(FORMATS[fmt], math, M, N, K, UNITS, 1) == -1
+        assert lib.dromos_plan_ring(FORMATS[fmt], M, N, K, UNITS, 1, None) == 0 and lib.dromos_plan_fed(FORMATS[fmt], M, N, K, UNITS, 1) == 0
+
+
 @pytest.mark.parametrize("fmt,math", [("bf16", 0), ("int8", 1), ("fp8", 0), ("fp8", 2), ("nvfp4", 0)])
 def test_the_variant_table_has_the_last_word(lib, fmt, math):
     # An entry is for a row count (the next power of two) of a matrix: "block" asks for the block kernel at any count, every other
