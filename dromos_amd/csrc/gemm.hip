@@ -1418,24 +1418,28 @@ int ring_cols(const GemmArgs& a, int n_tiles) {
 }
 
 // Whether NVFP4 rows go to the ring kernel with loader wavefronts (gemm_ring.h: fed_kernel), of the calls that ring_cols() leaves: more than
-// 512 tiles (fewer are up to 1.6 times the present time: 192 workgroups at 384 tiles) in up to four slices. From 6200 random calls on
-// cold weights (9 .. 64 rows, 128 .. 1536 tiles, K 1024 .. 14336 in steps of 64, f32 and bf16 outputs), times over the kernels it replaces: the 3014
-// calls of them that this takes 0.69 on average, none above 1.01.
+// 512 tiles (fewer are up to 1.6 times the present time: 96 workgroups at 384 tiles) in up to four slices. The lines come from 6200 random calls
+// on cold weights to 1536 tiles and 2500 to 9500 tiles; 1500 others, drawn afterwards over all that this takes (9 .. 64 rows, 513 .. 9500 tiles, K 1024 ..
+// 14336, f32 and bf16 outputs), need 0.69 of the time of the kernels it replaces, one of them 1.03 and none more.
 // - Rows of a cut load step (K % 128), where no walk kernel applies, from 17 rows 0.23 .. 0.95; at 9 .. 16 rows 0.75 .. 1.0 to 1024 tiles
-//   (beyond, a second round of workgroups, 0.96 .. 1.26).
-// - Whole steps from 33 rows 0.29 .. 1.0, but not slices of 32 steps (1.04 .. 1.14).
-// - At 17 .. 32 rows the walk kernels' bytes count for more: beyond 1024 tiles 0.65 .. 0.99; to 1024 where K leaves slices unfilled, which this kernel
-//   does not walk (filled ones 0.92 .. 1.13), not three slices of 16 steps that are four fifths full, nor four of 24 and more (to 1.46).
+//   (beyond, a second round of workgroups, 0.96 .. 1.26), but not three or four slices of eight steps that are full (0.98 .. 1.03).
+// - Whole steps from 33 rows 0.29 .. 1.0, but not four slices of more than 24 steps (1.04 .. 1.14). One slice (more than 1810 tiles: a
+//   vocabulary's; half of this kernel's wavefronts have no slice then) is behind on long rows: to 48 rows below K = 6144 to 1.03, from there to 1.09;
+//   at 49 .. 64 rows 0.32 .. 0.93.
+// - At 17 .. 32 rows the walk kernels' bytes count for more. Beyond 1024 tiles in two slices and more 0.55 .. 1.03 below K = 9216, from there 0.88 .. 1.08; in
+//   one slice 0.65 .. 1.02 below K = 3584, but not of whole walks (K = 2048, to 1.15) or eight steps (to 1.16); from there 0.78 .. 1.25, the longer the worse
+//   (32000 x 14336 at 17 rows 88 / 110 us, 50304 x 8192 at 32 rows 108 / 129). To 1024 tiles where K leaves slices unfilled, which this kernel does not
+//   walk (filled ones 0.92 .. 1.13), not three slices of 16 steps that are four fifths full, nor four of 24 and more (to 1.46).
 bool fed_wanted(const GemmArgs& a, int n_tiles) {
-  if (a.M <= 8 || n_tiles <= 512 || a.K < 1024 || a.K > 14336) return false;
+  if (a.M <= 8 || n_tiles <= 512 || n_tiles > 9500 || a.K < 1024 || a.K > 14336) return false;
   if (a.scale_row_bytes % 4 != 0 || reinterpret_cast<uintptr_t>(a.scale) % 4 != 0) return false;  // (loaded four bytes at a time)
   const int slices = (a.steps + a.steps_per_wave - 1) / a.steps_per_wave;
   if (slices > 4) return false;
-  if (a.K % 128 != 0) return a.M > 16 || n_tiles <= 1024;
-  if (a.M <= 16) return false;
-  if (a.M > 32) return slices < 4 || a.steps_per_wave <= 24;
-  if (n_tiles > 1024) return true;
   const int filled = a.steps * 100 / (a.steps_per_wave * slices);  // percent of the slices
+  if (a.K % 128 != 0) return a.M > 16 || (n_tiles <= 1024 && (slices < 3 || a.steps_per_wave > 8 || filled <= 94));
+  if (a.M <= 16) return false;
+  if (a.M > 32) return slices == 4 ? a.steps_per_wave <= 24 : slices > 1 || a.M > 48 || a.K < 6144;
+  if (n_tiles > 1024) return slices > 1 ? a.K < 9216 : a.K > 1024 && a.K < 3584 && a.K % 2048 != 0;
   if (filled > 94) return false;
   return slices == 3 ? a.steps_per_wave != 16 || filled < 80 : slices < 4 || a.steps_per_wave <= 16;
 }

@@ -55,6 +55,16 @@ def test_what_the_form_with_loaders_takes(lib, M, N, K, slices):
     assert slices == 0 or lib.dromos_plan_ring(FORMATS["nvfp4"], M, N, K, UNITS, 1, None) == 0
 
 
+# Where that form was measured slower: few rows in one slice (more than 1810 tiles, as vocabularies have) or two long ones; and beyond what was
+# measured.
+@pytest.mark.parametrize("M,N,K,slices", [
+    (32, 32000, 4096, 0), (17, 128256, 4096, 0), (24, 151936, 8192, 0), (20, 30001, 14336, 0), (25, 68208, 2048, 0), (31, 49872, 1024, 0), (17, 32000, 3072, 1), (32, 128256, 1536, 1),
+    (24, 18656, 1024, 0), (32, 50304, 4160, 1), (48, 32000, 14336, 0), (34, 50848, 8192, 0), (33, 152000, 4096, 1), (49, 32000, 14336, 1), (64, 128256, 4096, 1), (64, 152016, 4096, 0), (30, 18480, 14208, 0),
+    (32, 20480, 8192, 2), (23, 16574, 13952, 0), (13, 13614, 3008, 0), (14, 11888, 4032, 0), (9, 9600, 2112, 3)])
+def test_what_the_form_with_loaders_leaves(lib, M, N, K, slices):
+    assert lib.dromos_plan_fed(FORMATS["nvfp4"], M, N, K, UNITS, 1) == slices
+
+
 # A feeder of that form passes a stage's barrier with the stage's loads here, and ends its walk with nothing on its way: behind it the ring
 # is overwritten, and what it asked for ahead of the walk counts too (one without any stage, where K is one slice, asks for that only).
 @pytest.mark.parametrize("weights", [0, 1])
