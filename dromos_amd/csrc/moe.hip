@@ -48,7 +48,8 @@ __device__ __forceinline__ uint32_t wave_max_key(uint32_t v) {
 // A launch's latency is what counts (a token is one wavefront): a round is 0.25 us, the ranks 1.3, 3.5 and 12 us at 64, 128 and 256
 // experts, so they are for more than 6, 16 and 40 picks. Eight of 128 experts 5.8 -> 4.1 us, of 256 14.0 -> 5.2 (by ranks before), of 512
 // 16.2 -> 11.6 (rounds through LDS before); 2048 tokens' 7.3 -> 4.7; two of 64 3.0 -> 2.1.
-template <int NPL>
+// (Two kernels: with the rounds behind a branch the ranks were up to 1.21 times as slow, 48 of 160 experts 16.0 / 19.3 us.)
+template <int NPL, bool RANKS>
 __global__ void __launch_bounds__(kThreads) route_kernel(const float* __restrict__ logits, const float* __restrict__ bias,
                                                          int32_t* __restrict__ ids, float* __restrict__ weights,
                                                          float* __restrict__ entropy, float* __restrict__ confidence, int T,
@@ -90,7 +91,7 @@ __global__ void __launch_bounds__(kThreads) route_kernel(const float* __restrict
     entropy[t] = h;
     confidence[t] = 1.0f / z;  // the largest probability is exp(0) / z
   }
-  if (NPL <= 4 && top_k > (NPL == 1 ? 6 : NPL == 2 ? 16 : 40)) {
+  if constexpr (RANKS) {
     // Element (u, ~index) as one 64-bit number: another element is picked before this one exactly when its number
     // is the greater (a greater biased logit, or the same and a lower index).
     uint32_t key[NPL];
@@ -525,11 +526,12 @@ int route(const float* logits, const float* selection_bias, int32_t* ids, float*
   // One token: one wavefront, not a workgroup of sixteen of which fifteen leave at once.
   const int waves = T < kWaves ? T : kWaves;
   const dim3 grid((T + waves - 1) / waves), block(waves * kWave);
-  if (E <= 64) hipLaunchKernelGGL(route_kernel<1>, grid, block, 0, s, logits, selection_bias, ids, weights, entropy, confidence, T, E, top_k);
-  else if (E <= 128) hipLaunchKernelGGL(route_kernel<2>, grid, block, 0, s, logits, selection_bias, ids, weights, entropy, confidence, T, E, top_k);
-  else if (E <= 256) hipLaunchKernelGGL(route_kernel<4>, grid, block, 0, s, logits, selection_bias, ids, weights, entropy, confidence, T, E, top_k);
-  else if (E <= 1024) hipLaunchKernelGGL(route_kernel<16>, grid, block, 0, s, logits, selection_bias, ids, weights, entropy, confidence, T, E, top_k);
-  else hipLaunchKernelGGL(route_kernel<64>, grid, block, 0, s, logits, selection_bias, ids, weights, entropy, confidence, T, E, top_k);
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, logits, selection_bias, ids, weights, entropy, confidence, T, E, top_k); };
+  if (E <= 64) top_k > 6 ? go(route_kernel<1, true>) : go(route_kernel<1, false>);
+  else if (E <= 128) top_k > 16 ? go(route_kernel<2, true>) : go(route_kernel<2, false>);
+  else if (E <= 256) top_k > 40 ? go(route_kernel<4, true>) : go(route_kernel<4, false>);
+  else if (E <= 1024) go(route_kernel<16, false>);
+  else go(route_kernel<64, false>);
   return status_of(hipGetLastError());
 }
 
