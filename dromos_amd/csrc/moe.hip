@@ -47,7 +47,7 @@ __device__ __forceinline__ uint32_t wave_max_key(uint32_t v) {
 // many picks of up to 256 experts instead every element's rank among all (its pick number), which takes as long whatever top_k is.
 // A launch's latency is what counts (a token is one wavefront): a round is 0.25 us, the ranks 1.3, 3.5 and 12 us at 64, 128 and 256
 // experts, so they are for more than 6, 16 and 40 picks. Eight of 128 experts 5.8 -> 4.1 us, of 256 14.0 -> 5.2 (by ranks before), of 512
-// 16.2 -> 11.6 (rounds through LDS before); 2048 tokens' 7.3 -> 4.7; two of 64 3.0 -> 2.1.
+// 15.5 -> 7.6 (rounds through LDS before); 2048 tokens' 7.3 -> 4.7; two of 64 3.0 -> 2.1.
 // (Two kernels: with the rounds behind a branch the ranks were up to 1.21 times as slow, 48 of 160 experts 16.0 / 19.3 us.)
 template <int NPL, bool RANKS>
 __global__ void __launch_bounds__(kThreads) route_kernel(const float* __restrict__ logits, const float* __restrict__ bias,
@@ -149,16 +149,39 @@ __global__ void __launch_bounds__(kThreads) route_kernel(const float* __restrict
         }
         break;
       }
-      bool found = false;
+      // The lowest index that holds it. With more elements a lane its own lowest, then the lanes' by the same maximum: a look at every element's
+      // lanes, which is less for four and fewer (6000 tokens' eight of 128 7.4 / 8.2 us), was slower there than the search through LDS before
+      // (one of 2048 experts 14.6 / 15.5; now 14.4, eight of 512 11.1 -> 7.6).
+      if constexpr (NPL <= 4) {
+        bool found = false;
 #pragma unroll
-      for (int j = 0; j < NPL; ++j) {
-        const uint64_t holds = __ballot(key[j] == most);
-        if (!found && holds != 0 && lane == __ffsll(static_cast<unsigned long long>(holds)) - 1) {
-          ids[t * top_k + r] = lane + j * kWave;
-          picked_logit[wave][r] = v[j];
-          key[j] = 0;
+        for (int j = 0; j < NPL; ++j) {
+          const uint64_t holds = __ballot(key[j] == most);
+          if (!found && holds != 0 && lane == __ffsll(static_cast<unsigned long long>(holds)) - 1) {
+            ids[t * top_k + r] = lane + j * kWave;
+            picked_logit[wave][r] = v[j];
+            key[j] = 0;
+          }
+          found = found || holds != 0;
         }
-        found = found || holds != 0;
+      } else {
+        int own = NPL;
+        float logit = 0.0f;
+#pragma unroll
+        for (int j = NPL - 1; j >= 0; --j) {
+          const bool holds = key[j] == most;
+          own = holds ? j : own;
+          logit = holds ? v[j] : logit;
+        }
+        const uint32_t index = own * kWave + lane;
+        const uint32_t first = ~static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(wave_max_key(~index))));
+        if (index == first) {
+          ids[t * top_k + r] = static_cast<int>(index);
+          picked_logit[wave][r] = logit;
+        }
+        own = index == first ? own : NPL;
+#pragma unroll
+        for (int j = 0; j < NPL; ++j) key[j] = j == own ? 0u : key[j];
       }
     }
   }

@@ -50,6 +50,15 @@ def test_route_either_side_of_the_rounds(hip, oracle, E, top_k):
         checks.same_routes(ops.route(hip, logits.cuda(), None if b is None else b.cuda(), top_k), ops.route(oracle, logits, b, top_k), E)
 
 
+# More than 256 experts: a lane's own lowest of several that hold the maximum, then the lanes'; every number of elements a lane, its last ones missing.
+@pytest.mark.parametrize("E,top_k", [(257, 1), (321, 8), (1023, 64), (1025, 64), (2048, 1), (2049, 16), (4095, 7), (4096, 64)])
+def test_route_on_many_experts(hip, oracle, E, top_k):
+    logits, bias = checks.awkward_logits(E, top_k)
+    logits = torch.cat([logits, torch.zeros(1, E), torch.arange(E).remainder(3).float()[None], torch.full((1, E), float("nan")).scatter(1, torch.tensor([[E - 1, 64]]), 1.0)])
+    for b in (None, bias):
+        checks.same_routes(ops.route(hip, logits.cuda(), None if b is None else b.cuda(), top_k), ops.route(oracle, logits, b, top_k), E)
+
+
 def test_route_empty_and_invalid(hip):
     logits = torch.zeros(2, 8, device="cuda")
     ids = torch.zeros(2, 2, dtype=torch.int32, device="cuda")
