@@ -22,21 +22,17 @@ constexpr int kSpecRows = 8;  // engine/cpu/spec.cpp:12
 
 // Rows that allow 16-byte loads, R (1, 2, 4, 8) of them at a time (one past the last repeats it and is not stored). Bound by latency: a
 // router is a few workgroups (64 experts: 16), and a loop that waited for a piece of the row before it asked for the next took a memory
-// latency per 256 values. All of a row's pieces of 256, up to C (4, 8), are asked for together, and the activations against as many
+// latency per 256 values. All of a row's pieces of 256, up to C (1, 2, 4, 6, 8), are asked for together, and the activations against as many
 // pieces as R rows leave registers for: 64 x 1024 at one row 2.9 -> 1.9 us (a launch is 1.6), 128 x 2048 at eight 9.8 -> 4.4, 4096 x 2048
-// at eight 22.4 -> 14.9.
+// at eight 22.4 -> 14.9. C is the least that takes a row in as many turns: with 4 and 8 only, pieces that the row does not have cost wide and short ones
+// more than the turns (4096 x 256 at nine rows 4.85 us piece by piece, 5.55, now 4.9; 1600 x 1168 at 29 12.0, 12.65, 12.1). Of 820 random calls (1 .. 64
+// rows, N 2 .. 4096, K 64 .. 8192) against piece by piece 0.69 of the time, two above 1.03 (41 x 1215 x 2128 18.6 / 20.5, rows, N, K: more workgroups than its
+// registers let a unit hold at once).
 template <int R, int C>
-__global__ void __launch_bounds__(kThreads) spec_gemv_f32_kernel(const float* __restrict__ x, int64_t ld_x, const float* __restrict__ w,
-                                                                 const float* __restrict__ bias, float* __restrict__ y, int64_t ld_y,
-                                                                 int rows, int N, int K) {
-  constexpr int kAtOnce = R == 1 ? C : R == 2 ? 4 : R == 4 ? 2 : 1;
+__device__ __forceinline__ void spec_rows(const float* __restrict__ x, int64_t ld_x, const float* __restrict__ wrow, const float* __restrict__ bias,
+                                          float* __restrict__ y, int64_t ld_y, int M, int64_t n, int K) {
+  constexpr int kPairs = C % 2 == 0 ? 2 : 1, kAtOnce = R == 1 ? C : R == 2 ? (C % 4 == 0 ? 4 : kPairs) : R == 4 ? kPairs : 1;
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t n = static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + threadIdx.x / kWave;
-  if (n >= N) return;
-  const int m0 = blockIdx.y * kSpecRows, M = min(kSpecRows, rows - m0);
-  x += m0 * ld_x;
-  y += m0 * ld_y;
-  const float* wrow = w + n * K;
   float acc[R];
 #pragma unroll
   for (int m = 0; m < R; ++m) acc[m] = 0.0f;
@@ -73,6 +69,23 @@ __global__ void __launch_bounds__(kThreads) spec_gemv_f32_kernel(const float* __
   }
 }
 
+// REST: the last block has at most half of R rows and takes as many. On wide products only, where eight rows' work for one counts (4096 x 2048 at nine
+// rows 21.6 -> 18.6, 3207 x 6652 at 20 79 -> 72); the two paths in one kernel cost narrow ones 5 .. 10 %.
+template <int R, int C, bool REST = false>
+__global__ void __launch_bounds__(kThreads) spec_gemv_f32_kernel(const float* __restrict__ x, int64_t ld_x, const float* __restrict__ w,
+                                                                 const float* __restrict__ bias, float* __restrict__ y, int64_t ld_y,
+                                                                 int rows, int N, int K) {
+  const int64_t n = static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + threadIdx.x / kWave;
+  if (n >= N) return;
+  const int m0 = blockIdx.y * kSpecRows, M = min(kSpecRows, rows - m0);
+  x += m0 * ld_x;
+  y += m0 * ld_y;
+  const float* wrow = w + n * K;
+  if constexpr (REST)
+    if (M <= R / 2) return spec_rows<R / 2, C>(x, ld_x, wrow, bias, y, ld_y, M, n, K);
+  spec_rows<R, C>(x, ld_x, wrow, bias, y, ld_y, M, n, K);
+}
+
 // The same assignment of k to lanes and the same order, element by element.
 __global__ void __launch_bounds__(kThreads) spec_gemv_f32_plain_kernel(const float* __restrict__ x, int64_t ld_x, const float* __restrict__ w,
                                                                        const float* __restrict__ bias, float* __restrict__ y, int64_t ld_y,
@@ -106,12 +119,21 @@ int spec_gemv(const float* x, int ld_x, const float* w, const float* bias, float
   const bool vec = K % 4 == 0 && ld_x % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
   const dim3 grid((N + kThreads / kWave - 1) / (kThreads / kWave), (M + kSpecRows - 1) / kSpecRows);
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, s, x, ld_x, w, bias, y, ld_y, M, N, K); };
-  const bool few = K <= 4 * kWave * 4;
+  auto rows = [&](auto c) {
+    constexpr int C = decltype(c)::value;
+    if (M == 1) go(spec_gemv_f32_kernel<1, C>);
+    else if (M == 2) go(spec_gemv_f32_kernel<2, C>);
+    else if (M <= 4) go(spec_gemv_f32_kernel<4, C>);
+    else if (C >= 6 && M > kSpecRows && (M - 1) % kSpecRows < kSpecRows / 2 && N > 1024) go(spec_gemv_f32_kernel<8, C, (C >= 6)>);
+    else go(spec_gemv_f32_kernel<8, C>);
+  };
+  const int pieces = K / (kWave * 4) + (K % (kWave * 4) != 0);
   if (!vec) go(spec_gemv_f32_plain_kernel);
-  else if (M == 1) few ? go(spec_gemv_f32_kernel<1, 4>) : go(spec_gemv_f32_kernel<1, 8>);
-  else if (M == 2) few ? go(spec_gemv_f32_kernel<2, 4>) : go(spec_gemv_f32_kernel<2, 8>);
-  else if (M <= 4) few ? go(spec_gemv_f32_kernel<4, 4>) : go(spec_gemv_f32_kernel<4, 8>);
-  else few ? go(spec_gemv_f32_kernel<8, 4>) : go(spec_gemv_f32_kernel<8, 8>);
+  else if (pieces <= 1) rows(std::integral_constant<int, 1>{});
+  else if (pieces <= 2) rows(std::integral_constant<int, 2>{});
+  else if (pieces <= 4) rows(std::integral_constant<int, 4>{});
+  else if ((pieces + 7) / 8 * 6 >= pieces) rows(std::integral_constant<int, 6>{});
+  else rows(std::integral_constant<int, 8>{});
   return status_of(hipGetLastError());
 }
 

@@ -57,16 +57,25 @@ def test_gemm_f32(hip, oracle, M, N, K, pad):
 
 
 # Rows that 16-byte loads can read give the bits of the same rows one float off, which are read element by element: around the pieces of 256
-# values, the pieces asked for together (four to 1024 values, eight beyond), and the rows taken at a time.
-@pytest.mark.parametrize("K", [4, 252, 256, 260, 1020, 1024, 1028, 2044, 2048, 2052, 5000])
+# values, the pieces asked for together (one, two, four, six or eight of them), and the rows taken at a time.
+@pytest.mark.parametrize("K", [4, 252, 256, 260, 508, 512, 516, 1020, 1024, 1028, 1532, 1536, 1540, 2044, 2048, 2052, 3072, 3076, 5000])
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 9, 19])
 def test_gemm_f32_read_either_way_gives_the_same_bits(hip, M, K):
-    N = 21
+    either_way(hip, M, 21, K)
+
+
+def either_way(hip, M, N, K):
     x, w, bias, _ = router_inputs(M, N, K, M + K)
     x, w, bias = x.cuda(), w.cuda(), bias.cuda()
     off = torch.empty(N * K + 1, device="cuda")[1:].view(N, K).copy_(w)
     assert off.data_ptr() % 16 == 4
     assert torch.equal(ops.gemm_f32(hip, x, w, bias).view(torch.int32), ops.gemm_f32(hip, x, off, bias).view(torch.int32))
+
+
+# Wide products whose last rows are one to four of a block of eight.
+@pytest.mark.parametrize("M,N,K", [(9, 1025, 1028), (12, 1030, 2048), (17, 1101, 2308), (20, 1025, 3076), (27, 1201, 1540), (13, 1025, 2048), (9, 1024, 2048)])
+def test_gemm_f32_wide_products_with_few_rows_behind_the_eights(hip, M, N, K):
+    either_way(hip, M, N, K)
 
 
 def test_gemm_f32_arguments(hip):
