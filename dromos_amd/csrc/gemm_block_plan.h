@@ -3,6 +3,7 @@
 #pragma once
 
 #include <math.h>
+#include <stdint.h>
 
 #include "gemm_args.h"
 
@@ -65,15 +66,20 @@ struct Plan {
   int mode, shape, tiles, slice_tiles;
 };
 
+// Blocks of shape `i` a unit takes one behind the other, for `slices` launches of the product's.
+template <int F, int MATH>
+int64_t turns(const GemmArgs& a, int i, int slices, int units) {
+  const Shape s = shape<F, MATH>(i);
+  return (static_cast<int64_t>((a.M + s.bm - 1) / s.bm) * ((a.N + s.bn - 1) / s.bn) * slices + units - 1) / units;
+}
+
 // The shape that is estimated to take least for `slices` launches of `tiles` K tiles a block, and that time.
 template <int F, int MATH>
 int best_shape(const GemmArgs& a, int tiles, int slices, int units, float* us) {
   int best = 0;
   for (int i = 0; i < kShapes<F, MATH>; ++i) {
     const Shape s = shape<F, MATH>(i);
-    const int64_t blocks = static_cast<int64_t>((a.M + s.bm - 1) / s.bm) * ((a.N + s.bn - 1) / s.bn) * slices;
-    const int64_t a_unit = (blocks + units - 1) / units;
-    const float t = (s.per_block * a_unit + s.once) * tiles * (1.0f / 64);
+    const float t = (s.per_block * turns<F, MATH>(a, i, slices, units) + s.once) * tiles * (1.0f / 64);
     if (i == 0 || t < *us) {
       best = i;
       *us = t;
@@ -116,15 +122,20 @@ Plan plan(const GemmArgs& a, int units, int most) {
     // 13312 13 -> 4 slices, 57.1 -> 40.5 us; 437 x 2608 x 10016 10 -> 3, 54.6 -> 36.9; 515 x 592 x 2656 6 -> 4 18.7 -> 17.2: rows, N, K; more
     // slices lost where they were estimated ahead, 79 x 1328 x 2240 5 -> 9 11.6 / 12.7). Where a workgroup walks all of K it stays so unless
     // its block is a large one and slices are estimated at 0.85 of the time: 515 x 4096 x 11008 in three 59.7 -> 53.1, 418 x 5216 x 13344 82 -> 70; of 14
-    // others that the estimate alone moved eight lost (66 x 5360 x 2464 12.4 / 16.7). 250 random calls of 65 .. 2048 rows, N 512 .. 16384, K 1024 ..
-    // 14336: 0.95 on average, none above 1.03; fewer columns were not measured.
+    // others that the estimate alone moved eight lost (66 x 5360 x 2464 12.4 / 16.7). Nor do a row's own slices make way for blocks of more turns: one of 128 x
+    // 256 a unit is as good as two of 64 x 128 (44 calls estimated at 0.85 .. 0.99: 0.91 .. 1.06, 154 x 6263 x 7584 37.4 / 39.8); and for 128 x 128 only where
+    // that is estimated at 0.94 (18 calls above that: 0.91 .. 1.11, 112 x 11455 x 8192 41.7 / 46.3). 600 calls in slices drawn
+    // afterwards (65 .. 4096 rows, N 512 .. 32768, K 1024 .. 14336): 0.87 on average with the sums' wider stores, none above 1.03; fewer columns were not measured.
     const bool own = best.mode == kPart;
     if (a.N >= 512 && (own || best.shape == 2 || best.shape == 3)) {
+      const int64_t most_turns = own ? turns<F, MATH>(a, best.shape, slices, units) : INT64_MAX;
+      const float large_us = own && best.shape == 3 ? 0.94f * us : INFINITY;
       if (!own) us *= 0.85f;
       for (int s = 2; s <= (own ? slices - 1 : most) && s * 2 <= tiles; ++s) {
         const int cut = ((tiles + s - 1) / s + 1) / 2 * 2;
+        const int cuts = (tiles + cut - 1) / cut;
         int part;
-        if (const float t = parts(cut, (tiles + cut - 1) / cut, &part); t < us) {
+        if (const float t = parts(cut, cuts, &part); t < us && (part != 2 || t < large_us) && turns<F, MATH>(a, part, cuts, units) <= most_turns) {
           best = {kPart, part, tiles, cut};
           us = t;
         }

@@ -58,6 +58,14 @@ def test_sums_of_slices_that_do_not_fit_the_buffer_stay_in_the_workgroup(lib):
     assert not part(8192)
 
 
+# The INT8 math's own cuts of K: not into small blocks that a unit would take two of, where one large one was as good, nor for little; one small block a
+# unit is ahead.
+@pytest.mark.parametrize("M,N,K,plan", [(154, 6263, 7584, {10, 11}), (191, 4148, 12320, {10, 11}), (183, 4240, 13376, {10, 11}), (172, 5984, 6048, {10, 11}), (112, 11455, 8192, {11}), (211, 8030, 13344, {11}), (639, 618, 5632, {9}), (142, 3376, 8448, {9}),
+                                          (100, 2826, 13824, {10})])
+def test_int8_math_slices_take_no_more_turns(lib, M, N, K, plan):
+    assert lib.dromos_plan_gemm(FORMATS["int8"], 1, M, N, K, UNITS, 1) in plan
+
+
 # Sizes that are no product have no plan (the slices that fit the buffer are a quotient by the rows and columns).
 @pytest.mark.parametrize("M,N,K", [(128, 0, 4096), (0, 4096, 4096), (128, 4096, 0), (-5, 4096, 4096), (128, -16, 4096), (128, 4096, -64), (32, 0, 4096), (32, 4096, 0)])
 def test_nothing_to_compute(lib, M, N, K):
