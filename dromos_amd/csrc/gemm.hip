@@ -1890,6 +1890,32 @@ int slab_release(hipStream_t stream) {
   return status_of(hipFree(buffer));
 }
 
+// The block kernel's plan for a call as dromos_plan_gemm() takes it.
+block::Plan plan_of(int format, int math, int M, int N, int K, int units, int buffer) {
+  if (M < 1 || N < 1 || K < 1) return {-1, 0, 0, 0};
+  if (units <= 0) units = compute_units();
+  auto ask = [&](auto f, auto m) {
+    GemmArgs a{};
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.xs.ld = K;
+    cut_rows<f()>(a);
+    return block_plan<f(), m()>(a, tuned_variant(gemm_key<f()>(), M, N, K), units, buffer != 0);
+  };
+  constexpr std::integral_constant<int, LX_MATH_BF16> bf16{};
+  switch (format) {
+    case LX_W_BF16: return ask(std::integral_constant<int, LX_W_BF16>{}, bf16);
+    case LX_W_INT8:
+      if (math == LX_MATH_INT8) return ask(std::integral_constant<int, LX_W_INT8>{}, std::integral_constant<int, LX_MATH_INT8>{});
+      return ask(std::integral_constant<int, LX_W_INT8>{}, bf16);
+    case LX_W_FP8:
+      if (math == LX_MATH_FP8) return ask(std::integral_constant<int, LX_W_FP8>{}, std::integral_constant<int, LX_MATH_FP8>{});
+      return ask(std::integral_constant<int, LX_W_FP8>{}, bf16);
+    default: return ask(std::integral_constant<int, LX_W_NVFP4>{}, bf16);
+  }
+}
+
 // What a feeder (gemm_ring.h) asks for and waits for, counted on the host.
 struct FeedOnHost {
   int loads, stages, ahead, asked;  // a stage's loads, the stages, what was asked for before the walk and so far
@@ -1918,29 +1944,14 @@ extern "C" {
 // where the kernels for up to 64 rows take it or there is nothing to compute. For tests of the rule: nothing is launched, and with
 // `units` given no device is needed.
 LX_API int dromos_plan_gemm(int format, int math, int M, int N, int K, int units, int buffer) {
-  if (M < 1 || N < 1 || K < 1) return -1;
-  if (units <= 0) units = compute_units();
-  auto ask = [&](auto f, auto m) {
-    GemmArgs a{};
-    a.M = M;
-    a.N = N;
-    a.K = K;
-    a.xs.ld = K;
-    cut_rows<f()>(a);
-    const block::Plan p = block_plan<f(), m()>(a, tuned_variant(gemm_key<f()>(), M, N, K), units, buffer != 0);
-    return p.mode < 0 ? -1 : 4 * p.mode + p.shape;
-  };
-  constexpr std::integral_constant<int, LX_MATH_BF16> bf16{};
-  switch (format) {
-    case LX_W_BF16: return ask(std::integral_constant<int, LX_W_BF16>{}, bf16);
-    case LX_W_INT8:
-      if (math == LX_MATH_INT8) return ask(std::integral_constant<int, LX_W_INT8>{}, std::integral_constant<int, LX_MATH_INT8>{});
-      return ask(std::integral_constant<int, LX_W_INT8>{}, bf16);
-    case LX_W_FP8:
-      if (math == LX_MATH_FP8) return ask(std::integral_constant<int, LX_W_FP8>{}, std::integral_constant<int, LX_MATH_FP8>{});
-      return ask(std::integral_constant<int, LX_W_FP8>{}, bf16);
-    default: return ask(std::integral_constant<int, LX_W_NVFP4>{}, bf16);
-  }
+  const block::Plan p = plan_of(format, math, M, N, K, units, buffer);
+  return p.mode < 0 ? -1 : 4 * p.mode + p.shape;
+}
+
+// The slices of K whose sums that plan leaves in the partial-tile buffer, or 0.
+LX_API int dromos_plan_slices(int format, int math, int M, int N, int K, int units, int buffer) {
+  const block::Plan p = plan_of(format, math, M, N, K, units, buffer);
+  return p.mode == block::kPart ? (p.tiles + p.slice_tiles - 1) / p.slice_tiles : 0;
 }
 
 // The same of the ring kernel, for a pass of up to 64 bf16 rows under the BF16 math: 8 * its weight rows a workgroup + the slices of K, or

@@ -2,6 +2,8 @@
 were measured faster there go, those that were measured slower do not."""
 
 import ctypes
+import math
+import random
 
 import pytest
 
@@ -64,6 +66,23 @@ def test_sums_of_slices_that_do_not_fit_the_buffer_stay_in_the_workgroup(lib):
                                           (100, 2826, 13824, {10})])
 def test_int8_math_slices_take_no_more_turns(lib, M, N, K, plan):
     assert lib.dromos_plan_gemm(FORMATS["int8"], 1, M, N, K, UNITS, 1) in plan
+
+
+# Slices' sums stay inside the 64 MiB of the buffer that a stream has, whatever the sizes: 1 KB for 16 rows by 16 columns of each slice, of
+# which there are sixteen at most.
+@pytest.mark.parametrize("fmt,math_id", [("bf16", 0), ("int8", 0), ("int8", 1), ("fp8", 0), ("fp8", 2), ("nvfp4", 0)])
+def test_the_sums_of_slices_fit_the_buffer(lib, fmt, math_id):
+    rng = random.Random(fmt)
+    cut, most = 0, 0
+    for _ in range(20000):
+        M, N, K = (int(2 ** rng.uniform(math.log2(low), math.log2(high))) for low, high in ((1, 70000), (1, 70000), (64, 70000)))
+        slices = lib.dromos_plan_slices(FORMATS[fmt], math_id, M, N, K // 32 * 32, UNITS, 1)
+        assert (slices > 0) == (lib.dromos_plan_gemm(FORMATS[fmt], math_id, M, N, K // 32 * 32, UNITS, 1) // 4 == 2)
+        used = slices * -(-N // 16) * -(-M // 16) * 1024
+        assert slices <= 16 and used <= 64 << 20, (M, N, K)
+        assert lib.dromos_plan_slices(FORMATS[fmt], math_id, M, N, K // 32 * 32, UNITS, 0) == 0
+        cut, most = cut + (slices > 1), max(most, used)
+    assert cut > 1000 and most > 60 << 20
 
 
 # Sizes that are no product have no plan (the slices that fit the buffer are a quotient by the rows and columns).
