@@ -106,7 +106,7 @@ bool launch_ring_bf16(const GemmArgs& a, int cols, int* status, hipStream_t stre
 bool launch_ring_int8(const GemmArgs& a, int cols, int* status, hipStream_t stream);
 bool launch_ring_fp8(const GemmArgs& a, int cols, int* status, hipStream_t stream);
 bool launch_ring_nvfp4(const GemmArgs& a, int cols, int* status, hipStream_t stream);
-// The same of its form with loader wavefronts, for 17 .. 64 rows on NVFP4 weights in up to four slices. Returns the launch's status.
+// The same of its form with loader wavefronts, for 9 .. 64 rows on NVFP4 weights in up to four slices. Returns the launch's status.
 int launch_fed_nvfp4(const GemmArgs& a, hipStream_t stream);
 
 // gemm_block_<format>.hip: the block kernel (gemm_block.h) for any number of bf16 activation rows, gemm_block_<format>_math.hip the

@@ -146,9 +146,7 @@ __global__ void __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(
     }
 #pragma unroll
     for (int u = 0; u < R::kSLoads; ++u) {
-      uint8_t* const s = to + own_at + R::kWBytes + u * 256 + lane * 4;
-      if (spiece + t * 8 >= sbytes) *reinterpret_cast<uint32_t*>(s) = 0;
-      else if (spiece + t * 8 + 2 >= sbytes) *reinterpret_cast<uint16_t*>(s + 2) = 0;
+      if (spiece + t * 8 >= sbytes) *reinterpret_cast<uint32_t*>(to + own_at + R::kWBytes + u * 256 + lane * 4) = 0;  // (four bytes are all or none of a row)
     }
   };
   uint32_t xat[J];
@@ -405,17 +403,15 @@ __global__ void __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
               for (int u = 0; u < R::kWLoads; ++u) *reinterpret_cast<u32x4*>(to + u * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
             }
-            uint8_t* const s = to + R::kWBytes + lane * 4;
-            if (spiece + t * 8 >= sbytes) *reinterpret_cast<uint32_t*>(s) = 0;
-            else if (spiece + t * 8 + 2 >= sbytes) *reinterpret_cast<uint16_t*>(s + 2) = 0;
+            if (spiece + t * 8 >= sbytes) *reinterpret_cast<uint32_t*>(to + R::kWBytes + lane * 4) = 0;  // (four bytes are all or none of a row)
           }
         }));
   } else if (wave >= R::kWaves) {
     // Slice ks's activations, 256 bytes of every row a stage. Places in a row as in ring_kernel.
     const Rsrc xbuf = block::buffer_of(a.xs.x, (a.M - 1) * ld + xbytes);
     uint32_t xrow[D::kXL];
-    int xpiece[D::kXL > 3 ? 4 : D::kXL];
-    static_assert(R::kXRow == 256 && J == 4);
+    int xpiece[4];
+    static_assert(R::kXRow == 256 && J == 4 && D::kXL >= 4);
 #pragma unroll
     for (int u = 0; u < D::kXL; ++u) {
       const int row = u * 4 + (lane >> 4), place = (lane ^ row) & 15;
