@@ -330,7 +330,7 @@ __host__ __device__ __forceinline__ void wait_stages(int behind, Walk& walk) {
 
 // A feeder's walk over `stages` stages of L loads each by a ring of STAGES; stage `cut` is finished once it has arrived. `all` stages have a
 // barrier. Whatever was asked for before the walk (a look-ahead) is here when it ends, as the walk's own loads are: a feeder that has no
-// stage waits for nothing else, and behind the walk the ring's bytes are the sums'.
+// stage has waited for nothing else, and behind the walk the ring's bytes are the sums'.
 template <int L, int STAGES, class Walk>
 __host__ __device__ __forceinline__ void feed(int stages, int all, int cut, Walk&& walk) {
   for (int st = 0; st < STAGES - 1; ++st)
@@ -348,7 +348,7 @@ __host__ __device__ __forceinline__ void feed(int stages, int all, int cut, Walk
     free = free + 1 == STAGES ? 0 : free + 1;
   }
   for (int st = stages; st < all; ++st) walk.barrier();
-  if (stages == 0) walk.template wait<0>();
+  walk.template wait<0>();
 }
 
 template <int MT, int PER>
