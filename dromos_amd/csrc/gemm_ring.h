@@ -281,9 +281,11 @@ __global__ void __launch_bounds__(4 * kWave) __attribute__((amdgpu_waves_per_eu(
 // memory; here the two wait apart, and the weights' ring is as deep as LDS allows. What the row does not fill of the last slices is not
 // walked (ring_kernel multiplies zeros there).
 // 14336 x 4096 at 64 rows 28.3 -> 21.1 us (by gemm_walk.h before), 16384 x 4096 28.4 -> 21.0, 8256 x 4416 at 50 rows 67 -> 26 (by the windows before).
-// Bound by what a multiplying wavefront, alone on its SIMD but for a feeder, issues: an instruction every four cycles whatever its kind, about
-// 300 a stage of which 32 are matrix instructions and 128 conversions. (With every load from one row, out of L2, 16.7 us; the loads on
-// the multiplying wavefronts the same time at 64 rows and 1 us more at 32; a stage's codes read a quarter earlier 1 us more.)
+// Bound by no one thing. Counters of that launch (45500 cycles): a SIMD issues in half of them at most (its multiplying wavefront about 220 vector
+// instructions a stage, 32 of them matrix instructions and 128 conversions, and 22 LDS reads; its feeder hardly any), the matrix cores are busy in 0.18,
+// LDS in 0.13, without a bank conflict. A third is the launch, the first loads and the sums' way out, and the walk waits for memory besides: with
+// every load from one row, out of L2, 16.7 us. (The loads on the multiplying wavefronts the same time at 64 rows and 1 us more at 32; a stage's
+// codes read a quarter earlier 1 us more.)
 // A barrier a stage: behind stage st's it is in LDS, and nobody reads stage st - 1 any more.
 template <int MT_, int PER_>
 struct Fed {
