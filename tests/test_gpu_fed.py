@@ -13,10 +13,11 @@ from dromos_amd.formats import random_weight
 
 pytestmark = pytest.mark.gpu
 NVFP4 = FORMATS["nvfp4"]
-# Rows, columns, K; slices.
+# Rows, columns, K; slices. The last three: one slice of many stages, where the other slice's wavefronts have none, and of 64 x 30001 x 4096's loaders of activations
+# the one without stages asks for lines ahead (70 a workgroup, the first 64 are the other's).
 CASES = [(9, 8209, 1088, 2), (16, 8250, 4416, 3), (17, 8241, 3200, 4), (32, 8211, 6464, 4), (20, 16401, 4096, 2), (25, 16433, 1088, 2), (33, 12301, 6464, 4), (48, 8207, 8704, 3),
          (40, 8225, 4416, 3), (34, 30001, 1024, 1), (49, 30001, 1088, 1), (64, 14336, 4096, 4), (63, 14330, 4160, 3), (50, 12301, 2176, 3), (64, 17003, 2176, 2), (57, 16385, 1024, 1),
-         (64, 8197, 10304, 4)]
+         (64, 8197, 10304, 4), (17, 29003, 3392, 1), (49, 28977, 6208, 1), (64, 30001, 4096, 1)]
 
 
 def plan(hip, M, N, K):
