@@ -25,9 +25,7 @@ constexpr int kSpecRows = 8;  // engine/cpu/spec.cpp:12
 // latency per 256 values. All of a row's pieces of 256, up to C (1, 2, 4, 6, 8), are asked for together, and the activations against as many
 // pieces as R rows leave registers for: 64 x 1024 at one row 2.9 -> 1.9 us (a launch is 1.6), 128 x 2048 at eight 9.8 -> 4.4, 4096 x 2048
 // at eight 22.4 -> 14.9. C is the least that takes a row in as many turns: with 4 and 8 only, pieces that the row does not have cost wide and short ones
-// more than the turns (4096 x 256 at nine rows 4.85 us piece by piece, 5.55, now 4.9; 1600 x 1168 at 29 12.0, 12.65, 12.1). Of 820 random calls (1 .. 64
-// rows, N 2 .. 4096, K 64 .. 8192) against piece by piece 0.69 of the time, two above 1.03 (41 x 1215 x 2128 18.6 / 20.5, rows, N, K: more workgroups than its
-// registers let a unit hold at once).
+// more than the turns (4096 x 256 at nine rows 4.85 us piece by piece, 5.55, now 4.9; 1600 x 1168 at 29 12.0, 12.65, 12.1).
 template <int R, int C>
 __device__ __forceinline__ void spec_rows(const float* __restrict__ x, int64_t ld_x, const float* __restrict__ wrow, const float* __restrict__ bias,
                                           float* __restrict__ y, int64_t ld_y, int M, int64_t n, int K) {
@@ -69,8 +67,12 @@ __device__ __forceinline__ void spec_rows(const float* __restrict__ x, int64_t l
   }
 }
 
-// REST: the last block has at most half of R rows and takes as many. On wide products only, where eight rows' work for one counts (4096 x 2048 at nine
-// rows 21.6 -> 18.6, 3207 x 6652 at 20 79 -> 72); the two paths in one kernel cost narrow ones 5 .. 10 %.
+// REST: the last block has at most half of R rows and takes as many. Where eight rows' work for one counts: on wide products (4096 x 2048 at nine rows 21.6 ->
+// 18.6 us, 3207 x 6652 at 20 79 -> 72) and on more than four workgroups a unit; the two paths in one kernel cost narrow ones 5 .. 10 %. From four
+// to eight workgroups a unit hold all at once by C = 2's registers only (64; six and eight pieces' let it hold five and four): on rows to sixteen pieces it
+// is ahead of them there. Without either, calls there had been up to 1.17 times as slow as piece by piece: 10 x 3704 x 684 (rows, N, K) 7.5 / 8.8 us, now
+// 7.6; 41 x 701 x 2152 13.0 / 14.2, 12.9. Of 900 random calls (1 .. 200 rows, N 2 .. 4096, K 64 .. 8192, half of them around 1000 .. 5000 workgroups) against piece by
+// piece 0.76 of the time, three above 1.03 (41 x 1215 x 2128 18.2 / 18.9, 33 x 1898 x 3812 42.3 / 44.2, 5 x 4006 x 716 5.3 / 5.7).
 template <int R, int C, bool REST = false>
 __global__ void __launch_bounds__(kThreads) spec_gemv_f32_kernel(const float* __restrict__ x, int64_t ld_x, const float* __restrict__ w,
                                                                  const float* __restrict__ bias, float* __restrict__ y, int64_t ld_y,
@@ -119,16 +121,20 @@ int spec_gemv(const float* x, int ld_x, const float* w, const float* bias, float
   const bool vec = K % 4 == 0 && ld_x % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
   const dim3 grid((N + kThreads / kWave - 1) / (kThreads / kWave), (M + kSpecRows - 1) / kSpecRows);
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, s, x, ld_x, w, bias, y, ld_y, M, N, K); };
+  const bool rest = M > kSpecRows && (M - 1) % kSpecRows < kSpecRows / 2;  // one to four rows behind the eights
   auto rows = [&](auto c) {
     constexpr int C = decltype(c)::value;
     if (M == 1) go(spec_gemv_f32_kernel<1, C>);
     else if (M == 2) go(spec_gemv_f32_kernel<2, C>);
     else if (M <= 4) go(spec_gemv_f32_kernel<4, C>);
-    else if (C >= 6 && M > kSpecRows && (M - 1) % kSpecRows < kSpecRows / 2 && N > 1024) go(spec_gemv_f32_kernel<8, C, (C >= 6)>);
+    else if (C >= 6 && rest && N > 1024) go(spec_gemv_f32_kernel<8, C, (C >= 6)>);
     else go(spec_gemv_f32_kernel<8, C>);
   };
   const int pieces = K / (kWave * 4) + (K % (kWave * 4) != 0);
+  const int64_t blocks = static_cast<int64_t>(grid.x) * grid.y;
   if (!vec) go(spec_gemv_f32_plain_kernel);
+  else if (rest && blocks > 1024 && (pieces == 2 || (pieces > 4 && pieces <= 16 && blocks <= 2048))) go(spec_gemv_f32_kernel<8, 2, true>);
+  else if (rest && blocks > 1024 && (pieces == 3 || pieces == 4)) go(spec_gemv_f32_kernel<8, 4, true>);
   else if (pieces <= 1) rows(std::integral_constant<int, 1>{});
   else if (pieces <= 2) rows(std::integral_constant<int, 2>{});
   else if (pieces <= 4) rows(std::integral_constant<int, 4>{});

@@ -72,8 +72,10 @@ def either_way(hip, M, N, K):
     assert torch.equal(ops.gemm_f32(hip, x, w, bias).view(torch.int32), ops.gemm_f32(hip, x, off, bias).view(torch.int32))
 
 
-# Wide products whose last rows are one to four of a block of eight.
-@pytest.mark.parametrize("M,N,K", [(9, 1025, 1028), (12, 1030, 2048), (17, 1101, 2308), (20, 1025, 3076), (27, 1201, 1540), (13, 1025, 2048), (9, 1024, 2048)])
+# Wide products whose last rows are one to four of a block of eight; the second line's are of more than 1024 workgroups, by two and by four pieces a turn, and either
+# side of the lines between them.
+@pytest.mark.parametrize("M,N,K", [(9, 1025, 1028), (12, 1030, 2048), (17, 1101, 2308), (20, 1025, 3076), (27, 1201, 1540), (13, 1025, 2048), (9, 1024, 2048),
+                                   (9, 2049, 512), (12, 2049, 508), (9, 2048, 512), (17, 1365, 1024), (20, 1367, 516), (10, 2051, 256), (41, 690, 1028), (12, 2049, 4096), (9, 2053, 4100), (18, 2730, 1284), (18, 2733, 1284), (13, 2049, 512)])
 def test_gemm_f32_wide_products_with_few_rows_behind_the_eights(hip, M, N, K):
     either_way(hip, M, N, K)
 
