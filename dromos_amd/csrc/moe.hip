@@ -151,7 +151,7 @@ __global__ void __launch_bounds__(kThreads) route_kernel(const float* __restrict
       }
       // The lowest index that holds it. With more elements a lane its own lowest, then the lanes' by the same maximum: a look at every element's
       // lanes, which is less for four and fewer (6000 tokens' eight of 128 7.4 / 8.2 us), was slower there than the search through LDS before
-      // (one of 2048 experts 14.6 / 15.5; now 14.4, eight of 512 11.1 -> 7.6).
+      // (one of 2048 experts 14.6 / 15.5 us; eight of 512 11.1 -> 7.6).
       if constexpr (NPL <= 4) {
         bool found = false;
 #pragma unroll
@@ -179,6 +179,7 @@ __global__ void __launch_bounds__(kThreads) route_kernel(const float* __restrict
           ids[t * top_k + r] = static_cast<int>(index);
           picked_logit[wave][r] = logit;
         }
+        if (r + 1 == top_k) break;
         own = index == first ? own : NPL;
 #pragma unroll
         for (int j = 0; j < NPL; ++j) key[j] = j == own ? 0u : key[j];
@@ -554,6 +555,9 @@ int route(const float* logits, const float* selection_bias, int32_t* ids, float*
   else if (E <= 128) top_k > 16 ? go(route_kernel<2, true>) : go(route_kernel<2, false>);
   else if (E <= 256) top_k > 40 ? go(route_kernel<4, true>) : go(route_kernel<4, false>);
   else if (E <= 1024) go(route_kernel<16, false>);
+  // (A round looks at all of a lane's elements, also those that E does not fill: one pick of 1025 .. 2048 experts was up to 1.09 times as slow by 64 as the
+  // search before it, 239 tokens' of 1073 13.1 / 14.2 us; one of 2048 15.5 -> 10.1, eight 47.2 -> 15.0.)
+  else if (E <= 2048) go(route_kernel<32, false>);
   else go(route_kernel<64, false>);
   return status_of(hipGetLastError());
 }
